@@ -729,7 +729,8 @@ class EngineBase : public Engine, protected BufRegistry {
     HIP_CHECK(hipStreamSynchronize(stream_));
     for (DevBuf *b : bufs_)
       if (!b->model_data) b->release();
-    scal_.ensure(8 * sizeof(double));    // grown by a batch upload: an empty pass still clears and reads one record
+    have_sid_ = false;
+    scal_.ensure((size_t) 8 * kRecordCopies * sizeof(double));    // an empty pass still clears and reads the records of one structure
     chunk_laid_out_ = 0;
     n_peak_ = 0;
     n_ = 0;
@@ -886,7 +887,7 @@ class EngineBase : public Engine, protected BufRegistry {
     nstruct_ = in.sid ? in.nstruct : 1;
     have_sid_ = in.sid != nullptr;
     sid_sorted_ = !in.sid || std::is_sorted(in.sid, in.sid + n);
-    scal_.ensure((size_t) 8 * nstruct_ * sizeof(double));
+    scal_.ensure((size_t) 8 * records() * sizeof(double));
     have_rij_ = in.rij != nullptr;
     auto put = [&](DevBuf &b, const void *src, size_t bytes) {
       b.ensure(std::max<size_t>(bytes, 8));
@@ -937,7 +938,7 @@ class EngineBase : public Engine, protected BufRegistry {
     have_sid_ = in.sid != nullptr;
     sid_sorted_ = !in.sid || std::is_sorted(in.sid, in.sid + n);
     have_rij_ = in.rij != nullptr;
-    scal_.ensure((size_t) 8 * nstruct_ * sizeof(double));
+    scal_.ensure((size_t) 8 * records() * sizeof(double));
     auto put = [&](DevBuf &b, const void *src, size_t bytes, hipMemcpyKind kind) {
       b.ensure(std::max<size_t>(bytes, 8));
       if (bytes) HIP_CHECK(hipMemcpyAsync(b.p, src, bytes, kind, stream_));
@@ -1018,9 +1019,9 @@ class EngineBase : public Engine, protected BufRegistry {
     if (!ran_) throw Error("fetch() before run()");
     if (nstruct != nstruct_) throw InvalidArgument("fetch_batch: the uploaded list holds " + std::to_string(nstruct_) + " structures");
     // everything the call returns goes to pinned memory as asynchronous copies behind the pass, with one wait:
-    // [records 8 nstruct][forces 3 n_nodes][per-atom energies n]; the zero-bond flag of the pass is in pin_flag_ already
+    // [records 8 records()][forces 3 n_nodes][per-atom energies n]; the zero-bond flag of the pass is in pin_flag_ already
     const bool wf = forces && ran_forces_ && n_nodes_ > 0, we = eatom && ran_eatom_ && n_ > 0;
-    const size_t nrec = (size_t) 8 * nstruct_, nf = wf ? (size_t) 3 * n_nodes_ : 0, ne = we ? (size_t) n_ : 0;
+    const size_t nrec = (size_t) 8 * records(), nf = wf ? (size_t) 3 * n_nodes_ : 0, ne = we ? (size_t) n_ : 0;
     pin_out_.ensure((nrec + nf + ne) * sizeof(double));
     double *rec = pin_out_.as<double>(), *pf = rec + nrec, *pe = pf + nf;
     HIP_CHECK(hipMemcpyAsync(rec, scal_.p, nrec * sizeof(double), hipMemcpyDeviceToHost, stream_));
@@ -1029,9 +1030,11 @@ class EngineBase : public Engine, protected BufRegistry {
     HIP_CHECK(hipStreamSynchronize(stream_));
     check_zero_bond();
     for (int q = 0; q < nstruct_; q++) {
-      if (energy) energy[q] = rec[8 * (size_t) q];
+      double s[7];
+      add_records(rec, q, s);
+      if (energy) energy[q] = s[0];
       if (virial && ran_forces_)
-        for (int k = 0; k < 6; k++) virial[6 * (size_t) q + k] = rec[8 * (size_t) q + 1 + k];
+        for (int k = 0; k < 6; k++) virial[6 * (size_t) q + k] = s[1 + k];
     }
     if (wf) std::memcpy(forces, pf, nf * sizeof(double));
     if (we) std::memcpy(eatom, pe, ne * sizeof(double));
@@ -1043,7 +1046,7 @@ class EngineBase : public Engine, protected BufRegistry {
     if (nstruct != nstruct_) throw InvalidArgument("fetch_batch: the uploaded list holds " + std::to_string(nstruct_) + " structures");
     HIP_CHECK(hipStreamSynchronize(stream_));
     check_zero_bond();    // before anything is written to the caller's arrays
-    hipLaunchKernelGGL(k_unpack_records, dim3((unsigned) ((nstruct_ + 255) / 256)), dim3(256), 0, stream_, scal_.as<double>(), nstruct_, energy,
+    hipLaunchKernelGGL(k_unpack_records, dim3((unsigned) ((nstruct_ + 255) / 256)), dim3(256), 0, stream_, scal_.as<double>(), nstruct_, record_copies(), energy,
                        ran_forces_ ? virial : nullptr);
     if (forces && ran_forces_ && n_ > 0) HIP_CHECK(hipMemcpyAsync(forces, f_.p, sizeof(double) * 3 * n_, hipMemcpyDeviceToDevice, stream_));
     if (eatom && ran_eatom_ && n_ > 0) HIP_CHECK(hipMemcpyAsync(eatom, eatom_.p, sizeof(double) * n_, hipMemcpyDeviceToDevice, stream_));
@@ -1072,9 +1075,11 @@ class EngineBase : public Engine, protected BufRegistry {
     if (n_ > 0 && (wf || we))
       hipLaunchKernelGGL(k_add_results, dim3((unsigned) ((n_nodes_ + 255) / 256)), dim3(256), 0, stream_, atom, n_nodes_, n_, f_.as<double>(),
                          wf ? forces : nullptr, eatom_.as<double>(), we ? eatom : nullptr);
-    double s[8];
-    HIP_CHECK(hipMemcpyAsync(s, scal_.p, sizeof(s), hipMemcpyDeviceToHost, stream_));
+    pin_out_.ensure((size_t) 8 * records() * sizeof(double));
+    HIP_CHECK(hipMemcpyAsync(pin_out_.p, scal_.p, (size_t) 8 * records() * sizeof(double), hipMemcpyDeviceToHost, stream_));
     HIP_CHECK(hipStreamSynchronize(stream_));
+    double s[7];
+    add_records(pin_out_.as<double>(), 0, s);
     if (energy) *energy = s[0];
     if (virial && ran_forces_)
       for (int k = 0; k < 6; k++) virial[k] = s[1 + k];
@@ -1159,7 +1164,7 @@ class EngineBase : public Engine, protected BufRegistry {
     f_.ensure(std::max<size_t>((size_t) 3 * n_nodes_, 1) * sizeof(double));
     eatom_.ensure(std::max<size_t>(n, 1) * sizeof(double));
     HIP_CHECK(hipMemsetAsync(f_.p, 0, (size_t) 3 * n_nodes_ * sizeof(double), stream_));
-    HIP_CHECK(hipMemsetAsync(scal_.p, 0, (size_t) 8 * nstruct_ * sizeof(double), stream_));
+    HIP_CHECK(hipMemsetAsync(scal_.p, 0, (size_t) 8 * records() * sizeof(double), stream_));
     ran_ = true;
     n_peak_ = std::max(n_peak_, n_);
     ran_forces_ = !fl.energy_only;
@@ -1206,7 +1211,7 @@ class EngineBase : public Engine, protected BufRegistry {
     ncu_ = prop.multiProcessorCount;
     arch_ = prop.gcnArchName;
     check(hipStreamCreate(&stream_), "hipStreamCreate");
-    scal_.ensure(8 * sizeof(double));
+    scal_.ensure((size_t) 8 * kRecordCopies * sizeof(double));
     zero_.ensure(2 * sizeof(int));
   }
   ~EngineBase() override
@@ -1590,6 +1595,16 @@ class EngineBase : public Engine, protected BufRegistry {
     });
   }
   const int *sid_ptr() const { return have_sid_ ? sid_.as<int>() : nullptr; }
+  // records (energy, virial[6], unused) of the pass: one per structure of a list with structure indices, kRecordCopies of one
+  // structure (record_of)
+  int record_copies() const { return have_sid_ ? 1 : kRecordCopies; }
+  size_t records() const { return (size_t) nstruct_ * record_copies(); }
+  void add_records(const double *rec, int structure, double *sum) const
+  {
+    for (int k = 0; k < 7; k++) sum[k] = 0.0;
+    for (int q = 0; q < record_copies(); q++)
+      for (int k = 0; k < 7; k++) sum[k] += rec[8 * ((size_t) structure * record_copies() + q) + k];
+  }
   // edges of the pass and its outputs (scal: energy, virial[6])
   DevBuf count_, eoff_, zero_, ei_, ej_, emu_, rh_, r_, xr_, rc_, f_, eatom_, scal_;
   bool ran_ = false, ran_forces_ = false, ran_eatom_ = false, ran_uq_ = false;

@@ -278,7 +278,7 @@ __global__ void k_pair_bwd(const long long *__restrict__ eoff, const int *__rest
         for (int k = 0; k < 9; k++) ord.fcen[9 * ((long long) (a0 + i) * ord.ngrp + grp) + k] = vsum[k];
     } else if (lane == 0 && e1 > e0) {
       for (int k = 0; k < 3; k++) atomicAdd(&f[3 * (long long) (a0 + i) + k], vsum[k]);
-      for (int k = 0; k < 6; k++) atomicAdd(&virial[(sid ? 8 * sid[a0 + i] : 0) + k], vsum[3 + k]);
+      for (int k = 0; k < 6; k++) atomicAdd(&virial[record_of(sid, a0 + i) + k], vsum[3 + k]);
       if (vatom)
         for (int k = 0; k < 6; k++) atomicAdd(&vatom[9 * (long long) (a0 + i) + k], 0.5 * vsum[3 + k]);
     }
@@ -554,7 +554,7 @@ __global__ void k_pair_bwd_async(const long long *__restrict__ eoff, const int *
       for (int o = 32; o > 0; o >>= 1) vsum[k] += __shfl_xor(vsum[k], o, 64);
     if (lane == 0 && e1 > e0) {
       for (int k = 0; k < 3; k++) atomicAdd(&f[3 * (long long) (a0 + i) + k], vsum[k]);
-      for (int k = 0; k < 6; k++) atomicAdd(&virial[(sid ? 8 * sid[a0 + i] : 0) + k], vsum[3 + k]);
+      for (int k = 0; k < 6; k++) atomicAdd(&virial[record_of(sid, a0 + i) + k], vsum[3 + k]);
       if (vatom)
         for (int k = 0; k < 6; k++) atomicAdd(&vatom[9 * (long long) (a0 + i) + k], 0.5 * vsum[3 + k]);
     }
@@ -833,7 +833,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
     for (int q = 0; q < 16; q++) sum += fsum[q][t];      // written by threads of this wave
     if (t < 3) atomicAdd(&a.f[3 * (long long) (a.a0 + i) + t], sum);
     else {
-      atomicAdd(&a.virial[(a.sid ? 8 * a.sid[a.a0 + i] : 0) + t - 3], sum);
+      atomicAdd(&a.virial[record_of(a.sid, a.a0 + i) + t - 3], sum);
       if (a.vatom) atomicAdd(&a.vatom[9 * (long long) (a.a0 + i) + t - 3], 0.5 * sum);
     }
   }
@@ -967,7 +967,7 @@ static __global__ void k_energy_2l(Energy2Dev M, const int *mu, int natoms, cons
   const double Ei = (act(M.nlay, 0) + r[0] + i2[0] / s0 * M.ln0[0]) * M.out_scale + M.shift[mu[at]];
   if (lane == 0) {
     if (eatom) eatom[at] = Ei;
-    if (energy) atomicAdd(energy + (sid ? 8 * sid[at] : 0), Ei);    // null: ordered sums, the records are added from eatom afterwards
+    if (energy) atomicAdd(energy + record_of(sid, at), Ei);    // null: ordered sums, the records are added from eatom afterwards
   }
   if (!want_grad) return;
   int cur = 0;
