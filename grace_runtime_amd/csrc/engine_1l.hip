@@ -129,13 +129,13 @@ template<class T> class Engine1L final : public EngineBase {
   // the atom tiles of the chunk that is being evaluated (all atoms when there is one chunk)
   const int *cur_tiles_ = nullptr;
   int cur_ntiles_ = 0;
-  void run_chunk(const RunFlags &fl, int a0, int nc, long long e_begin, long long e_count);
+  void run_chunk(const RunFlags &fl, int chunk, int a0, int nc, long long e_begin, long long e_count);
   void launch_gemm(DevJobs<T> &J, int kb0, int kb1, int nb, const T *X0, int nf0, const T *X1, int nf1, T *out, int nfo, int accumulate)
   {
     EngineBase::launch_gemm<T>(J, kb0, kb1, nb, X0, nf0, X1, nf1, out, nfo, accumulate, cur_tiles_, cur_ntiles_);
   }
   void launch_radial(long long e_begin, long long e_count, const double *x, const int *emu, T *Rz, T *dRz,
-                     const long long *n_edges, bool tables = false);
+                     const long long *n_edges, bool tables = false, const PairedRows &rows = {});
   void apply_spline(int n) override { rad_.spline_n = n; }
 };
 
@@ -348,15 +348,16 @@ template<class T> void Engine1L<T>::build()
 
 template<class T>
 void Engine1L<T>::launch_radial(long long e_begin, long long e_count, const double *x, const int *emu, T *Rz, T *dRz,
-                                const long long *n_edges, bool tables)
+                                const long long *n_edges, bool tables, const PairedRows &rows)
 {
-  rad_.launch(stream_, ncu_, z_.as<T>(), e_begin, e_count, x, emu, Rz, dRz, n_edges, nullptr, tables);
+  rad_.launch(stream_, ncu_, z_.as<T>(), e_begin, e_count, x, emu, Rz, dRz, n_edges, nullptr, tables, rows);
 }
 
 template<class T> void Engine1L<T>::run(const RunFlags &fl)
 {
   const int n = n_;
   ordered_check(fl);
+  want_pairs_ = !(rad_.has_tables() && tables_inside_);
   if (!begin_pass(fl)) return;
   if (ordered_ && !fl.energy_only) ordered_begin();
 
@@ -380,7 +381,9 @@ template<class T> void Engine1L<T>::run(const RunFlags &fl)
   // rows of the per-atom tensors: the generated chain kernels run whole blocks of atoms and neither guard their loads nor
   // their stores, so the tensors hold rows up to the end of the last block
   const size_t na = (size_t) round_up(cs, 16);
+  paired_ = false;
   if (!(rad_.has_tables() && tables_inside_)) {    // with tables evaluated inside the kernels the rows do not exist
+    pair_rows(cs, ecap, noutp_, ebound);
     Rz_.ensure(ecap * noutp_ * sizeof(T));
     dRz_.ensure(ecap * noutp_ * sizeof(T));
   }
@@ -416,11 +419,11 @@ template<class T> void Engine1L<T>::run(const RunFlags &fl)
     if (nchunks == 1) {
       cur_tiles_ = tiles_.as<int>();
       cur_ntiles_ = ntiles_;
-      run_chunk(fl, 0, n, 0, -1);
+      run_chunk(fl, 0, 0, n, 0, -1);
     } else {
       cur_tiles_ = chunk_tiles_.as<int>() + (size_t) 16 * chunk_tile_off_[(size_t) k];
       cur_ntiles_ = chunk_tile_off_[(size_t) k + 1] - chunk_tile_off_[(size_t) k];
-      run_chunk(fl, a0, nc, ebound[(size_t) k], ebound[(size_t) k + 1] - ebound[(size_t) k]);
+      run_chunk(fl, k, a0, nc, ebound[(size_t) k], ebound[(size_t) k + 1] - ebound[(size_t) k]);
     }
   }
   if (ordered_) ordered_finish(fl);
@@ -428,7 +431,7 @@ template<class T> void Engine1L<T>::run(const RunFlags &fl)
 
 // One chunk: atoms [a0, a0 + nc) and their bonds [e_begin, e_begin + e_count) (e_count < 0: all bonds, counted on the
 // device).  Per-atom tensors hold the chunk's atoms from row 0; cur_tiles_ names them by that row.
-template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int a0, int nc, long long e_begin, long long e_count)
+template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int chunk, int a0, int nc, long long e_begin, long long e_count)
 {
   const int n = nc;
   const int ntiles = cur_ntiles_;
@@ -442,12 +445,14 @@ template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int a0, int nc
   // (GRACE_HIP_TABLE_ROWS=1: the rows are written by the table kernel and read back, as without tables)
   const bool tab_inside = rad_.has_tables() && tables_inside_ && (nl_ * (CP_ / 16) <= 10 || (nl_ <= 7 && CP_ == 16));
   RadialTable<T> tb{};
+  const PairedRows rows = paired(chunk, e_begin);
   if (tab_inside) tb = rad_.table(stream_, ncu_, xr_.as<double>(), emu_.as<int>(), z_.as<T>());
-  else stage("radial_mlp", [&] { launch_radial(e_begin, e_count, xr_.as<double>(), emu_.as<int>(), Rz, dRz, eoff_.as<long long>() + n_, true); });
+  else stage("radial_mlp", [&] { launch_radial(e_begin, e_count, xr_.as<double>(), emu_.as<int>(), Rz, dRz, eoff_.as<long long>() + n_, true, rows); });
 
   ScatterArgs<T> sa{};
   sa.tb = tb;
   sa.eoff = eoff_.as<long long>(); sa.rh = rh_.as<double>(); sa.Rz = Rz; sa.A = A_.as<T>();
+  sa.erow = rows.erow; sa.emu = emu_.as<int>(); sa.z = z_.as<T>();
   sa.a0 = a0; sa.C = CP_; sa.nl = nl_; sa.nlm = nlm_; sa.noutp = noutp_; sa.sh = sh_;
   stage("scatter_A", [&] { launch_scatter<T>(sa, n, lmax_); });
 
@@ -626,6 +631,7 @@ template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int a0, int nc
   BondBwdArgs<T> ba{};
   ba.eoff = eoff_.as<long long>(); ba.ej = ej_.as<int>(); ba.rh = rh_.as<double>(); ba.r = r_.as<double>(); ba.rc = rc_.as<double>();
   ba.Rz = Rz; ba.dRz = dRz; ba.gA = gA;
+  ba.erow = rows.erow; ba.emu = emu_.as<int>(); ba.z = z_.as<T>();
   ba.tb = tb;
   ba.f = f_.as<double>(); ba.virial = scal_.as<double>() + 1; ba.sid = sid_ptr(); ba.vatom = vatom_ptr();
   ba.fedge = ordered_ ? fedge_.as<double>() : nullptr; ba.fcen = ordered_ ? fcen_.as<double>() : nullptr;

@@ -69,7 +69,7 @@ template<class T> class Engine2L final : public EngineBase {
   int lmax_ = 0, nl_ = 0, nlm_ = 0, nel_ = 0, C1P_ = 0, CRP_ = 0, C2P_ = 0, PI1_ = 0, nI1_ = 0, nI_ = 0, nslot_ = 0, nB_ = 0, nrho_ = 0;
   bool order4_ = false;
   ShCoef sh_{};
-  DevBuf zA_, zB0_, ones_, shift_, lnI_, ln0_, eW_[7];
+  DevBuf zA_, zB0_, shift_, lnI_, ln0_, eW_[7];
   DevRadial<T> radR_, radR1_;
   Chain<T> c1_, c2_;
   DevReduce<T> redrho_, redI2_;
@@ -243,7 +243,6 @@ template<class T> void Engine2L<T>::build()
     };
     upload_vec(zA_, ztab(m.A_lin_transform_W, m.A_lin_transform_norm, m.A_inv_avg_n_neigh, m.C1, C1P_));
     upload_vec(zB0_, ztab(m.B0_lin_transform_W, m.B0_lin_transform_norm, m.B0_inv_avg_n_neigh, m.CR, CRP_));
-    upload_vec(ones_, std::vector<T>((size_t) nel_ * CRP_, (T) 1));
     upload_vec(shift_, m.shift_values);
   }
   sink_.ensure(64);
@@ -610,6 +609,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
 {
   const int n = n_;
   ordered_check(fl);
+  want_pairs_ = !radR1_.has_tables();
   if (!begin_pass(fl)) return;
   const size_t ecap_all = (size_t) std::max<int64_t>(nb_, 1);
   const long long *n_edges = eoff_.as<long long>() + n;
@@ -654,7 +654,9 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     for (int q = 0; q < nchunks; q++) ecap = std::max(ecap, (size_t) (ebound[(size_t) q + 1] - ebound[(size_t) q]));
   }
   long long eb = 0, ecnt = -1;
+  PairedRows rows;
   auto set_chunk = [&](int q) {
+    rows = paired(q, nchunks == 1 ? 0 : ebound[(size_t) q]);
     if (nchunks == 1) {
       a0_ = 0; cn_ = n; eb = 0; ecnt = -1;
       cur_tiles_ = tiles_.as<int>(); cur_ntiles_ = ntiles_;
@@ -668,6 +670,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     cur_ntiles_ = chunk_tile_off_[(size_t) q + 1] - chunk_tile_off_[(size_t) q];
   };
   const size_t na = cap_, nnodes = (size_t) n_nodes_;
+  pair_rows(cs, ecap, std::max(radR_.noutp, radR1_.noutp), ebound);
 
   // buffers of the whole structure
   rho_.ensure((size_t) n * nrho_ * sizeof(double));
@@ -702,10 +705,11 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
   auto layer1_chain = [&] {
     T *Rz = moved_back(Rz_.as<T>(), eb * radR_.noutp), *dRz = moved_back(dRz_.as<T>(), eb * radR_.noutp);
     if (!tab_inside)
-      stage("radial_R", [&] { radR_.launch(stream_, ncu_, zA_.as<T>(), eb, ecnt, xr_.as<double>(), emu_.as<int>(), Rz, dRz, n_edges, nullptr, true); });
+      stage("radial_R", [&] { radR_.launch(stream_, ncu_, zA_.as<T>(), eb, ecnt, xr_.as<double>(), emu_.as<int>(), Rz, dRz, n_edges, nullptr, true, rows); });
     ScatterArgs<T> sa{};
     sa.tb = tbR;
     sa.eoff = eoff_.as<long long>(); sa.rh = rh_.as<double>(); sa.Rz = Rz; sa.A = A;
+    if (!tab_inside) { sa.erow = rows.erow; sa.emu = emu_.as<int>(); sa.z = zA_.as<T>(); }
     sa.a0 = a0_; sa.C = C1P_; sa.nl = nl_; sa.nlm = nlm_; sa.noutp = radR_.noutp; sa.sh = sh_;
     stage("scatter_A", [&] { launch_scatter<T>(sa, cn_, lmax_); });
     chain_forward(c1_, "_L1", A);
@@ -811,11 +815,11 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     const long long *eoff = eoff_.as<long long>() + a0_;
     const int *mu = mu_.as<int>() + a0_;
     T *R1 = moved_back(R1_.as<T>(), eb * radR1_.noutp), *dR1 = moved_back(dR1_.as<T>(), eb * radR1_.noutp);
-    stage("radial_R1", [&] { radR1_.launch(stream_, ncu_, ones_.as<T>(), eb, ecnt, xr_.as<double>(), emu_.as<int>(), R1, dR1, n_edges, nullptr, true); });
+    stage("radial_R1", [&] { radR1_.launch(stream_, ncu_, nullptr, eb, ecnt, xr_.as<double>(), emu_.as<int>(), R1, dR1, n_edges, nullptr, true, rows); });
     stage("pair_fwd", [&] {
       const size_t lds = (size_t) 2 * kAsyncChunkFwd * (pthreads + radR1_.noutp) * sizeof(T);
       GR_PAIR(k_pair_fwd, dim3(nc), dim3(pthreads), lds, stream_, eoff, ej_.as<int>(), YG_.as<T>(), (const T *) R1, (const T *) M, P, nslot_, CRP_,
-              nl_, radR1_.noutp, yw, sink_.as<T>(), 0, nc, nslot_);
+              nl_, radR1_.noutp, yw, sink_.as<T>(), 0, nc, nslot_, rows.erow);
     });
     stage("reduce_B", [&] { gemm(jB_, CRP_ / 16, C2P_ / 16, P, npf, B, nB_, 0); });
     chain_forward(c2_, "_L2", B);
@@ -855,7 +859,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
 #define GR_ARGS_ASYNC                                                                                                                   \
   dim3(nc), dim3(pthreads), lds, stream_, eoff, ej_.as<int>(), YG_.as<T>(), (const T *) R1, (const T *) dR1, (const T *) M, (const T *) gP_.as<T>(),        \
       rh_.as<double>(), r_.as<double>(), rc_.as<double>(), gM_.as<T>(), f_.as<double>(), scal_.as<double>() + 1, nslot_, nI_, CRP_, nl_, radR1_.noutp, \
-      sink_.as<T>(), 1, sid_ptr(), nslot_, 0, nc, a0_, vatom_ptr(), yw
+      sink_.as<T>(), 1, sid_ptr(), nslot_, 0, nc, a0_, vatom_ptr(), yw, rows.erow
 #define GR_ARGS GR_ARGS_ASYNC, po
       // ordered sums: the staged kernel without atomics; the message adjoints of the chunk's bonds are gathered afterwards
       PairOrdered<T> po{};
@@ -865,7 +869,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
       const PairMfmaPlan mp = pair_mfma_plan(nslot_, CRP_, nl_, sizeof(T), pair_mfma_waves(sizeof(T), pair_waves_));
       if (!ordered_ && mp.ok && pair_mfma_ != 0) {
         PairMfmaArgs<T> pa{};
-        pa.eoff = eoff; pa.ej = ej_.as<int>(); pa.YG = YG_.as<T>(); pa.R1 = R1; pa.dR1 = dR1; pa.M = M; pa.gP = gP_.as<T>();
+        pa.eoff = eoff; pa.ej = ej_.as<int>(); pa.erow = rows.erow; pa.YG = YG_.as<T>(); pa.R1 = R1; pa.dR1 = dR1; pa.M = M; pa.gP = gP_.as<T>();
         pa.rh = rh_.as<double>(); pa.rlen = r_.as<double>(); pa.rcut = rc_.as<double>();
         pa.gM = gM_.as<T>(); pa.f = f_.as<double>(); pa.virial = scal_.as<double>() + 1; pa.vatom = vatom_ptr(); pa.sid = sid_ptr();
         pa.nslot = nslot_; pa.nI = nI_; pa.C = CRP_; pa.noutp = radR1_.noutp; pa.natoms = nc; pa.a0 = a0_;
@@ -935,6 +939,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     ba.Rz = moved_back(Rz_.as<T>(), eb * radR_.noutp); ba.dRz = moved_back(dRz_.as<T>(), eb * radR_.noutp); ba.gA = c1_.gX.template as<T>();
     ba.f = f_.as<double>(); ba.virial = scal_.as<double>() + 1; ba.sid = sid_ptr(); ba.vatom = vatom_ptr();
     ba.tb = tbR;
+    if (!tab_inside) { ba.erow = rows.erow; ba.emu = emu_.as<int>(); ba.z = zA_.as<T>(); }
     ba.a0 = a0_; ba.C = C1P_; ba.nl = nl_; ba.nlm = nlm_; ba.noutp = radR_.noutp; ba.sh = sh_;
     if (ordered_) {    // added to what the pair kernel of layer 2 stored for the same bonds and atoms
       ba.fedge = fedge_.as<double>(); ba.fcen = fcen_.as<double>(); ba.ordered_add = 1;

@@ -788,7 +788,7 @@ template<class T> void Engine3L<T>::layer_forward(int k, bool forces, int yw, bo
       if ((L.CP * s) % 16 || (L.rad.noutp * s) % 16) throw Error("GRACE-3L: pair kernels need rows that are multiples of 16 bytes");
       const size_t lds = (size_t) 2 * kAsyncChunkFwd * (pt + L.rad.noutp) * s;
       GR_PAIR(k_pair_fwd, dim3((unsigned) ((n + 7) / 8 * 8 * ngrp)), dim3(pt), lds, stream_, eoff, ej_.as<int>(), YG_.as<T>(), (const T *) Rl,
-              (const T *) M_.as<T>(), pairP_.as<T>(), L.nlmi, L.CP, nl_, L.rad.noutp, yw, sink_.as<T>(), ngrp, n, spb);
+              (const T *) M_.as<T>(), pairP_.as<T>(), L.nlmi, L.CP, nl_, L.rad.noutp, yw, sink_.as<T>(), ngrp, n, spb, (const int *) nullptr);
     });
     stage(tg(k, "couple_YI").c_str(), [&] {
       const int AT = 64 / L.CP;
@@ -1007,7 +1007,7 @@ template<class T> void Engine3L<T>::layer_backward(int k, int yw)
 #define GR_ARGS                                                                                                                          \
   dim3((unsigned) ((n + 7) / 8 * 8 * ngrp)), dim3(pthreads), lds, stream_, eoff, ej_.as<int>(), YG_.as<T>(), (const T *) Rl, (const T *) dRl,     \
       (const T *) M_.as<T>(), (const T *) gpairP_.as<T>(), rh_.as<double>(), r_.as<double>(), rc_.as<double>(), gM_.as<T>(), f_.as<double>(),   \
-      scal_.as<double>() + 1, L.nlmi, L.nlmi, L.CP, nl_, L.rad.noutp, sink_.as<T>(), 1, sid_ptr(), spb, ngrp, n, a0_, vatom_ptr(), yw
+      scal_.as<double>() + 1, L.nlmi, L.nlmi, L.CP, nl_, L.rad.noutp, sink_.as<T>(), 1, sid_ptr(), spb, ngrp, n, a0_, vatom_ptr(), yw, (const int *) nullptr
     const PairMfmaPlan mp = pair_mfma_plan(L.nlmi, L.CP, nl_, s, pair_mfma_waves(s, pair_waves_));
     if (!ordered_ && mp.ok && pair_mfma_ != 0) {
       PairMfmaArgs<T> pa{};

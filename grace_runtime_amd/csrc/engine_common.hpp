@@ -385,6 +385,15 @@ template<class T> struct DevFcPairBwd {
 };
 
 
+// The bonds of a pass whose radial rows are evaluated (k_edge_pairs): uid / x [*n], erow [bonds]; on == false: every bond has
+// its own row
+struct PairedRows {
+  bool on = false;
+  const int *uid = nullptr, *erow = nullptr;
+  const double *x = nullptr;
+  const long long *n = nullptr;
+};
+
 // A 3-layer radial MLP in MFMA fragment order and the launch of the persistent radial kernel (radial_x.h:11-60 of the
 // reference; its spline tables are replaced by the exact network).  Output column l * CP + n of an edge holds
 // R_{n,l}(x) z[mu_j][n] (file order of the last layer: o = n nl + l, libgrace/src/fused_1l.cpp:123).
@@ -516,19 +525,27 @@ template<class T> struct DevRadial {
   // emi: element of the central atom of every edge (species form only)
   // tables: use the radial tables when the engine was asked for them (the plain form only); otherwise, and for the debug
   // entry points, the MLP is evaluated for every bond
+  // rows: only the listed rows are written, without the species weights (z, e_begin, e_count and x are not used)
   void launch(hipStream_t stream, int ncu, const T *z, long long e_begin, long long e_count, const double *x, const int *emu, T *Rz, T *dRz,
-              const long long *n_edges, const int *emi = nullptr, bool tables = false)
+              const long long *n_edges, const int *emi = nullptr, bool tables = false, const PairedRows &rows = {})
   {
+    if (rows.on) {
+      z = nullptr;
+      e_begin = 0;
+      e_count = -1;
+      x = rows.x;
+      n_edges = rows.n;
+    }
     if (tables && has_tables()) {
       ensure_tables(stream, ncu);
       const long long bound = e_count >= 0 ? e_count : (long long) 1 << 40;
       const unsigned grid = (unsigned) std::max<long long>(1, std::min<long long>(bound, (long long) ncu * 32));
       hipLaunchKernelGGL((k_radial_spline<T, sizeof(T) == 4>), dim3(grid), dim3(round_up(noutp, 64)), 0, stream, n_edges, e_begin, e_count, x, emu,
                          (const T *) tabF.template as<T>(), (const T *) tabD.template as<T>(), table_n, z, CP, noutp, Rz, dRz,
-                         mode == 1 ? emi : (const int *) nullptr, (const int *) sp_of_mu.as<int>(), (int) species_mu.size());
+                         mode == 1 ? emi : (const int *) nullptr, (const int *) sp_of_mu.as<int>(), (int) species_mu.size(), rows.uid);
       return;
     }
-    launch_mlp(stream, ncu, z, e_begin, e_count, x, emu, Rz, dRz, n_edges, emi);
+    launch_mlp(stream, ncu, z, e_begin, e_count, x, emu, Rz, dRz, n_edges, emi, rows.uid);
   }
   // tables requested (spline_n > 0) and, in the species form, within the memory they may take
   bool has_tables()
@@ -600,9 +617,10 @@ template<class T> struct DevRadial {
   }
   // the radial MLP itself for every edge of the range
   void launch_mlp(hipStream_t stream, int ncu, const T *z, long long e_begin, long long e_count, const double *x, const int *emu, T *Rz, T *dRz,
-                  const long long *n_edges, const int *emi)
+                  const long long *n_edges, const int *emi, const int *uid = nullptr)
   {
     RadialArgs<T> ra{};
+    ra.uid = uid;
     ra.n_edges = n_edges;
     ra.e_begin = e_begin;
     ra.e_count = e_count;
@@ -1190,7 +1208,12 @@ class EngineBase : public Engine, protected BufRegistry {
     ei_.ensure(ecap * sizeof(int)); ej_.ensure(ecap * sizeof(int)); emu_.ensure(ecap * sizeof(int));
     rh_.ensure(ecap * 3 * sizeof(double)); r_.ensure(ecap * sizeof(double)); xr_.ensure(ecap * sizeof(double));
     rc_.ensure(ecap * sizeof(double));
-    Edges ed{ei_.as<int>(), ej_.as<int>(), emu_.as<int>(), rh_.as<double>(), r_.as<double>(), xr_.as<double>(), rc_.as<double>()};
+    Edges ed{ei_.as<int>(), ej_.as<int>(), emu_.as<int>(), rh_.as<double>(), r_.as<double>(), xr_.as<double>(), rc_.as<double>(), nullptr};
+    want_pairs_ = want_pairs_ && nb_ >= kPairRowsMin && nb_ < INT32_MAX;
+    if (want_pairs_) {
+      erow_.ensure(ecap * sizeof(int));
+      ed.erow = erow_.as<int>();
+    }
     const int wpb = 4;
     stage("edge_count", [&] { hipLaunchKernelGGL(k_edge_count, dim3((n + wpb - 1) / wpb), dim3(64 * wpb), 0, stream_, src, n, count_.as<int>(), zero_.as<int>()); });
     stage("edge_scan", [&] { hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, stream_, count_.as<int>(), n, eoff_.as<long long>()); });
@@ -1443,6 +1466,49 @@ class EngineBase : public Engine, protected BufRegistry {
     HIP_CHECK(hipGetLastError());
     if (host && (mode == 0 || mode == 2)) HIP_CHECK(hipMemcpyAsync(buf, db, count * sizeof(double), hipMemcpyDeviceToHost, stream_));
     HIP_CHECK(hipStreamSynchronize(stream_));
+  }
+
+  // ---- one radial row for both directions of a bond (k_edge_pairs) ----
+  // want_pairs_: set by an engine before begin_pass(), kept by it from kPairRowsMin bonds of the list on.  Measured: GRACE-1L
+  // with 475 136 bonds, network 0.548 -> 0.296 ms, search 0.035 ms; GRACE-2L with 2.5 M bonds, both networks 6.0 -> 2.95 ms,
+  // search 0.16 ms (the kernels that gather the rows: + 0.15 ms).  A pass over fewer bonds has fewer tiles of 16 than the
+  // GPU has SIMDs for them twice over, and half as many tiles save less than the two launches cost.  Not with tables,
+  // where a row costs its stores only (312 018 bonds: 0.080 -> 0.047 ms, less than the search and the gathers).  The rows of
+  // a chunk are addressed with 32-bit offsets (k_pair_bwd_mfma), which bounds it from above.
+  static constexpr int64_t kPairRowsMin = 32768;
+  DevBuf erow_, uid_, ux_, nrows_;
+  bool want_pairs_ = false, paired_ = false;
+  // chunks of cs atoms; chunk_edges: bonds of the largest; bounds: first bond of every chunk (empty: one chunk of all atoms)
+  void pair_rows(int cs, size_t chunk_edges, int noutp, const std::vector<long long> &bounds)
+  {
+    paired_ = want_pairs_ && (double) chunk_edges * noutp < 2147483647.0;
+    if (!paired_) return;
+    const int n = n_, nch = (n + cs - 1) / cs;
+    uid_.ensure((size_t) nb_ * sizeof(int));
+    ux_.ensure((size_t) nb_ * sizeof(double));
+    nrows_.ensure((size_t) nch * sizeof(long long));
+    stage("edge_pairs", [&] {
+      HIP_CHECK(hipMemsetAsync(nrows_.p, 0, (size_t) nch * sizeof(long long), stream_));
+      for (int k = 0; k < nch; k++) {
+        const int a0 = k * cs, nc = std::min(n, a0 + cs) - a0;
+        const long long eb = bounds.empty() ? 0 : bounds[(size_t) k], ne = bounds.empty() ? nb_ : bounds[(size_t) k + 1] - eb;
+        hipLaunchKernelGGL(k_edge_pairs, dim3((unsigned) ((nc + 3) / 4)), dim3(256), 0, stream_, eoff_.as<long long>(), a0, nc, ej_.as<int>(),
+                           rh_.as<double>(), xr_.as<double>(), erow_.as<int>());
+        hipLaunchKernelGGL(k_edge_rows, dim3((unsigned) ((ne + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(1024), 0, stream_, eoff_.as<long long>(), a0,
+                           nc, erow_.as<int>(), xr_.as<double>(), uid_.as<int>() + eb, ux_.as<double>() + eb, nrows_.as<unsigned long long>() + k);
+      }
+    });
+  }
+  PairedRows paired(int chunk, long long eb) const
+  {
+    PairedRows p;
+    if (!paired_) return p;
+    p.on = true;
+    p.uid = uid_.as<int>() + eb;
+    p.erow = erow_.as<int>();
+    p.x = ux_.as<double>() + eb;
+    p.n = nrows_.as<long long>() + chunk;
+    return p;
   }
 
   // ---- chunks of atoms ---------------------------------------------------------------------------------------

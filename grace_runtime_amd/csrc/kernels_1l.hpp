@@ -282,6 +282,7 @@ struct Edges {
   int *ei, *ej, *emu;         // central atom, neighbour, neighbour element
   double *rh;                 // [E][3] unit vectors
   double *r, *x, *rc;         // length, r / rc, rc
+  int *erow;                  // its own number (k_edge_pairs), or null
 };
 
 // one wave per atom: in-cutoff bonds in list order -> compact edge arrays at eoff[i]
@@ -316,8 +317,135 @@ static __global__ void k_edge_fill(BondSrc s, int n, const long long *eoff, Edge
       e.r[p] = r;
       e.rc[p] = rc;
       e.x[p] = r / rc;
+      if (e.erow) e.erow[p] = (int) p;
     }
     w += __popcll(m);
+  }
+}
+
+// One row of radial functions for the two directions of a bond.  The radial network of GRACE-1L and 2L sees only r / rc, and
+// the bonds i -> j and j -> i have the same length, so a pass over many bonds evaluates the network once per pair: erow[e] is
+// the bond whose row bond e uses (a row stands at its own bond's place); k_edge_rows lists the bonds that have a row.
+// k_edge_fill has set erow[e] = e.  Of two atoms the one that pair_owner() names looks for the counterparts of its bonds --
+// the bonds of the other atom with the opposite unit vector and the same argument to 16 ulp (bond vectors that a caller
+// computed for each direction round differently) -- and points them at its own bond, which nobody points elsewhere.  A bond
+// without a counterpart in the list (a ghost's row, another chunk of atoms, a list that is not symmetric) and a bond of an
+// atom with its own image keep their rows.
+// One wave per atom.  What the search waits for is memory latency (index of the neighbour, start of its row, the row, the
+// counterpart's vector), so a lane first fetches the row of its own bond's neighbour for 64 bonds at a time, and then 16 bonds
+// are looked up together, 16 lanes each, 80 entries of every row in flight.
+__device__ inline bool pair_owner(int i, int j) { return ((i + j) & 1) ? i < j : i > j; }    // half of the bonds of every atom
+static __global__ __launch_bounds__(256) void k_edge_pairs(const long long *__restrict__ eoff, int a0, int natoms, const int *__restrict__ ej,
+                                                           const double *__restrict__ rh, const double *__restrict__ x, int *__restrict__ erow)
+{
+  __shared__ int s_row[4][64], s_len[4][64], s_e[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, gq = lane >> 4, lq = lane & 15;
+  const int ia = blockIdx.x * 4 + wave, i = a0 + ia;
+  if (ia >= natoms) return;
+  const int e0 = (int) eoff[i], e1 = (int) eoff[i + 1];
+  for (int b0 = e0; b0 < e1; b0 += 64) {
+    const int e = b0 + lane;
+    const int j = e < e1 ? ej[e] : -1;
+    const bool look = j >= a0 && j < a0 + natoms && j != i && pair_owner(i, j);
+    const unsigned long long mask = __ballot(look);
+    const int nlook = __popcll(mask);
+    __builtin_amdgcn_wave_barrier();
+    if (look) {
+      const int r = __popcll(mask & ((1ull << lane) - 1ull)), start = (int) eoff[j];
+      s_row[wave][r] = start;
+      s_len[wave][r] = (int) eoff[j + 1] - start;
+      s_e[wave][r] = e;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int t = 0; t < nlook; t += 16) {
+      int row[4], n[4], eb[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const int q = t + 4 * k + gq;
+        row[k] = q < nlook ? s_row[wave][q] : 0;
+        n[k] = q < nlook ? s_len[wave][q] : 0;
+        eb[k] = q < nlook ? s_e[wave][q] : 0;
+      }
+      int base = 0;
+      bool more;
+      do {    // one round per 80 entries of the longest of the 16 rows
+        int nb[4][5];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+          for (int m = 0; m < 5; m++) {
+            const int at = base + 16 * m + lq;
+            nb[k][m] = at < n[k] ? ej[row[k] + at] : -1;
+          }
+        unsigned hit[4], any = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          hit[k] = 0;
+#pragma unroll
+          for (int m = 0; m < 5; m++) hit[k] |= nb[k][m] == i ? 1u << m : 0u;
+          any |= hit[k];
+        }
+        while (__ballot(any != 0)) {    // one round unless a row names atom i more than once (images of a small cell)
+          any = 0;
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            if (hit[k]) {
+              const long long m = row[k] + base + 16 * (__ffs(hit[k]) - 1) + lq, ek = eb[k];
+              const double d = fabs(rh[3 * m] + rh[3 * ek]) + fabs(rh[3 * m + 1] + rh[3 * ek + 1]) + fabs(rh[3 * m + 2] + rh[3 * ek + 2]);
+              const double xm = x[m], xe = x[ek];
+              if (d < 1e-9 && fabs(xm - xe) <= 1.8e-15 * (xm + xe)) erow[m] = (int) ek;
+              hit[k] &= hit[k] - 1;
+              any |= hit[k];
+            }
+        }
+        base += 80;
+        more = base < n[0] || base < n[1] || base < n[2] || base < n[3];
+      } while (__ballot(more));
+    }
+  }
+}
+// The bonds of [e_begin, e_end) that have a row of their own (erow[e] == e): uid[q], ux[q] = their numbers and arguments,
+// *nrows their count (cleared by the caller).  A block lists kRowsPerBlock bonds and takes its place in the list with one
+// atomic addition (additions to one address follow each other at 12 ns).
+constexpr int kRowsPerBlock = 4096;
+static __global__ __launch_bounds__(1024) void k_edge_rows(const long long *__restrict__ eoff, int a0, int natoms, const int *__restrict__ erow,
+                                                           const double *__restrict__ x, int *__restrict__ uid, double *__restrict__ ux,
+                                                           unsigned long long *nrows)
+{
+  __shared__ int cnt[16];
+  __shared__ unsigned long long first;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const long long e0 = eoff[a0] + (long long) blockIdx.x * kRowsPerBlock, e1 = eoff[a0 + natoms];
+  if (e0 >= e1) return;
+  unsigned long long mask[kRowsPerBlock / 1024];
+  int own = 0;
+#pragma unroll
+  for (int k = 0; k < kRowsPerBlock / 1024; k++) {
+    const long long e = e0 + wave * (kRowsPerBlock / 16) + k * 64 + lane;
+    mask[k] = __ballot(e < e1 && erow[e] == (int) e);
+    own += __popcll(mask[k]);
+  }
+  if (lane == 0) cnt[wave] = own;
+  __syncthreads();
+  if (t == 0) {
+    int total = 0;
+    for (int w = 0; w < 16; w++) total += cnt[w];
+    first = atomicAdd(nrows, (unsigned long long) total);
+  }
+  __syncthreads();
+  long long u = (long long) first;
+  for (int w = 0; w < wave; w++) u += cnt[w];
+#pragma unroll
+  for (int k = 0; k < kRowsPerBlock / 1024; k++) {
+    const long long e = e0 + wave * (kRowsPerBlock / 16) + k * 64 + lane;
+    if (mask[k] >> lane & 1) {
+      const long long q = u + __popcll(mask[k] & ((1ull << lane) - 1ull));
+      uid[q] = (int) e;
+      ux[q] = x[e];
+    }
+    u += __popcll(mask[k]);
   }
 }
 
@@ -349,8 +477,9 @@ template<class T> struct RadialArgs {
   long long e_begin, e_count; // e_count < 0: take *n_edges - e_begin
   const double *x;            // [E] r / rc
   const int *emu;             // [E] neighbour element
+  const int *uid;             // [count] row that entry q of the pass writes (k_edge_pairs), or null: row e_begin + q
   const T *w0, *w1, *w2;      // fragment-ordered weights (norms folded in)
-  const T *z;                 // [nel][C]
+  const T *z;                 // [nel][C], or null: rows without species weights
   T *Rz, *dRz;                // [E][noutp]  columns l * C + n
   int nrb, p, ks0;            // basis functions, envelope order, k-steps of layer 0
   int nob, noutp;             // 16-column blocks and padded width of the output
@@ -427,7 +556,7 @@ template<class T, bool COEF>
 __global__ void k_radial_spline(const long long *__restrict__ n_edges, long long e_begin, long long e_count, const double *__restrict__ x,
                                 const int *__restrict__ emu, const T *__restrict__ F, const T *__restrict__ D, int N, const T *__restrict__ z, int C,
                                 int noutp, T *__restrict__ Rz, T *__restrict__ dRz, const int *__restrict__ emi = nullptr,
-                                const int *__restrict__ sp = nullptr, int nsp = 1)
+                                const int *__restrict__ sp = nullptr, int nsp = 1, const int *__restrict__ uid = nullptr)
 {
   const long long cnt = e_count >= 0 ? e_count : *n_edges - e_begin;
   const int col = threadIdx.x;
@@ -444,7 +573,7 @@ __global__ void k_radial_spline(const long long *__restrict__ n_edges, long long
       int k = (int) sx;
       k = k > N - 1 ? N - 1 : (k < 0 ? 0 : k);
       t[u] = (T) (sx - k);
-      zc[u] = z[emu[e] * C + n];
+      zc[u] = z ? z[emu[e] * C + n] : (T) 1;
       const long long pair = emi ? (long long) sp[emi[e]] * nsp + sp[emu[e]] : 0;
       if (COEF) {
         const T *c = F + (pair * N + k) * 4 * noutp + col;
@@ -457,7 +586,7 @@ __global__ void k_radial_spline(const long long *__restrict__ n_edges, long long
 #pragma unroll
     for (int u = 0; u < U; u++) {
       if (el0 + u >= cnt) break;
-      const long long e = e_begin + el0 + u;
+      const long long e = uid ? uid[el0 + u] : e_begin + el0 + u;
       T a0 = c0[u], a1 = c1[u], a2 = c2[u], a3 = c3[u];
       if (!COEF) {
         const T f1 = a2, d1 = a3 * h;
@@ -514,10 +643,13 @@ template<class T, int HB, int ACT, int MODE, bool W2L> __global__ __launch_bound
   // to complete.  The per-edge inputs of the NEXT tile (x of this lane's column, element and x of this lane's four
   // output rows) are therefore requested before the first store of the current tile.
   const int KZ = a.C >> 4;                        // distinct columns n = (16 cb + c) mod C of a lane: c + 16 k, k < KZ <= 4
+  // Tiles go to the blocks in turn: a pass of few tiles then runs on as many CUs as there are tiles instead of filling the
+  // waves of the first blocks (464 tiles: 39 blocks of 12 waves before).
   const long long tstep = (long long) gridDim.x * nw;
-  long long tile = (long long) blockIdx.x * nw + wave;
+  long long tile = (long long) wave * gridDim.x + blockIdx.x;
   double x_n = 0.5, xv_n[4] = {0.5, 0.5, 0.5, 0.5};
-  int emu_n[4] = {0, 0, 0, 0};
+  int emu_n[4] = {0, 0, 0, 0};    // element of the neighbour, or, with uid, the row
+  const int *const emu_src = MODE == 0 && a.uid ? a.uid : a.emu + a.e_begin;
   auto fetch_edge_inputs = [&](long long tl) {
     const long long el = tl * 16 + c;
     x_n = (tl < ntiles && el < cnt) ? a.x[a.e_begin + el] : 0.5;
@@ -525,7 +657,7 @@ template<class T, int HB, int ACT, int MODE, bool W2L> __global__ __launch_bound
     for (int v = 0; v < 4; v++) {
       const long long er = tl * 16 + a.drow[g * 4 + v];
       const bool ok = tl < ntiles && er < cnt;
-      emu_n[v] = ok ? a.emu[a.e_begin + er] : 0;
+      emu_n[v] = ok ? emu_src[er] : 0;
       if (MODE == 1) xv_n[v] = ok ? a.x[a.e_begin + er] : 0.5;
     }
   };
@@ -630,16 +762,16 @@ template<class T, int HB, int ACT, int MODE, bool W2L> __global__ __launch_bound
     // single dependent accumulator chain keeps the matrix pipe full, and one block's weights are all that is in flight)
     // The z values of a column block are requested one block ahead and the inputs of the next tile before the first
     // store of this one: no load is issued behind a store whose completion it would then wait for.
-    // rows of the tile as 32-bit offsets from its first row (the tile is wave-uniform), -1: no such edge
-    T *const Rt = a.Rz + (a.e_begin + tile * 16) * a.noutp, *const dRt = a.dRz + (a.e_begin + tile * 16) * a.noutp;
+    // rows of the tile as 32-bit numbers from the first row of the pass (k_edge_pairs: from the first bond), -1: no such edge
+    T *const Rt = a.Rz + (a.uid ? 0 : a.e_begin * a.noutp), *const dRt = a.dRz + (a.uid ? 0 : a.e_begin * a.noutp);
     int zrow[4], row_v[4];
     T env_v[4], denv_v[4], zc[4];
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       const int rl = a.drow[g * 4 + v];
-      row_v[v] = tile * 16 + rl < cnt ? rl * a.noutp : -1;
+      row_v[v] = tile * 16 + rl < cnt ? (MODE == 0 && a.uid ? emu_n[v] : (int) (tile * 16) + rl) : -1;
       zrow[v] = emu_n[v] * a.C + c;
-      zc[v] = a.z[zrow[v]];
+      zc[v] = a.z ? a.z[zrow[v]] : (T) 1;
       if (MODE == 1) {
         const double xpm = ipow(xv[v], p - 1), xp = xpm * xv[v], xp1 = xp * xv[v], xp2 = xp1 * xv[v];
         env_v[v] = (T) (1.0 - cf0 * xp + cf1 * xp1 - cf2 * xp2);
@@ -661,7 +793,7 @@ template<class T, int HB, int ACT, int MODE, bool W2L> __global__ __launch_bound
       T zn[4];
       const int kn = ((cb + 1) & (KZ - 1)) * 16;       // column n = c + 16 k of z in the next block
 #pragma unroll
-      for (int v = 0; v < 4; v++) zn[v] = a.z[zrow[v] + kn];
+      for (int v = 0; v < 4; v++) zn[v] = a.z ? a.z[zrow[v] + kn] : (T) 1;
       v4 acc = {0, 0, 0, 0}, dacc = {0, 0, 0, 0};
       const T *wc = wl + (long long) cb * NQ * 64;
 #pragma unroll
@@ -677,13 +809,14 @@ template<class T, int HB, int ACT, int MODE, bool W2L> __global__ __launch_bound
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         if (row_v[v] >= 0) {
+          const long long o = (long long) row_v[v] * a.noutp + col;
           // streaming stores: the rows are read by other kernels after the whole array has been written
           if (MODE == 1) {
-            __builtin_nontemporal_store((T) (acc[v] * env_v[v] * zc[v]), &Rt[row_v[v] + col]);
-            __builtin_nontemporal_store((T) ((dacc[v] * env_v[v] + acc[v] * denv_v[v]) * zc[v]), &dRt[row_v[v] + col]);
+            __builtin_nontemporal_store((T) (acc[v] * env_v[v] * zc[v]), &Rt[o]);
+            __builtin_nontemporal_store((T) ((dacc[v] * env_v[v] + acc[v] * denv_v[v]) * zc[v]), &dRt[o]);
           } else {
-            __builtin_nontemporal_store((T) (acc[v] * zc[v]), &Rt[row_v[v] + col]);
-            __builtin_nontemporal_store((T) (dacc[v] * zc[v]), &dRt[row_v[v] + col]);
+            __builtin_nontemporal_store((T) (acc[v] * zc[v]), &Rt[o]);
+            __builtin_nontemporal_store((T) (dacc[v] * zc[v]), &dRt[o]);
           }
         }
         zc[v] = zn[v];
@@ -744,6 +877,9 @@ template<class T> struct ScatterArgs {
   const long long *eoff;      // [n + 1]
   const double *rh;           // [E][3]
   const T *Rz;                // [E][noutp]
+  // erow set: bond e uses row erow[e] (k_edge_pairs), whose values times z[emu[e]][n] are the radial functions of the bond
+  const int *erow, *emu;
+  const T *z;                 // [nel][C]
   RadialTable<T> tb;          // tb.F set: the radial functions come from the tables, Rz is not read
   T *A;                       // [chunk atoms][nlm][C]
   int a0, natoms;             // first atom of the chunk, atoms in it
@@ -786,10 +922,15 @@ template<class T, int MAXM> __global__ void k_scatter_a(ScatterArgs<T> a)
   for (int m = 0; m < MAXM; m++) acc[m] = (T) 0;
   for (long long base = e0; base < e1; base += kScatterBonds) {
     const int nb = (int) (e1 - base < kScatterBonds ? e1 - base : kScatterBonds);
-    const T *rp = a.Rz + base * a.noutp + (t < ncol ? t : 0);
+    const T *rp = a.Rz + (t < ncol ? t : 0);
+    auto value = [&](int b) {
+      const long long e = base + (b < nb ? b : 0);
+      if (!a.erow) return rp[e * a.noutp];
+      return rp[(long long) a.erow[e] * a.noutp] * a.z[a.emu[e] * a.C + n];
+    };
     T r0[kScatterGroup], r1[kScatterGroup];
 #pragma unroll
-    for (int u = 0; u < kScatterGroup; u++) r0[u] = rp[(long long) (u < nb ? u : 0) * a.noutp];
+    for (int u = 0; u < kScatterGroup; u++) r0[u] = value(u);
     __syncthreads();
     for (int b = t; b < nb; b += blockDim.x) {
       const double *u = a.rh + 3 * (base + b);
@@ -799,10 +940,10 @@ template<class T, int MAXM> __global__ void k_scatter_a(ScatterArgs<T> a)
     for (int b0 = 0; b0 < nb; b0 += 2 * kScatterGroup) {
       const int b1 = b0 + kScatterGroup, b2 = b1 + kScatterGroup;
 #pragma unroll
-      for (int u = 0; u < kScatterGroup; u++) r1[u] = rp[(long long) (b1 + u < nb ? b1 + u : 0) * a.noutp];
+      for (int u = 0; u < kScatterGroup; u++) r1[u] = value(b1 + u);
       scatter_group<T, MAXM>(Ysh, b0, nb, lm0, nm, r0, acc);
 #pragma unroll
-      for (int u = 0; u < kScatterGroup; u++) r0[u] = rp[(long long) (b2 + u < nb ? b2 + u : 0) * a.noutp];
+      for (int u = 0; u < kScatterGroup; u++) r0[u] = value(b2 + u);
       scatter_group<T, MAXM>(Ysh, b1, nb, lm0, nm, r1, acc);
     }
   }
@@ -840,21 +981,46 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256) __attribute_
   for (int l = 0; l < NL; l++)
 #pragma unroll
     for (int cb = 0; cb < KB; cb++) acc[l][cb] = v4{0, 0, 0, 0};
-  T breg[4][NL][KB];
+  T breg[4][NL][KB], zreg[4][KB];
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+#pragma unroll
+    for (int cb = 0; cb < KB; cb++) zreg[s][cb] = (T) 1;
+  // paired rows: row and element of the lane's four bonds, fetched a tile ahead of the rows themselves
+  int rown[4], mun[4];
+  auto rows_of = [&](long long eb) {
+    const int nb = (int) (w1 - eb < 16 ? w1 - eb : 16);
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int b = 4 * s + g;
+      const long long e = eb + (b < nb ? b : 0);
+      rown[s] = a.erow[e];
+      mun[s] = a.emu[e];
+    }
+  };
   auto request = [&](long long eb, int h) {
     const int nb = (int) (w1 - eb < 16 ? w1 - eb : 16);
 #pragma unroll
     for (int s = 2 * h; s < 2 * h + 2; s++) {
       if (4 * s >= nb) continue;                      // a step with no bond: neither loaded nor multiplied
       const int b = 4 * s + g;                        // k index of this lane in step s = bond of the tile
-      const T *row = a.Rz + (eb + (b < nb ? b : 0)) * a.noutp + c;      // rows beyond the range: any valid row (Y = 0 there)
+      // rows beyond the range: any valid row (Y = 0 there)
+      const T *row = a.Rz + (a.erow ? (long long) rown[s] : eb + (b < nb ? b : 0)) * a.noutp + c;
 #pragma unroll
       for (int l = 0; l < NL; l++)
 #pragma unroll
         for (int cb = 0; cb < KB; cb++) breg[s][l][cb] = row[l * C + cb * 16];
+      if (a.erow) {
+#pragma unroll
+        for (int cb = 0; cb < KB; cb++) zreg[s][cb] = a.z[mun[s] * C + cb * 16 + c];
+      }
     }
   };
-  if (w0 < w1) { request(w0, 0); request(w0, 1); }
+  if (w0 < w1) {
+    if (a.erow) rows_of(w0);
+    request(w0, 0);
+    request(w0, 1);
+  }
   for (long long eb = w0; eb < w1; eb += 16) {
     const int nb = (int) (w1 - eb < 16 ? w1 - eb : 16);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -871,6 +1037,7 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256) __attribute_
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const bool more = eb + 16 < w1;
+    if (a.erow && more) rows_of(eb + 16);
 #pragma unroll
     for (int h = 0; h < 2; h++) {
 #pragma unroll
@@ -881,7 +1048,7 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256) __attribute_
         for (int l = 0; l < NL; l++) {
           const T y = c < 2 * l + 1 ? yb[l * l + c] : (T) 0;       // A operand: row m = c
 #pragma unroll
-          for (int cb = 0; cb < KB; cb++) acc[l][cb] = Mfma<T>::mma(y, breg[s][l][cb], acc[l][cb]);
+          for (int cb = 0; cb < KB; cb++) acc[l][cb] = Mfma<T>::mma(y, breg[s][l][cb] * zreg[s][cb], acc[l][cb]);
         }
       }
       if (more) request(eb + 16, h);
@@ -1648,6 +1815,8 @@ template<class T> struct BondBwdArgs {
   const int *ej;
   const double *rh, *r, *rc;
   const T *Rz, *dRz;          // [E][noutp]
+  const int *erow, *emu;      // as ScatterArgs
+  const T *z;
   RadialTable<T> tb;          // tb.F set: value and derivative of the radial functions come from the tables, Rz / dRz are not read
   const T *gA;                // [chunk atoms][nlm][C]
   double *f;                  // [n][3]  (+=, atomics)
@@ -1709,14 +1878,15 @@ template<class T, int KB, int NL, bool TAB> __global__ __launch_bounds__(256) vo
     const bool colok = c < nb;                      // B operand column = bond c of the tile
     // rows read by this lane: without tables step s of lane group g is channel 8 (s / 2) + 2 g + s % 2 (CH), so that the
     // four lane groups read 64 consecutive bytes of a bond's row in one instruction; with tables channel g KS + s
-    const T *rp = a.Rz + (eb + (colok ? c : 0)) * a.noutp + (TAB ? g * KS : 2 * g);
-    const T *dp = a.dRz + (eb + (colok ? c : 0)) * a.noutp + (TAB ? g * KS : 2 * g);
+    const long long ec = eb + (colok ? c : 0), erow = !TAB && a.erow ? (long long) a.erow[ec] : ec;
+    const T *rp = a.Rz + erow * a.noutp + (TAB ? g * KS : 2 * g);
+    const T *dp = a.dRz + erow * a.noutp + (TAB ? g * KS : 2 * g);
 #define CH(s_) (TAB ? (s_) : 8 * ((s_) >> 1) + ((s_) & 1))
     T x[2][KS], dx[2][KS];
     // tables: interval, offset and species weights of bond c, and the entries of l = 0
     // (four columns at a time: the entries of the next four are requested before the products of these four)
     constexpr int KH = 4;
-    T raw[TAB ? KH : 1][4], zc[TAB ? KS : 1], tt = (T) 0;
+    T raw[TAB ? KH : 1][4], zc[KS], tt = (T) 0;
     int tk = 0;
     const T th = TAB ? (T) (1.0 / a.tb.N) : (T) 0, tN = TAB ? (T) a.tb.N : (T) 0;
     if constexpr (TAB) {
@@ -1730,6 +1900,9 @@ template<class T, int KB, int NL, bool TAB> __global__ __launch_bounds__(256) vo
     } else {
 #pragma unroll
       for (int s = 0; s < KS; s++) { x[0][s] = rp[CH(s)]; dx[0][s] = dp[CH(s)]; }
+      const int mu = a.erow ? a.emu[ec] : 0;
+#pragma unroll
+      for (int s = 0; s < KS; s++) zc[s] = a.erow ? a.z[mu * C + 2 * g + CH(s)] : (T) 1;
     }
     // geometry of bond `lane` (lanes below nb), kept for the end of the tile
     double u0 = 0, u1 = 0, u2 = 1, br = 1, brc = 1;
@@ -1794,8 +1967,8 @@ template<class T, int KB, int NL, bool TAB> __global__ __launch_bounds__(256) vo
 #pragma unroll
         for (int s = 0; s < KS; s++) {
           const T w = c < 2 * l + 1 ? ga[CH(s)] : (T) 0;
-          aP = Mfma<T>::mma(w, x[cur][s], aP);
-          aQ = Mfma<T>::mma(w, dx[cur][s], aQ);
+          aP = Mfma<T>::mma(w, x[cur][s] * zc[s], aP);
+          aQ = Mfma<T>::mma(w, dx[cur][s] * zc[s], aQ);
         }
       }
       if (colok) {

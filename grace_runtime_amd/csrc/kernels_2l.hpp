@@ -99,13 +99,13 @@ __device__ inline bool pair_block(int ngrp, int natoms, int &atom, int &grp)
 }
 
 // Stages what a chunk of nb bonds (edges base .. base + nb) needs into LDS with all loads in flight at once: the
-// neighbour rows M_j[slot][n] of this thread, the radial rows (contiguous in memory), and touches the harmonics of the
+// neighbour rows M_j[slot][n] of this thread, the radial rows (contiguous in memory, or row erow[e] of bond e), and touches the harmonics of the
 // chunk (the first yuse values of every row of ylen) so that the uniform (scalar) reads of the bond loop find them in
 // the L2.
 template<class T>
 __device__ inline T pair_stage(const int *__restrict__ ej, const T *__restrict__ M, const T *__restrict__ R1, const T *__restrict__ dR1,
                                const T *__restrict__ Yu, int ylen, int yuse, long long base, int nb, int nslot, int C, int nrow, bool active, int slot,
-                               int n, T *Msh, T *Rsh, T *dRsh, int NT)
+                               int n, T *Msh, T *Rsh, T *dRsh, int NT, const int *__restrict__ erow)
 {
   const int t = threadIdx.x;
   T mv[kPairChunk];
@@ -114,10 +114,20 @@ __device__ inline T pair_stage(const int *__restrict__ ej, const T *__restrict__
     const int j = b < nb ? ej[base + b] : 0;
     mv[b] = (active && b < nb) ? M[((long long) j * nslot + slot) * C + n] : (T) 0;
   }
-  const T *rs = R1 + base * nrow, *drs = dR1 ? dR1 + base * nrow : nullptr;
-  for (int q = t; q < nb * nrow; q += blockDim.x) {
-    Rsh[q] = rs[q];
-    if (drs) dRsh[q] = drs[q];
+  if (erow) {
+    for (int b = 0; b < nb; b++) {
+      const long long row = (long long) erow[base + b] * nrow;
+      for (int q = t; q < nrow; q += blockDim.x) {
+        Rsh[b * nrow + q] = R1[row + q];
+        if (dR1) dRsh[b * nrow + q] = dR1[row + q];
+      }
+    }
+  } else {
+    const T *rs = R1 + base * nrow, *drs = dR1 ? dR1 + base * nrow : nullptr;
+    for (int q = t; q < nb * nrow; q += blockDim.x) {
+      Rsh[q] = rs[q];
+      if (drs) dRsh[q] = drs[q];
+    }
   }
   T touch = (T) 0;
   const T *yu = Yu + base * ylen;
@@ -171,7 +181,7 @@ __global__ void k_pair_bwd(const long long *__restrict__ eoff, const int *__rest
                            const double *__restrict__ rh, const double *__restrict__ rlen, const double *__restrict__ rcut,
                            T *__restrict__ gM, double *__restrict__ f, double *__restrict__ virial, int nslot, int nI, int C, int nl,
                            int noutp, T *__restrict__ sink, int one, const int *__restrict__ sid, int spb, int ngrp, int natoms, int a0,
-                           double *__restrict__ vatom, int ystr, PairOrdered<T> ord)
+                           double *__restrict__ vatom, int ystr, const int *__restrict__ erow, PairOrdered<T> ord)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double bsum[kPairChunk][4];
@@ -196,7 +206,7 @@ __global__ void k_pair_bwd(const long long *__restrict__ eoff, const int *__rest
   for (long long base = e0; base < e1; base += kPairChunk) {
     const int nb = (int) (e1 - base < kPairChunk ? e1 - base : kPairChunk);
     __syncthreads();
-    touch += pair_stage<T>(ej, M, R1, dR1, YG, ystr, nlm * 3, base, nb, nslot, C, noutp, active, slot, n, Msh, Rsh, dRsh, NT);
+    touch += pair_stage<T>(ej, M, R1, dR1, YG, ystr, nlm * 3, base, nb, nslot, C, noutp, active, slot, n, Msh, Rsh, dRsh, NT, erow);
     if (t < kPairChunk * 4) bsum[t >> 2][t & 3] = 0.0;
     __syncthreads();
     for (int b = 0; b < nb; b++) {
@@ -352,6 +362,20 @@ __device__ inline void block_copy_async(const void *src, void *dst, int nbytes, 
   }
 }
 
+// the same for nb rows of nbytes each (multiples of 16), row b from src + row[b] * nbytes, one after another at dst
+__device__ inline void block_copy_rows_async(const void *src, const int *__restrict__ row, void *dst, int nb, int nbytes, int wave, int nw, int lane)
+{
+  const int ppr = nbytes >> 4, total = nb * ppr;    // 16-byte pieces of a row, of the chunk
+  for (int p = wave; p * 64 < total; p += nw) {
+    const int q = p * 64 + lane;
+    if (q < total) {
+      const int b = q / ppr;
+      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *) (reinterpret_cast<const char *>(src) + (long long) row[b] * nbytes + 16 * (q - b * ppr)),
+                                       (void __attribute__((address_space(3))) *) (reinterpret_cast<char *>(dst) + 1024 * (size_t) p), 16, 0, 0);
+    }
+  }
+}
+
 __device__ inline void wait_async_loads() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // The neighbour gather: spb slots per block, spb C threads rounded up to whole waves (a copy is the work
@@ -359,7 +383,7 @@ __device__ inline void wait_async_loads() { __asm__ volatile("s_waitcnt vmcnt(0)
 template<class T, int NLM>
 __global__ void k_pair_fwd(const long long *__restrict__ eoff, const int *__restrict__ ej, const T *__restrict__ Y,
                            const T *__restrict__ R1, const T *__restrict__ M, T *__restrict__ P, int nslot, int C, int nl, int noutp,
-                           int ystride, T *__restrict__ sink, int ngrp, int natoms, int spb)
+                           int ystride, T *__restrict__ sink, int ngrp, int natoms, int spb, const int *__restrict__ erow)
 {
   constexpr int CH = kAsyncChunkFwd;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -386,7 +410,8 @@ __global__ void k_pair_fwd(const long long *__restrict__ eoff, const int *__rest
     for (int b = 0; b < nb; b++)
       block_copy_async(M + ((long long) ej[base + b] * nslot + grp * spb) * C, Msh + (size_t) (buf * CH + b) * NT, nact * (int) sizeof(T), (wave + b) % nw,
                        nw, lane);
-    block_copy_async(R1 + base * noutp, Rsh + (size_t) buf * CH * noutp, nb * noutp * (int) sizeof(T), wave, nw, lane);
+    if (erow) block_copy_rows_async(R1, erow + base, Rsh + (size_t) buf * CH * noutp, nb, noutp * (int) sizeof(T), wave, nw, lane);
+    else block_copy_async(R1 + base * noutp, Rsh + (size_t) buf * CH * noutp, nb * noutp * (int) sizeof(T), wave, nw, lane);
   };
   T touch = (T) 0;
   const bool works = __ballot(active) != 0;      // a wave without a slot (the last group of an atom) only copies
@@ -432,7 +457,7 @@ __global__ void k_pair_bwd_async(const long long *__restrict__ eoff, const int *
                                  const double *__restrict__ rh, const double *__restrict__ rlen, const double *__restrict__ rcut,
                                  T *__restrict__ gM, double *__restrict__ f, double *__restrict__ virial, int nslot, int nI, int C, int nl,
                                  int noutp, T *__restrict__ sink, int one, const int *__restrict__ sid, int spb, int ngrp, int natoms, int a0,
-                                 double *__restrict__ vatom, int ystr)
+                                 double *__restrict__ vatom, int ystr, const int *__restrict__ erow)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double bsum[2][CH][4];
@@ -467,8 +492,13 @@ __global__ void k_pair_bwd_async(const long long *__restrict__ eoff, const int *
     for (int b = 0; b < nb; b++)
       block_copy_async(M + ((long long) ej[base + b] * nslot + grp * spb) * C, Msh + (size_t) (buf * CH + b) * NT, nact * (int) sizeof(T), (wave + b) % nw,
                        nw, lane);
-    block_copy_async(R1 + base * noutp, Rsh + (size_t) buf * CH * noutp, nb * noutp * (int) sizeof(T), (wave + 1) % nw, nw, lane);
-    block_copy_async(dR1 + base * noutp, dRsh + (size_t) buf * CH * noutp, nb * noutp * (int) sizeof(T), (wave + 2) % nw, nw, lane);
+    if (erow) {
+      block_copy_rows_async(R1, erow + base, Rsh + (size_t) buf * CH * noutp, nb, noutp * (int) sizeof(T), (wave + 1) % nw, nw, lane);
+      block_copy_rows_async(dR1, erow + base, dRsh + (size_t) buf * CH * noutp, nb, noutp * (int) sizeof(T), (wave + 2) % nw, nw, lane);
+    } else {
+      block_copy_async(R1 + base * noutp, Rsh + (size_t) buf * CH * noutp, nb * noutp * (int) sizeof(T), (wave + 1) % nw, nw, lane);
+      block_copy_async(dR1 + base * noutp, dRsh + (size_t) buf * CH * noutp, nb * noutp * (int) sizeof(T), (wave + 2) % nw, nw, lane);
+    }
     if (wave == 0) {
       if (lane < nb * 6) lds_load_word(reinterpret_cast<const char *>(rh + 3 * base) + 4 * lane, &g_rh[buf][0]);
       if (lane < nb * 2) lds_load_word(reinterpret_cast<const char *>(rlen + base) + 4 * lane, &g_r[buf][0]);
@@ -581,7 +611,7 @@ __global__ void k_pair_bwd_async(const long long *__restrict__ eoff, const int *
 // dynamic LDS: 2 * 16 * (spb C + ystr) values.
 template<class T> struct PairMfmaArgs {
   const long long *eoff;
-  const int *ej;
+  const int *ej, *erow;    // erow: radial row of every bond (k_edge_pairs), or null: row e
   const T *YG, *R1, *dR1, *M, *gP;
   const double *rh, *rlen, *rcut;
   T *gM;
@@ -617,7 +647,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double bsum[2][16][4], fsum[16][9];    // fsum: what thread t < 16 has summed over its bonds (3 force, 6 virial)
   __shared__ __align__(16) double g_rh[2][48], g_r[2][16], g_rc[2][16];
-  __shared__ __align__(16) int g_j[2][16];
+  __shared__ __align__(16) int g_j[2][16], g_row[2][16];
   int i, grp;
   if (!pair_block(a.ngrp, a.natoms, i, grp)) return;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, NT = blockDim.x;
@@ -684,6 +714,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
       if (lane < nb * 2) lds_load_word(reinterpret_cast<const char *>(a.rlen + base) + 4 * lane, &g_r[buf][0]);
       if (lane < nb * 2) lds_load_word(reinterpret_cast<const char *>(a.rcut + base) + 4 * lane, &g_rc[buf][0]);
       if (lane < nb) lds_load_word(reinterpret_cast<const char *>(a.ej + base) + 4 * lane, &g_j[buf][0]);
+      if (a.erow && lane < nb) lds_load_word(reinterpret_cast<const char *>(a.erow + base) + 4 * lane, &g_row[buf][0]);
     }
     if (ch + 1 < nchunk) neighbours(ch + 1);
   };
@@ -696,9 +727,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
       const T *Yc = Ysh + (size_t) (buf * 16 + c) * a.ystr + g;          // A operand: row = bond c of the chunk, k = 4 s + g
       const T *Mc = Msh + (size_t) buf * 16 * mrow + n0 + c;
       // the radial rows of the lane's four bonds (rows beyond the chunk: its last bond; their results are not used)
-      int ro[4];
+      int ro[4];    // in values, counted from the row of the chunk's first bond (paired_rows() sees to it that they fit)
 #pragma unroll
-      for (int v = 0; v < 4; v++) ro[v] = (int) ((rows[v] < nb ? rows[v] : nb - 1) * a.noutp) + n0 + c;
+      for (int v = 0; v < 4; v++) {
+        const int rl = rows[v] < nb ? rows[v] : nb - 1;
+        ro[v] = (a.erow ? g_row[buf][rl] - (int) base : rl) * a.noutp + n0 + c;
+      }
       const T *Rb = a.R1 + base * a.noutp, *dRb = a.dR1 + base * a.noutp;
       T sI[TPW][4], pE[4], p1[4], p2[4];
       // the message values of the lane's bonds: rows of nloc C values, as copied (a row beyond the chunk: its last bond;
