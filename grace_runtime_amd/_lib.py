@@ -25,7 +25,7 @@ SYMBOLS = [
     "gr_lammps_add_vatom_device", "gr_neighbor_build", "gr_nlist_nbonds", "gr_nlist_nimages", "gr_nlist_get",
     "gr_nlist_free", "gr_compute", "gr_compute_batch", "gr_engine_upload_batch", "gr_engine_fetch_batch",
     "gr_system_create", "gr_system_free", "gr_system_compute", "gr_system_rebuilds", "gr_system_list_on_device",
-    "gr_system_list_sizes", "gr_system_list_get", "gr_compute_lammps", "gr_compute_batch_device", "gr_compute_batch_uq", "gr_compute_batch_device_uq", "gr_engine_reset", "gr_engine_release_buffers", "gr_set_memory_limit", "gr_memory_in_use", "gr_compute_lammps_device", "gr_model_has_uq", "gr_model_validate_uq", "gr_engine_fetch_uq",
+    "gr_system_list_sizes", "gr_system_list_get", "gr_compute_lammps", "gr_compute_batch_device", "gr_compute_batch_uq", "gr_compute_batch_device_uq", "gr_engine_reset", "gr_engine_release_buffers", "gr_engine_recycle_buffers", "gr_memory_pooled", "gr_set_memory_limit", "gr_memory_in_use", "gr_compute_lammps_device", "gr_model_has_uq", "gr_model_validate_uq", "gr_engine_fetch_uq",
     "gr_system_fetch_uq", "gr_engine_atoms_that_fit", "gr_engine_set_exchange", "gr_engine_comm_layers", "gr_engine_comm_width", "gr_engine_pack_forward", "gr_engine_unpack_forward", "gr_engine_pack_reverse", "gr_engine_unpack_reverse", "gr_engine_pack_forward_host", "gr_engine_unpack_forward_host", "gr_engine_pack_reverse_host", "gr_engine_unpack_reverse_host", "gr_engine_set_chunksize", "gr_engine_chunksize", "gr_system_set_chunksize", "gr_system_chunksize",
     "gr_engine_set_ordered_sums", "gr_engine_ordered_sums", "gr_engine_fetch_cvatom", "gr_system_fetch_cvatom", "gr_lammps_add_cvatom",
     "gr_lammps_add_cvatom_device", "gr_engine_set_spline", "gr_engine_spline",
@@ -72,6 +72,9 @@ def lib():
     L.gr_engine_free.argtypes = [vp]
     L.gr_engine_reset.argtypes = [vp]
     L.gr_engine_release_buffers.argtypes = [vp]
+    L.gr_engine_recycle_buffers.argtypes = [vp]
+    L.gr_memory_pooled.restype = i64
+    L.gr_memory_pooled.argtypes = []
     L.gr_set_memory_limit.restype = None
     L.gr_set_memory_limit.argtypes = [i64]
     L.gr_memory_in_use.restype = i64

@@ -65,6 +65,7 @@ struct gr_engine {
     lmp.reset();
     forget_lammps_call();
     eng.reset();    // frees every device buffer of the engine before the new one allocates
+    grhip::device_pool().give_back();
     generation++;
     make();
     if (has_exchange) eng->set_exchange(exchange);
@@ -76,8 +77,16 @@ struct gr_engine {
   std::unique_ptr<grhip::BatchDeviceNeighbors> bnl;    // lists of gr_compute_batch_device (buffers kept between calls)
   std::unique_ptr<grhip::LammpsDeviceList> lmp;       // converted list of gr_compute_lammps_device
   hipStream_t bnl_stream = nullptr;                    // stream of the list builds of the device entry points
+  gr_engine() { alive()++; }
+  gr_engine(const gr_engine &) = delete;
+  static std::atomic<int> &alive()
+  {
+    static std::atomic<int> n{0};
+    return n;
+  }
   ~gr_engine()
   {
+    if (--alive() == 0) grhip::device_pool().give_back();
     if (bnl_stream) (void) hipStreamDestroy(bnl_stream);
   }
 };
@@ -288,7 +297,24 @@ int gr_engine_release_buffers(gr_engine *e)
     e->lmp.reset();
     e->forget_lammps_call();
     live(e).release_buffers();
+    grhip::device_pool().give_back();
     e->generation++;    // a gr_system on this engine uploads its structure again
+  });
+}
+
+int gr_engine_recycle_buffers(gr_engine *e)
+{
+  return guarded([&] {
+    if (!e) throw grhip::InvalidArgument("null engine");
+    grhip::Engine &eng = live(e);
+    eng.synchronize();
+    if (e->bnl_stream && hipStreamSynchronize(e->bnl_stream) != hipSuccess) throw grhip::Error("hipStreamSynchronize failed");
+    grhip::RecycleScope scope;
+    e->bnl.reset();
+    e->lmp.reset();
+    e->forget_lammps_call();
+    eng.release_buffers();
+    e->generation++;
   });
 }
 
@@ -302,6 +328,7 @@ int gr_engine_reset(gr_engine *e)
 
 void gr_set_memory_limit(int64_t bytes) { grhip::dev_bytes_limit().store(bytes > 0 ? bytes : 0); }
 int64_t gr_memory_in_use(void) { return grhip::dev_bytes_in_use().load(); }
+int64_t gr_memory_pooled(void) { return grhip::device_pool().held(); }
 
 void gr_engine_free(gr_engine *e) { delete e; }
 

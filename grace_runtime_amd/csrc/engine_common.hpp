@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <atomic>
 #include <functional>
+#include <mutex>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -55,6 +56,80 @@ inline std::atomic<long long> &dev_bytes_limit()
   return v;
 }
 
+// Device memory that a finished job gave back to the process instead of to the device (gr_engine_recycle_buffers), for the
+// next job to take.  A batch call holds some 45 buffers; returning them with hipFree (0.1 ms each) and getting them again from
+// memory that the driver has to clear first (about 30 GB/s once the clean memory of the GPU is used up) took 60 to 80 ms for
+// the 2 GB of a call whose kernels take 0.8 ms.  Bounded by kPoolBytes (16 of 288 GB; the block that would pass it goes to
+// the device), not counted as in use, and given back to the device when an allocation fails or would pass the cap, on
+// gr_engine_release_buffers and gr_engine_reset, and with the last engine of the process.  Blocks come here only after
+// their stream has been waited for, so any stream and thread may take them.
+constexpr long long kPoolBytes = 16ll << 30;
+class DevicePool {
+ public:
+  // a block of at least `want` bytes on the current device, at most a quarter larger; null when there is none
+  void *take(size_t want, size_t *bytes)
+  {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    std::lock_guard<std::mutex> lock(mutex_);
+    auto best = blocks_.end();
+    for (auto it = blocks_.begin(); it != blocks_.end(); ++it)
+      if (it->dev == dev && it->bytes >= want && it->bytes <= want + want / 4 && (best == blocks_.end() || it->bytes < best->bytes)) best = it;
+    if (best == blocks_.end()) return nullptr;
+    void *p = best->p;
+    *bytes = best->bytes;
+    held_ -= (long long) best->bytes;
+    blocks_.erase(best);
+    return p;
+  }
+  // false: the pool is full, the caller frees the block
+  bool put(void *p, size_t bytes, int dev)
+  {
+    std::lock_guard<std::mutex> lock(mutex_);
+    if (held_ + (long long) bytes > kPoolBytes) return false;
+    blocks_.push_back({p, bytes, dev});
+    held_ += (long long) bytes;
+    return true;
+  }
+  void give_back()
+  {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (const Block &b : blocks_) (void) hipFree(b.p);
+    blocks_.clear();
+    held_ = 0;
+  }
+  long long held()
+  {
+    std::lock_guard<std::mutex> lock(mutex_);
+    return held_;
+  }
+
+ private:
+  struct Block {
+    void *p;
+    size_t bytes;
+    int dev;
+  };
+  std::mutex mutex_;
+  std::vector<Block> blocks_;
+  long long held_ = 0;
+};
+inline DevicePool &device_pool()
+{
+  static DevicePool *p = new DevicePool;    // never destroyed: what it holds at the end of the process goes with the process
+  return *p;
+}
+// while one exists on this thread, buffers that are released go to the pool
+struct RecycleScope {
+  static bool &on()
+  {
+    static thread_local bool v = false;
+    return v;
+  }
+  RecycleScope() { on() = true; }
+  ~RecycleScope() { on() = false; }
+};
+
 // The buffers of the engine under construction on this thread register themselves here (BufRegistry below): the engine
 // can then give back the memory of its work buffers without knowing each of them.
 struct DevBuf;
@@ -68,6 +143,7 @@ inline std::vector<DevBuf *> *&building_registry()
 struct DevBuf {
   void *p = nullptr;
   size_t bytes = 0;
+  int dev = 0;
   bool model_data = false;              // allocated while the engine was built (weights, tables): kept by release_work()
   std::vector<DevBuf *> *reg = nullptr;
   DevBuf() : reg(building_registry())
@@ -87,7 +163,7 @@ struct DevBuf {
   void release()
   {
     if (p) {
-      (void) hipFree(p);
+      if (!RecycleScope::on() || !device_pool().put(p, bytes, dev)) (void) hipFree(p);
       dev_bytes_in_use() -= (long long) bytes;
     }
     p = nullptr;
@@ -100,16 +176,28 @@ struct DevBuf {
     release();
     const size_t want = std::max<size_t>(need + need / 8, 256);
     const long long cap = dev_bytes_limit().load();
-    if (cap > 0 && dev_bytes_in_use().load() + (long long) want > cap) throw std::bad_alloc();
-    hipError_t e = hipMalloc(&p, want);
-    if (e != hipSuccess) {
-      p = nullptr;
-      (void) hipGetLastError();
-      throw std::bad_alloc();
+    if (cap > 0 && dev_bytes_in_use().load() + (long long) want + device_pool().held() > cap) {
+      device_pool().give_back();
+      if (dev_bytes_in_use().load() + (long long) want > cap) throw std::bad_alloc();
     }
-    bytes = want;
+    (void) hipGetDevice(&dev);
+    p = device_pool().take(need, &bytes);
+    if (!p) {
+      hipError_t e = hipMalloc(&p, want);
+      if (e != hipSuccess && device_pool().held() > 0) {
+        (void) hipGetLastError();
+        device_pool().give_back();
+        e = hipMalloc(&p, want);
+      }
+      if (e != hipSuccess) {
+        p = nullptr;
+        (void) hipGetLastError();
+        throw std::bad_alloc();
+      }
+      bytes = want;
+    }
     model_data = building_registry() != nullptr;
-    dev_bytes_in_use() += (long long) want;
+    dev_bytes_in_use() += (long long) bytes;
   }
   template<class U> U *as() const { return static_cast<U *>(p); }
 };
@@ -794,7 +882,7 @@ class EngineBase : public Engine, protected BufRegistry {
       if (!b->model_data) held += (double) b->bytes;
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
-    double avail = (double) free_b;
+    double avail = (double) free_b + (double) device_pool().held();
     const long long cap = dev_bytes_limit().load();
     if (cap > 0) avail = std::min(avail, (double) (cap - dev_bytes_in_use().load()));
     // the buffers grew to the largest pass since they were last released: that pass fits, and sets the bytes per atom
@@ -1522,7 +1610,7 @@ class EngineBase : public Engine, protected BufRegistry {
     if (chunk_request_ > 0) return std::min(n, chunk_request_);
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
-    double avail = (double) free_b;
+    double avail = (double) free_b + (double) device_pool().held();
     const long long cap = dev_bytes_limit().load();
     if (cap > 0) avail = std::min(avail, (double) (cap - dev_bytes_in_use().load()));
     double held = 0.0;

@@ -83,6 +83,12 @@ def memory_in_use() -> int:
     return int(_lib.lib().gr_memory_in_use())
 
 
+def memory_pooled() -> int:
+    """bytes of device memory that finished batch calls left for the next one (at most 16 GiB; `release_buffers` of any engine,
+    System or Batch returns it to the device)"""
+    return int(_lib.lib().gr_memory_pooled())
+
+
 def set_memory_limit(nbytes: int):
     """cap on memory_in_use(): an allocation beyond it fails like one the device refuses (MemoryError, or the smaller
     passes of Batch); 0 removes the cap"""
@@ -733,10 +739,11 @@ class Batch:
         self.engine.release_buffers()
 
     def _done(self):
-        # a batch is a job: its device memory goes back after the call unless keep_buffers is set (an MD loop over the
-        # same batch), python/kk/kk_core.cpp:1466-1469
+        # a batch is a job: it keeps no device memory after the call unless keep_buffers is set (an MD loop over the same
+        # batch), python/kk/kk_core.cpp:1466-1469; the memory waits in the library's bounded pool for the next job
         if not self.keep_buffers:
-            self.release_buffers()
+            check(_lib.lib().gr_engine_recycle_buffers(self.engine._h))
+            self.engine._n = 0
 
     def compute(self, natoms, types, positions, cells, pbc, energies=False, uq=False, energy_only=False,
                 max_nall=1 << 21, dispersion_parts=False):

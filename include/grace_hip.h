@@ -97,12 +97,19 @@ int gr_engine_reset(gr_engine *e);
  * Batch.release_buffers() of the reference's GPU module (python/kk/kk_api.h:66-156; engines: release_buffers(),
  * kk/grace_1l_kk.h:72-113). */
 int gr_engine_release_buffers(gr_engine *e);
+/* The same at the end of a job that is likely to be followed by another (Batch.compute without keep_buffers): the memory goes
+ * to a pool of the process, at most 16 GiB, from which the next allocations are served; what does not fit the pool is
+ * freed.  The pool is returned to the device when an allocation fails or would pass the cap below, by
+ * gr_engine_release_buffers and gr_engine_reset, and with the last engine. */
+int gr_engine_recycle_buffers(gr_engine *e);
 /* Bytes of device memory the library's buffers hold (all engines of the process), and a cap on them: with a cap an
  * allocation that would pass it fails as one the device refuses (GR_NOMEM, or the retry of gr_compute_batch_device).
  * 0: no cap.  The part of the reference module's memory_info() / chunk-by-free-memory policy (kk/support.h:415-450) that
  * the caller controls; it also lets the allocation-failure paths be tested without exhausting a GPU. */
 void gr_set_memory_limit(int64_t bytes);
 int64_t gr_memory_in_use(void);
+/* Bytes that the pool of gr_engine_recycle_buffers holds (not part of gr_memory_in_use). */
+int64_t gr_memory_pooled(void);
 /* Grace1LFused::cutoff(t1, t2): fused_1l.h:32 */
 double gr_engine_cutoff(const gr_engine *e, int t1, int t2);
 

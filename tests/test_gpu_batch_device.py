@@ -224,6 +224,11 @@ def test_release_buffers_gives_the_work_memory_back(model_dir):
     assert kk.memory_in_use() <= built + 4096
     _compare(_device_run(b, natoms, types, pos, cells, pbc), ref)
     assert kk.memory_in_use() <= built + 4096
+    # a job's memory waits in the bounded pool for the next one, and goes back to the device with an explicit release
+    assert 0 < kk.memory_pooled() <= 16 << 30
+    _compare(b.compute(natoms, types, pos, cells, pbc, energies=True), ref)      # on buffers that another call has used
+    b.release_buffers()
+    assert kk.memory_pooled() == 0
     # a System on a released engine builds its list again
     s = kk.System(model, ["Mo", "W"], skin=0.3)
     p, c, pb, t = structs[0]
