@@ -477,16 +477,9 @@ template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int chunk, int
   const T *Ar = aaa_a_ ? A : A1;
   const bool fused = chain_.ok();
   const T *chainW = chainW_.as<T>();
-  const unsigned chain_blocks = fused ? (unsigned) ((n + chain_.atoms_per_block - 1) / chain_.atoms_per_block) : 0;
   if (fused) {
     // A -> A1 -> AA -> AA1 / AA2 -> AAA / AAAA in one kernel: AA is written for the functions the rho reduce collects only
-    stage("chain_fwd", [&] {
-      const T *x0 = A;
-      void *args[] = {(void *) &x0, (void *) &A1, (void *) &AA, (void *) &AA1, (void *) &AA2, (void *) &AAA, (void *) &AAAA, (void *) &chainW, (void *) &nat,
-                      (void *) &one};
-      HIP_CHECK(hipModuleLaunchKernel(chain_.fwd, chain_blocks, 1, 1, 256, 1, 1, 0, stream_, args, nullptr));
-      cur_flops_ += chain_.flops_per_atom * n;
-    });
+    stage("chain_fwd", [&] { launch_chain_fwd<T>(chain_, n, A, A1, AA, AA1, AA2, AAA, AAAA, chainW); });
   } else {
     stage("fc_A1", [&] { launch_gemm(fcA1_.fwd, ka, ka, kf, A, nlm_, A, nlm_, A1, nlm_, 0); });
     prod_fwd("prod_AA", pAA_, A1, A1, AA, nlm_, nlm_);
@@ -552,12 +545,7 @@ template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int chunk, int
                            gAAA, gAAAA, 0, red_writes_ ? 1 : 0);
     });
     stage("chain_bwd", [&] {
-      const T *x0 = A, *x1 = A1, *p21 = AA1, *p22 = AA2, *g2 = gAA, *g3 = gAAA, *g4 = gAAAA, *g21 = nullptr;    // P3 is inside the kernel
-      void *args[] = {(void *) &x0, (void *) &x1, (void *) &p21, (void *) &p22, (void *) &g2, (void *) &g3, (void *) &g4, (void *) &g21, (void *) &gA,
-                      (void *) &chainW,
-                      (void *) &nat, (void *) &one};
-      HIP_CHECK(hipModuleLaunchKernel(chain_.bwd, chain_blocks, 1, 1, 256, 1, 1, 0, stream_, args, nullptr));
-      cur_flops_ += chain_.flops_per_atom * n;
+      launch_chain_bwd<T>(chain_, n, A, A1, AA1, AA2, gAA, gAAA, gAAAA, nullptr, gA, chainW);    // P3 is inside the kernel
     });
   } else {
   stage("zero_grads", [&] {

@@ -449,12 +449,7 @@ template<class T> void Engine2L<T>::chain_forward(Chain<T> &c, const char *tag, 
   if (c.fused.ok()) {
     // X -> X1 -> XX -> XX1 / XX2 -> XXX / XXXX in one kernel; XX is written for the functions the reduces collect only
     stage(tagged(tag, "chain_fwd").c_str(), [&] {
-      const T *w = c.fusedW.template as<T>();
-      void *args[] = {(void *) &X, (void *) &X1, (void *) &XX, (void *) &XX1, (void *) &XX2, (void *) &XXX, (void *) &XXXX, (void *) &w, (void *) &nat,
-                      (void *) &one};
-      const unsigned blocks = (unsigned) ((n + c.fused.atoms_per_block - 1) / c.fused.atoms_per_block);
-      HIP_CHECK(hipModuleLaunchKernel(c.fused.fwd, blocks, 1, 1, 256, 1, 1, 0, stream_, args, nullptr));
-      cur_flops_ += c.fused.flops_per_atom * n;
+      launch_chain_fwd<T>(c.fused, n, X, X1, XX, XX1, XX2, XXX, XXXX, c.fusedW.template as<T>());
     });
     if (!c.fuse3) prod(tagged(tag, "prod_3"), c.p3, XX1, X, XXX, c.nXX, c.nf);
     return;
@@ -556,12 +551,7 @@ template<class T> void Engine2L<T>::chain_backward(Chain<T> &c, const char *tag,
     reduces_x_xx();    // the adjoints the reduces leave on X and on the collected functions of XX come first
     if (!c.fuse3) prod_bwd(tagged(tag, "prod_3_bwd"), c.p3, XX1, X, gXXX, gXX1, gX, c.nXX, c.nf, 0, 1);
     stage(tagged(tag, "chain_bwd").c_str(), [&] {
-      const T *w = c.fusedW.template as<T>(), *g2 = gXX, *g3 = gXXX, *g4 = gXXXX, *g21 = gXX1;
-      void *args[] = {(void *) &X, (void *) &X1, (void *) &XX1, (void *) &XX2, (void *) &g2, (void *) &g3, (void *) &g4, (void *) &g21, (void *) &gX,
-                      (void *) &w, (void *) &nat, (void *) &one};
-      const unsigned blocks = (unsigned) ((n + c.fused.atoms_per_block - 1) / c.fused.atoms_per_block);
-      HIP_CHECK(hipModuleLaunchKernel(c.fused.bwd, blocks, 1, 1, 256, 1, 1, 0, stream_, args, nullptr));
-      cur_flops_ += c.fused.flops_per_atom * n;
+      launch_chain_bwd<T>(c.fused, n, X, X1, XX1, XX2, gXX, gXXX, gXXXX, gXX1, gX, c.fusedW.template as<T>());
     });
     return;
   }

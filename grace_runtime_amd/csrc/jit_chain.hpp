@@ -25,6 +25,12 @@
 // * P4 couples functions of different paths: paths are joined into groups (connected components of the P4 term list:
 //   the paths of one L), a group's P22 functions stay in registers until the group's P4 outputs are formed.
 //
+// A block walks the steps of the chain one after the other, so a pass over few atoms takes as long as one block (GRACE-1L with
+// 128 atoms: 69 us forward, 87 us reverse on 16 of 256 CUs).  For those the same kernels exist in a second form, chain_fwd_part
+// and chain_bwd_part: blockIdx.y names a set of groups (a bit mask per part), every part repeats FC1, which is a few steps, and
+// runs its own groups; the reverse is linear, so a part takes its share of the adjoint of X1 through the reverse of FC1 by
+// itself and k_chain_sum adds the parts' adjoints of X0.  Groups that share an output of P3 stay in one part.
+//
 // The generator refuses (returns false with a reason) what it does not cover: channel widths other than 32, FC
 // functions with other than one right connection, groups too large for the register file.  The engine then keeps its
 // stage-by-stage kernels.
@@ -74,25 +80,43 @@ struct ChainSpec {
   int drow[16];                 // accumulator row of (lane / 16, register) of the 16x16x4 MFMA
 };
 
+constexpr int kChainMaxParts = 8;
+struct ChainParts {
+  bool used = false;
+  unsigned long long mask[kChainMaxParts] = {};    // groups of every part
+};
+
 struct ChainCode {
   std::string src;
   std::vector<double> weights;    // fragment-ordered weight units of both kernels
   std::string why;
   int atoms_per_block = 0;
   double flops_per_atom = 0.0;    // of the FC layers of one direction (live functions, padded widths; 2 per multiply-add)
+  ChainParts parts[kChainMaxParts + 1];    // [p]: the groups dealt to p parts (p >= 2); used == false: not available
 };
 
 struct ChainKernels {
+  std::shared_ptr<LoadedModule> owner;
   hipModule_t mod = nullptr;
-  hipFunction_t fwd = nullptr, bwd = nullptr;
-  int atoms_per_block = 0;
+  hipFunction_t fwd = nullptr, bwd = nullptr, fwd_part = nullptr, bwd_part = nullptr;
+  int atoms_per_block = 0, nf0 = 0, C = 0;
   double flops_per_atom = 0.0;
+  ChainParts parts[kChainMaxParts + 1];
+  unsigned long long keep0 = 0;    // functions of X0 whose stored adjoint the reverse adds to
   bool ok() const { return mod != nullptr; }
+  // parts of a launch over n atoms: as many as leave every block its own CU (the LDS of a block fills one)
+  int parts_for(int n, int ncu) const
+  {
+    const int blocks = (n + atoms_per_block - 1) / atoms_per_block;
+    int p = blocks > 0 ? std::min(kChainMaxParts, ncu / blocks) : 1;
+    while (p > 1 && !parts[p].used) p--;
+    return std::max(p, 1);
+  }
   void release()
   {
-    if (mod) (void) hipModuleUnload(mod);
+    owner.reset();
     mod = nullptr;
-    fwd = bwd = nullptr;
+    fwd = bwd = fwd_part = bwd_part = nullptr;
   }
 };
 
@@ -487,9 +511,10 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   };
   // begin_step: template and call arguments of fc_rows that name this step's buffer and the next step's request
   struct StepArgs { std::string nnext, bufs; };
-  auto begin_step = [&]() {
+  // last: the step after this one may not be the next to run (the end of a group in the kernels that run a set of groups)
+  auto begin_step = [&](bool last = false) {
     StepArgs a;
-    const bool more = step + 1 < steps.size();
+    const bool more = step + 1 < steps.size() && !last;
     a.nnext = std::to_string(more ? steps[step + 1]->nseg * KS : 0);
     const std::string cur = (step & 1) ? "wf1" : "wf0", nxt = (step & 1) ? "wf0" : "wf1";
     a.bufs = cur + ", " + nxt + ", W + " + (more ? woff(*steps[step + 1]) : std::string("0")) + " + lane";
@@ -523,9 +548,36 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   auto xr = [&](int f) { return (sp.prod3_right_x0 ? "x0_" : "x1_") + std::to_string(f); };
   auto v2 = [](int f) { return "v2_" + std::to_string(f); };
 
+  // groups that give to one output of P3 are never in two parts
+  std::vector<int> cluster(order.size());
+  std::iota(cluster.begin(), cluster.end(), 0);
+  std::function<int(int)> root = [&](int x) { return cluster[x] == x ? x : cluster[x] = root(cluster[x]); };
+  std::vector<int> owner_of_p3(std::max(nP3, 1), 0);
+  for (const auto &kv : p3_by_o)
+    for (const ProdTerm *t : kv.second) {
+      const int g = paths[path_of[t->l]].group;
+      if (t == kv.second[0]) owner_of_p3[kv.first] = g;
+      cluster[root(g)] = root(owner_of_p3[kv.first]);
+    }
   // =========================================================== forward
-  s << "extern \"C\" __global__ __launch_bounds__(256) void chain_fwd(const T *__restrict__ X0, T *__restrict__ X1, T *__restrict__ P2, "
-       "T *__restrict__ P21, T *__restrict__ P22, T *__restrict__ P3, T *__restrict__ P4, const T *__restrict__ W, int natoms, int one)\n{\n";
+  auto mask_args = [&](bool split) {
+    std::string a;
+    if (split)
+      for (int q = 0; q < kChainMaxParts; q++) a += ", unsigned long long m" + std::to_string(q);
+    return a;
+  };
+  auto mask_pick = [&] {
+    s << "  const unsigned long long mask = ";
+    for (int q = 0; q + 1 < kChainMaxParts; q++) s << "blockIdx.y == " << q << " ? m" << q << " : ";
+    s << "m" << kChainMaxParts - 1 << ";\n";
+  };
+  auto guard = [&](bool split, size_t gi) { return split ? "if (mask >> " + std::to_string(gi) + " & 1) " : std::string(); };
+  // cluster_of_p3[o]: a group whose part owns output o of P3 (all groups that give to o are in one part)
+  auto emit_forward = [&](bool split) {
+  s << "extern \"C\" __global__ __launch_bounds__(256) void chain_fwd" << (split ? "_part" : "") << "(const T *__restrict__ X0, T *__restrict__ X1, T *__restrict__ P2, "
+       "T *__restrict__ P21, T *__restrict__ P22, T *__restrict__ P3, T *__restrict__ P4, const T *__restrict__ W, int natoms, int one"
+    << mask_args(split) << ")\n{\n";
+  if (split) mask_pick();
   {
     std::ostringstream d;
     d << "__shared__ T L0[" << nf0 * NA * S << "], LX[" << XR * S << "], LY1[" << XR * S << "], LY2[" << XR * S << "];";
@@ -549,7 +601,7 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   for (size_t q = 0; q < f1.size(); q++) {
     const Fc1Path &p = f1[q];
     s << "  {    // FC1, functions " << p.f0 << " .. " << p.f0 + p.M - 1 << "\n";
-    const StepArgs wf = begin_step();
+    const StepArgs wf = begin_step(split && q + 1 == f1.size());
     s << "    SYNC();\n";
     s << "    fc_rows<2, " << p.M * NA << ", 2, " << wf.nnext << ", 0>(" << wf.bufs << ", L0 + " << p.f0 * NA * S << ", L0 + " << p.r0 * NA * S << ", LY1, wave >> 1, wave & 1, 0, lane);\n";
     s << "    SYNC();\n";
@@ -560,13 +612,19 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
     s << "  }\n";
   }
   // P2 paths, group by group
-  for (const auto &g : order) {
+  for (size_t gi = 0; gi < order.size(); gi++) {
+    const auto &g = order[gi];
     bool any = false;
-    for (int q : g) any = any || paths[q].any;
+    int last_step = -1;
+    for (int q : g) {
+      any = any || paths[q].any;
+      if (paths[q].any && (paths[q].l21 || paths[q].l22)) last_step = q;
+    }
     if (!any) continue;
-    s << "  {    // group of paths";
+    s << "  " << guard(split, gi) << "{    // group of paths";
     for (int q : g) s << " " << q;
     s << "\n";
+    if (split && last_step >= 0) request_wf(step);
     for (int q : g)
       if (paths[q].l22)
         for (int i = 0; i < paths[q].M; i++) s << "    T " << v2(paths[q].f0 + i) << ";\n";
@@ -576,7 +634,7 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
       if (!p.any) continue;
       const bool gemm = p.l21 || p.l22;
       s << "    {    // path " << q << ": functions " << p.f0 << " .. " << p.f0 + p.M - 1 << "\n";
-      const StepArgs wf = gemm ? begin_step() : StepArgs();
+      const StepArgs wf = gemm ? begin_step(split && q == last_step) : StepArgs();
       for (int i = 0; i < p.M; i++) {
         const int f = p.f0 + i;
         const auto it = p2_by_o.find(f);
@@ -630,16 +688,23 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   }
   s << "  {\n";
   if (sp.fuse3)
-    for (int o = 0; o < nP3; o++) s << "    P3[" << o << " * C] = p3_" << o << ";\n";
+    for (int o = 0; o < nP3; o++) s << "    " << guard(split, (size_t) owner_of_p3[o]) << "P3[" << o << " * C] = p3_" << o << ";\n";
   for (int o = 0; o < nP4; o++)
-    if (!p4_by_o.count(o)) s << "    P4[" << o << " * C] = (T) 0;\n";
+    if (!p4_by_o.count(o)) s << "    " << (split ? "if (blockIdx.y == 0) " : "") << "P4[" << o << " * C] = (T) 0;\n";
   s << "  }\n}\n\n";
+  };
 
   // =========================================================== reverse
-  s << "extern \"C\" __global__ __launch_bounds__(256) void chain_bwd(const T *__restrict__ X0, const T *__restrict__ X1, const T *__restrict__ P21, "
+  auto emit_reverse = [&](bool split) -> bool {
+  s << "extern \"C\" __global__ __launch_bounds__(256) void chain_bwd" << (split ? "_part" : "") << "(const T *__restrict__ X0, const T *__restrict__ X1, const T *__restrict__ P21, "
        "const T *__restrict__ P22, const T *__restrict__ gP2, const T *__restrict__ gP3, const T *__restrict__ gP4, const T *__restrict__ gP21, "
        "T *__restrict__ gX0, "
-       "const T *__restrict__ W, int natoms, int one)\n{\n";
+       "const T *__restrict__ W, int natoms, int one"
+    << (split ? ", long long part_stride" : "") << mask_args(split) << ")\n{\n";
+  if (split) {
+    mask_pick();
+    s << "  gX0 += blockIdx.y * part_stride;\n";
+  }
   {
     std::ostringstream d;
     d << "__shared__ T LG[" << nf0 * NA * S << "], LX1[" << XR * S << "], LX2[" << XR * S << "], LY[" << XR * S << "];";
@@ -664,9 +729,21 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   if (sp.fuse3) {
     if (sp.prod3_right_x0)
       for (int f = 0; f < nf0; f++) s << "    T gx0_" << f << " = (T) 0;\n";
-    for (const auto &kv : p3_by_l) s << "    const T p_" << kv.first << " = P21[" << kv.first << " * C];\n";
-    for (const auto &kv : p3_by_l)
-      for (const ProdTerm *t : kv.second) s << "    " << gr(t->r) << " += (T) " << lit(t->c, f32) << " * g3_" << t->o << " * p_" << kv.first << ";\n";
+    if (split) {
+      for (size_t gi = 0; gi < order.size(); gi++) {
+        std::ostringstream l, u;
+        for (const auto &kv : p3_by_l) {
+          if (paths[path_of[kv.first]].group != (int) gi) continue;
+          l << "      const T p_" << kv.first << " = P21[" << kv.first << " * C];\n";
+          for (const ProdTerm *t : kv.second) u << "      " << gr(t->r) << " += (T) " << lit(t->c, f32) << " * g3_" << t->o << " * p_" << kv.first << ";\n";
+        }
+        if (!l.str().empty()) s << "    " << guard(true, gi) << "{\n" << l.str() << u.str() << "    }\n";
+      }
+    } else {
+      for (const auto &kv : p3_by_l) s << "    const T p_" << kv.first << " = P21[" << kv.first << " * C];\n";
+      for (const auto &kv : p3_by_l)
+        for (const ProdTerm *t : kv.second) s << "    " << gr(t->r) << " += (T) " << lit(t->c, f32) << " * g3_" << t->o << " * p_" << kv.first << ";\n";
+    }
   }
   for (int f = 0; f < nf0; f++)
     s << "    LG[" << f * NA * S << " + col] = " << (sp.prod3_right_x0 && sp.fuse3 ? "gx0_" + std::to_string(f) : std::string("(T) 0")) << ";\n";
@@ -698,7 +775,7 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
         }
     for (int o : outs4) s << indent << "g4_" << o << " = " << g4p << "[" << o << " * C];\n";
   };
-  if (!live_groups.empty()) {
+  if (!live_groups.empty() && !split) {
     s << "  for (int it = 0; it < one; it++) {\n    const T *P22v = P22 + it, *gP4v = gP4 + it;\n";
     group_loads(live_groups[0], "P22v", "gP4v", "    ");
     s << "  }\n";
@@ -710,15 +787,16 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
     for (int q : g)
       if (paths[q].any && (paths[q].l21 || paths[q].l22)) steps.push_back(&wu_pb[q]);
   for (size_t q = 0; q < f1.size(); q++) steps.push_back(&wu_f1b[q]);
-  request_wf(0);
-  for (const auto &g : order) {
+  if (!split) request_wf(0);
+  for (size_t gi = 0; gi < order.size(); gi++) {
+    const auto &g = order[gi];
     bool any = false;
     for (int q : g) any = any || paths[q].any;
     if (!any) continue;
     // every group is the body of a loop that runs `one` (= 1, a kernel argument) times and reads global memory through
     // pointers that depend on the loop counter: the compiler then keeps the loads of a group inside it (it otherwise
     // starts them groups ahead and spills what they return)
-    s << "  for (int it = 0; it < one; it++) {    // group of paths";
+    s << "  " << guard(split, gi) << "for (int it = 0; it < one; it++) {    // group of paths";
     for (int q : g) s << " " << q;
     s << "\n";
     s << "    const T *P22v = P22 + it, *gP4v = gP4 + it;\n";
@@ -726,7 +804,12 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
     int last_gemm = -1;
     for (int q : g)
       if (paths[q].any && (paths[q].l21 || paths[q].l22)) last_gemm = q;
+    if (split) {
+      group_loads(gi, "P22v", "gP4v", "    ");
+      if (last_gemm >= 0) request_wf(step);
+    }
     size_t next_group = order.size();
+    if (!split)
     for (size_t k = 0; k + 1 < live_groups.size(); k++)
       if (&order[live_groups[k]] == &g) next_group = live_groups[k + 1];
     bool next_requested = false;
@@ -739,7 +822,7 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
       // the adjoints that the reduces left on this path's functions: requested here, used behind the matrix phase
       for (int i = 0; i < p.M; i++)
         if (keep2[p.f0 + i] && p2_by_o.count(p.f0 + i)) s << "      const T gk_" << p.f0 + i << " = gP2w[" << p.f0 + i << " * C];\n";
-      const StepArgs wf = gemm ? begin_step() : StepArgs();
+      const StepArgs wf = gemm ? begin_step(split && q == last_gemm) : StepArgs();
       if (gemm) {
         for (int i = 0; i < p.M; i++) {
           const int f = p.f0 + i;
@@ -814,6 +897,7 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
     s << "  }\n";
   }
   // reverse of FC1
+  if (split && !f1.empty()) request_wf(step);
   for (size_t q = 0; q < f1.size(); q++) {
     const Fc1Path &p = f1[q];
     const bool same = p.r0 == p.f0;
@@ -840,10 +924,46 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   keep0.resize(nf0, 0);
   for (int f = 0; f < nf0; f++) {
     s << "    gX0[" << f << " * C] = LG[" << f * NA * S << " + col]";
-    if (keep0[f] || !sp.fuse3) s << " + gX0[" << f << " * C]";
+    if (!split && (keep0[f] || !sp.fuse3)) s << " + gX0[" << f << " * C]";
     s << ";\n";
   }
   s << "  }\n}\n";
+  return true;
+  };
+  // the parts of p-part launches: clusters by falling work (a step costs about as much as four functions), each to the part
+  // with the least
+  bool splittable = order.size() <= 64;
+  if (splittable) {
+    std::map<int, double> work;
+    std::map<int, unsigned long long> bits;
+    for (size_t gi = 0; gi < order.size(); gi++) {
+      const int c = root((int) gi);
+      bits[c] |= 1ull << gi;
+      for (int q : order[gi])
+        if (paths[q].any) work[c] += paths[q].M + 4.0;
+    }
+    std::vector<std::pair<double, int>> by_work;
+    for (const auto &kv : work) by_work.push_back({-kv.second, kv.first});
+    std::sort(by_work.begin(), by_work.end());
+    splittable = by_work.size() >= 2;
+    for (int np = 2; np <= std::min<int>(kChainMaxParts, (int) by_work.size()); np++) {
+      std::vector<double> load(np, 0.0);
+      out.parts[np].used = true;
+      for (const auto &kv : bits)
+        if (!work.count(kv.first)) out.parts[np].mask[0] |= kv.second;    // groups without a step
+      for (const auto &w : by_work) {
+        const int p = (int) (std::min_element(load.begin(), load.end()) - load.begin());
+        load[p] -= w.first;
+        out.parts[np].mask[p] |= bits[w.second];
+      }
+    }
+  }
+  emit_forward(false);
+  if (!emit_reverse(false)) return false;
+  if (splittable) {
+    emit_forward(true);
+    if (!emit_reverse(true)) return false;
+  }
   out.src = s.str();
   out.atoms_per_block = NA;
   {
@@ -872,10 +992,20 @@ inline bool jit_compile_chain(const char *name, const ChainSpec &sp, const std::
   }
   JitKernels jk;
   if (!jit_compile_source(name, code.src, sp.f32, arch, jk, why, false, "chain_fwd", "chain_bwd")) return false;
+  k.owner = jk.owner;
   k.mod = jk.mod;
   k.fwd = jk.fwd;
   k.bwd = jk.bwd;
   k.atoms_per_block = code.atoms_per_block;
+  k.nf0 = sp.nf0;
+  k.C = sp.C;
+  for (int f = 0; f < sp.nf0 && f < 64; f++)
+    if (!sp.fuse3 || (f < (int) sp.keepX0.size() && sp.keepX0[f])) k.keep0 |= 1ull << f;
+  if (code.parts[2].used && sp.nf0 <= 64 && hipModuleGetFunction(&k.fwd_part, k.mod, "chain_fwd_part") == hipSuccess &&
+      hipModuleGetFunction(&k.bwd_part, k.mod, "chain_bwd_part") == hipSuccess)
+    for (int p = 0; p <= kChainMaxParts; p++) k.parts[p] = code.parts[p];
+  else
+    (void) hipGetLastError();
   k.flops_per_atom = code.flops_per_atom;
   weights = std::move(code.weights);
   return true;

@@ -1472,6 +1472,18 @@ __global__ __launch_bounds__(64) void k_reduce_bwd(ReduceDev<T> R, const int *mu
 }
 
 
+// gX[atom][f][c] = sum of the parts of chain_bwd_part (part p at parts + p * stride), plus what gX holds for the functions of
+// keep (the reduces' adjoints)
+template<class T> __global__ void k_chain_sum(const T *__restrict__ parts, long long stride, int nparts, unsigned long long keep, int nf, int C,
+                                              long long total, T *__restrict__ gX)
+{
+  const long long q = blockIdx.x * (long long) blockDim.x + threadIdx.x;
+  if (q >= total) return;
+  T v = keep >> ((q / C) % nf) & 1 ? gX[q] : (T) 0;
+  for (int p = 0; p < nparts; p++) v += parts[p * stride + q];
+  gX[q] = v;
+}
+
 struct EnergyDev {
   const double *W[7];         // [n_in][n_out]
   double norm[7];

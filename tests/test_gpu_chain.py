@@ -142,3 +142,25 @@ def test_compiled_kernels_are_kept_on_disk_for_the_next_process(model_dir, tmp_p
     res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env0, timeout=300)
     assert res.returncode == 0, res.stderr
     assert not os.path.exists(tmp_path / "home" / ".cache" / "grace_hip")
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("natoms", [9, 350, 1020, 1030])
+@pytest.mark.parametrize("model", ["ch20", "config3"])
+def test_chain_in_parts(model_dir, model, natoms, precision):
+    """few atoms: the groups of the chain dealt to 2 .. 8 blocks (jit_chain.hpp: chain_fwd_part, chain_bwd_part, k_chain_sum);
+    256 CUs hold 8 parts up to 256 atoms, 2 parts up to 1024, one block per 8 atoms above"""
+    from grace_runtime_amd import synth
+    from oracle import grace_oracle_2l as g2
+    path = cases.model_file(model_dir, model)
+    om = g1.Model1L(path) if model == "ch20" else g2.Model2L(path)
+    pos, cell = synth.bcc_supercell(3.165, 9)
+    rng = np.random.default_rng(natoms)
+    pos = synth.jitter(pos, 0.05, 3)[np.sort(rng.permutation(len(pos))[:natoms])]      # dilute: the atoms stay in the full box
+    types = rng.integers(1, om.n_elements + 1, natoms).astype(np.int32)
+    perm, offset, j, image, shifts = kk.neighbor_search(pos, cell, [True] * 3, float(np.max(om.cut)))
+    rij = cases.bond_vectors(pos, perm, offset, j, image, shifts)
+    species = [s.decode() for s in om.d["element_names"]]
+    out = _engine(path, species, precision, True).compute(types[perm], offset, j, rij=rij, energies=True)
+    ref = (g1.compute_1l if model == "ch20" else g2.compute_2l)(om, types[perm] - 1, offset, j, rij)
+    cases.check_against(out, ref, natoms, *((1e-10, 1e-9, 1e-10, 1e-9) if precision == 64 else (1e-6, 2e-5, 1e-5, 1e-5)))
