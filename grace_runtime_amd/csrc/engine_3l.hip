@@ -36,10 +36,15 @@ template<class T> struct DevContract {
   size_t wstride = 0, wtstride = 0;             // values of one weight set, forward / transposed
   int kin = 0, kout = 0, nsrc = 0, ndst = 0;    // padded widths, functions of the source and destination tensors
   bool all_dst = false, all_src = false;        // every destination / source function has a connection
+  std::vector<Conn> conns;                      // kept with dscale for the job lists that join several contractions
+  std::vector<double> dscale;
+  double scale_of(int d) const { return dscale.empty() ? 1.0 : dscale[d]; }
   template<class WGet>
-  void build(int nin, int nout, int nt, const std::vector<Conn> &conns, WGet wget, const std::vector<double> &dscale, int nsrc_, int ndst_,
+  void build(int nin, int nout, int nt, const std::vector<Conn> &conns_, WGet wget, const std::vector<double> &dscale_, int nsrc_, int ndst_,
              const int *drow, const std::string &what, int nel_ = 1)
   {
+    conns = conns_;
+    dscale = dscale_;
     nel = nel_;
     kin = pad_width(nin);
     kout = pad_width(nout);
@@ -71,7 +76,7 @@ template<class T> struct DevContract {
     all_dst = all_src = true;
     for (const auto &v : by_dst) all_dst = all_dst && !v.empty();
     for (const auto &v : by_src) all_src = all_src && !v.empty();
-    auto sc = [&](int d) { return dscale.empty() ? 1.0 : dscale[d]; };
+    auto sc = [&](int d) { return scale_of(d); };
     typename DevJobs<T>::Host hf, hb;
     for (int d = 0; d < ndst; d++) {
       if (by_dst[d].empty()) continue;
@@ -127,8 +132,63 @@ struct Ten {
   size_t bytes(size_t na, size_t s) const { return na * nf * w * s; }
 };
 
+// Several contractions of 64 x 64 channels as ONE launch (k_gemm_few / k_gemm_wide; a launch of a small structure takes
+// some 5 us whatever it does, and two launches that add to one tensor pass over it twice).  `joined` false (other widths,
+// weights per element): every contraction is its own launch.
+template<class T> bool joinable(std::initializer_list<const DevContract<T> *> cs)
+{
+  for (const DevContract<T> *c : cs)
+    if (c->kin != 64 || c->kout != 64 || c->nel != 1) return false;
+  return true;
+}
+// rows of `io` that a contraction fills: source q reads X with the weights W
+template<class T> void io_source(GemmIO<T> &io, int q, const T *X, int nf, const T *W)
+{
+  io.X[q] = X;
+  io.nf[q] = nf;
+  io.WF[q] = W;
+}
+template<class T> void io_output(GemmIO<T> &io, int q, T *out, int nf, bool accumulate)
+{
+  io.out[q] = out;
+  io.nfo[q] = nf;
+  if (accumulate) io.accumulate |= 1u << q;
+}
+
 template<class T> struct ProdStage {
   DevContract<T> U, V, red;
+  bool joined = false, one_input = false;    // one_input: both projections read one tensor
+  DevJobs<T> proj, projb;                    // both projections; their reverse, a job per function of the input if there is one
+  void join(const int *drow)
+  {
+    joined = joinable<T>({&U, &V});
+    if (!joined) return;
+    typename DevJobs<T>::Host h, hb;
+    std::vector<std::vector<std::pair<int, typename DevContract<T>::Conn>>> by_src(one_input ? U.nsrc : U.nsrc + V.nsrc);
+    const DevContract<T> *side[2] = {&U, &V};
+    for (int q = 0; q < 2; q++) {
+      std::vector<std::vector<typename DevContract<T>::Conn>> by_dst(side[q]->ndst);
+      for (const auto &c : side[q]->conns) {
+        by_dst[c.dst].push_back(c);
+        by_src[one_input || q == 0 ? c.src : U.nsrc + c.src].push_back({q, c});
+      }
+      for (int d = 0; d < side[q]->ndst; d++) {
+        h.job(d, side[q]->scale_of(d), q);
+        for (const auto &c : by_dst[d]) h.seg(q, c.src, c.tile, 1.0);
+        h.end_job();
+      }
+    }
+    for (int f = 0; f < (int) by_src.size(); f++) {
+      const bool right = f >= U.nsrc;
+      hb.job(right ? f - U.nsrc : f, 1.0, right ? 1 : 0);
+      for (const auto &c : by_src[f]) hb.seg(c.first, c.second.dst, c.second.tile, side[c.first]->scale_of(c.second.dst));
+      hb.end_job();
+    }
+    proj.build(h, nullptr, nullptr);
+    projb.build(hb, nullptr, nullptr);
+    proj.set_rows(drow);
+    projb.set_rows(drow);
+  }
   DevProd cp;
   DevBuf tl, tr, to, tc;    // the terms sorted by output, for the LDS couple kernels
   CoupleDev cd{};
@@ -141,6 +201,40 @@ template<class T> struct FcStage {
   DevContract<T> right;
   DevBuf nof;
   int nf = 0;
+  bool joined = false;
+  DevJobs<T> fwd, bwd;    // the right input with the scaled rows of the left one added; both adjoints (0: left, 1: right)
+  void join(const std::vector<double> &factor, const int *drow)
+  {
+    joined = joinable<T>({&right});
+    if (!joined) return;
+    typename DevJobs<T>::Host h, hb;
+    std::vector<std::vector<typename DevContract<T>::Conn>> by_dst(right.ndst), by_src(right.nsrc);
+    for (const auto &c : right.conns) {
+      by_dst[c.dst].push_back(c);
+      by_src[c.src].push_back(c);
+    }
+    for (int d = 0; d < right.ndst; d++) {
+      h.job(d, right.scale_of(d));
+      h.job_add.push_back((T) factor[d]);
+      for (const auto &c : by_dst[d]) h.seg(0, c.src, c.tile, 1.0);
+      h.end_job();
+    }
+    for (int d = 0; d < right.ndst; d++) {
+      hb.job(d, 1.0, 0);
+      hb.job_add.push_back((T) factor[d]);
+      hb.end_job();
+    }
+    for (int f = 0; f < right.nsrc; f++) {
+      hb.job(f, 1.0, 1);
+      hb.job_add.push_back((T) 0);
+      for (const auto &c : by_src[f]) hb.seg(0, c.dst, c.tile, right.scale_of(c.dst));
+      hb.end_job();
+    }
+    fwd.build(h, nullptr, nullptr);
+    bwd.build(hb, nullptr, nullptr);
+    fwd.set_rows(drow);
+    bwd.set_rows(drow);
+  }
 };
 
 template<class T> struct Layer3 {
@@ -156,6 +250,32 @@ template<class T> struct Layer3 {
   ProdStage<T> p2, p3, p4;
   FcStage<T> fa, fb;
   std::vector<std::unique_ptr<DevContract<T>>> eq;    // sources X, R2, R3, R4
+  bool eq_joined = false;
+  DevJobs<T> eq_fwd, eq_bwd;          // the four of them; their reverse (every row of the four adjoints is set)
+  void join_eq(const int *drow)
+  {
+    eq_joined = eq.size() == 4 && joinable<T>({eq[0].get(), eq[1].get(), eq[2].get(), eq[3].get()});
+    if (!eq_joined) return;
+    typename DevJobs<T>::Host h, hb;
+    for (int d = 0; d < eq[0]->ndst; d++) {
+      h.job(d, 1.0);
+      for (int q = 0; q < 4; q++)
+        for (const auto &c : eq[q]->conns)
+          if (c.dst == d) h.seg(q, c.src, c.tile, eq[q]->scale_of(d));
+      h.end_job();
+    }
+    for (int q = 0; q < 4; q++)
+      for (int f = 0; f < eq[q]->nsrc; f++) {
+        hb.job(f, 1.0, q);
+        for (const auto &c : eq[q]->conns)
+          if (c.src == f) hb.seg(q, c.dst, c.tile, eq[q]->scale_of(c.dst));
+        hb.end_job();
+      }
+    eq_fwd.build(h, nullptr, nullptr);
+    eq_bwd.build(hb, nullptr, nullptr);
+    eq_fwd.set_rows(drow);
+    eq_bwd.set_rows(drow);
+  }
   DevBuf eq_dw, eq_mask, eq_aff, eq_grp;
   EqNormDev eqn{};
   DevReduce<T> rho;
@@ -509,7 +629,7 @@ template<class T> void Engine3L<T>::build_layer(int k)
     L.X.w = L.CP;
   const int nX = L.X.nf;
   // ---- cp_l products with their reduces
-  auto build_prod = [&](ProdStage<T> &P, const std::string &q, int nfl, int wl, int nfr, int wr, Ten &Lp, Ten &Rp, int &nfred) {
+  auto build_prod = [&](ProdStage<T> &P, const std::string &q, int nfl, int wl, int nfr, int wr, Ten &Lp, Ten &Rp, int &nfred, bool one_input) {
     const Model3L::Cpl &c = Model3L::by_name(m.prod, K + "_" + q);
     const Model3L::Reduce &r = Model3L::by_name(m.reduce, K + "_" + q + "_red");
     if (r.instr.size() != 1 || r.only_invar) throw Error("GRACE-3L: " + r.name + " must be one instruction on the product");
@@ -523,6 +643,8 @@ template<class T> void Engine3L<T>::build_layer(int k)
               nfr, nfr, drow_, c.name + "_V");
     P.nfunc = c.nfunc;
     P.rankP = P.U.kout;
+    P.one_input = one_input;
+    P.join(drow_);
     const HostProd h = grhip::build_prod(c.cg, std::vector<char>(c.nfunc, 1), nfl, nfr);
     P.cp.build(h);
     // The shorter term lists run with the operands of both sides in registers (that generator writes only outputs with
@@ -568,12 +690,13 @@ template<class T> void Engine3L<T>::build_layer(int k)
                   nX, f.n_funcs_left, drow_, "fc_" + name);
     F.nf = f.n_funcs_left;
     upload_vec(F.nof, std::vector<T>(f.norm_out_factor.begin(), f.norm_out_factor.end()));
+    F.join(f.norm_out_factor, drow_);
   };
-  build_prod(L.p2, "2", nX, L.X.w, nX, L.X.w, L.L2, L.R2p, L.nR2);
+  build_prod(L.p2, "2", nX, L.X.w, nX, L.X.w, L.L2, L.R2p, L.nR2, true);
   build_fc(L.fa, K + "_2a");
-  build_prod(L.p3, "3", L.nR2, L.wR, nX, L.X.w, L.L3, L.R3p, L.nR3);
+  build_prod(L.p3, "3", L.nR2, L.wR, nX, L.X.w, L.L3, L.R3p, L.nR3, false);
   build_fc(L.fb, K + "_2b");
-  build_prod(L.p4, "4", L.nR2, L.wR, L.nR2, L.wR, L.L4, L.R4p, L.nR4);
+  build_prod(L.p4, "4", L.nR2, L.wR, L.nR2, L.wR, L.L4, L.R4p, L.nR4, true);
   // ---- eq (layers 1-2) and rho reduces of (X, R2, R3, R4)
   const std::string xname = L.equiv ? K + "_red" : K;
   const std::string srcs[4] = {xname, K + "_2_red", K + "_3_red", K + "_4_red"};
@@ -586,6 +709,7 @@ template<class T> void Engine3L<T>::build_layer(int k)
       L.eq.emplace_back(new DevContract<T>());
       instr_contract(*L.eq.back(), r, Model3L::by_name(r.instr, srcs[s]), src_nf[s], "eq" + ks);
     }
+    L.join_eq(drow_);
     const Model3L::EqNorm &e = Model3L::by_name(m.eqnorm, "eq" + ks + "_norm");
     L.EQ.nf = L.I.nf = e.M;
     L.EQ.w = L.I.w = L.eq[0]->kout;
@@ -815,6 +939,14 @@ template<class T> void Engine3L<T>::layer_forward(int k, bool forces, int yw, bo
     (void) nfred;
     T *lp = Lp.buf.template as<T>(), *rp = Rp.buf.template as<T>();
     stage(tg(k, (std::string("proj_") + name).c_str()).c_str(), [&] {
+      if (p.joined) {
+        GemmIO<T> io{};
+        io_source(io, 0, XL, p.U.nsrc, p.U.WF.template as<T>());
+        io_source(io, 1, XR, p.V.nsrc, p.V.WF.template as<T>());
+        io_output(io, 0, lp, p.U.ndst, false);
+        io_output(io, 1, rp, p.V.ndst, false);
+        return EngineBase::launch_gemm_io<T>(p.proj, 4, 4, io, cur_tiles_, cur_ntiles_);
+      }
       cfwd(p.U, XL, lp, 0);
       cfwd(p.V, XR, rp, 0);
     });
@@ -823,6 +955,13 @@ template<class T> void Engine3L<T>::layer_forward(int k, bool forces, int yw, bo
   };
   auto fc = [&](const char *name, FcStage<T> &F, T *out) {
     stage(tg(k, name).c_str(), [&] {
+      if (F.joined) {
+        GemmIO<T> io{};
+        io_source(io, 0, (const T *) X, F.right.nsrc, F.right.WF.template as<T>());
+        io_output(io, 0, out, F.right.ndst, false);
+        io.add = R2;
+        return EngineBase::launch_gemm_io<T>(F.fwd, 4, 4, io, cur_tiles_, cur_ntiles_);
+      }
       scale_rows(R2, F.nof, out, F.nf, wR, 0);
       cfwd(F.right, X, out, 1);
     });
@@ -837,6 +976,12 @@ template<class T> void Engine3L<T>::layer_forward(int k, bool forces, int yw, bo
     L.EQ.buf.ensure(L.EQ.bytes(na, s));
     L.I.buf.ensure(L.I.bytes((size_t) n_nodes_, s));    // rows of the ghost atoms too: the exchange fills them
     stage(tg(k, "reduce_eq").c_str(), [&] {
+      if (L.eq_joined) {
+        GemmIO<T> io{};
+        for (int q = 0; q < 4; q++) io_source(io, q, srcs[q], L.eq[q]->nsrc, L.eq[q]->WF.template as<T>());
+        io_output(io, 0, L.EQ.buf.template as<T>(), L.eq[0]->ndst, false);
+        return EngineBase::launch_gemm_io<T>(L.eq_fwd, 4, 4, io, cur_tiles_, cur_ntiles_);
+      }
       zero(L.EQ.buf.p, L.EQ.bytes((size_t) n, s));
       for (int q = 0; q < 4; q++) cfwd(*L.eq[q], srcs[q], L.EQ.buf.template as<T>(), 1);
     });
@@ -916,12 +1061,15 @@ template<class T> void Engine3L<T>::layer_backward(int k, int yw)
   T *gsrc[4] = {gX, gR2, gR3, gR4};
   const size_t nn = (size_t) n;
   stage(tg(k, "zero_grads").c_str(), [&] {
-    zero(gX, nn * nX * wX * s);
-    zero(gR2, nn * L.nR2 * wR * s);
-    zero(gR3, nn * L.nR3 * wR * s);
-    zero(gR4, nn * L.nR4 * wR * s);
-    zero(gFA, nn * L.nR2 * wR * s);
-    zero(gFB, nn * L.nR2 * wR * s);
+    if (!L.eq_joined) {              // else the reverse of the eq reduces sets them
+      zero(gX, nn * nX * wX * s);
+      zero(gR2, nn * L.nR2 * wR * s);
+      zero(gR3, nn * L.nR3 * wR * s);
+      zero(gR4, nn * L.nR4 * wR * s);
+    }
+    // set by the reverse of the projections that read them where that is one launch
+    if (!L.p3.joined) zero(gFA, nn * L.nR2 * wR * s);
+    if (!L.p4.joined) zero(gFB, nn * L.nR2 * wR * s);
   });
   if (L.has_eq) {
     gEQ_.ensure(L.EQ.bytes(na, s));
@@ -930,6 +1078,14 @@ template<class T> void Engine3L<T>::layer_backward(int k, int yw)
                          (const T *) gMin_.as<T>() + (size_t) a0_ * L.eqn.M * L.eqn.C, gEQ_.as<T>(), 0);
     });
     stage(tg(k, "reduce_eq_bwd").c_str(), [&] {
+      if (L.eq_joined) {
+        GemmIO<T> io{};
+        for (int q = 0; q < 4; q++) {
+          io_source(io, q, (const T *) gEQ_.as<T>(), L.eq[q]->ndst, L.eq[q]->WT.template as<T>());
+          io_output(io, q, gsrc[q], L.eq[q]->nsrc, false);
+        }
+        return EngineBase::launch_gemm_io<T>(L.eq_bwd, 4, 4, io, cur_tiles_, cur_ntiles_);
+      }
       for (int q = 0; q < 4; q++) cbwd(*L.eq[q], gEQ_.as<T>(), gsrc[q], 1);
     });
   }
@@ -938,8 +1094,9 @@ template<class T> void Engine3L<T>::layer_backward(int k, int yw)
       hipLaunchKernelGGL(k_reduce_bwd<T>, dim3(cur_ntiles_, L.rho.njobs), dim3(64), 0, stream_, L.rho.d, mu, cur_tiles_,
                          (const double *) L.grho.template as<double>() + (size_t) a0_ * nrho_, gX, gR2, gR3, gR4);
   });
-  // gXL / gXR: where the adjoints of the product's inputs are added
-  auto prod_bwd = [&](const char *name, ProdStage<T> &p, Ten &Lp, Ten &Rp, const T *gR, T *gXL, T *gXR) {
+  // gXL / gXR: where the adjoints of the product's inputs are added; first_left: gXL has no other part yet (a joined launch
+  // sets it; else it was cleared)
+  auto prod_bwd = [&](const char *name, ProdStage<T> &p, Ten &Lp, Ten &Rp, const T *gR, T *gXL, T *gXR, bool first_left) {
     const T *lp = Lp.buf.template as<T>(), *rp = Rp.buf.template as<T>();
     stage(tg(k, (std::string("reduce_") + name + "_bwd").c_str()).c_str(), [&] { cbwd_set(p.red, gR, gP); });
     stage(tg(k, (std::string("couple_") + name + "_bwd").c_str()).c_str(), [&] {
@@ -950,21 +1107,37 @@ template<class T> void Engine3L<T>::layer_backward(int k, int yw)
       couple_bwd(p, lp, Lp.nf, rp, Rp.nf, gP, gLp, gRp);
     });
     stage(tg(k, (std::string("proj_") + name + "_bwd").c_str()).c_str(), [&] {
+      if (p.joined) {
+        GemmIO<T> io{};
+        io_source(io, 0, (const T *) gLp, p.U.ndst, p.U.WT.template as<T>());
+        io_source(io, 1, (const T *) gRp, p.V.ndst, p.V.WT.template as<T>());
+        io_output(io, 0, gXL, p.U.nsrc, !first_left);
+        if (!p.one_input) io_output(io, 1, gXR, p.V.nsrc, true);
+        return EngineBase::launch_gemm_io<T>(p.projb, 4, 4, io, cur_tiles_, cur_ntiles_);
+      }
       cbwd(p.U, gLp, gXL, 1);
       cbwd(p.V, gRp, gXR, 1);
     });
   };
   auto fc_bwd = [&](const char *name, FcStage<T> &F, const T *gout) {
     stage(tg(k, name).c_str(), [&] {
+      if (F.joined) {
+        GemmIO<T> io{};
+        io_source(io, 0, gout, F.right.ndst, F.right.WT.template as<T>());
+        io_output(io, 0, gR2, F.right.ndst, true);
+        io_output(io, 1, gX, F.right.nsrc, true);
+        io.add = gout;
+        return EngineBase::launch_gemm_io<T>(F.bwd, 4, 4, io, cur_tiles_, cur_ntiles_);
+      }
       scale_rows(gout, F.nof, gR2, F.nf, wR, 1);
       cbwd(F.right, gout, gX, 1);
     });
   };
-  prod_bwd("4", L.p4, L.L4, L.R4p, gR4, gFB, gFB);
+  prod_bwd("4", L.p4, L.L4, L.R4p, gR4, gFB, gFB, true);
   fc_bwd("fc_2b_bwd", L.fb, gFB);
-  prod_bwd("3", L.p3, L.L3, L.R3p, gR3, gFA, gX);
+  prod_bwd("3", L.p3, L.L3, L.R3p, gR3, gFA, gX, true);
   fc_bwd("fc_2a_bwd", L.fa, gFA);
-  prod_bwd("2", L.p2, L.L2, L.R2p, gR2, gX, gX);
+  prod_bwd("2", L.p2, L.L2, L.R2p, gR2, gX, gX, false);
   if (!L.equiv) {
     BondBwdArgs<T> ba{};
     ba.eoff = eoff_.as<long long>(); ba.ej = ej_.as<int>(); ba.rh = rh_.as<double>(); ba.r = r_.as<double>(); ba.rc = rc_.as<double>();

@@ -307,7 +307,8 @@ struct DevProd {
 
 // weights W[K][N] (row-major) of a tile GEMM in MFMA fragment order [cb][s][lane]: lane (g, c) holds
 // W[g * (K / 4) + s][cb * 16 + c]
-template<class T> void pack_fragments(const std::vector<double> &W, int K, int N, int Kp, int Np, std::vector<T> &out)
+// (k index frag_k<T>, or g * Kp / 4 + s with plain: inputs that are no rows of a multiple of 16 channels)
+template<class T> void pack_fragments(const std::vector<double> &W, int K, int N, int Kp, int Np, std::vector<T> &out, bool plain = false)
 {
   const int ks = Kp / 4, nb = Np / 16;
   const size_t base = out.size();
@@ -315,19 +316,20 @@ template<class T> void pack_fragments(const std::vector<double> &W, int K, int N
   for (int cb = 0; cb < nb; cb++)
     for (int s = 0; s < ks; s++)
       for (int lane = 0; lane < 64; lane++) {
-        const int g = lane >> 4, c = lane & 15, k = g * ks + s, n = cb * 16 + c;
+        const int g = lane >> 4, c = lane & 15, k = plain ? g * ks + s : frag_k<T>(g, s), n = cb * 16 + c;
         if (k < K && n < N) out[base + ((size_t) cb * ks + s) * 64 + lane] = (T) W[(size_t) k * N + n];
       }
 }
 
 template<class T> struct DevJobs {
-  DevBuf job_out, job_scale, seg_off, seg_src, seg_fn, seg_w, seg_scale;
+  DevBuf job_out, job_scale, job_dst, job_add, seg_off, seg_src, seg_fn, seg_w, seg_scale, seg;
   GemmJobs<T> d{};
   long long nseg[2] = {0, 0};    // segments that read source 0 / source 1
+  long long seg_count = 0;
   struct Host {
-    std::vector<int> job_out, seg_off{0}, seg_src, seg_fn, seg_w;
-    std::vector<T> job_scale, seg_scale;
-    void job(int out, double scale) { job_out.push_back(out); job_scale.push_back((T) scale); }
+    std::vector<int> job_out, job_dst, seg_off{0}, seg_src, seg_fn, seg_w;
+    std::vector<T> job_scale, job_add, seg_scale;     // job_add: empty, or a factor for every job
+    void job(int out, double scale, int dst = 0) { job_out.push_back(out); job_scale.push_back((T) scale); job_dst.push_back(dst); }
     void seg(int src, int fn, int w, double scale) { seg_src.push_back(src); seg_fn.push_back(fn); seg_w.push_back(w); seg_scale.push_back((T) scale); }
     void end_job() { seg_off.push_back((int) seg_src.size()); }
   };
@@ -337,9 +339,17 @@ template<class T> struct DevJobs {
     upload_vec(seg_src, h.seg_src); upload_vec(seg_fn, h.seg_fn); upload_vec(seg_w, h.seg_w); upload_vec(seg_scale, h.seg_scale);
     d.job_out = job_out.as<int>(); d.job_scale = job_scale.as<T>(); d.seg_off = seg_off.as<int>();
     d.seg_src = seg_src.as<int>(); d.seg_fn = seg_fn.as<int>(); d.seg_w = seg_w.as<int>(); d.seg_scale = seg_scale.as<T>();
+    upload_vec(job_dst, h.job_dst);
+    if (!h.job_add.empty()) upload_vec(job_add, h.job_add);
+    std::vector<int4> sv;
+    for (size_t q = 0; q < h.seg_src.size(); q++) sv.push_back(int4{h.seg_src[q], h.seg_fn[q], h.seg_w[q], 0});
+    if (sv.empty()) sv.push_back(int4{0, 0, 0, 0});
+    upload_vec(seg, sv);
+    d.job_dst = job_dst.as<int>(); d.seg = seg.as<int4>(); d.job_add = h.job_add.empty() ? nullptr : job_add.as<T>();
     d.WF0 = WF0; d.WF1 = WF1;
     d.njobs = (int) h.job_out.size();
     nseg[0] = nseg[1] = 0;
+    seg_count = (long long) h.seg_src.size();
     for (int src : h.seg_src) nseg[src ? 1 : 0]++;
     d.max_seg = 0;
     for (size_t q = 0; q + 1 < h.seg_off.size(); q++) d.max_seg = std::max(d.max_seg, h.seg_off[q + 1] - h.seg_off[q]);
@@ -792,7 +802,7 @@ template<class T> struct DevReduce {
           for (int k = 0; k < nout; k++)
             for (int n = 0; n < nin; n++) Mt[(size_t) k * nin + n] = M[(size_t) n * nout + k];
           pack_fragments<T>(M, nin, nout, w.ninp, d.nbr * 16, vF);      // X[atom][n] . M[n][k]
-          pack_fragments<T>(Mt, nout, nin, krp, w.ninp, vB);             // g[atom][k] . Mt[k][n]
+          pack_fragments<T>(Mt, nout, nin, krp, w.ninp, vB, true);       // g[atom][k] . Mt[k][n]
         }
       upload_vec(WF[s], vF);
       upload_vec(WB[s], vB);
@@ -1451,6 +1461,47 @@ class EngineBase : public Engine, protected BufRegistry {
 #undef GR_BB_NL
 #undef GR_BB
   }
+  // Which launches with one input width take k_gemm_few / k_gemm_wide: all of 64 x 64 channels, and those whose blocks of
+  // k_gemm_jobs (16 atom tiles each) would leave CUs idle.
+  bool gemm_io_shape(int njobs, int kb, int nb, int ntiles) const
+  {
+    return (kb == 4 && nb == 4) || (long long) njobs * ((ntiles + 15) / 16) < ncu_;
+  }
+  template<class T> void launch_gemm_io(DevJobs<T> &J, int kb, int nb, const GemmIO<T> &io, const int *tiles, int ntiles)
+  {
+    if (J.d.njobs == 0 || ntiles == 0) return;
+    cur_flops_ += 2.0 * 16.0 * ntiles * (double) (nb * 16) * (double) (kb * 16) * (double) J.seg_count;
+    // groups of k_gemm_wide: four waves of two atom tiles.  It takes over where its blocks fill the chip twice, or half of it
+    // when the jobs are long enough for its better use of the weights to count.  Measured, k_gemm_few / k_gemm_wide, 36 jobs: one
+    // segment, 47 tiles (216 blocks, fp32) 9.5 / 10.0 us plain and 11.3 / 17.8 adding, 190 tiles (864 blocks, fp64) 51 / 36;
+    // 47 segments, 8 tiles (36 blocks) 25 / 50, 47 tiles 42 / 35, 190 tiles 369 / 185.
+    const int groups = (ntiles + 7) / 8;
+    const bool longer = J.seg_count >= 4ll * J.d.njobs;
+    if (kb == 4 && nb == 4 && (long long) J.d.njobs * groups >= (longer ? ncu_ / 2 : 2 * ncu_)) {
+      const int reps = J.d.max_seg == 1 && !io.accumulate && !J.d.job_add ? std::max(1, std::min(8, (int) ((long long) J.d.njobs * groups / (8 * ncu_)))) : 1;
+      hipLaunchKernelGGL(k_gemm_wide<T>, dim3(J.d.njobs, (groups + reps - 1) / reps), dim3(256), 0, stream_, J.d, io, tiles, ntiles, reps);
+      return;
+    }
+    const dim3 grid(J.d.njobs, ntiles);
+#define GR_FEW(K_, N_)                                                                                                              \
+  {                                                                                                                                 \
+    if (J.d.max_seg >= 4) hipLaunchKernelGGL((k_gemm_few<T, K_, N_, 4>), grid, dim3(64 * N_ * 4), 0, stream_, J.d, io, tiles);      \
+    else hipLaunchKernelGGL((k_gemm_few<T, K_, N_, 1>), grid, dim3(64 * N_), 0, stream_, J.d, io, tiles);                           \
+  }
+    switch (kb * 10 + nb) {
+      case 11: GR_FEW(1, 1) break;
+      case 12: GR_FEW(1, 2) break;
+      case 14: GR_FEW(1, 4) break;
+      case 21: GR_FEW(2, 1) break;
+      case 22: GR_FEW(2, 2) break;
+      case 24: GR_FEW(2, 4) break;
+      case 41: GR_FEW(4, 1) break;
+      case 42: GR_FEW(4, 2) break;
+      case 44: GR_FEW(4, 4) break;
+      default: throw Error("unsupported channel widths");
+    }
+#undef GR_FEW
+  }
   // out[tile atoms][job output] = GEMM jobs over X0 (kb0 16-channel blocks) and X1 (kb1), nb output blocks
   static constexpr size_t kGemmLdsBudget = 24 * 1024;    // measured on the benchmarks: 24 kB beats 16, 40 and 64 kB (blocks per CU)
   template<class T>
@@ -1458,6 +1509,12 @@ class EngineBase : public Engine, protected BufRegistry {
                    const int *tiles, int ntiles)
   {
     if (J.d.njobs == 0 || ntiles == 0) return;
+    if (kb0 == kb1 && gemm_io_shape(J.d.njobs, kb0, nb, ntiles)) {
+      GemmIO<T> io{};
+      io.X[0] = X0; io.X[1] = X1; io.nf[0] = nf0; io.nf[1] = nf1; io.WF[0] = J.d.WF0; io.WF[1] = J.d.WF1;
+      io.out[0] = out; io.nfo[0] = nfo; io.accumulate = accumulate ? 1 : 0;
+      return launch_gemm_io<T>(J, kb0, nb, io, tiles, ntiles);
+    }
     // multiply-adds of the launch: every segment is a [16 atoms x K] . [K x N] product per atom tile
     cur_flops_ += 2.0 * 16.0 * ntiles * (double) (nb * 16) * ((double) J.nseg[0] * kb0 * 16 + (double) J.nseg[1] * kb1 * 16);
     const int ksm = std::max(kb0, kb1) * 4;
@@ -1468,17 +1525,15 @@ class EngineBase : public Engine, protected BufRegistry {
     const size_t lds = (size_t) mseg * tile_bytes;
     // single-segment jobs (one weight tile each: projections, reverse of the product reduces) walk several groups of
     // atom tiles per block when the grid is large: the staging of the tile is what they spend their time on
-    const bool widest = kb0 == 4 && kb1 == 4 && nb == 4;
-    const int tpw = widest ? 1 : 2;      // = gemm_tiles_per_wave<kb0, kb1, nb>()
-    // waves of a block: a staged weight set is shared by 8 waves at fp64 and for the widest tiles, by 4 at fp32 with
-    // narrower tiles (measured: 8 instead of 4 gives -1.3 % of a pass on the fp64 benchmarks, +1.8 % at fp32)
-    const int nwave = widest || sizeof(T) == 8 ? 8 : 4;
-    const int groups = (ntiles + nwave * tpw - 1) / (nwave * tpw);
+    // waves of a block: a staged weight set is shared by 8 waves at fp64, by 4 at fp32 (measured: 8 instead of 4 gives
+    // -1.3 % of a pass on the fp64 benchmarks, +1.8 % at fp32)
+    const int nwave = sizeof(T) == 8 ? 8 : 4;
+    const int groups = (ntiles + nwave * kGemmTilesPerWave - 1) / (nwave * kGemmTilesPerWave);
     const int reps = J.d.max_seg == 1 ? std::max(1, std::min(8, (int) ((long long) J.d.njobs * groups / 8192))) : 1;
     const dim3 grid(J.d.njobs, (groups + reps - 1) / reps);
 #define GR_GEMM(A_, B_, C_)                                                                                            \
   {                                                                                                                    \
-    auto kern = k_gemm_jobs<T, A_, B_, C_, gemm_tiles_per_wave<A_, B_, C_>()>;                                         \
+    auto kern = k_gemm_jobs<T, A_, B_, C_>;                                                                            \
     if (lds > 48 * 1024)                                                                                               \
       HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds)); \
     hipLaunchKernelGGL(kern, grid, dim3(64 * nwave), lds, stream_, J.d, X0, nf0, X1, nf1, out, nfo, tiles, ntiles, accumulate, reps, mseg); \
@@ -1499,7 +1554,9 @@ class EngineBase : public Engine, protected BufRegistry {
       case 24: GR_GEMM_C(2, 4) break;
       case 41: GR_GEMM_C(4, 1) break;
       case 42: GR_GEMM_C(4, 2) break;
-      case 44: GR_GEMM_C(4, 4) break;
+      case 44:    // 64 outputs: k_gemm_few, k_gemm_wide
+        if (nb == 1) { GR_GEMM(4, 4, 1) } else if (nb == 2) { GR_GEMM(4, 4, 2) } else throw Error("unsupported channel widths");
+        break;
       default: throw Error("unsupported channel widths");
     }
 #undef GR_GEMM_C

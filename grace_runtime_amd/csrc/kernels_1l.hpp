@@ -1182,8 +1182,27 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256) __attribute_
 // FC forward:        job f,  segments (Xl, f, Wl[tile_l f]) and (Xr, from c, Wr[tile c]) for every connection c -> f
 // FC reverse, left:  job f,  segment  (g, f, Wl^T[tile_l f]), accumulated into gXl
 // FC reverse, right: job r,  segments (g, to c, nof[to c] Wr^T[tile c]) for the connections c from r, accumulated
-// Rows of the A operand are the 16 atoms (lane % 16), its k index g * (K / 4) + s (g = lane / 16), so that a lane
-// reads K / 4 consecutive channels; weights are stored in that fragment order ([tile][cb][s][lane]) and staged in LDS.
+// Rows of the A operand are the 16 atoms (lane % 16).  The channel that step s takes from lane group g = lane / 16 is
+// frag_k<T>: 16 bytes of the row per group in turn, so that one load instruction reads 64 consecutive bytes of each of the 16
+// rows (with K / 4 consecutive channels per group it touched four times as many cache lines).  Weights are stored in that
+// order ([tile][cb][s][lane]).
+template<class T> __host__ __device__ constexpr int frag_k(int g, int s)
+{
+  constexpr int V = 16 / (int) sizeof(T);    // values of a 16-byte piece
+  return (s / V) * 4 * V + g * V + s % V;
+}
+// KS values of the A operand of lane group g, from the row xp (16-byte aligned: rows hold a multiple of 16 channels)
+template<int KS, class T> __device__ inline void frag_load(const T *xp, int g, T (&x)[KS])
+{
+  constexpr int V = 16 / (int) sizeof(T);
+  typedef T piece __attribute__((ext_vector_type(16 / sizeof(T))));
+#pragma unroll
+  for (int p = 0; p < KS / V; p++) {
+    const piece w = *reinterpret_cast<const piece *>(xp + (p * 4 + g) * V);
+#pragma unroll
+    for (int q = 0; q < V; q++) x[p * V + q] = w[q];
+  }
+}
 template<class T> struct GemmJobs {
   const int *job_out;         // [njobs] output function
   const T *job_scale;         // [njobs]
@@ -1196,14 +1215,24 @@ template<class T> struct GemmJobs {
   int njobs;
   int max_seg;                // most segments of one job
   int drow[16];               // accumulator row of (lane / 16, register), probed on the device
+  const int4 *seg;            // [nseg] source, function, weight tile as one entry (k_gemm_few, k_gemm_wide)
+  const int *job_dst;         // [njobs] output tensor
+  const T *job_add;           // [njobs] factor of the row of GemmIO::add that is added, or null
+};
+// The tensors of a launch whose job list reads up to four sources and writes up to four outputs, all of one width
+template<class T> struct GemmIO {
+  const T *X[4], *WF[4];
+  int nf[4];
+  T *out[4];
+  int nfo[4];
+  const T *add;               // out[0] += job_add x this row (shape of out[0])
+  unsigned accumulate;        // bit d: added to out[d], not set
 };
 
 constexpr int kGemmMaxSeg = 4;      // most weight tiles staged in LDS at a time (the launch passes the number, mseg)
-// atom tiles of a wave (TPW): 2, and 1 for the widest tiles (64 channels in, 64 out), whose accumulators and operands
-// of two atom tiles would leave two waves per SIMD
-template<int KB0, int KB1, int NB> constexpr int gemm_tiles_per_wave() { return KB0 == 4 && KB1 == 4 && NB == 4 ? 1 : 2; }
+constexpr int kGemmTilesPerWave = 2;
 
-template<class T, int KB0, int KB1, int NB, int TPW>
+template<class T, int KB0, int KB1, int NB>
 __global__ __launch_bounds__(512) void k_gemm_jobs(GemmJobs<T> J, const T *X0, int nf0, const T *X1, int nf1, T *out, int nfo,
                                                    const int *tile_atoms, int ntiles, int accumulate, int reps, int mseg)
 {
@@ -1211,6 +1240,7 @@ __global__ __launch_bounds__(512) void k_gemm_jobs(GemmJobs<T> J, const T *X0, i
   // time so that several blocks fit a CU).  reps > 1 (only when every job has one segment): the block stages its
   // weight tile once and walks `reps` groups of atom tiles with it
   typedef typename Mfma<T>::v4 v4;
+  constexpr int TPW = kGemmTilesPerWave;
   constexpr int KS0 = KB0 * 4, KS1 = KB1 * 4, KSM = KS0 > KS1 ? KS0 : KS1, K0 = KB0 * 16, K1 = KB1 * 16, N = NB * 16;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *wl = reinterpret_cast<T *>(smem_raw);      // [mseg][NB][KSM][64]
@@ -1258,9 +1288,9 @@ __global__ __launch_bounds__(512) void k_gemm_jobs(GemmJobs<T> J, const T *X0, i
           if (s_src[q] == 0) {
             T x[KS0];
             if (arow[i] >= 0) {
-              const T *xp = X0 + ((long long) arow[i] * nf0 + s_fn[q]) * K0 + g * KS0;
+              frag_load<KS0>(X0 + ((long long) arow[i] * nf0 + s_fn[q]) * K0, g, x);
 #pragma unroll
-              for (int s = 0; s < KS0; s++) x[s] = xp[s] * sc;
+              for (int s = 0; s < KS0; s++) x[s] *= sc;
             } else {
 #pragma unroll
               for (int s = 0; s < KS0; s++) x[s] = (T) 0;
@@ -1272,9 +1302,9 @@ __global__ __launch_bounds__(512) void k_gemm_jobs(GemmJobs<T> J, const T *X0, i
           } else {
             T x[KS1];
             if (arow[i] >= 0) {
-              const T *xp = X1 + ((long long) arow[i] * nf1 + s_fn[q]) * K1 + g * KS1;
+              frag_load<KS1>(X1 + ((long long) arow[i] * nf1 + s_fn[q]) * K1, g, x);
 #pragma unroll
-              for (int s = 0; s < KS1; s++) x[s] = xp[s] * sc;
+              for (int s = 0; s < KS1; s++) x[s] *= sc;
             } else {
 #pragma unroll
               for (int s = 0; s < KS1; s++) x[s] = (T) 0;
@@ -1305,6 +1335,296 @@ __global__ __launch_bounds__(512) void k_gemm_jobs(GemmJobs<T> J, const T *X0, i
       }
     }
   }
+}
+
+// ---- the jobs of a launch with one width of inputs and one of outputs, in the two shapes that few and many atom tiles need ----
+// barrier of a block that exchanges through LDS only: __syncthreads would also wait for the loads and stores in flight
+__device__ inline void lds_barrier()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// k_gemm_few: a wave owns ONE 16 x 16 tile of the output (an atom tile and a column block), so that a structure of a few
+// atom tiles still puts a wave on every SIMD, and the segments of a job are dealt to S waves whose sums meet in LDS (in the
+// order of the waves).  No operand passes through LDS and no wave waits for another before the end: both operands come from
+// L1 / L2, 8 steps of them requested while the 8 before are multiplied, the description of a segment one request earlier.
+// What bounds it: the L1 (16 kB of operands per 16 x 16 x 64 tile, as many cycles as its matrix instructions take with all
+// four SIMDs busy) and, for jobs of one segment, the latency of a launch.  GRACE-3L, 96 atoms (8 tiles): 36 jobs of 47
+// segments 80 us as k_gemm_jobs (36 blocks), 50 as k_gemm_wide, 25 so; 36 jobs of one segment 12.4 / 11.4 / 7.2 us.
+template<class T, int KB, int NB, int S>
+__global__ __launch_bounds__(64 * NB * S) void k_gemm_few(GemmJobs<T> J, GemmIO<T> io, const int *tile_atoms)
+{
+  typedef typename Mfma<T>::v4 v4;
+  constexpr int KS = KB * 4, K = KB * 16, N = NB * 16, HS = KS > 8 ? 8 : KS, U = KS / HS, V = 16 / (int) sizeof(T);
+  typedef T piece __attribute__((ext_vector_type(16 / sizeof(T))));
+  __shared__ T part[S > 1 ? (S - 1) * NB * 256 : 1];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4, cb = wave % NB, pt = wave / NB;
+  const int job = blockIdx.x, tile = blockIdx.y;
+  const int sg0 = J.seg_off[job] + pt, sg1 = J.seg_off[job + 1];
+  const int first = tile_atoms[tile * 16], mine = tile_atoms[tile * 16 + c];
+  const int row = mine >= 0 ? mine : first;           // a row without an atom: computed from the tile's first, never stored
+  const int nu = sg1 > sg0 ? (sg1 - sg0 + S - 1) / S * U : 0;      // units of HS steps of this wave
+  const int fo = J.job_out[job], dst = J.job_dst[job];
+  const T js = J.job_scale[job];
+  T *out = io.out[dst] + fo * N + cb * 16 + c;
+  const long long nfoN = (long long) io.nfo[dst] * N;
+  int at[4];
+#pragma unroll
+  for (int v = 0; v < 4; v++) at[v] = tile_atoms[tile * 16 + J.drow[4 * g + v]];
+  // what is added to the sum: requested first, added last (in fp32 a sum that starts from it is 20 % less accurate)
+  v4 acc = {0, 0, 0, 0}, y = {0, 0, 0, 0};
+  if (pt == 0) {
+    const bool accumulate = io.accumulate >> dst & 1;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const long long o = (at[v] >= 0 ? at[v] : first) * nfoN;
+      if (accumulate) y[v] = out[o];
+      if (J.job_add && dst == 0) y[v] += J.job_add[job] * io.add[o + fo * N + cb * 16 + c];
+    }
+  }
+  T xa[HS], wa[HS], xb[HS], wb[HS], sa = 0, sb = 0, scn = 0;
+  int4 mn = {0, 0, 0, 0};
+  auto describe = [&](int u) {
+    const int sg = sg0 + (u / U) * S;
+    mn = J.seg[sg];
+    scn = J.seg_scale[sg];
+  };
+  auto load = [&](int u, T (&x)[HS], T (&w)[HS], T &sc) {
+    const int src = mn.x, h = U == 1 ? 0 : u % U;
+    const T *xp = io.X[src] + ((long long) row * io.nf[src] + mn.y) * K + (h * (HS / V) * 4 + g) * V;
+    const T *wp = io.WF[src] + (((long long) mn.z * NB + cb) * KS + h * HS) * 64 + lane;
+#pragma unroll
+    for (int p = 0; p < HS / V; p++) {
+      const piece q = *reinterpret_cast<const piece *>(xp + p * 4 * V);
+#pragma unroll
+      for (int e = 0; e < V; e++) x[p * V + e] = q[e];
+    }
+#pragma unroll
+    for (int s = 0; s < HS; s++) w[s] = wp[s * 64];
+    sc = scn;
+    if (u + 1 < nu) describe(u + 1);
+  };
+  auto multiply = [&](const T (&x)[HS], const T (&w)[HS], T sc) {
+#pragma unroll
+    for (int s = 0; s < HS; s++) acc = Mfma<T>::mma(x[s] * sc, w[s], acc);
+  };
+  if (nu > 0) {
+    describe(0);
+    load(0, xa, wa, sa);
+  }
+  for (int u = 0; u < nu; u += 2) {
+    if (u + 1 < nu) load(u + 1, xb, wb, sb);
+    multiply(xa, wa, sa);
+    if (u + 2 < nu) load(u + 2, xa, wa, sa);
+    if (u + 1 < nu) multiply(xb, wb, sb);
+  }
+  if (S > 1) {
+    if (pt > 0) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) part[((pt - 1) * NB + cb) * 256 + v * 64 + lane] = acc[v];
+    }
+    lds_barrier();
+    if (pt > 0) return;
+#pragma unroll
+    for (int q = 0; q < S - 1; q++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) acc[v] += part[(q * NB + cb) * 256 + v * 64 + lane];
+  }
+#pragma unroll
+  for (int v = 0; v < 4; v++)
+    if (at[v] >= 0) out[at[v] * nfoN] = js * acc[v] + y[v];
+}
+
+// k_gemm_wide (64 channels in, 64 out): a wave owns two atom tiles and all 64 columns, the four waves of a block share the
+// weight tile of a segment in LDS (two tiles of 32 kB in fp64, one filled while the other is read).  The rows of the next
+// segment are requested into the registers that hold this one's, each piece as soon as its last product has been issued,
+// and the next weight tile waits in registers until the products are done: every load has a whole segment (8192 cycles of
+// matrix work in fp64) to arrive, which k_gemm_jobs, whose loads stood at the head of every segment, left exposed.
+// GRACE-3L, 3001 atoms fp64: 72 jobs of 23 segments 1281 -> 857 us (49 TF; the rows of its source are read once: 2.6 GB, 0.5
+// ms at the copy rate), 1685 jobs of one segment 1119 -> 909 us (writes 2.6 GB).
+// Jobs of one segment walk `reps` groups of atom tiles with the tile they have staged.
+template<class T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 2))) void k_gemm_wide(GemmJobs<T> J, GemmIO<T> io, const int *tile_atoms, int ntiles,
+                                                                                        int reps)
+{
+  typedef typename Mfma<T>::v4 v4;
+  constexpr int KS = 16, K = 64, N = 64, NB = 4, MT = 2, V = 16 / (int) sizeof(T), NP = KS / V, WT = NB * KS * 64, WP = WT / V / 256;
+  typedef T piece __attribute__((ext_vector_type(16 / sizeof(T))));
+  __shared__ __align__(16) T wl[2][WT];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int job = blockIdx.x;
+  const int sg0 = J.seg_off[job], nseg = J.seg_off[job + 1] - sg0;
+  const int fo = J.job_out[job], dst = J.job_dst[job];
+  const T js = J.job_scale[job];
+  T *out = io.out[dst];
+  const int nfo = io.nfo[dst];
+  const bool accumulate = io.accumulate >> dst & 1;
+  auto tile_of = [&](int rep, int i) { return ((blockIdx.y * reps + rep) * 4 + wave) * MT + i; };
+  // groups of atom tiles this block walks (jobs of one segment), or segments
+  const int left = ntiles - (int) blockIdx.y * reps * 4 * MT, ngroups = left >= reps * 4 * MT ? reps : (left + 4 * MT - 1) / (4 * MT);
+  const int steps = reps > 1 ? ngroups : nseg;
+  int row[MT];
+  auto rows_of = [&](int rep) {
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int tile = tile_of(rep, i), tc = tile < ntiles ? tile : ntiles - 1;
+      const int first = tile_atoms[tc * 16], mine = tile_atoms[tc * 16 + c];
+      row[i] = mine >= 0 ? mine : first;              // rows without an atom: never stored
+    }
+  };
+  v4 acc[MT][NB];
+  T x[MT][KS];
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int cb = 0; cb < NB; cb++) acc[i][cb] = v4{0, 0, 0, 0};
+  };
+  // What is added to the sums (value (cb, v) of a tile at x[i][4 cb + v]): requested into the registers of the operands as the
+  // last segment frees them.  (Sums that start from it are as quick and, in fp32, 20 % less accurate.)
+  const bool add = J.job_add && dst == 0, added = accumulate || add;
+  auto added_request = [&](int rep, int q) {
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int tile = tile_of(rep, i), tc = tile < ntiles ? tile : ntiles - 1;
+      const int at = tile_atoms[tc * 16 + J.drow[4 * g + q % 4]];
+      const long long o = ((long long) (at >= 0 ? at : tile_atoms[tc * 16]) * nfo + fo) * N + c + (q / 4) * 16;
+      x[i][q] = accumulate ? out[o] : (T) 0;
+      if (add) x[i][q] += J.job_add[job] * io.add[o];
+    }
+  };
+  auto store = [&](int rep) {
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int tile = tile_of(rep, i);
+      if (tile >= ntiles) continue;
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int at = tile_atoms[tile * 16 + J.drow[4 * g + v]];
+        if (at < 0) continue;
+        const long long o = ((long long) at * nfo + fo) * N + c;
+#pragma unroll
+        for (int cb = 0; cb < NB; cb++) out[o + cb * 16] = added ? js * acc[i][cb][v] + x[i][4 * cb + v] : js * acc[i][cb][v];
+      }
+    }
+  };
+  // fp32: the sum of every segment is added to the total by itself.  One long chain of accumulations over the segments of
+  // joined contractions was 5 % less accurate than the separate launches (forces of 701 and 1500 atoms against fp64).
+  v4 total[MT][NB];
+  auto take = [&]() {
+    if (sizeof(T) == 4) {
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int cb = 0; cb < NB; cb++) total[i][cb] += acc[i][cb];
+      clear();
+    }
+  };
+  clear();
+  if (sizeof(T) == 4) {
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int cb = 0; cb < NB; cb++) total[i][cb] = v4{0, 0, 0, 0};
+  }
+  if (nseg == 0) {                                    // a job that only clears, or adds a row of io.add
+    for (int rep = 0; rep < (reps > 1 ? ngroups : 1); rep++) {
+      if (added) {
+#pragma unroll
+        for (int q = 0; q < KS; q++) added_request(rep, q);
+      }
+      store(rep);
+    }
+    return;
+  }
+  piece wn[WP];
+  auto weights_request = [&](const int4 &m) {
+    const T *wf = io.WF[m.x] + (long long) m.z * WT;
+#pragma unroll
+    for (int p = 0; p < WP; p++) wn[p] = *reinterpret_cast<const piece *>(wf + (p * 256 + threadIdx.x) * V);
+  };
+  auto weights_store = [&](int buf) {
+#pragma unroll
+    for (int p = 0; p < WP; p++) *reinterpret_cast<piece *>(&wl[buf][(p * 256 + threadIdx.x) * V]) = wn[p];
+  };
+  const T *xp[MT];
+  auto sources = [&](const int4 &m) {
+    const T *X = io.X[m.x];
+    const int nf = io.nf[m.x];
+#pragma unroll
+    for (int i = 0; i < MT; i++) xp[i] = X + ((long long) row[i] * nf + m.y) * K + g * V;
+  };
+  auto x_request = [&](int p) {
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const piece q = *reinterpret_cast<const piece *>(xp[i] + p * 4 * V);
+#pragma unroll
+      for (int e = 0; e < V; e++) x[i][p * V + e] = q[e];
+    }
+  };
+  int4 m = J.seg[sg0];
+  T sc = J.seg_scale[sg0];
+  rows_of(0);
+  weights_request(m);
+  sources(m);
+#pragma unroll
+  for (int p = 0; p < NP; p++) x_request(p);
+  weights_store(0);
+  for (int t = 0; t < steps; t++) {
+    if (reps == 1 || t == 0) lds_barrier();
+    const bool more = t + 1 < steps;
+    const T scn = reps == 1 && more ? J.seg_scale[sg0 + t + 1] : sc;
+    if (more) {
+      if (reps == 1) {
+        m = J.seg[sg0 + t + 1];
+        weights_request(m);
+      } else {
+        rows_of(t + 1);
+      }
+      sources(m);
+    }
+    const T *wq = wl[reps == 1 ? t & 1 : 0] + lane;
+    T w[2][NB];
+#pragma unroll
+    for (int cb = 0; cb < NB; cb++) w[0][cb] = wq[cb * KS * 64];
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+      if (s + 1 < KS) {
+#pragma unroll
+        for (int cb = 0; cb < NB; cb++) w[(s + 1) & 1][cb] = wq[(cb * KS + s + 1) * 64];
+      }
+#pragma unroll
+      for (int i = 0; i < MT; i++) {
+        const T xs = x[i][s] * sc;
+#pragma unroll
+        for (int cb = 0; cb < NB; cb++) acc[i][cb] = Mfma<T>::mma(xs, w[s & 1][cb], acc[i][cb]);
+      }
+      if (more) {
+        if ((s + 1) % V == 0) x_request(s / V);
+      } else if (added) {
+        added_request(0, s);       // launches with several groups add nothing
+      }
+    }
+    if (reps > 1) {
+      store(t);
+      clear();
+    } else {
+      if (nseg > 1) take();
+      if (more) weights_store((t + 1) & 1);
+    }
+    sc = scn;
+  }
+  if (sizeof(T) == 4 && nseg > 1) {
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int cb = 0; cb < NB; cb++) acc[i][cb] = total[i][cb];
+  }
+  if (reps == 1) store(0);
 }
 
 // Block index -> (function q, atom group) for grids of nq * 8 * ceil(groups / 8) blocks.  Workgroups go to the 8 XCDs
@@ -1364,7 +1684,7 @@ template<class T> __global__ void k_prod_bwd(ProdDev P, int side, const T *other
 
 template<class T> struct ReduceDev {
   // per source s: collected functions fn[s][c] (unique), weights in fragment order
-  //   forward WF[s][mu][c][cb][ks][lane]  = W_s[mu][c][n = g KS + ks][k = cb 16 + lane % 16]    (norm folded, k >= nrho zero)
+  //   forward WF[s][mu][c][cb][ks][lane]  = W_s[mu][c][n = frag_k(g, ks)][k = cb 16 + lane % 16] (norm folded, k >= nrho zero)
   //   reverse WB[s][mu][c][cb][ks][lane]  = W_s[mu][c][n = cb 16 + lane % 16][k = g KSR + ks]
   const T *WF[4], *WB[4];
   const int *fn[4];
@@ -1400,9 +1720,9 @@ __global__ __launch_bounds__(64 * kReduceWaves) void k_reduce_fwd(ReduceDev<T> R
       const T *wf = R.WF[s] + ((long long) m * R.ncol[s] + cc) * R.nbr * ks * 64 + lane;
       T x[(KBA > KBF ? KBA : KBF) * 4];
       if (arow >= 0) {
-        const T *xp = X[s] + ((long long) arow * R.stride[s] + R.fn[s][cc]) * K + g * ks;
+        const T *xp = X[s] + ((long long) arow * R.stride[s] + R.fn[s][cc]) * K;
 #pragma unroll
-        for (int q = 0; q < (KBA > KBF ? KBA : KBF) * 4; q++) x[q] = q < ks ? xp[q] : (T) 0;
+        for (int q = 0; q < (KBA > KBF ? KBA : KBF) * 4; q++) x[q] = q < ks ? xp[frag_k<T>(g, q)] : (T) 0;
       } else {
 #pragma unroll
         for (int q = 0; q < (KBA > KBF ? KBA : KBF) * 4; q++) x[q] = (T) 0;
