@@ -605,6 +605,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
   const long long *n_edges = eoff_.as<long long>() + n;
   const bool forces = !fl.energy_only;
   if (ordered_ && forces) ordered_begin();
+  bsum_begin(forces && !ordered_ && pair_mfma_ != 0 && pair_mfma_plan(nslot_, CRP_, nl_, sizeof(T), pair_mfma_waves(pair_waves_)).ok);
   // row of an edge: Y[nlm] and, for forces, the two tangential gradients D1[nlm], D2[nlm] and padding (pair_row_stride)
   const int yw = forces ? pair_row_stride(nlm_, sizeof(T)) : nlm_;
   YG_.ensure(ecap_all * yw * sizeof(T));
@@ -630,7 +631,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
   const double per_atom = sizeof(T) * (chain_values(c1_) + chain_values(c2_) + (double) nlm_ * C1P_ + 2.0 * npf * CRP_ + (double) nB_ * C2P_ +
                                        bonds_per_atom * 2.0 * (radR_.noutp + radR1_.noutp)) +
                           (2.0 * nI1_ * PI1_ + 2.0 * nrho_) * sizeof(double) + 2.0 * nI1_ * PI1_ * (sizeof(T) == 4 ? 4.0 : 0.0);
-  const double kept = bonds_per_atom * (60.0 + yw * sizeof(T)) + (double) (nslot_ + nI_) * CRP_ * sizeof(T) + 32.0 * nrho_ + 64.0;
+  const double kept = bonds_per_atom * ((bsum_on_ ? 84.0 : 60.0) + yw * sizeof(T)) + (double) (nslot_ + nI_) * CRP_ * sizeof(T) + 32.0 * nrho_ + 64.0;
   const int cs = plan_chunk(n, per_atom, kept);
   const int nchunks = (n + cs - 1) / cs;
   chunk_used_ = nchunks > 1 ? cs : 0;
@@ -856,13 +857,12 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
       if (ordered_) {
         po.gMe = gMe_.as<T>(); po.fedge = fedge_.as<double>(); po.fcen = fcen_.as<double>(); po.e_base = eb; po.ngrp = 1;
       }
-      const PairMfmaPlan mp = pair_mfma_plan(nslot_, CRP_, nl_, sizeof(T), pair_mfma_waves(sizeof(T), pair_waves_));
+      const PairMfmaPlan mp = pair_mfma_plan(nslot_, CRP_, nl_, sizeof(T), pair_mfma_waves(pair_waves_));
       if (!ordered_ && mp.ok && pair_mfma_ != 0) {
         PairMfmaArgs<T> pa{};
         pa.eoff = eoff; pa.ej = ej_.as<int>(); pa.erow = rows.erow; pa.YG = YG_.as<T>(); pa.R1 = R1; pa.dR1 = dR1; pa.M = M; pa.gP = gP_.as<T>();
-        pa.rh = rh_.as<double>(); pa.rlen = r_.as<double>(); pa.rcut = rc_.as<double>();
-        pa.gM = gM_.as<T>(); pa.f = f_.as<double>(); pa.virial = scal_.as<double>() + 1; pa.vatom = vatom_ptr(); pa.sid = sid_ptr();
-        pa.nslot = nslot_; pa.nI = nI_; pa.C = CRP_; pa.noutp = radR1_.noutp; pa.natoms = nc; pa.a0 = a0_;
+        pa.gM = gM_.as<T>(); pa.bsum = bsum_ptr();
+        pa.nslot = nslot_; pa.nI = nI_; pa.C = CRP_; pa.noutp = radR1_.noutp; pa.natoms = nc;
         for (int q = 0; q < 16; q++) pa.drow[q] = drow_[q];
         launch_pair_bwd_mfma(mp, pa, nl_, stream_);
       } else if (ordered_) {
@@ -927,7 +927,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     BondBwdArgs<T> ba{};
     ba.eoff = eoff_.as<long long>(); ba.ej = ej_.as<int>(); ba.rh = rh_.as<double>(); ba.r = r_.as<double>(); ba.rc = rc_.as<double>();
     ba.Rz = moved_back(Rz_.as<T>(), eb * radR_.noutp); ba.dRz = moved_back(dRz_.as<T>(), eb * radR_.noutp); ba.gA = c1_.gX.template as<T>();
-    ba.f = f_.as<double>(); ba.virial = scal_.as<double>() + 1; ba.sid = sid_ptr(); ba.vatom = vatom_ptr();
+    ba.f = f_.as<double>(); ba.virial = scal_.as<double>() + 1; ba.sid = sid_ptr(); ba.vatom = vatom_ptr(); ba.bsum = bsum_ptr();
     ba.tb = tbR;
     if (!tab_inside) { ba.erow = rows.erow; ba.emu = emu_.as<int>(); ba.z = zA_.as<T>(); }
     ba.a0 = a0_; ba.C = C1P_; ba.nl = nl_; ba.nlm = nlm_; ba.noutp = radR_.noutp; ba.sh = sh_;

@@ -1142,7 +1142,7 @@ template<class T> void Engine3L<T>::layer_backward(int k, int yw)
     BondBwdArgs<T> ba{};
     ba.eoff = eoff_.as<long long>(); ba.ej = ej_.as<int>(); ba.rh = rh_.as<double>(); ba.r = r_.as<double>(); ba.rc = rc_.as<double>();
     ba.Rz = Rl; ba.dRz = dRl; ba.gA = gX;
-    ba.f = f_.as<double>(); ba.virial = scal_.as<double>() + 1; ba.sid = sid_ptr(); ba.vatom = vatom_ptr();
+    ba.f = f_.as<double>(); ba.virial = scal_.as<double>() + 1; ba.sid = sid_ptr(); ba.vatom = vatom_ptr(); ba.bsum = bsum_ptr();
     ba.a0 = a0_; ba.C = L.CP; ba.nl = nl_; ba.nlm = nlm_; ba.noutp = L.rad.noutp; ba.sh = sh_;
     if (ordered_) {
       ba.fedge = fedge_.as<double>(); ba.fcen = fcen_.as<double>(); ba.ordered_add = ordered_first_ ? 0 : 1;
@@ -1181,13 +1181,12 @@ template<class T> void Engine3L<T>::layer_backward(int k, int yw)
   dim3((unsigned) ((n + 7) / 8 * 8 * ngrp)), dim3(pthreads), lds, stream_, eoff, ej_.as<int>(), YG_.as<T>(), (const T *) Rl, (const T *) dRl,     \
       (const T *) M_.as<T>(), (const T *) gpairP_.as<T>(), rh_.as<double>(), r_.as<double>(), rc_.as<double>(), gM_.as<T>(), f_.as<double>(),   \
       scal_.as<double>() + 1, L.nlmi, L.nlmi, L.CP, nl_, L.rad.noutp, sink_.as<T>(), 1, sid_ptr(), spb, ngrp, n, a0_, vatom_ptr(), yw, (const int *) nullptr
-    const PairMfmaPlan mp = pair_mfma_plan(L.nlmi, L.CP, nl_, s, pair_mfma_waves(s, pair_waves_));
+    const PairMfmaPlan mp = pair_mfma_plan(L.nlmi, L.CP, nl_, s, pair_mfma_waves(pair_waves_));
     if (!ordered_ && mp.ok && pair_mfma_ != 0) {
       PairMfmaArgs<T> pa{};
       pa.eoff = eoff; pa.ej = ej_.as<int>(); pa.YG = YG_.as<T>(); pa.R1 = Rl; pa.dR1 = dRl; pa.M = M_.as<T>(); pa.gP = gpairP_.as<T>();
-      pa.rh = rh_.as<double>(); pa.rlen = r_.as<double>(); pa.rcut = rc_.as<double>();
-      pa.gM = gM_.as<T>(); pa.f = f_.as<double>(); pa.virial = scal_.as<double>() + 1; pa.vatom = vatom_ptr(); pa.sid = sid_ptr();
-      pa.nslot = pa.nI = L.nlmi; pa.C = L.CP; pa.noutp = L.rad.noutp; pa.natoms = n; pa.a0 = a0_;
+      pa.gM = gM_.as<T>(); pa.bsum = bsum_ptr();
+      pa.nslot = pa.nI = L.nlmi; pa.C = L.CP; pa.noutp = L.rad.noutp; pa.natoms = n;
       for (int q = 0; q < 16; q++) pa.drow[q] = drow_[q];
       launch_pair_bwd_mfma(mp, pa, nl_, stream_);
     } else if (ordered_) {
@@ -1247,6 +1246,9 @@ template<class T> void Engine3L<T>::run(const RunFlags &fl)
   const long long *n_edges = eoff_.as<long long>() + n;
   const bool forces = !fl.energy_only;
   if (ordered_ && forces) ordered_begin();
+  bool sums = false;
+  for (int k = 1; k < 3; k++) sums = sums || pair_mfma_plan(L_[k].nlmi, L_[k].CP, nl_, sizeof(T), pair_mfma_waves(pair_waves_)).ok;
+  bsum_begin(forces && !ordered_ && pair_mfma_ != 0 && sums);
   emi_.ensure(ecap * sizeof(int));
   stage("edge_center", [&] { hipLaunchKernelGGL(k_edge_center, dim3(n), dim3(64), 0, stream_, eoff_.as<long long>(), mu_.as<int>(), emi_.as<int>()); });
   // row of an edge: Y[nlm] and, for forces, the two tangential gradients D1[nlm], D2[nlm] and padding (pair_row_stride)
@@ -1274,7 +1276,7 @@ template<class T> void Engine3L<T>::run(const RunFlags &fl)
   // layer repeats that layer's forward pass for the chunk first (the reference's store_l1 = false, libgrace/include/grace/
   // system.h:79-80, extended to every layer).
   const double bonds_per_atom = (double) ecap / n;
-  double kept = bonds_per_atom * (60.0 + yw * sizeof(T)) + 64.0;
+  double kept = bonds_per_atom * ((bsum_on_ ? 84.0 : 60.0) + yw * sizeof(T)) + 64.0;
   for (int k = 0; k < 3; k++) kept += 3.0 * (double) L_[k].I.nf * L_[k].I.w * sizeof(T) + 16.0 * nrho_;
   const int cs = plan_chunk(n, chunk_bytes_per_atom(), kept);
   const int nchunks = (n + cs - 1) / cs;

@@ -1880,7 +1880,19 @@ class EngineBase : public Engine, protected BufRegistry {
     const char *e = std::getenv("GRACE_HIP_PAIR_MFMA");
     return e && e[0] == '0' ? 0 : 1;
   }
-  int pair_waves_ = pair_waves_switch();    // waves of a block of that kernel; 0: 8 in fp64, 4 in fp32 (pair_mfma_waves)
+  // the sums of the bonds that kernel leaves for k_bond_bwd of the first layer (BondBwdArgs::bsum): cleared once per pass
+  DevBuf bsum_;
+  bool bsum_on_ = false;
+  double *bsum_ptr() const { return bsum_on_ ? bsum_.as<double>() : nullptr; }
+  void bsum_begin(bool on)
+  {
+    bsum_on_ = on;
+    if (!on) return;
+    const size_t bytes = (size_t) 3 * std::max<int64_t>(nb_, 1) * sizeof(double);
+    bsum_.ensure(bytes);
+    stage("zero_bond_sums", [&] { HIP_CHECK(hipMemsetAsync(bsum_.p, 0, bytes, stream_)); });
+  }
+  int pair_waves_ = pair_waves_switch();    // waves of a block of that kernel; 0: those of one group of slots
   static int pair_waves_switch()
   {
     const char *e = std::getenv("GRACE_HIP_PAIR_WAVES");

@@ -2158,6 +2158,9 @@ template<class T> struct BondBwdArgs {
   // ordered mode (both set, no atomics, vatom null): fedge[e][3] = force of bond e on its central atom; fcen[i][9] = sum of
   // these over the bonds of atom i, then the six virial sums of its bonds; k_ordered_forces / k_ordered_records finish
   double *fedge, *fcen;
+  // sums of a bond left by the reverse pair kernels of the layers above ([e][3]: against Y dR, D1 R and D2 R as px, p1, p2 here),
+  // or null: their part of the bond's force is finished with this layer's, in one addition to each of its atoms
+  const double *bsum;
   int ordered_add;            // ordered mode: add to what fedge / fcen hold (a later layer of the same pass) instead of storing
   int a0;
   int C, nl, nlm, noutp;
@@ -2320,6 +2323,10 @@ template<class T, int KB, int NL, bool TAB> __global__ __launch_bounds__(256) vo
     px += __shfl_xor(px, 16, 64); p1 += __shfl_xor(p1, 16, 64); p2 += __shfl_xor(p2, 16, 64);
     px += __shfl_xor(px, 32, 64); p1 += __shfl_xor(p1, 32, 64); p2 += __shfl_xor(p2, 32, 64);
     if (lane < nb) {
+      if (a.bsum) {
+        const double *b = a.bsum + 3 * (eb + lane);
+        px += b[0]; p1 += b[1]; p2 += b[2];
+      }
       const double dEdr = px / brc, t1 = p1 / br, t2 = p2 / br;
       const double fv[3] = {dEdr * u0 + t1 * e1[0] + t2 * e2[0], dEdr * u1 + t1 * e1[1] + t2 * e2[1], dEdr * u2 + t1 * e1[2] + t2 * e2[2]};
       for (int d = 0; d < 3; d++) {
