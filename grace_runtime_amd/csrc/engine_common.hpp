@@ -1680,6 +1680,7 @@ class EngineBase : public Engine, protected BufRegistry {
       for (int k = 0; k < nch; k++) {
         const int a0 = k * cs, nc = std::min(n, a0 + cs) - a0;
         const long long eb = bounds.empty() ? 0 : bounds[(size_t) k], ne = bounds.empty() ? nb_ : bounds[(size_t) k + 1] - eb;
+        if (ne <= 0) continue;    // a chunk of isolated atoms
         hipLaunchKernelGGL(k_edge_pairs, dim3((unsigned) ((nc + 3) / 4)), dim3(256), 0, stream_, eoff_.as<long long>(), a0, nc, ej_.as<int>(),
                            rh_.as<double>(), xr_.as<double>(), erow_.as<int>());
         hipLaunchKernelGGL(k_edge_rows, dim3((unsigned) ((ne + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(1024), 0, stream_, eoff_.as<long long>(), a0,

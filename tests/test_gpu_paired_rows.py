@@ -1,7 +1,7 @@
 """Lists with enough bonds for the two directions of a bond to share one row of radial functions (k_edge_pairs): symmetric
 lists, lists in which one direction of a bond is missing, lists that hold bonds twice, bond vectors that were rounded
-differently in the two directions, atoms with more than 80 neighbours, chunks that cut bonds, against the oracle on the
-same list."""
+differently in the two directions, atoms with more than 80 neighbours, chunks that cut bonds, chunks of isolated atoms, against
+the oracle on the same list."""
 import numpy as np
 import pytest
 
@@ -31,16 +31,21 @@ def _list(variant):
         i, j, rij = i[order], j[order], rij[order]
     if variant == "rounded":
         rij = rij * (1.0 + 2e-16 * rng.integers(-2, 3, rij.shape))
-    offset = np.concatenate([[0], np.cumsum(np.bincount(i, minlength=len(pos)))]).astype(np.int64)
+    types = types[perm]
+    if variant == "gas":    # 700 atoms without a neighbour: chunks of 300 atoms that hold no bond, between others and at the end
+        late = i >= 512
+        i, j = i + 700 * late, j + 700 * (j >= 512)
+        types = np.concatenate([types[:512], rng.integers(1, 3, 700).astype(np.int32), types[512:], np.ones(700, np.int32)])
+    offset = np.concatenate([[0], np.cumsum(np.bincount(i, minlength=len(types)))]).astype(np.int64)
     assert len(j) > 32768
-    return types[perm], offset, j.astype(np.int32), rij
+    return types, offset, j.astype(np.int32), rij
 
 
 _oracle = {}
 
 
 @pytest.mark.parametrize("precision,chunk", [(64, 0), (32, 0), (64, 300)])
-@pytest.mark.parametrize("variant", ["plain", "holes", "twice", "rounded", "long"])
+@pytest.mark.parametrize("variant", ["plain", "holes", "twice", "rounded", "long", "gas"])
 @pytest.mark.parametrize("model", ["mix2", "l2mix"])
 def test_shared_rows_equal_the_oracle(model_dir, model, variant, precision, chunk):
     path = cases.model_file(model_dir, model)
