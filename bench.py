@@ -41,14 +41,15 @@ HBM_PEAK = 8000.0                 # GB/s
 # HBM bytes per launch of the dominant kernel measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (two runs of this
 # script, counters scaled by what they read for the 1 GiB copy kernel; summaries under profiles/): (workload, kernel)
 MEASURED_TRAFFIC = {
-    ("config2", "radial_mlp"): 14.3e6 + 1175.4e6,       # fetch + write of k_radial<double,4,0,0,true> (its launches on the full edge list)
-    ("config3", "pair_bwd"): 10754.5e6 + 2764.4e6,      # fetch + write of k_pair_bwd_mfma<double,5,2>
-    ("config4", "pair_bwd_L3"): 44870e6 + 31121e6,      # the layer-3 launches of k_pair_bwd_mfma<double,6,2> (layer 2: 24.5 + 15.6 GB)
-    ("config5", "pair_bwd"): 8993.2e6 + 2467.7e6,       # fetch + write of k_pair_bwd_mfma<double,5,2> over the ragged batch
+    ("config2", "radial_mlp"): 10.9e6 + 585.4e6,        # fetch + write of k_radial<double,4,0,0,true> (one row per pair of atoms)
+    ("config2", "chain_bwd"): 670.3e6 + 52.4e6,
+    ("config3", "pair_bwd"): 10770.7e6 + 3292.8e6,      # fetch + write of k_pair_bwd_mfma<double,5>
+    ("config4", "pair_bwd_L3"): 43831e6 + 30158e6,      # the layer-3 launches of k_pair_bwd_mfma<double,6> (layer 2: 24.2 + 15.1 GB)
+    ("config5", "pair_bwd"): 9670.6e6 + 2934.6e6,       # fetch + write of k_pair_bwd_mfma<double,5> over the ragged batch
 }
 # the per-atom dense chain of configuration 2 (chain_fwd 0.72 GB, k_reduce_fwd 0.19, k_energy < 0.01, k_reduce_bwd 0.19, chain_bwd
-# 0.79 GB: every launch between the A basis and the bond reverse), same counters
-DENSE_TRAFFIC = {"config2": 1.90e9}
+# 0.72 GB: every launch between the A basis and the bond reverse), same counters
+DENSE_TRAFFIC = {"config2": 1.83e9}
 DENSE_PREFIXES = ("fc_", "prod_", "reduce_", "energy_mlp", "zero_grads", "chain_")
 
 
@@ -390,6 +391,8 @@ def run_workload(a, light=False):
                  stream_bytes=couple_stream_bytes(workloads.model_config4(), N, s)) if three else {}
     if a.spline > 0 and not three:
         extra = dict(radial_flops=0.0)    # the radial stages are table look-ups: a stream, not a GEMM
+    elif "edge_pairs" in stages:
+        extra = dict(radial_flops=0.5 * 59392.0)    # the network runs once for both directions of a bond
     # FC / reduce tile GEMMs: flops of the live functions as the engine counts them
     dense_flops = dict(gemm_flops)
     roof = {}
