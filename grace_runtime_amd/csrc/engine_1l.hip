@@ -116,8 +116,7 @@ template<class T> class Engine1L final : public EngineBase {
   bool tables_inside_ = true;  // radial tables evaluated by the kernels that use the radial functions
   // ... where their kernel of the A basis has a form for the channel width; else k_radial_spline writes the rows of the bonds
   bool tables_in_kernels() { return rad_.has_tables() && tables_inside_ && nl_ * (CP_ / 16) <= 10; }
-  bool red_writes_ = false;    // the reverse of the rho reduce may overwrite the adjoints (every function collected at most once)
-  DevReduce<T> redrho_;
+  DevReduces<T> redrho_;
   UqDev<T> uq_{};             // UQ head (models that carry a valid one)
   DevBuf uqR_, uqCen_, uqIcov_, uqNcl_, uqThr_, uqCi_[4];
   DevBuf eW_[7];
@@ -262,12 +261,6 @@ template<class T> void Engine1L<T>::build()
       } else {
         log_message(1, "GRACE-1L: the dense chain runs stage by stage (" + chain_note_ + ")");
       }
-      // the reverse of the rho reduce may write its rows instead of adding to cleared ones when no function is collected twice
-      red_writes_ = true;
-      for (const ReduceWeights *rw : {&m.red_A, &m.red_AA, &m.red_AAA, &m.red_AAAA}) {
-        std::set<int> seen;
-        for (int c : rw->collect_ind) red_writes_ = red_writes_ && seen.insert(c).second;
-      }
     }
     fcA1_.build(m.fc_A1, liveA1, nlm_, CP_, CP_, CFP_, drow_, false, true);    // both inputs are A: one reverse launch
     fcAA1_.build(m.fc_AA1, liveAA1, nlm_, CFP_, CP_, CFP_, drow_);
@@ -285,7 +278,7 @@ template<class T> void Engine1L<T>::build()
     for (int s = 0; s < (order4_ ? 4 : 3); s++)
       src.push_back({&rw[s]->W, rw[s]->norm, rw[s]->n_in, rw[s]->w_shape, &rw[s]->collect_ind, &rw[s]->w_l_tile, nullptr, nfun[s],
                      s == 0 ? CP_ : CFP_});
-    redrho_.build(src, nel_, nrho_, -1, nrho_, 0, drow_);
+    redrho_.build({ReduceSpec{src, nrho_, -1, 0, nrho_, 0}}, nel_, drow_);
   }
 
   // ---- UQ head: a head that does not validate leaves the model usable without UQ (libgrace/src/model_1l.cpp:216-271)
@@ -494,15 +487,7 @@ template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int chunk, int
     }
   }
   stage("reduce_rho", [&] {
-#define GR_RED(KA, KF) hipLaunchKernelGGL((k_reduce_fwd<T, KA, KF>), dim3(ntiles), dim3(64 * kReduceWaves), 0, stream_, redrho_.d, mu, tiles, \
-                                          (const T *) A, (const T *) AA, (const T *) AAA, (const T *) AAAA, rho_.as<double>())
-    switch (ka * 10 + kf) {
-      case 11: GR_RED(1, 1); break; case 12: GR_RED(1, 2); break; case 14: GR_RED(1, 4); break;
-      case 21: GR_RED(2, 1); break; case 22: GR_RED(2, 2); break; case 24: GR_RED(2, 4); break;
-      case 41: GR_RED(4, 1); break; case 42: GR_RED(4, 2); break; case 44: GR_RED(4, 4); break;
-      default: throw Error("unsupported channel widths");
-    }
-#undef GR_RED
+    launch_reduce_fwd<T>(redrho_, ka, kf, mu, A, AA, AAA, AAAA, rho_.as<double>(), nullptr, tiles, ntiles);
   });
   stage("energy_mlp", [&] {
     const size_t lds = (size_t) (4 * (2 * en_.nlay + 4) * en_.width + en_.wlds) * sizeof(double);
@@ -533,19 +518,9 @@ template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int chunk, int
     *gAAA = gAAA_.as<T>(), *gAAAA = gAAAA_.as<T>();
   if (fused) {
     // the reverse of the rho reduce leaves the adjoints of AAA, AAAA and of the collected functions of A and AA; the chain
-    // kernel takes them to the adjoint of A.  Rows the reduce does not visit are not read by it, so nothing is cleared
-    // when the reduce may write its rows.
-    if (!red_writes_)
-      stage("zero_grads", [&] {
-        HIP_CHECK(hipMemsetAsync(gA, 0, na * nlm_ * CP_ * sizeof(T), stream_));
-        HIP_CHECK(hipMemsetAsync(gAA, 0, na * nAA_ * CFP_ * sizeof(T), stream_));
-        HIP_CHECK(hipMemsetAsync(gAAA, 0, na * nAAA_ * CFP_ * sizeof(T), stream_));
-        if (order4_) HIP_CHECK(hipMemsetAsync(gAAAA, 0, na * nAAAA_ * CFP_ * sizeof(T), stream_));
-      });
+    // kernel takes them to the adjoint of A.  The reduce writes its rows and the others are not read, so nothing is cleared.
     stage("reduce_rho_bwd", [&] {
-      if (redrho_.njobs > 0)
-        hipLaunchKernelGGL(k_reduce_bwd<T>, dim3(ntiles, redrho_.njobs), dim3(64), 0, stream_, redrho_.d, mu, tiles, grho_.as<double>(), gA, gAA,
-                           gAAA, gAAAA, 0, red_writes_ ? 1 : 0);
+      launch_reduce_bwd<T>(redrho_, redrho_.all, mu, grho_.as<double>(), nullptr, gA, gAA, gAAA, gAAAA, tiles, ntiles, true);
     });
     int parts = 1;
     stage("chain_bwd", [&] {
@@ -567,12 +542,8 @@ template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int chunk, int
       HIP_CHECK(hipMemsetAsync(gAAAA, 0, na * nAAAA_ * CFP_ * sizeof(T), stream_));
     }
   });
-  const int jobs_a_aa = redrho_.d.ncol[0] + redrho_.d.ncol[1];    // jobs of the sources A and AA (the first two)
   stage("reduce_rho_bwd", [&] {
-    const int first = order4_ ? jobs_a_aa : 0;
-    if (redrho_.njobs > first)
-      hipLaunchKernelGGL(k_reduce_bwd<T>, dim3(ntiles, redrho_.njobs - first), dim3(64), 0, stream_, redrho_.d, mu, tiles, grho_.as<double>(),
-                         gA, gAA, gAAA, gAAAA, first);
+    launch_reduce_bwd<T>(redrho_, order4_ ? redrho_.high : redrho_.all, mu, grho_.as<double>(), nullptr, gA, gAA, gAAA, gAAAA, tiles, ntiles, false);
   });
   // accL / accR: add to the stored adjoint or overwrite it (specialised kernels; the table-driven ones always add)
   auto prod_bwd = [&](const char *name, DevProd &P, const T *L, const T *R, const T *g, T *gL, T *gR, int sl, int sr, int accL, int accR) {
@@ -610,9 +581,7 @@ template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int chunk, int
       launch_gemm(fcAA12_.bwd_r, kf, kf, ka, gAA1, nAA_, gAA2, nAA_, gA, nlm_, 1);
     });
     stage("reduce_rho_bwd_A_AA", [&] {
-      if (jobs_a_aa > 0)
-        hipLaunchKernelGGL(k_reduce_bwd<T>, dim3(ntiles, jobs_a_aa), dim3(64), 0, stream_, redrho_.d, mu, tiles, grho_.as<double>(), gA, gAA,
-                           gAAA, gAAAA, 0);
+      launch_reduce_bwd<T>(redrho_, redrho_.low, mu, grho_.as<double>(), nullptr, gA, gAA, gAAA, gAAAA, tiles, ntiles, false);
     });
   } else {
     fc_bwd("fc_AA1_bwd", fcAA1_, gAA1, gAA, gA, nAA_, kf);

@@ -22,8 +22,7 @@ template<class T> struct Chain {
   DevProd p2, p3, p4;
   // the whole chain as one generated kernel per direction (jit_chain.hpp); not ok(): the stage-by-stage kernels run
   ChainKernels fused;
-  DevBuf fusedW, keepXX;    // fragment-ordered weights; the functions of XX the reduces collect (their adjoint rows are cleared)
-  int nkeepXX = 0;
+  DevBuf fusedW;            // fragment-ordered weights
   bool fuse3 = true;        // P3 = XX1 x X inside the chain kernels (few outputs) or as the product kernels below (many)
   std::string fused_note;
   ~Chain() { fused.release(); }
@@ -72,15 +71,14 @@ template<class T> class Engine2L final : public EngineBase {
   DevBuf zA_, zB0_, ones_, shift_, lnI_, ln0_, eW_[7];
   DevRadial<T> radR_, radR1_;
   Chain<T> c1_, c2_;
-  DevReduce<T> redrho_, redI2_;
+  DevReduces<T> red1_, red2_;    // of layer 1: rho and the functions of I1; of layer 2: I2
   UqDev<T> uq_{};             // UQ head: blocks [I2 (layer 2), rho (layer 1)]
   DevBuf uqR_, uqCen_, uqIcov_, uqNcl_, uqThr_, uqCi_[kUqMaxSrc];
-  std::vector<std::unique_ptr<DevReduce<T>>> redI1_;    // one per output function of I1
   DevBuf WI_, WIT_, WB_, WBT_;
   DevJobs<T> jI_, jIb_, jB_, jBb_;
   Energy2Dev en_{};
   // pass buffers
-  DevBuf sink_, Rz_, dRz_, R1_, dR1_, YG_, A_, rho_, grho_, I1_, gI1_, I1t_, gI1t_, M_, gM_, P_, gP_, B_, I2_, gI2_;
+  DevBuf sink_, Rz_, dRz_, R1_, dR1_, YG_, A_, rho_, grho_, I1_, gI1_, M_, gM_, P_, gP_, B_, I2_, gI2_;
   DevBuf gMe_;    // ordered sums: the message adjoints of a chunk's bonds, [bond][nI][CRP]
   // the chunk of atoms the chain and reduce functions act on: cn_ atoms from a0_, the chunk's element tiles (atoms counted
   // from a0_), the capacity the chunk buffers are sized for
@@ -99,8 +97,8 @@ template<class T> class Engine2L final : public EngineBase {
   void chain_forward(Chain<T> &c, const char *tag, const T *X);
   void chain_zero(Chain<T> &c, const char *tag);
   void chain_backward(Chain<T> &c, const char *tag, const T *X, const std::function<void()> &reduces_x_xx);
-  void reduce_fwd(DevReduce<T> &R, int kb, const Chain<T> &c, const T *X, double *out);
-  void reduce_bwd(DevReduce<T> &R, const Chain<T> &c, const double *g, bool high);
+  void reduce_fwd(DevReduces<T> &R, const Chain<T> &c, const T *X, double *out0, T *out1);
+  void reduce_bwd(DevReduces<T> &R, const Chain<T> &c, const double *g0, const T *g1, bool late);
   std::string tagged(const char *tag, const char *name) { return std::string(name) + tag; }
 };
 
@@ -172,12 +170,6 @@ void Engine2L<T>::build_chain(Chain<T> &c, const char *tag, int nf, int KP, cons
     if (jit_compile_chain(("chain" + t).c_str(), sp, arch_, c.fused, w, c.fused_note)) {
       std::vector<T> wt(w.begin(), w.end());
       upload_vec(c.fusedW, wt);
-      std::vector<int> keep;
-      for (int q = 0; q < c.nXX; q++)
-        if (sp.keepP2[q]) keep.push_back(q);
-      c.nkeepXX = (int) keep.size();
-      if (keep.empty()) keep.push_back(0);
-      upload_vec(c.keepXX, keep);
     } else {
       log_message(1, std::string("GRACE-2L: the dense chain") + tag + " runs stage by stage (" + c.fused_note + ")");
     }
@@ -276,8 +268,13 @@ template<class T> void Engine2L<T>::build()
                    c.nfun(s), KP});
     return v;
   };
-  redrho_.build(sources(m.rho_red, c1_, C1P_, false), nel_, nrho_, -1, nrho_, 0, drow_);
-  redI2_.build(sources(m.I2_red, c2_, C2P_, false), nel_, nrho_, -1, nrho_, 0, drow_);
+  {
+    // a P3 outside the chain kernel adds to the adjoint of any function of X, so all its rows have to be there
+    std::vector<ReduceSpec> specs{ReduceSpec{sources(m.rho_red, c1_, C1P_, false), nrho_, -1, 0, nrho_, 0}};
+    for (int fo = 0; fo < nI1_; fo++) specs.push_back(ReduceSpec{sources(m.I1_red, c1_, C1P_, true), m.I1_n_out, fo, 1, nI1_ * PI1_, fo * PI1_});
+    red1_.build(specs, nel_, drow_, std::vector<char>(c1_.fuse3 ? 0 : c1_.nf, 1));
+    red2_.build({ReduceSpec{sources(m.I2_red, c2_, C2P_, false), nrho_, -1, 0, nrho_, 0}}, nel_, drow_, std::vector<char>(c2_.fuse3 ? 0 : c2_.nf, 1));
+  }
   // ---- UQ head: a head that does not validate leaves the model usable without UQ (libgrace/src/model_2l.cpp:404-478)
   if (m.uq.has_uq) {
     try {
@@ -313,10 +310,6 @@ template<class T> void Engine2L<T>::build()
     }
   } else {
     uq_why_ = "the model file carries none";
-  }
-  for (int fo = 0; fo < nI1_; fo++) {
-    redI1_.emplace_back(new DevReduce<T>());
-    redI1_.back()->build(sources(m.I1_red, c1_, C1P_, true), nel_, m.I1_n_out, fo, nI1_ * PI1_, fo * PI1_, drow_);
   }
   // ---- I from I1 and B from (YI, B0): tile-GEMM job lists (weights not element dependent).  W: [n_out][n_in][w_shape]
   auto tile_frags = [&](const ReduceEq &r, int nout, int KinP, int NoutP, std::vector<T> &F, std::vector<T> &Ft) {
@@ -469,24 +462,14 @@ template<class T> void Engine2L<T>::chain_zero(Chain<T> &c, const char *tag)
 {
   const size_t nc = cap_, KP = c.kb * 16;
   if (c.fused.ok()) {
-    // the reduces add their adjoints to gX, gXXX, gXXXX and to the collected rows of gXX; the chain kernel reads those rows
-    // only and writes gX
+    // the reduces write the rows of gX, gXX, gXXX and gXXXX that are read
     c.gX.ensure(nc * c.nf * KP * sizeof(T));
     c.gXX.ensure(nc * c.nXX * KP * sizeof(T));
     c.gXXX.ensure(nc * c.nXXX * KP * sizeof(T));
     if (c.order4) c.gXXXX.ensure(nc * std::max(c.nXXXX, 1) * KP * sizeof(T));
     if (!c.fuse3) c.gXX1.ensure(nc * c.nXX * KP * sizeof(T));
-    const size_t na = (size_t) cn_;
-    stage(tagged(tag, "zero_grads").c_str(), [&] {
-      HIP_CHECK(hipMemsetAsync(c.gX.p, 0, na * c.nf * KP * sizeof(T), stream_));
-      if (!c.fuse3 && !c.jit_all) HIP_CHECK(hipMemsetAsync(c.gXX1.p, 0, na * c.nXX * KP * sizeof(T), stream_));
-      HIP_CHECK(hipMemsetAsync(c.gXXX.p, 0, na * c.nXXX * KP * sizeof(T), stream_));
-      if (c.order4) HIP_CHECK(hipMemsetAsync(c.gXXXX.p, 0, na * std::max(c.nXXXX, 1) * KP * sizeof(T), stream_));
-      const long long total = (long long) na * c.nkeepXX * (long long) KP;
-      if (total > 0)
-        hipLaunchKernelGGL(k_clear_functions<T>, dim3((unsigned) ((total + 255) / 256)), dim3(256), 0, stream_, c.gXX.template as<T>(), c.nXX, (int) KP,
-                           c.keepXX.template as<int>(), c.nkeepXX, total);
-    });
+    if (!c.fuse3 && !c.jit_all)
+      stage(tagged(tag, "zero_grads").c_str(), [&] { HIP_CHECK(hipMemsetAsync(c.gXX1.p, 0, (size_t) cn_ * c.nXX * KP * sizeof(T), stream_)); });
     return;
   }
   c.gX.ensure(nc * c.nf * KP * sizeof(T));
@@ -513,8 +496,8 @@ template<class T> void Engine2L<T>::chain_zero(Chain<T> &c, const char *tag)
   });
 }
 
-// reverse of the chain; the reduces have added their adjoints to gXXX and gXXXX.  The FC reverse WRITES gXX (no fill, no
-// read of the largest adjoint); reduces_x_xx then adds the reduces' adjoints of X and XX.  Result in c.gX.
+// reverse of the chain; the reduces have left their adjoints (fused chain: of every source; else of XXX and XXXX: the FC
+// reverse WRITES gXX, and reduces_x_xx then adds the reduces' adjoints of X and XX).  Result in c.gX.
 template<class T> void Engine2L<T>::chain_backward(Chain<T> &c, const char *tag, const T *X, const std::function<void()> &reduces_x_xx)
 {
   const int n = cn_, KP = c.kb * 16;
@@ -549,7 +532,6 @@ template<class T> void Engine2L<T>::chain_backward(Chain<T> &c, const char *tag,
   T *gX = c.gX.template as<T>(), *gX1 = c.gX1.template as<T>(), *gXX = c.gXX.template as<T>(), *gXX1 = c.gXX1.template as<T>(),
     *gXXX = c.gXXX.template as<T>(), *gXX2 = c.gXX2.template as<T>(), *gXXXX = c.gXXXX.template as<T>();
   if (c.fused.ok()) {
-    reduces_x_xx();    // the adjoints the reduces leave on X and on the collected functions of XX come first
     if (!c.fuse3) prod_bwd(tagged(tag, "prod_3_bwd"), c.p3, XX1, X, gXXX, gXX1, gX, c.nXX, c.nf, 0, 1);
     int parts = 1;
     stage(tagged(tag, "chain_bwd").c_str(), [&] {
@@ -574,28 +556,18 @@ template<class T> void Engine2L<T>::chain_backward(Chain<T> &c, const char *tag,
   fc_bwd(tagged(tag, "fc_1_bwd"), c.fc1, gX1, gX, gX, c.nf, 1);
 }
 
-template<class T> void Engine2L<T>::reduce_fwd(DevReduce<T> &R, int kb, const Chain<T> &c, const T *X, double *out)
+template<class T> void Engine2L<T>::reduce_fwd(DevReduces<T> &R, const Chain<T> &c, const T *X, double *out0, T *out1)
 {
-  const int *tiles = cur_tiles_;
-#define GR_RED(KA) hipLaunchKernelGGL((k_reduce_fwd<T, KA, KA>), dim3(cur_ntiles_), dim3(64 * kReduceWaves), 0, stream_, R.d, mu_.as<int>() + a0_, tiles, \
-                                      c.src(0, X), c.src(1, X), c.src(2, X), c.src(3, X), out)
-  switch (kb) {
-    case 1: GR_RED(1); break;
-    case 2: GR_RED(2); break;
-    case 4: GR_RED(4); break;
-    default: throw Error("unsupported channel widths");
-  }
-#undef GR_RED
+  EngineBase::launch_reduce_fwd<T>(R, c.kb, c.kb, mu_.as<int>() + a0_, c.src(0, X), c.src(1, X), c.src(2, X), c.src(3, X), out0, out1, cur_tiles_, cur_ntiles_);
 }
 
-// high: the sources XXX and XXXX (before the chain's reverse reads their adjoints); else X and XX (after the FC reverse
-// has written the adjoint of XX)
-template<class T> void Engine2L<T>::reduce_bwd(DevReduce<T> &R, const Chain<T> &c, const double *g, bool high)
+// before the chain's reverse: every adjoint row of a fused chain is written, of the others those of XXX and XXXX are added;
+// after its FC reverse (late): those of X and XX are added
+template<class T> void Engine2L<T>::reduce_bwd(DevReduces<T> &R, const Chain<T> &c, const double *g0, const T *g1, bool late)
 {
-  const int low = R.d.ncol[0] + R.d.ncol[1], first = high ? low : 0, count = high ? R.njobs - low : low;
-  if (count <= 0) return;
-  hipLaunchKernelGGL(k_reduce_bwd<T>, dim3(cur_ntiles_, count), dim3(64), 0, stream_, R.d, mu_.as<int>() + a0_, cur_tiles_, g, c.gsrc(0), c.gsrc(1),
-                     c.gsrc(2), c.gsrc(3), first);
+  const bool fused = c.fused.ok();
+  EngineBase::launch_reduce_bwd<T>(R, fused ? R.all : late ? R.low : R.high, mu_.as<int>() + a0_, g0, g1, c.gsrc(0), c.gsrc(1), c.gsrc(2), c.gsrc(3), cur_tiles_,
+                                   cur_ntiles_, fused);
 }
 
 template<class T> void Engine2L<T>::run(const RunFlags &fl)
@@ -633,7 +605,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
   const int npf = nslot_ * nlm_;
   const double per_atom = sizeof(T) * (chain_values(c1_) + chain_values(c2_) + (double) nlm_ * C1P_ + 2.0 * npf * CRP_ + (double) nB_ * C2P_ +
                                        bonds_per_atom * 2.0 * (radR_.noutp + radR1_.noutp)) +
-                          (2.0 * nI1_ * PI1_ + 2.0 * nrho_) * sizeof(double) + 2.0 * nI1_ * PI1_ * (sizeof(T) == 4 ? 4.0 : 0.0);
+                          2.0 * nI1_ * PI1_ * sizeof(T) + 2.0 * nrho_ * sizeof(double);
   const double kept = bonds_per_atom * ((bsum_on_ ? 84.0 : 60.0) + yw * sizeof(T)) + (double) (nslot_ + nI_) * CRP_ * sizeof(T) + 32.0 * nrho_ + 64.0;
   const int cs = plan_chunk(n, per_atom, kept);
   const int nchunks = (n + cs - 1) / cs;
@@ -688,11 +660,10 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
   if (tab_inside) tbR = radR_.table(stream_, ncu_, xr_.as<double>(), emu_.as<int>(), zA_.as<T>());
   A_.ensure(na * nlm_ * C1P_ * sizeof(T));
   T *A = A_.as<T>();
-  if (I1_.bytes < na * nI1_ * PI1_ * sizeof(double)) {
-    I1_.ensure(na * nI1_ * PI1_ * sizeof(double));
+  if (I1_.bytes < na * nI1_ * PI1_ * sizeof(T)) {
+    I1_.ensure(na * nI1_ * PI1_ * sizeof(T));
     HIP_CHECK(hipMemsetAsync(I1_.p, 0, I1_.bytes, stream_));    // the padding channels stay zero
   }
-  if constexpr (sizeof(T) == 4) I1t_.ensure(na * nI1_ * PI1_ * sizeof(T));
 
   // layer 1 of the current chunk up to its chain (radial rows from row 0 of Rz_ / dRz_; kernels index bonds by their number
   // in the structure)
@@ -716,19 +687,8 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
   for (int q = 0; q < nchunks; q++) {
     set_chunk(q);
     layer1_chain();
-    stage("reduce_rho", [&] { reduce_fwd(redrho_, c1_.kb, c1_, A, rho_.as<double>() + (size_t) a0_ * nrho_); });
-    stage("reduce_I1", [&] {
-      for (auto &r : redI1_) reduce_fwd(*r, c1_.kb, c1_, A, I1_.as<double>());
-    });
-    // I1 leaves the scalar reduce in fp64; the fp32 engine hands the GEMM a copy in fp32
-    const long long nI1v = (long long) cn_ * nI1_ * PI1_;
-    const T *I1t = I1_.as<T>();
-    if constexpr (sizeof(T) == 4) I1t = I1t_.as<T>();
-    stage("reduce_I", [&] {
-      if constexpr (sizeof(T) == 4)
-        hipLaunchKernelGGL((k_convert<double, T>), dim3((unsigned) ((nI1v + 255) / 256)), dim3(256), 0, stream_, I1_.as<double>(), I1t_.as<T>(), nI1v);
-      gemm(jI_, PI1_ / 16, CRP_ / 16, I1t, nI1_, M + (size_t) a0_ * nslot_ * CRP_, nslot_, 0);
-    });
+    stage("reduce_rho_I1", [&] { reduce_fwd(red1_, c1_, A, rho_.as<double>() + (size_t) a0_ * nrho_, I1_.as<T>()); });
+    stage("reduce_I", [&] { gemm(jI_, PI1_ / 16, CRP_ / 16, (const T *) I1_.as<T>(), nI1_, M + (size_t) a0_ * nslot_ * CRP_, nslot_, 0); });
   }
   stage("fill_slot", [&] {
     hipLaunchKernelGGL(k_fill_slot<T>, dim3((unsigned) ((nnodes * CRP_ + 255) / 256)), dim3(256), 0, stream_, mu_.as<int>(), zB0_.as<T>(), M, n_nodes_,
@@ -823,7 +783,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     });
     stage("reduce_B", [&] { gemm(jB_, CRP_ / 16, C2P_ / 16, P, npf, B, nB_, 0); });
     chain_forward(c2_, "_L2", B);
-    stage("reduce_I2", [&] { reduce_fwd(redI2_, c2_.kb, c2_, B, I2_.as<double>()); });
+    stage("reduce_I2", [&] { reduce_fwd(red2_, c2_, B, I2_.as<double>(), nullptr); });
     if (fl.uq) {
       if (nchunks > 1) layer1_chain();    // the head reads layer 1's tensors of these atoms as well
       stage("uq", [&] {
@@ -847,8 +807,8 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     if (!forces) continue;
     // layer 2 reverse: dE/dB -> dE/dP -> bond forces of layer 2 and dE/dI of the neighbours
     chain_zero(c2_, "_L2");
-    stage("reduce_I2_bwd", [&] { reduce_bwd(redI2_, c2_, gI2_.as<double>(), true); });
-    chain_backward(c2_, "_L2", B, [&] { stage("reduce_I2_bwd_X_XX", [&] { reduce_bwd(redI2_, c2_, gI2_.as<double>(), false); }); });
+    stage("reduce_I2_bwd", [&] { reduce_bwd(red2_, c2_, gI2_.as<double>(), nullptr, false); });
+    chain_backward(c2_, "_L2", B, [&] { stage("reduce_I2_bwd_X_XX", [&] { reduce_bwd(red2_, c2_, gI2_.as<double>(), nullptr, true); }); });
     stage("reduce_B_bwd", [&] { gemm(jBb_, C2P_ / 16, CRP_ / 16, c2_.gX.template as<T>(), nB_, gP_.as<T>(), npf, 0); });    // gP: every row is written
     stage("pair_bwd", [&] {
       // fp32: the next chunk is copied to a second LDS buffer while this one is worked on (chunks of 8 bonds in the large
@@ -906,33 +866,16 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
   exchange_reverse(1);
 
   // ---- sweep 3: layer 1 reverse
-  gI1_.ensure(na * nI1_ * PI1_ * sizeof(double));
-  if constexpr (sizeof(T) == 4) gI1t_.ensure(na * nI1_ * PI1_ * sizeof(T));
+  gI1_.ensure(na * nI1_ * PI1_ * sizeof(T));
   for (int q = 0; q < nchunks; q++) {
     set_chunk(q);
     if (nchunks > 1) layer1_chain();
-    const long long nI1v = (long long) cn_ * nI1_ * PI1_;
     const T *gMc = gM_.as<T>() + (size_t) a0_ * nI_ * CRP_;
     const double *grho = grho_.as<double>() + (size_t) a0_ * nrho_;
     chain_zero(c1_, "_L1");
-    stage("reduce_I_bwd", [&] {
-      if constexpr (sizeof(T) == 4) {
-        gemm(jIb_, CRP_ / 16, PI1_ / 16, gMc, nI_, gI1t_.as<T>(), nI1_, 0);
-        hipLaunchKernelGGL((k_convert<T, double>), dim3((unsigned) ((nI1v + 255) / 256)), dim3(256), 0, stream_, gI1t_.as<T>(), gI1_.as<double>(), nI1v);
-      } else {
-        gemm(jIb_, CRP_ / 16, PI1_ / 16, gMc, nI_, gI1_.as<T>(), nI1_, 0);
-      }
-    });
-    stage("reduce_rho_bwd", [&] { reduce_bwd(redrho_, c1_, grho, true); });
-    stage("reduce_I1_bwd", [&] {
-      for (auto &r : redI1_) reduce_bwd(*r, c1_, gI1_.as<double>(), true);
-    });
-    chain_backward(c1_, "_L1", A, [&] {
-      stage("reduce_rho_bwd_X_XX", [&] { reduce_bwd(redrho_, c1_, grho, false); });
-      stage("reduce_I1_bwd_X_XX", [&] {
-        for (auto &r : redI1_) reduce_bwd(*r, c1_, gI1_.as<double>(), false);
-      });
-    });
+    stage("reduce_I_bwd", [&] { gemm(jIb_, CRP_ / 16, PI1_ / 16, gMc, nI_, gI1_.as<T>(), nI1_, 0); });
+    stage("reduce_rho_I1_bwd", [&] { reduce_bwd(red1_, c1_, grho, gI1_.as<T>(), false); });
+    chain_backward(c1_, "_L1", A, [&] { stage("reduce_rho_I1_bwd_X_XX", [&] { reduce_bwd(red1_, c1_, grho, gI1_.as<T>(), true); }); });
     BondBwdArgs<T> ba{};
     ba.eoff = eoff_.as<long long>(); ba.ej = ej_.as<int>(); ba.rh = rh_.as<double>(); ba.r = r_.as<double>(); ba.rc = rc_.as<double>();
     ba.Rz = moved_back(Rz_.as<T>(), eb * radR_.noutp); ba.dRz = moved_back(dRz_.as<T>(), eb * radR_.noutp); ba.gA = c1_.gX.template as<T>();

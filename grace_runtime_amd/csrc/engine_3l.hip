@@ -282,7 +282,7 @@ template<class T> struct Layer3 {
   }
   DevBuf eq_dw, eq_mask, eq_aff, eq_grp;
   EqNormDev eqn{};
-  DevReduce<T> rho;
+  DevReduces<T> rho;
   // forward tensors kept for the reverse
   DevBuf R, dR;
   Ten X, L2, R2p, L3, R3p, L4, R4p, EQ, I;
@@ -750,7 +750,7 @@ template<class T> void Engine3L<T>::build_layer(int k)
       }
       v.push_back({W, ins.norm, ins.n_in, ins.w_shape, &ins.collect_ind, &ins.w_l_tile, nullptr, src_nf[s], s == 0 ? L.X.w : L.wR});
     }
-    L.rho.build(v, nel_, nrho_, -1, nrho_, 0, drow_);
+    L.rho.build({ReduceSpec{v, nrho_, -1, 0, nrho_, 0}}, nel_, drow_);
   }
 }
 
@@ -1001,22 +1001,8 @@ template<class T> void Engine3L<T>::layer_forward(int k, bool forces, int yw, bo
   (void) nX;
   if (again) return;    // the densities, the energy and the UQ rows come from the first forward pass
   stage(tg(k, "reduce_rho").c_str(), [&] {
-    const int *tiles = cur_tiles_;
-#define GR_RED(KA, KF) hipLaunchKernelGGL((k_reduce_fwd<T, KA, KF>), dim3(cur_ntiles_), dim3(64 * kReduceWaves), 0, stream_, L.rho.d, mu, tiles, srcs[0], srcs[1], \
-                                          srcs[2], srcs[3], L.rho_raw.template as<double>() + (size_t) a0_ * nrho_)
-    switch ((wX / 16) * 10 + wR / 16) {
-      case 11: GR_RED(1, 1); break;
-      case 12: GR_RED(1, 2); break;
-      case 14: GR_RED(1, 4); break;
-      case 21: GR_RED(2, 1); break;
-      case 22: GR_RED(2, 2); break;
-      case 24: GR_RED(2, 4); break;
-      case 41: GR_RED(4, 1); break;
-      case 42: GR_RED(4, 2); break;
-      case 44: GR_RED(4, 4); break;
-      default: throw Error("unsupported channel widths");
-    }
-#undef GR_RED
+    launch_reduce_fwd<T>(L.rho, wX / 16, wR / 16, mu, srcs[0], srcs[1], srcs[2], srcs[3], L.rho_raw.template as<double>() + (size_t) a0_ * nrho_, nullptr,
+                         cur_tiles_, cur_ntiles_);
   });
   if (uq_on_) {    // this layer's rows of the basis while its tensors exist; the last layer finishes the GMM (fused_3l.cpp:1158-1201)
     stage(tg(k, "uq").c_str(), [&] {
@@ -1095,9 +1081,7 @@ template<class T> void Engine3L<T>::layer_backward(int k, int yw)
     });
   }
   stage(tg(k, "reduce_rho_bwd").c_str(), [&] {
-    if (L.rho.njobs)
-      hipLaunchKernelGGL(k_reduce_bwd<T>, dim3(cur_ntiles_, L.rho.njobs), dim3(64), 0, stream_, L.rho.d, mu, cur_tiles_,
-                         (const double *) L.grho.template as<double>() + (size_t) a0_ * nrho_, gX, gR2, gR3, gR4);
+    launch_reduce_bwd<T>(L.rho, L.rho.all, mu, L.grho.template as<double>() + (size_t) a0_ * nrho_, nullptr, gX, gR2, gR3, gR4, cur_tiles_, cur_ntiles_, false);
   });
   // gXL / gXR: where the adjoints of the product's inputs are added; first_left: gXL has no other part yet (a joined launch
   // sets it; else it was cleared)

@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <atomic>
 #include <functional>
+#include <map>
 #include <mutex>
 #include <cmath>
 #include <cstring>
@@ -607,62 +608,136 @@ struct ReduceSrc {
   int nfun, ninp;                                            // functions of the source tensor, its padded channel width
 };
 
-// Element-dependent reduce of up to 4 sources into `nout` channels of ONE output function (fused_cpu.h:1202-1273 of the
-// reference): weights per collected function in MFMA fragment order, for k_reduce_fwd / k_reduce_bwd.
-// fo >= 0 keeps the connections whose output function is fo.
-template<class T> struct DevReduce {
-  DevBuf WF[4], WB[4], Fn[4];
-  ReduceDev<T> d{};
-  int njobs = 0;
-  void build(const std::vector<ReduceSrc> &src, int nel, int nout, int fo, int ostride, int ooff, const int *drow)
+// functions of source w that the reduce collects (fo >= 0: through the connections whose output function is fo)
+inline std::vector<int> reduce_functions(const ReduceSrc &w, int fo)
+{
+  std::vector<int> fn;
+  for (size_t c = 0; c < w.collect_ind->size(); c++)
+    if (fo < 0 || !w.out_fn || (*w.out_fn)[c] == fo) fn.push_back((*w.collect_ind)[c]);
+  std::sort(fn.begin(), fn.end());
+  fn.erase(std::unique(fn.begin(), fn.end()), fn.end());
+  return fn;
+}
+// M[n][k] of function fn for element mu: the sum of its connections' weight tiles
+inline void reduce_matrix(const ReduceSrc &w, int fo, int fn, int mu, int nout, std::vector<double> &M)
+{
+  const int nin = w.n_in;
+  M.assign((size_t) nin * nout, 0.0);
+  for (size_t c = 0; c < w.collect_ind->size(); c++) {
+    if ((*w.collect_ind)[c] != fn || (fo >= 0 && w.out_fn && (*w.out_fn)[c] != fo)) continue;
+    const int tile = (*w.w_l_tile)[c];
+    for (int k = 0; k < nout; k++)
+      for (int n = 0; n < nin; n++) M[(size_t) n * nout + k] += w.norm * (*w.W)[(((size_t) mu * nout + k) * nin + n) * w.w_shape + tile];
+  }
+}
+
+// One element-dependent reduce of a set: up to 4 sources into `nout` channels of ONE output function
+// (fused_cpu.h:1202-1273 of the reference).  fo >= 0 keeps the connections whose output function is fo.  sel: array of the
+// result (0: fp64 rows, 1: rows of the engine's type), ostride / ooff: its row in that array.
+struct ReduceSpec {
+  std::vector<ReduceSrc> src;
+  int nout = 0, fo = -1, sel = 0, ostride = 0, ooff = 0;
+};
+
+// Reduces that read the same tensors: one launch forward, one launch in the reverse, where every adjoint row is visited once
+// whatever number of reduces feed it (k_reduce_fwd, k_reduce_bwd).
+template<class T> struct DevReduces {
+  std::vector<std::unique_ptr<DevBuf>> bufs;
+  std::vector<ReduceDev<T>> d;
+  int max_jobs = 0;    // collected functions of the longest reduce
+  // reverse: rows of the sources s >= 2, and of s < 2, and all of them.  A list is a sequence of launches (rows fed by more
+  // than two reduces take a second one, which adds)
+  struct List {
+    std::vector<ReduceBwdJob> host;
+    DevBuf dev;
+  };
+  std::vector<std::unique_ptr<List>> high, low, all;
+  DevBuf WB;
+  RowMap drow{};
+
+  // cover: functions of source 0 whose adjoint row the list `all` writes although no reduce collects them
+  void build(const std::vector<ReduceSpec> &specs, int nel, const int *drow_, const std::vector<char> &cover = {})
   {
-    d.nsrc = (int) src.size();
-    d.nrho = nout;
-    d.nbr = (nout + 15) / 16;
-    d.ksr = (nout + 3) / 4;
-    d.ostride = ostride;
-    d.ooff = ooff;
-    if (nout > 32) throw Error("reduce widths above 32 are not supported by the GPU reduce kernels");
-    for (int q = 0; q < 16; q++) d.drow[q] = drow[q];
-    const int krp = d.ksr * 4;
-    njobs = 0;
-    for (int s = 0; s < d.nsrc; s++) {
-      const ReduceSrc &w = src[s];
-      std::vector<int> fn;
-      for (size_t c = 0; c < w.collect_ind->size(); c++)
-        if (fo < 0 || !w.out_fn || (*w.out_fn)[c] == fo) fn.push_back((*w.collect_ind)[c]);
-      std::sort(fn.begin(), fn.end());
-      fn.erase(std::unique(fn.begin(), fn.end()), fn.end());
-      const int nc = (int) fn.size(), nin = w.n_in;
-      std::vector<T> vF, vB;
-      std::vector<double> M((size_t) nin * nout), Mt((size_t) nout * nin);
-      for (int mu = 0; mu < nel; mu++)
-        for (int u = 0; u < nc; u++) {
-          std::fill(M.begin(), M.end(), 0.0);
-          for (size_t c = 0; c < w.collect_ind->size(); c++) {
-            if ((*w.collect_ind)[c] != fn[u]) continue;
-            if (fo >= 0 && w.out_fn && (*w.out_fn)[c] != fo) continue;
-            const int tile = (*w.w_l_tile)[c];
-            for (int k = 0; k < nout; k++)
-              for (int n = 0; n < nin; n++)
-                M[(size_t) n * nout + k] += w.norm * (*w.W)[(((size_t) mu * nout + k) * nin + n) * w.w_shape + tile];
+    for (int q = 0; q < 16; q++) drow.r[q] = drow_[q];
+    const int ns = specs.empty() ? 0 : (int) specs[0].src.size();
+    std::map<std::pair<int, int>, std::vector<int>> fed;    // (source, function) -> the reduces that collect it
+    std::vector<double> M, Mt;
+    for (size_t r = 0; r < specs.size(); r++) {
+      const ReduceSpec &sp = specs[r];
+      if (sp.nout > 32) throw Error("reduce widths above 32 are not supported by the GPU reduce kernels");
+      ReduceDev<T> x{};
+      x.nsrc = ns;
+      x.nrho = sp.nout;
+      x.nbr = (sp.nout + 15) / 16;
+      x.sel = sp.sel;
+      x.ostride = sp.ostride;
+      x.ooff = sp.ooff;
+      for (int q = 0; q < 16; q++) x.drow[q] = drow_[q];
+      int jobs = 0;
+      for (int s = 0; s < ns; s++) {
+        const ReduceSrc &w = sp.src[s];
+        const std::vector<int> fn = reduce_functions(w, sp.fo);
+        std::vector<T> vF;
+        for (int mu = 0; mu < nel; mu++)
+          for (int f : fn) {
+            reduce_matrix(w, sp.fo, f, mu, sp.nout, M);
+            pack_fragments<T>(M, w.n_in, sp.nout, w.ninp, x.nbr * 16, vF);    // X[atom][n] . M[n][k]
           }
-          for (int k = 0; k < nout; k++)
-            for (int n = 0; n < nin; n++) Mt[(size_t) k * nin + n] = M[(size_t) n * nout + k];
-          pack_fragments<T>(M, nin, nout, w.ninp, d.nbr * 16, vF);      // X[atom][n] . M[n][k]
-          pack_fragments<T>(Mt, nout, nin, krp, w.ninp, vB, true);       // g[atom][k] . Mt[k][n]
-        }
-      upload_vec(WF[s], vF);
-      upload_vec(WB[s], vB);
-      upload_vec(Fn[s], fn);
-      d.WF[s] = WF[s].template as<T>();
-      d.WB[s] = WB[s].template as<T>();
-      d.fn[s] = Fn[s].template as<int>();
-      d.ncol[s] = nc;
-      d.nin[s] = w.ninp;
-      d.stride[s] = w.nfun;
-      njobs += nc;
+        for (int f : fn) fed[{s, f}].push_back((int) r);
+        bufs.emplace_back(new DevBuf());
+        upload_vec(*bufs.back(), vF);
+        x.WF[s] = bufs.back()->template as<T>();
+        bufs.emplace_back(new DevBuf());
+        upload_vec(*bufs.back(), fn);
+        x.fn[s] = bufs.back()->template as<int>();
+        x.ncol[s] = (int) fn.size();
+        x.nin[s] = w.ninp;
+        x.stride[s] = w.nfun;
+        jobs += (int) fn.size();
+      }
+      max_jobs = std::max(max_jobs, jobs);
+      d.push_back(x);
     }
+    // reverse: g[atom][k] . W[k][n], weights [job][mu][con][cb < 2][step < 8][lane]
+    std::vector<T> vB;
+    auto add_rows = [&](int s, int f, const std::vector<int> &reds) {
+      const ReduceSrc &w0 = specs[0].src[s];
+      for (int cb0 = 0; cb0 < w0.ninp / 16; cb0 += 2)
+        for (size_t first = 0, round = 0; first == 0 || first < reds.size(); first += 2, round++) {
+          ReduceBwdJob j{};
+          j.s = s; j.fn = f; j.nin = w0.ninp; j.stride_out = w0.nfun; j.cb0 = cb0; j.nb = std::min(2, w0.ninp / 16 - cb0);
+          j.ncon = (int) std::min<size_t>(2, reds.size() - first);
+          j.w = (long long) vB.size();
+          j.wmu = (long long) j.ncon * 2 * 8 * 64;
+          vB.resize(vB.size() + (size_t) nel * j.wmu, (T) 0);
+          for (int q = 0; q < j.ncon; q++) {
+            const ReduceSpec &sp = specs[reds[first + q]];
+            j.sel[q] = sp.sel; j.stride[q] = sp.ostride; j.off[q] = sp.ooff; j.nout[q] = sp.nout; j.nks[q] = (sp.nout + 3) / 4;
+            for (int mu = 0; mu < nel; mu++) {
+              reduce_matrix(sp.src[s], sp.fo, f, mu, sp.nout, M);
+              for (int cb = 0; cb < j.nb; cb++)
+                for (int k4 = 0; k4 < j.nks[q]; k4++)
+                  for (int lane = 0; lane < 64; lane++) {
+                    const int k = 4 * k4 + (lane >> 4), n = (cb0 + cb) * 16 + (lane & 15);
+                    if (k < sp.nout && n < sp.src[s].n_in)
+                      vB[(size_t) (j.w + mu * j.wmu + ((q * 2 + cb) * 8 + k4) * 64 + lane)] = (T) M[(size_t) n * sp.nout + k];
+                  }
+            }
+          }
+          auto put = [&](std::vector<std::unique_ptr<List>> &l) {
+            while (l.size() <= round) l.emplace_back(new List());
+            l[round]->host.push_back(j);
+          };
+          put(all);
+          if (j.ncon > 0) put(s >= 2 ? high : low);
+        }
+    };
+    for (const auto &kv : fed) add_rows(kv.first.first, kv.first.second, kv.second);
+    for (size_t f = 0; f < cover.size(); f++)
+      if (cover[f] && !fed.count({0, (int) f})) add_rows(0, (int) f, {});
+    upload_vec(WB, vB);
+    for (auto *l : {&high, &low, &all})
+      for (auto &x : *l) upload_vec(x->dev, x->host);
   }
 };
 
@@ -1477,6 +1552,53 @@ class EngineBase : public Engine, protected BufRegistry {
                        ck.keep0, ck.nf0, ck.C, total, gX0);
   }
   DevBuf chain_part_;
+
+  // ---- element-dependent reduces ------------------------------------------------------------------------------
+  // The forward of a set: results to out0 (fp64 rows) and out1 (rows of T).  Few tiles: the functions of a reduce go to several
+  // blocks, as long as those fill the chip no more than twice, and k_reduce_sum (5 us) adds their parts (128 atoms of GRACE-1L: 34
+  // -> 11 us; the six reduces of GRACE-2L with 107 atoms: 69 -> 21 us in two sets; 251 tiles in two parts: 44 -> 41 us; 512 tiles:
+  // 75 us whole, 74 + 5 in parts).  One part with ordered sums, whose bits must not follow the number of tiles.
+  template<class T> void launch_reduce_fwd(DevReduces<T> &R, int ka, int kf, const int *mu, const T *X0, const T *X1, const T *X2, const T *X3, double *out0,
+                                           T *out1, const int *tiles, int ntiles)
+  {
+    if (ntiles == 0) return;
+    for (size_t first = 0; first < R.d.size(); first += kReduceSet) {
+      const int nr = (int) std::min<size_t>(kReduceSet, R.d.size() - first);
+      ReduceSet<T> set{};
+      std::copy(R.d.begin() + first, R.d.begin() + first + nr, set.r);
+      const int most = std::max(1, (R.max_jobs + kReduceWaves - 1) / kReduceWaves);
+      const int parts = ordered_ ? 1 : std::max(1, std::min(most, 2 * ncu_ / (nr * ntiles)));
+      if (parts > 1) red_part_.ensure((size_t) nr * ntiles * parts * 16 * 32 * sizeof(double));
+#define GR_RED(KA, KF)                                                                                                                      \
+  hipLaunchKernelGGL((k_reduce_fwd<T, KA, KF>), dim3(ntiles, nr, parts), dim3(64 * kReduceWaves), 0, stream_, set, mu, tiles, X0, X1, X2, X3, out0, out1, \
+                     parts, red_part_.as<double>())
+      switch (ka * 10 + kf) {
+        case 11: GR_RED(1, 1); break; case 12: GR_RED(1, 2); break; case 14: GR_RED(1, 4); break;
+        case 21: GR_RED(2, 1); break; case 22: GR_RED(2, 2); break; case 24: GR_RED(2, 4); break;
+        case 41: GR_RED(4, 1); break; case 42: GR_RED(4, 2); break; case 44: GR_RED(4, 4); break;
+        default: throw Error("unsupported channel widths");
+      }
+#undef GR_RED
+      if (parts > 1)
+        hipLaunchKernelGGL(k_reduce_sum<T>, dim3(ntiles, nr), dim3(512), 0, stream_, set, tiles, (const double *) red_part_.as<double>(), parts, out0, out1);
+    }
+  }
+  // The reverse of a set, rows of `list`: added to the adjoints, or (overwrite) written.  Tiles of a wave: as many as leave
+  // 16 waves per SIMD to deal out, eight at most.  As a launch per reduce with a wave per row and tile, added to cleared rows:
+  // GRACE-2L with 32 000 atoms 0.96 ms in 12 launches + 0.29 ms of fills, now 0.46 ms in two; 107 atoms 106 -> 14 us; GRACE-1L, one
+  // reduce: 8192 atoms 75 -> 55 us, 65 536 in fp32 470 -> 305 (389 with a tile per wave, 310 with 4 or 16 for all).
+  template<class T> void launch_reduce_bwd(DevReduces<T> &R, std::vector<std::unique_ptr<typename DevReduces<T>::List>> &list, const int *mu, const double *g0,
+                                           const T *g1, T *G0, T *G1, T *G2, T *G3, const int *tiles, int ntiles, bool overwrite)
+  {
+    for (size_t q = 0; q < list.size(); q++) {
+      const int njobs = (int) list[q]->host.size();
+      if (njobs == 0 || ntiles == 0) continue;
+      const int tpw = std::max(1, std::min(8, (int) ((long long) njobs * ntiles / (64 * ncu_))));
+      hipLaunchKernelGGL(k_reduce_bwd<T>, dim3(njobs, (ntiles + 4 * tpw - 1) / (4 * tpw)), dim3(256), 0, stream_, list[q]->dev.template as<ReduceBwdJob>(),
+                         R.WB.template as<T>(), R.drow, mu, tiles, ntiles, tpw, g0, g1, G0, G1, G2, G3, overwrite && q == 0 ? 1 : 0);
+    }
+  }
+  DevBuf red_part_;
 
   // ---- exchange with ghost atoms ------------------------------------------------------------------------------
   void exchange_forward(int layer)

@@ -1712,109 +1712,169 @@ template<class T> __global__ void k_prod_bwd(ProdDev P, int side, const T *other
 
 template<class T> struct ReduceDev {
   // per source s: collected functions fn[s][c] (unique), weights in fragment order
-  //   forward WF[s][mu][c][cb][ks][lane]  = W_s[mu][c][n = frag_k(g, ks)][k = cb 16 + lane % 16] (norm folded, k >= nrho zero)
-  //   reverse WB[s][mu][c][cb][ks][lane]  = W_s[mu][c][n = cb 16 + lane % 16][k = g KSR + ks]
-  const T *WF[4], *WB[4];
+  //   WF[s][mu][c][cb][ks][lane]  = W_s[mu][c][n = frag_k(g, ks)][k = cb 16 + lane % 16] (norm folded, k >= nrho zero)
+  const T *WF[4];
   const int *fn[4];
   int ncol[4], nin[4], stride[4];    // collected functions, (padded) channels, functions per atom of the source
-  int nsrc, nrho, nbr, ksr;          // rho width, its 16-column blocks, k-steps of the reverse (ceil(nrho / 4))
-  int ostride, ooff;                 // output row of an atom: rho[atom * ostride + ooff + k]
+  int nsrc, nrho, nbr;               // width of the result, its 16-column blocks
+  int sel, ostride, ooff;            // array of the result (0: fp64 rows, 1: rows of T) and its row: array[atom * ostride + ooff + k]
   int drow[16];                      // accumulator row of (lane / 16, register)
 };
+constexpr int kReduceSet = 8;        // reduces of one launch
+template<class T> struct ReduceSet { ReduceDev<T> r[kReduceSet]; };
 
-// rho[atom][k] = sum_s sum_c sum_n W_s[mu][c][n][k] X_s[atom][fn c][n] on the matrix cores: one block per tile of
-// 16 atoms, its kReduceWaves waves split the (s, c) list, partial tiles summed through LDS.  KBA / KBF: 16-channel blocks of
-// source 0 (A) and of the other sources.
-constexpr int kReduceWaves = 8;    // waves of a k_reduce_fwd block: each takes every eighth collected function
+// out[atom][k] = sum_s sum_c sum_n W_s[mu][c][n][k] X_s[atom][fn c][n] on the matrix cores.  Grid (tiles of 16 atoms, reduces
+// of the set, parts): the kReduceWaves waves of the `nparts` blocks of a (tile, reduce) split its (s, c) list, partial tiles are
+// summed through LDS; with several parts they go to part_sums [reduce][part][tile][16][32] and k_reduce_sum adds them.
+// KBA / KBF: 16-channel blocks of source 0 (A) and of the other sources.
+// A wave waits some 2 us for the operands of one collected function, so what bounds few atoms is the length of a wave's
+// list: 89 functions over one block of eight waves took 34 us with 128 atoms.
+constexpr int kReduceWaves = 8;    // waves of a k_reduce_fwd block
 template<class T, int KBA, int KBF>
-__global__ __launch_bounds__(64 * kReduceWaves) void k_reduce_fwd(ReduceDev<T> R, const int *mu, const int *tile_atoms, const T *X0, const T *X1,
-                                                    const T *X2, const T *X3, double *rho)
+__global__ __launch_bounds__(64 * kReduceWaves) void k_reduce_fwd(ReduceSet<T> set, const int *mu, const int *tile_atoms, const T *X0, const T *X1,
+                                                    const T *X2, const T *X3, double *out0, T *out1, int nparts, double *part_sums)
 {
   typedef typename Mfma<T>::v4 v4;
+  constexpr int KSM = (KBA > KBF ? KBA : KBF) * 4;
   __shared__ double part[kReduceWaves][2][16][17];
+  const ReduceDev<T> &R = set.r[blockIdx.y];
   const int tile = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, g = lane >> 4;
   const int arow = tile_atoms[tile * 16 + c];
   const int a0 = tile_atoms[tile * 16];
   const int m = mu[a0];
   const T *X[4] = {X0, X1, X2, X3};
   v4 acc[2] = {v4{0, 0, 0, 0}, v4{0, 0, 0, 0}};
-  int job = 0;
-  for (int s = 0; s < R.nsrc; s++) {
+  int s = 0, cc = wave + kReduceWaves * blockIdx.z;
+  while (true) {
+    while (s < R.nsrc && cc >= R.ncol[s]) cc -= R.ncol[s++];
+    if (s >= R.nsrc) break;
     const int ks = (s == 0 ? KBA : KBF) * 4, K = ks * 4;
-    for (int cc = 0; cc < R.ncol[s]; cc++, job++) {
-      if (job % kReduceWaves != wave) continue;
-      const T *wf = R.WF[s] + ((long long) m * R.ncol[s] + cc) * R.nbr * ks * 64 + lane;
-      T x[(KBA > KBF ? KBA : KBF) * 4];
-      if (arow >= 0) {
-        const T *xp = X[s] + ((long long) arow * R.stride[s] + R.fn[s][cc]) * K;
+    const T *wf = R.WF[s] + ((long long) m * R.ncol[s] + cc) * R.nbr * ks * 64 + lane;
+    T x[KSM];
+    if (arow >= 0) {
+      const T *xp = X[s] + ((long long) arow * R.stride[s] + R.fn[s][cc]) * K;
 #pragma unroll
-        for (int q = 0; q < (KBA > KBF ? KBA : KBF) * 4; q++) x[q] = q < ks ? xp[frag_k<T>(g, q)] : (T) 0;
-      } else {
+      for (int q = 0; q < KSM; q++) x[q] = q < ks ? xp[frag_k<T>(g, q)] : (T) 0;
+    } else {
 #pragma unroll
-        for (int q = 0; q < (KBA > KBF ? KBA : KBF) * 4; q++) x[q] = (T) 0;
-      }
-#pragma unroll
-      for (int cb = 0; cb < 2; cb++)
-        if (cb < R.nbr) {
-#pragma unroll
-          for (int q = 0; q < (KBA > KBF ? KBA : KBF) * 4; q++)
-            if (q < ks) acc[cb] = Mfma<T>::mma(x[q], wf[(cb * ks + q) * 64], acc[cb]);
-        }
+      for (int q = 0; q < KSM; q++) x[q] = (T) 0;
     }
+#pragma unroll
+    for (int cb = 0; cb < 2; cb++)
+      if (cb < R.nbr) {
+#pragma unroll
+        for (int q = 0; q < KSM; q++)
+          if (q < ks) acc[cb] = Mfma<T>::mma(x[q], wf[(cb * ks + q) * 64], acc[cb]);
+      }
+    cc += kReduceWaves * nparts;
   }
 #pragma unroll
   for (int cb = 0; cb < 2; cb++)
 #pragma unroll
     for (int v = 0; v < 4; v++) part[wave][cb][R.drow[4 * g + v]][c] = (double) acc[cb][v];
   __syncthreads();
+  double *sums = part_sums + (((long long) blockIdx.y * nparts + blockIdx.z) * gridDim.x + tile) * (16 * 32);
   for (int e = threadIdx.x; e < 16 * R.nrho; e += 64 * kReduceWaves) {
     const int r = e / R.nrho, k = e % R.nrho;
     const int at = tile_atoms[tile * 16 + r];
     if (at < 0) continue;
     double v = 0.0;
     for (int w = 0; w < kReduceWaves; w++) v += part[w][k >> 4][r][k & 15];
-    rho[(long long) at * R.ostride + R.ooff + k] = v;
+    const long long to = (long long) at * R.ostride + R.ooff + k;
+    if (nparts > 1) sums[r * 32 + k] = v;
+    else if (R.sel == 0) out0[to] = v;
+    else out1[to] = (T) v;
   }
 }
 
-// gX_s[atom][fn c][n] += sum_k grho[atom][k] W_s[mu][c][n][k]: grid (tiles, jobs), one wave per block; the jobs are all
-// (s, c) in the order of the sources, this launch takes those from job_first on.  overwrite: the rows are written, not
-// added to (for callers that know every row is visited once and read no row that is not visited)
+// the parts of k_reduce_fwd, added in their order: grid (tiles, reduces of the set), 512 threads
 template<class T>
-__global__ __launch_bounds__(64) void k_reduce_bwd(ReduceDev<T> R, const int *mu, const int *tile_atoms, const double *grho, T *G0, T *G1,
-                                                   T *G2, T *G3, int job_first = 0, int overwrite = 0)
+__global__ __launch_bounds__(512) void k_reduce_sum(ReduceSet<T> set, const int *tile_atoms, const double *part_sums, int nparts, double *out0, T *out1)
+{
+  const ReduceDev<T> &R = set.r[blockIdx.y];
+  const int tile = blockIdx.x, r = threadIdx.x >> 5, k = threadIdx.x & 31;
+  const int at = tile_atoms[tile * 16 + r];
+  if (at < 0 || k >= R.nrho) return;
+  const double *p = part_sums + ((long long) blockIdx.y * nparts * gridDim.x + tile) * (16 * 32) + threadIdx.x;
+  double v = 0.0;
+#pragma unroll 4
+  for (int q = 0; q < nparts; q++) v += p[(long long) q * gridDim.x * (16 * 32)];
+  const long long to = (long long) at * R.ostride + R.ooff + k;
+  if (R.sel == 0) out0[to] = v;
+  else out1[to] = (T) v;
+}
+
+struct RowMap { int r[16]; };    // accumulator row of (lane / 16, register)
+
+// One adjoint row of the reverse of a set of reduces: function fn of source s, its 16-channel blocks cb0 .. cb0 + nb - 1 (nb <= 2),
+// fed by up to two reduces (ncon; 0: the row is written as zeros): their result rows g_sel[atom * stride + off + k], k < nout,
+// nks MFMA steps each (step q takes k = 4 q + lane / 16).  Weights [mu][con][cb < 2][step < 8][lane] from w on.
+struct ReduceBwdJob {
+  int s, fn, nin, stride_out, cb0, nb, ncon;
+  int sel[2], stride[2], off[2], nout[2], nks[2];
+  long long w, wmu;    // first weight, weights of one element
+};
+
+// G_s[atom][fn][n] (+)= sum over the job's reduces of sum_k g[atom][k] W_s[mu][c][n][k]; overwrite: the rows are written.
+// Grid (jobs, groups of tiles), a wave per job and `tpw` tiles of 16 atoms: the weights of a job fed by one reduce stay in
+// registers for its tiles (of one element, mostly).  As a wave per (job, tile) the kernel was bound by the latency of its
+// chain tile -> element -> weights in 64-thread blocks: see launch_reduce_bwd for the figures.
+template<class T>
+__global__ __launch_bounds__(256) void k_reduce_bwd(const ReduceBwdJob *__restrict__ jobs, const T *__restrict__ W, RowMap drow, const int *__restrict__ mu,
+                                                    const int *__restrict__ tile_atoms, int ntiles, int tpw, const double *__restrict__ g0,
+                                                    const T *__restrict__ g1, T *G0, T *G1, T *G2, T *G3, int overwrite)
 {
   typedef typename Mfma<T>::v4 v4;
-  const int tile = blockIdx.x;
-  int job = blockIdx.y + job_first, s = 0;
-  while (job >= R.ncol[s]) { job -= R.ncol[s]; s++; }
-  const int lane = threadIdx.x, c = lane & 15, g = lane >> 4;
-  const int arow = tile_atoms[tile * 16 + c];
-  const int m = mu[tile_atoms[tile * 16]];
-  T *G[4] = {G0, G1, G2, G3};
-  T x[8];
+  const ReduceBwdJob J = jobs[blockIdx.x];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+  const int t0 = (blockIdx.y * 4 + wave) * tpw, t1 = min(ntiles, t0 + tpw);
+  if (t0 >= t1) return;
+  T *G = J.s == 0 ? G0 : J.s == 1 ? G1 : J.s == 2 ? G2 : G3;
+  T w[2][8];
+  int held = -1;    // element whose weights w holds (jobs fed by one reduce)
+  for (int t = t0; t < t1; t++) {
+    const int arow = tile_atoms[t * 16 + c];
+    const int m = __builtin_amdgcn_readfirstlane(mu[__builtin_amdgcn_readfirstlane(arow)]);    // a tile's first entry is an atom
+    v4 acc[2] = {v4{0, 0, 0, 0}, v4{0, 0, 0, 0}};
 #pragma unroll
-  for (int q = 0; q < 8; q++) {
-    const int k = g * R.ksr + q;
-    x[q] = (arow >= 0 && q < R.ksr && k < R.nrho) ? (T) grho[(long long) arow * R.ostride + R.ooff + k] : (T) 0;
-  }
-  const int nb = R.nin[s] / 16;
-  const T *wb = R.WB[s] + ((long long) m * R.ncol[s] + job) * nb * R.ksr * 64 + lane;
-  const int fn = R.fn[s][job];
-  for (int cb = 0; cb < nb; cb++) {
-    v4 acc = {0, 0, 0, 0};
+    for (int q = 0; q < 2; q++) {
+      if (q >= J.ncon) continue;
+      T x[8];
 #pragma unroll
-    for (int q = 0; q < 8; q++)
-      if (q < R.ksr) acc = Mfma<T>::mma(x[q], wb[(cb * R.ksr + q) * 64], acc);
+      for (int k4 = 0; k4 < 8; k4++) {
+        const int k = 4 * k4 + g;
+        x[k4] = (T) 0;
+        if (k4 < J.nks[q] && arow >= 0 && k < J.nout[q]) {
+          const long long at = (long long) arow * J.stride[q] + J.off[q] + k;
+          x[k4] = J.sel[q] == 0 ? (T) g0[at] : g1[at];
+        }
+      }
+      if (J.ncon > 1 || held != m) {
+        const T *wp = W + J.w + m * J.wmu + q * (2 * 8 * 64) + lane;
+#pragma unroll
+        for (int cb = 0; cb < 2; cb++)
+#pragma unroll
+          for (int k4 = 0; k4 < 8; k4++) w[cb][k4] = cb < J.nb && k4 < J.nks[q] ? wp[(cb * 8 + k4) * 64] : (T) 0;
+        held = m;
+      }
+#pragma unroll
+      for (int cb = 0; cb < 2; cb++)
+        if (cb < J.nb) {
+#pragma unroll
+          for (int k4 = 0; k4 < 8; k4++)
+            if (k4 < J.nks[q]) acc[cb] = Mfma<T>::mma(x[k4], w[cb][k4], acc[cb]);
+        }
+    }
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      const int at = tile_atoms[tile * 16 + R.drow[4 * g + v]];
-      if (at >= 0) {
-        T *out = &G[s][((long long) at * R.stride[s] + fn) * R.nin[s] + cb * 16 + c];
-        *out = overwrite ? acc[v] : *out + acc[v];
-      }
+      const int at = __shfl(arow, drow.r[4 * g + v], 64);
+      if (at < 0) continue;
+      T *out = G + ((long long) at * J.stride_out + J.fn) * J.nin + J.cb0 * 16 + c;
+#pragma unroll
+      for (int cb = 0; cb < 2; cb++)
+        if (cb < J.nb) out[cb * 16] = overwrite ? acc[cb][v] : out[cb * 16] + acc[cb][v];
     }
   }
 }

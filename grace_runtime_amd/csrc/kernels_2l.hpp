@@ -19,17 +19,6 @@
 
 namespace grhip {
 
-// rows (atom, listed function) of a per-atom tensor [atom][nfun][KP] set to zero; total = atoms x listed functions x KP
-template<class T> __global__ void k_clear_functions(T *G, int nfun, int KP, const int *list, int nlist, long long total)
-{
-  const long long i = (long long) blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  const int n = (int) (i % KP), q = (int) ((i / KP) % nlist);
-  const long long a = i / ((long long) KP * nlist);
-  G[(a * nfun + list[q]) * KP + n] = (T) 0;
-}
-
-
 // One thread per edge: YG[e] = (Y[nlm], D1[nlm], D2[nlm]) (row width W = 3 nlm), or Y[nlm] alone (W = nlm, no
 // gradients), in rows of `stride` >= W values, the rest of a row zero.  D1 = G . e1, D2 = G . e2 are the components of the gradient G of the polynomial extension of Y along the
 // tangent vectors of the bond (tangent_basis): the bond force only uses the part of sum_lm gY_lm G_lm normal to the bond,
@@ -71,14 +60,6 @@ template<class T> __global__ void k_fill_slot(const int *mu, const T *z, T *M, i
   const int at = (int) (q / C), n = (int) (q % C);
   M[((long long) at * nslot + slot) * C + n] = z[mu[at] * C + n];
 }
-
-// dst[q] = src[q] in another precision (the fp32 engine: the scalar reduces write and read fp64 rows, the GEMMs fp32 rows)
-template<class S, class D> __global__ void k_convert(const S *src, D *dst, long long count)
-{
-  const long long q = blockIdx.x * (long long) blockDim.x + threadIdx.x;
-  if (q < count) dst[q] = (D) src[q];
-}
-
 constexpr int kPairChunk = 8;    // bonds staged in LDS at a time by the pair kernel that stages through registers
 constexpr size_t kPairLdsMax = 158 * 1024;    // dynamic LDS a pair kernel may ask for
 
