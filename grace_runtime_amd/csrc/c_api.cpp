@@ -878,7 +878,7 @@ int gr_compute_lammps_device(gr_engine *e, int nlocal, int nall, int ntypes, con
       const dim3 grid((unsigned) ((n + 127) / 128)), block(128);
       hipLaunchKernelGGL(grhip::k_lmp_rows<false>, grid, block, 0, st, L, W.count.as<int>(), W.err.as<int>(), (const long long *) nullptr, (int *) nullptr,
                          (double *) nullptr);
-      hipLaunchKernelGGL(grhip::k_scan, dim3(1), dim3(1024), 0, st, W.count.as<int>(), n, W.offset.as<long long>());
+      grhip::launch_scan(st, W.count.as<int>(), n, W.offset.as<long long>());
       long long total = 0;
       int err = 0;
       if (hipMemcpyAsync(&total, W.offset.as<long long>() + n, sizeof(total), hipMemcpyDeviceToHost, st) != hipSuccess ||

@@ -1245,7 +1245,7 @@ class EngineBase : public Engine, protected BufRegistry {
     }
     const int wpb = 4;
     stage("edge_count", [&] { hipLaunchKernelGGL(k_edge_count, dim3((n + wpb - 1) / wpb), dim3(64 * wpb), 0, stream_, src, n, count_.as<int>(), zero_.as<int>()); });
-    stage("edge_scan", [&] { hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, stream_, count_.as<int>(), n, eoff_.as<long long>()); });
+    stage("edge_scan", [&] { launch_scan(stream_, count_.as<int>(), n, eoff_.as<long long>()); });
     stage("edge_fill", [&] { hipLaunchKernelGGL(k_edge_fill, dim3((n + wpb - 1) / wpb), dim3(64 * wpb), 0, stream_, src, n, eoff_.as<long long>(), ed); });
     pin_flag_.ensure(2 * sizeof(int));
     HIP_CHECK(hipMemcpyAsync(pin_flag_.p, zero_.p, 2 * sizeof(int), hipMemcpyDeviceToHost, stream_));    // read by check_zero_bond()
@@ -1845,7 +1845,7 @@ class EngineBase : public Engine, protected BufRegistry {
       const long long *n_edges = eoff_.as<long long>() + n;
       const dim3 egrid((unsigned) ((ne + 255) / 256)), agrid((unsigned) ((nn + 3) / 4));
       hipLaunchKernelGGL(k_tlist_count, egrid, dim3(256), 0, stream_, n_edges, ej_.as<int>(), tcount_.as<int>());
-      hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, stream_, tcount_.as<int>(), nn, toff_.as<long long>());
+      launch_scan(stream_, tcount_.as<int>(), nn, toff_.as<long long>());
       hipLaunchKernelGGL(k_tlist_fill, egrid, dim3(256), 0, stream_, n_edges, ej_.as<int>(), toff_.as<long long>(), tcount_.as<int>() + nn,
                          traw_.as<int>());
       hipLaunchKernelGGL(k_tlist_sort, agrid, dim3(256), 0, stream_, nn, toff_.as<long long>(), traw_.as<int>(), tsorted_.as<int>());

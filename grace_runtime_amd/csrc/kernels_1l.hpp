@@ -205,30 +205,51 @@ static __global__ void k_edge_count(BondSrc s, int n, int *count, int *zero_bond
   if (lane == 0) count[i] = c;
 }
 
-// exclusive scan of count[n] into eoff[n + 1] (single block; n up to a few million is a few passes of 1024)
-static __global__ void k_scan(const int *count, int n, long long *eoff)
+// Exclusive scan of count[n] into eoff[n + 1], a block of 1024 threads per kScanBlock counts (count: 16-byte aligned).  A block adds
+// up the counts in front of its own itself, so the blocks need neither a second launch nor each other: it reads 4 n / 2 bytes on
+// average from the L2.  One block that walked the list took 1.9 us per 1024 counts (65 536 atoms 122 us, 32 000 62, 4001 10);
+// now 8.9, 7.6 and 5.4 us.
+constexpr int kScanBlock = 8192;
+static __global__ __launch_bounds__(1024) void k_scan(const int *__restrict__ count, int n, long long *__restrict__ eoff)
 {
-  __shared__ long long part[1024];
-  __shared__ long long carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int base = 0; base < n; base += 1024) {
-    const int i = base + threadIdx.x;
-    long long v = i < n ? count[i] : 0;
-    part[threadIdx.x] = v;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-      long long t = threadIdx.x >= o ? part[threadIdx.x - o] : 0;
-      __syncthreads();
-      part[threadIdx.x] += t;
-      __syncthreads();
-    }
-    if (i < n) eoff[i] = carry + part[threadIdx.x] - v;
-    __syncthreads();
-    if (threadIdx.x == 1023) carry += part[1023];
-    __syncthreads();
+  __shared__ long long wsum[16], wpre[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const long long b0 = (long long) blockIdx.x * kScanBlock, base = b0 + 8 * t;
+  long long pre = 0;
+#pragma unroll 4
+  for (long long i = 4 * t; i < b0; i += 4096) {    // b0 is a multiple of 4096
+    const int4 v = *reinterpret_cast<const int4 *>(count + i);
+    pre += (long long) v.x + v.y + v.z + v.w;
   }
-  if (threadIdx.x == 0) eoff[n] = carry;
+  __align__(16) int v[8];
+  long long own = 0;
+  if (base + 8 <= n) {
+    *reinterpret_cast<int4 *>(v) = *reinterpret_cast<const int4 *>(count + base);
+    *reinterpret_cast<int4 *>(v + 4) = *reinterpret_cast<const int4 *>(count + base + 4);
+  } else {
+    for (int k = 0; k < 8; k++) v[k] = base + k < n ? count[base + k] : 0;
+  }
+  for (int k = 0; k < 8; k++) own += v[k];
+  long long inc = own;
+  for (int o = 1; o < 64; o <<= 1) {
+    const long long up = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += up;
+  }
+  for (int o = 32; o > 0; o >>= 1) pre += __shfl_xor(pre, o, 64);
+  if (lane == 63) wsum[wave] = inc;
+  if (lane == 0) wpre[wave] = pre;
+  __syncthreads();
+  long long at = inc - own;
+  for (int w = 0; w < 16; w++) at += wpre[w] + (w < wave ? wsum[w] : 0);
+  for (int k = 0; k < 8; k++) {
+    if (base + k < n) eoff[base + k] = at;
+    at += v[k];
+  }
+  if (blockIdx.x == gridDim.x - 1 && t == 1023) eoff[n] = at;
+}
+inline void launch_scan(hipStream_t stream, const int *count, int n, long long *eoff)
+{
+  hipLaunchKernelGGL(k_scan, dim3(n > 0 ? (unsigned) ((n - 1) / kScanBlock + 1) : 1u), dim3(1024), 0, stream, count, n, eoff);
 }
 
 // Energy and virial are added per atom with atomics to records of 8 doubles (energy, virial[6], unused).  Additions to one

@@ -131,7 +131,7 @@ class BatchDeviceNeighbors {
     const dim3 grid((unsigned) ((n + 3) / 4)), block(256);
     hipLaunchKernelGGL(k_bnl_pairs<false>, grid, block, 0, stream, tab_.as<BnlStruct>(), sid_.as<int>(), xw_.as<double>(), cutoff * cutoff, n,
                        count_.as<int>(), (const long long *) nullptr, (int *) nullptr, (double *) nullptr);
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, stream, count_.as<int>(), n, offset.as<long long>());
+    launch_scan(stream, count_.as<int>(), n, offset.as<long long>());
     long long total = 0;
     HIP_CHECK(hipMemcpyAsync(&total, offset.as<long long>() + n, sizeof(total), hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));    // also: the host tables above are free to go

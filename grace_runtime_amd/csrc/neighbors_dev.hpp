@@ -273,7 +273,7 @@ class DeviceNeighbors {
     HIP_CHECK(hipMemsetAsync(population_.p, 0, (size_t) nbins * sizeof(int), stream));
     HIP_CHECK(hipMemsetAsync(cursor_.p, 0, (size_t) nbins * sizeof(int), stream));
     hipLaunchKernelGGL(k_nl_bin, dim3(blocks), dim3(kNlBlock), 0, stream, G, u_.as<double>(), bin_.as<int>(), population_.as<int>());
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, stream, population_.as<int>(), (int) nbins, first_.as<long long>());
+    launch_scan(stream, population_.as<int>(), (int) nbins, first_.as<long long>());
     hipLaunchKernelGGL(k_nl_scatter, dim3(blocks), dim3(kNlBlock), 0, stream, (int) n, bin_.as<int>(), first_.as<long long>(), cursor_.as<int>(),
                        slot_atom_.as<int>());
     hipLaunchKernelGGL(k_nl_order_bins, dim3((unsigned) ((nbins + kNlBlock - 1) / kNlBlock)), dim3(kNlBlock), 0, stream, (int) nbins, first_.as<long long>(),
@@ -291,7 +291,7 @@ class DeviceNeighbors {
     const dim3 grid64((unsigned) ((n + 63) / 64)), block64(64);
     hipLaunchKernelGGL(k_nl_pairs<false>, grid64, block64, 0, stream, G, x_.as<double>(), bin3_.as<int>(), wrap3_.as<int>(), first_.as<long long>(),
                        count_.as<int>(), present_.as<unsigned char>(), (const long long *) nullptr, (const int *) nullptr, (int *) nullptr, (int *) nullptr);
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, stream, count_.as<int>(), (int) n, offset.as<long long>());
+    launch_scan(stream, count_.as<int>(), (int) n, offset.as<long long>());
     std::vector<unsigned char> met((size_t) tsize);
     long long total = 0;
     HIP_CHECK(hipMemcpyAsync(met.data(), present_.p, (size_t) tsize, hipMemcpyDeviceToHost, stream));

@@ -59,6 +59,17 @@ def test_device_list_at_benchmark_size(model):
     assert np.abs(out["forces"].sum(0)).max() < 1e-9
 
 
+@pytest.mark.parametrize("n", [8191, 8193, 16385])
+def test_device_list_at_the_edges_of_the_scan(model, n):
+    """the prefix sums of the rows go over blocks of 8192 counts"""
+    rng = np.random.default_rng(n)
+    grid = np.stack(np.meshgrid(*[np.arange(26)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    pos, cell, pbc = grid * 3.2 + rng.uniform(-0.3, 0.3, (n, 3)), 26 * 3.2 * np.eye(3), np.array([True] * 3)
+    s = kk.System(model, ["Mo", "W"], skin=0.0)
+    s.compute(rng.integers(1, 3, n).astype(np.int32), pos, cell, pbc, energy_only=True)
+    assert all(np.array_equal(a, b) for a, b in zip(kk.neighbor_search(pos, cell, pbc, s.cutoff, num_threads=8), s.neighbor_list()))
+
+
 def test_far_images_fall_back_to_the_host_search(model):
     """an atom shifted by 2^20 cells: the image differences do not fit the device table"""
     pos, cell, pbc, types = cases.structure_alloy54()
