@@ -817,11 +817,10 @@ int gr_compute_lammps_device(gr_engine *e, int nlocal, int nall, int ntypes, con
         W.nodes == L.nodes && W.neighmask == neighmask && W.stride_i == stride_i && W.stride_k == stride_k && W.neighbors == neighbors &&
         W.type == type && W.numneigh == numneigh && W.owner == owner) {
       // the steps between two reneighbourings: same rows, same bonds, new bond vectors written into the engine's array
-      L.idx = W.idx.as<int>(); L.atom = W.atom.as<int>(); L.mapped = W.mapped.as<unsigned char>(); L.n = W.n;
       if (W.n > 0 && W.nb > 0) {
         double *rij = eng.bond_vectors_device();
-        hipLaunchKernelGGL(grhip::k_lmp_rows<true>, dim3((unsigned) ((W.n + 127) / 128)), dim3(128), 0, st, L, (int *) nullptr, (int *) nullptr,
-                           (const long long *) W.offset.as<long long>(), W.j.as<int>(), rij);
+        hipLaunchKernelGGL(grhip::k_lmp_vectors, dim3((unsigned) ((W.n + 3) / 4)), dim3(256), 0, st, W.atom.as<int>(), W.n, W.offset.as<long long>(),
+                           W.named.as<int>(), x, rij);
         if (hipStreamSynchronize(st) != hipSuccess) throw grhip::Error("the renewal of the bond vectors failed");
       }
       eng.run(fl);
@@ -875,9 +874,9 @@ int gr_compute_lammps_device(gr_engine *e, int nlocal, int nall, int ntypes, con
     L.idx = W.idx.as<int>(); L.atom = W.atom.as<int>(); L.mapped = W.mapped.as<unsigned char>(); L.n = n;
     W.nb = 0;
     if (n > 0) {
-      const dim3 grid((unsigned) ((n + 127) / 128)), block(128);
+      const dim3 grid((unsigned) ((n + 3) / 4)), block(256);
       hipLaunchKernelGGL(grhip::k_lmp_rows<false>, grid, block, 0, st, L, W.count.as<int>(), W.err.as<int>(), (const long long *) nullptr, (int *) nullptr,
-                         (double *) nullptr);
+                         (double *) nullptr, (int *) nullptr);
       grhip::launch_scan(st, W.count.as<int>(), n, W.offset.as<long long>());
       long long total = 0;
       int err = 0;
@@ -890,8 +889,9 @@ int gr_compute_lammps_device(gr_engine *e, int nlocal, int nall, int ntypes, con
       W.nb = total;
       W.j.ensure(sizeof(int) * (size_t) std::max<int64_t>(W.nb, 1));
       W.rij.ensure(sizeof(double) * 3 * (size_t) std::max<int64_t>(W.nb, 1));
+      W.named.ensure(sizeof(int) * (size_t) std::max<int64_t>(W.nb, 1));
       hipLaunchKernelGGL(grhip::k_lmp_rows<true>, grid, block, 0, st, L, (int *) nullptr, (int *) nullptr, (const long long *) W.offset.as<long long>(),
-                         W.j.as<int>(), W.rij.as<double>());
+                         W.j.as<int>(), W.rij.as<double>(), W.named.as<int>());
     } else {
       const long long z = 0;
       put(W.offset, &z, sizeof(z));

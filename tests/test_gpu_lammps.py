@@ -132,6 +132,41 @@ def test_device_arrays_equal_host_arrays(model_dir, model, species, struct, layo
         eng.compute_lammps_device(n, td, torch.as_tensor(x), il, nn, nb, owner=od, forces=f)
 
 
+@pytest.mark.parametrize("entries", [1, 63, 64, 65, 128, 129])
+def test_rows_of_the_device_view_that_end_at_the_lanes_of_a_wave(model_dir, entries):
+    """the first `entries` of every row (one less of every second): the device list and the host list take the same bonds, also on
+    the step that only renews the vectors"""
+    import torch
+    eng = kk.Engine(kk.Model(cases.model_file(model_dir, "mix2")), ["Mo", "W"], 64)
+    pos, cell, pbc, types = cases.STRUCTURES["alloy54"]()
+    n = len(pos)
+    rc = max(eng.cutoff(a, b) for a in (1, 2) for b in (1, 2))
+    x, t, owner, rows = lammps_inputs(pos, cell, types, rc + 2.5)
+    assert min(len(r) for r in rows) > 129
+    rows = [list(r[:entries - i % 2]) for i, r in enumerate(rows)]
+    ref = eng.compute_lammps(n, t, x, np.arange(n), [len(r) for r in rows], rows, owner=owner)
+    dev = torch.device("cuda", 0)
+    nbh = np.full((n, entries + 1), -7, np.int32)
+    for i, r in enumerate(rows):
+        nbh[i, :len(r)] = r
+    args = [torch.as_tensor(a, device=dev) for a in (t, x, np.arange(n, dtype=np.int32), np.array([len(r) for r in rows], np.int32), nbh)]
+    od = torch.as_tensor(owner, device=dev)
+    for same in (False, True):
+        f = torch.zeros(len(x), 3, dtype=torch.float64, device=dev)
+        out = eng.compute_lammps_device(n, *args, owner=od, forces=f, same_list=same)
+        assert abs(out["energy"] - ref["energy"]) < 1e-10 * max(1.0, abs(ref["energy"]))
+        assert np.abs(f.cpu().numpy() - ref["forces"]).max() < 1e-9 * max(1.0, np.abs(ref["forces"]).max())
+        if not same:    # positions move within the same arrays
+            args[1] += 0.01 * torch.sin(torch.arange(args[1].numel(), dtype=torch.float64, device=dev)).reshape(-1, 3)
+            ref = eng2_compute(model_dir, n, t, args[1].cpu().numpy(), rows, owner)
+
+
+def eng2_compute(model_dir, n, t, x, rows, owner):
+    """the host form on an engine of its own (the kept list belongs to the engine that made it)"""
+    eng = kk.Engine(kk.Model(cases.model_file(model_dir, "mix2")), ["Mo", "W"], 64)
+    return eng.compute_lammps(n, t, x, np.arange(n), [len(r) for r in rows], rows, owner=owner)
+
+
 @pytest.mark.parametrize("model,species,struct", [("mix2", ["Mo", "W"], "alloy54"), ("l3mix", ["Mo", "W"], "triclinic")])
 def test_same_list_renews_only_the_bond_vectors(model_dir, model, species, struct):
     """the steps between two reneighbourings: the arrays stay, the positions in them move; a call with same_list gives what a
