@@ -53,6 +53,21 @@ def _compare(out, ref):
     assert np.abs(out["energies"] - ref["energies"]).max() < 1e-9 * fs
 
 
+def test_device_lists_over_few_and_many_images(model_dir):
+    """cells whose images number 1, 9, 27, 63, 64 or more per step of the search, 125 and 343 (more than the table of shifts holds)"""
+    rng = np.random.default_rng(5)
+    structs = []
+    for edges, pbc, n in [((9.0, 8.0, 7.0), (1, 1, 1), 5), ((2.9, 2.9, 2.9), (1, 1, 1), 1), ((2.4, 2.45, 2.5), (1, 1, 1), 1), ((2.4, 2.8, 9.0), (1, 1, 0), 3),
+                          ((2.4, 2.8, 6.0), (1, 1, 1), 2), ((9.0, 9.0, 9.0), (0, 0, 0), 4), ((9.0, 7.0, 5.5), (1, 0, 1), 4)]:
+        # sites 2.2 A apart along the last direction, outside the cell for some
+        pos = np.array([[0.1, 0.2, 2.2 * q] for q in range(n)]) + rng.uniform(-0.1, 0.1, (n, 3)) + np.array(edges) * np.array(pbc) * rng.integers(-2, 3, (n, 3))
+        structs.append((pos, np.diag(edges), np.array(pbc, bool), rng.integers(1, 3, n)))
+    natoms, types, pos, cells, pbc = _pack(structs)
+    b = kk.Batch(_engine(model_dir, "mix2", ["Mo", "W"]).model, ["Mo", "W"])
+    ref = b.compute(natoms, types, pos, cells, pbc, energies=True)
+    _compare(_device_run(b, natoms, types, pos, cells, pbc), ref)
+
+
 @pytest.mark.parametrize("name", ["mix2", "l2mix", "l3mix"])
 def test_device_batch_equals_host_batch(model_dir, name):
     eng = _engine(model_dir, name, ["Mo", "W"])
