@@ -194,7 +194,9 @@ template<class T> struct ProdStage {
   CoupleDev cd{};
   int nfunc = 0, rankP = 0;
   bool jit = false;
-  bool jit_sets = false;    // the specialised reverse kernel writes every row of both adjoints: nothing to clear before it
+  bool jit_sets = false;    // the block-structured kernels: the reverse writes every row of both adjoints, nothing to clear before it
+  DevBuf masks;             // [parts][kCoupleMaxParts] left groups of the parts of a launch (blocked_parts)
+  int max_parts = 1;
 };
 
 template<class T> struct FcStage {
@@ -408,6 +410,8 @@ template<class T> class Engine3L final : public EngineBase {
     if (!c.all_src) zero(gX, (size_t) cn_ * c.nsrc * c.kin * sizeof(T));
     cbwd(c, gout, gX, c.all_src ? 0 : 1);
   }
+  int couple_parts(const ProdStage<T> &p, int n) const;
+  DevBuf couple_part_;    // the right operand's adjoints of the parts of a reverse couple
   void couple_fwd(ProdStage<T> &p, const T *Lp, int nfl, const T *Rp, int nfr, T *out);
   void couple_bwd(ProdStage<T> &p, const T *Lp, int nfl, const T *Rp, int nfr, const T *g, T *gL, T *gR);
   void scale_rows(const T *in, const DevBuf &s, T *out, int nf, int w, int accumulate)
@@ -665,6 +669,16 @@ template<class T> void Engine3L<T>::build_layer(int k)
       P.jit_sets = jit_compile_blocked((c.name + "_cp").c_str(), h.terms, c.group_left, c.group_right, nfl, nfr, c.nfunc, P.rankP, sizeof(T) == 4,
                                        arch_, P.cp.jit, P.cp.jit_note);
     P.jit = P.cp.jit.ok();
+    if (P.jit && P.jit_sets) {
+      std::vector<unsigned long long> masks((size_t) (jit_detail::kCoupleMaxParts + 1) * jit_detail::kCoupleMaxParts, 0);
+      for (int np = 2; np <= jit_detail::kCoupleMaxParts; np++) {
+        const auto mk = jit_detail::blocked_parts(h.terms, c.group_left, c.group_right, np);
+        if (mk.empty()) break;
+        std::copy(mk.begin(), mk.end(), masks.begin() + (size_t) np * jit_detail::kCoupleMaxParts);
+        P.max_parts = np;
+      }
+      upload_vec(P.masks, masks);
+    }
     {
       std::vector<int> tl, tr, to;
       std::vector<double> tc;
@@ -754,14 +768,25 @@ template<class T> void Engine3L<T>::build_layer(int k)
   }
 }
 
+// Blocks that share the atoms of a couple: as many as keep 11 waves per CU (a wave runs one atom of 64 channels, and few atoms
+// wait for the loads of one wave each).  The nine couples of a pass, forward + reverse + sums of the parts, 1 / 2 / 4 / 8 parts:
+// 96 atoms fp64 1337, 801, 562, 523 us; 701 fp32 1134, 862, 771, 807; 3001 fp64 5253, 5378, 5799, 6406.
+template<class T> int Engine3L<T>::couple_parts(const ProdStage<T> &p, int n) const
+{
+  const int waves = std::max(1, n * p.rankP / 64);
+  return std::max(1, std::min(p.max_parts, 11 * ncu_ / waves));
+}
+
 template<class T> void Engine3L<T>::couple_fwd(ProdStage<T> &p, const T *Lp, int nfl, const T *Rp, int nfr, T *out)
 {
   const int n = cn_, KP = p.rankP;
   int one = 1, nat = n;
   if (p.jit) {
-    void *args[] = {(void *) &Lp, (void *) &Rp, (void *) &out, (void *) &nat, (void *) &one};
+    int parts = couple_parts(p, n);
+    const unsigned long long *masks = parts > 1 ? p.masks.template as<unsigned long long>() + parts * jit_detail::kCoupleMaxParts : nullptr;
+    void *args[] = {(void *) &Lp, (void *) &Rp, (void *) &out, (void *) &nat, (void *) &one, (void *) &parts, (void *) &masks};    // the last two: block-structured
     const long long cols = (long long) n * KP;
-    HIP_CHECK(hipModuleLaunchKernel(p.cp.jit.fwd, (unsigned) ((cols + 255) / 256), 1, 1, 256, 1, 1, 0, stream_, args, nullptr));
+    HIP_CHECK(hipModuleLaunchKernel(p.cp.jit.fwd, (unsigned) ((cols + 255) / 256 * parts), 1, 1, 256, 1, 1, 0, stream_, args, nullptr));
     return;
   }
   const int ATl = 64 / KP;
@@ -782,9 +807,20 @@ template<class T> void Engine3L<T>::couple_bwd(ProdStage<T> &p, const T *Lp, int
   const int n = cn_, KP = p.rankP;
   int one = 1, nat = n, acc = p.jit_sets ? 0 : 1;
   if (p.jit) {
-    void *args[] = {(void *) &Lp, (void *) &Rp, (void *) &g, (void *) &gL, (void *) &gR, (void *) &acc, (void *) &acc, (void *) &nat, (void *) &one};
+    int parts = couple_parts(p, n);
+    const unsigned long long *masks = parts > 1 ? p.masks.template as<unsigned long long>() + parts * jit_detail::kCoupleMaxParts : nullptr;
+    long long stride = (long long) n * nfr * KP;
+    T *gRp = gR;
+    if (parts > 1) {
+      couple_part_.ensure((size_t) parts * stride * sizeof(T));
+      gRp = couple_part_.as<T>();
+    }
+    void *args[] = {(void *) &Lp,  (void *) &Rp,  (void *) &g,     (void *) &gL,    (void *) &gRp,   (void *) &acc,
+                    (void *) &acc, (void *) &nat, (void *) &one,   (void *) &parts, (void *) &masks, (void *) &stride};    // the last three: block-structured
     const long long cols = (long long) n * KP;
-    HIP_CHECK(hipModuleLaunchKernel(p.cp.jit.bwd, (unsigned) ((cols + 255) / 256), 1, 1, 256, 1, 1, 0, stream_, args, nullptr));
+    HIP_CHECK(hipModuleLaunchKernel(p.cp.jit.bwd, (unsigned) ((cols + 255) / 256 * parts), 1, 1, 256, 1, 1, 0, stream_, args, nullptr));
+    if (parts > 1)
+      hipLaunchKernelGGL(k_chain_sum<T>, dim3((unsigned) ((stride + 255) / 256)), dim3(256), 0, stream_, (const T *) gRp, stride, parts, 0ull, nfr, KP, stride, gR);
     return;
   }
   const int ATl = 64 / KP;

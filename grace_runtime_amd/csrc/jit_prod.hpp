@@ -211,7 +211,41 @@ inline std::string generate(const std::vector<ProdTerm> &terms, int nfl, int nfr
 // and the operand adjoints once per block.  Blocks are ordered by left group, so the left rows and their adjoints stay
 // in registers over all blocks of the group.  Returns an empty string when the term list has no such structure (an
 // output fed by two blocks, a group with more than kBlockRows functions); the caller then keeps its other kernels.
+// Few atoms leave most of the GPU idle with one wave per atom, so a launch may deal the left groups to `nparts` blocks for the
+// same atoms (masks[part]: the left groups of a part, in ascending order of their numbers).  The parts of a forward launch write
+// different outputs; in the reverse every part writes all adjoint rows of the right operand to its own tensor (gR + part x
+// part_stride), and the caller adds them up.  Parts take accL = accR = 0.
 constexpr int kBlockRows = 16;
+constexpr int kCoupleMaxParts = 8;
+
+// Deals the left groups to n parts by falling work (outputs, and four more per block for its operands).  Empty: the list
+// cannot be dealt (more than 64 groups on a side, or fewer left groups than parts).
+inline std::vector<unsigned long long> blocked_parts(const std::vector<ProdTerm> &terms, const std::vector<int> &group_l, const std::vector<int> &group_r, int n)
+{
+  std::map<int, std::map<int, std::set<int>>> outs;    // left group -> right group -> outputs
+  std::set<int> right;
+  for (const auto &t : terms) {
+    outs[group_l[t.l]][group_r[t.r]].insert(t.o);
+    right.insert(group_r[t.r]);
+  }
+  if (outs.size() > 64 || right.size() > 64 || (int) outs.size() < n) return {};
+  std::vector<std::pair<double, int>> work;
+  int gi = 0;
+  for (const auto &a : outs) {
+    double w = 0.0;
+    for (const auto &b : a.second) w += 4.0 + (double) b.second.size();
+    work.push_back({-w, gi++});
+  }
+  std::sort(work.begin(), work.end());
+  std::vector<double> load(n, 0.0);
+  std::vector<unsigned long long> mask(n, 0);
+  for (const auto &w : work) {
+    const int q = (int) (std::min_element(load.begin(), load.end()) - load.begin());
+    load[q] -= w.first;
+    mask[q] |= 1ull << w.second;
+  }
+  return mask;
+}
 
 inline std::string generate_blocked(const std::vector<ProdTerm> &terms, const std::vector<int> &group_l, const std::vector<int> &group_r, int nfl,
                                     int nfr, int nout, int C, bool f32)
@@ -277,9 +311,16 @@ inline std::string generate_blocked(const std::vector<ProdTerm> &terms, const st
   std::ostringstream s;
   s << "typedef " << (f32 ? "float" : "double") << " T;\n";
   s << "#define C " << C << "\n";
-  auto header = [&](const char *name, const char *args) {
-    s << "extern \"C\" __global__ __launch_bounds__(256) void " << name << "(" << args << ", int natoms, int one)\n{\n"
-      << "  const long long col = (long long) blockIdx.x * blockDim.x + threadIdx.x;\n"
+  std::map<int, int> index_l, index_r;    // groups that any term uses, numbered in ascending order
+  for (const auto &kv : rows_l) index_l.emplace(kv.first, (int) index_l.size());
+  for (const auto &kv : rows_r) index_r.emplace(kv.first, (int) index_r.size());
+  const bool dealt = index_l.size() <= 64 && index_r.size() <= 64;    // else the list runs whole only
+  auto header = [&](const char *name, const char *args, const char *more) {
+    s << "extern \"C\" __global__ __launch_bounds__(256) void " << name << "(" << args
+      << ", int natoms, int one, int nparts = 1, const unsigned long long *__restrict__ masks = 0" << more << ")\n{\n"
+      << "  const unsigned part = nparts > 1 ? blockIdx.x % nparts : 0, block = nparts > 1 ? blockIdx.x / nparts : blockIdx.x;\n"
+      << "  const unsigned long long mask = masks ? masks[part] : ~0ull;\n"
+      << "  const long long col = (long long) block * blockDim.x + threadIdx.x;\n"
       << "  const long long at = col / C;\n  const int k = (int) (col % C);\n  if (at >= natoms) return;\n";
   };
   auto declare = [&](const char *stem, int n) {
@@ -292,7 +333,7 @@ inline std::string generate_blocked(const std::vector<ProdTerm> &terms, const st
   // compiler moves them, and the products that follow them, in front of the loop and keeps every product in a register.
   std::string vary = "    const T *Lv = L + it, *Rv = R + it;\n";
   // ---- forward
-  header("prod_fwd", "const T *__restrict__ L, const T *__restrict__ R, T *__restrict__ O");
+  header("prod_fwd", "const T *__restrict__ L, const T *__restrict__ R, T *__restrict__ O", "");
   s << "  L += at * " << nfl << " * C + k;\n  R += at * " << nfr << " * C + k;\n  O += at * " << nout << " * C + k;\n";
   declare("l", maxl);
   declare("r", maxr);
@@ -300,7 +341,7 @@ inline std::string generate_blocked(const std::vector<ProdTerm> &terms, const st
     bool any = false;
     for (int o = 0; o < nout; o++)
       if (owner[o] < 0) {
-        s << "  O[" << o << " * C] = (T) 0;\n";
+        s << "  if (part == 0) O[" << o << " * C] = (T) 0;\n";
         any = true;
       }
     if (any) s << "  __asm__ volatile(\"\" ::: \"memory\");\n";
@@ -309,6 +350,7 @@ inline std::string generate_blocked(const std::vector<ProdTerm> &terms, const st
   bool have_a = false;
   for (Block *Bp : order) {
     const Block &B = *Bp;
+    if (dealt && (!have_a || B.a != cur_a)) s << (have_a ? "  }\n" : "") << "  if (mask >> " << index_l[B.a] << " & 1) {\n";
     s << "  for (int it = 0; it < one; it++) {\n" << vary;
     if (!have_a || B.a != cur_a) {
       for (size_t i = 0; i < B.lrows.size(); i++) s << "    l" << i << " = Lv[" << B.lrows[i] << " * C];\n";
@@ -339,10 +381,12 @@ inline std::string generate_blocked(const std::vector<ProdTerm> &terms, const st
       s << "  }\n";
     }
   }
-  s << "}\n\n";
+  s << (dealt ? "  }\n}\n\n" : "}\n\n");
   vary = "    const T *Lv = L + it, *Rv = R + it, *Gv = G + it, *gLv = gL + it, *gRv = gR + it;\n";
   // ---- reverse.  accL / accR: add to the stored adjoint (1) or overwrite it (0)
-  header("prod_bwd", "const T *__restrict__ L, const T *__restrict__ R, const T *__restrict__ G, T *__restrict__ gL, T *__restrict__ gR, int accL, int accR");
+  header("prod_bwd", "const T *__restrict__ L, const T *__restrict__ R, const T *__restrict__ G, T *__restrict__ gL, T *__restrict__ gR, int accL, int accR",
+         ", long long part_stride = 0");
+  s << "  gR += part * part_stride;\n  unsigned long long seen = 0;    // right groups whose adjoint rows hold something\n";
   s << "  L += at * " << nfl << " * C + k;\n  R += at * " << nfr << " * C + k;\n  G += at * " << nout << " * C + k;\n"
     << "  gL += at * " << nfl << " * C + k;\n  gR += at * " << nfr << " * C + k;\n";
   declare("l", maxl);
@@ -354,7 +398,7 @@ inline std::string generate_blocked(const std::vector<ProdTerm> &terms, const st
     std::vector<char> usedl(nfl, 0), usedr(nfr, 0);
     for (const auto &t : terms) usedl[t.l] = usedr[t.r] = 1;
     for (int a = 0; a < nfl; a++)
-      if (!usedl[a]) s << "  if (!accL) gL[" << a << " * C] = (T) 0;\n";
+      if (!usedl[a]) s << "  if (!accL && part == 0) gL[" << a << " * C] = (T) 0;\n";
     for (int b = 0; b < nfr; b++)
       if (!usedr[b]) s << "  if (!accR) gR[" << b << " * C] = (T) 0;\n";
   }
@@ -362,16 +406,23 @@ inline std::string generate_blocked(const std::vector<ProdTerm> &terms, const st
   for (size_t q = 0; q < order.size(); q++) {
     const Block &B = *order[q];
     const bool first_of_a = q == 0 || order[q - 1]->a != B.a, last_of_a = q + 1 == order.size() || order[q + 1]->a != B.a;
+    if (dealt && first_of_a) s << "  if (mask >> " << index_l[B.a] << " & 1) {\n";
     s << "  for (int it = 0; it < one; it++) {\n" << vary;
     if (first_of_a)
       for (size_t i = 0; i < B.lrows.size(); i++)
         s << "    l" << i << " = Lv[" << B.lrows[i] << " * C]; gl" << i << " = accL ? gLv[" << B.lrows[i] << " * C] : (T) 0;\n";
-    const bool again = visited_r.count(B.b) != 0;
-    visited_r.insert(B.b);
-    for (size_t j = 0; j < B.rrows.size(); j++) {
-      s << "    r" << j << " = Rv[" << B.rrows[j] << " * C]; gr" << j << " = ";
-      if (again) s << "gRv[" << B.rrows[j] << " * C];\n";
-      else s << "accR ? gRv[" << B.rrows[j] << " * C] : (T) 0;\n";
+    const std::string bit = std::to_string(dealt ? index_r[B.b] : 0);
+    if (!dealt) {
+      const bool again = !visited_r.insert(B.b).second;
+      for (size_t j = 0; j < B.rrows.size(); j++)
+        s << "    r" << j << " = Rv[" << B.rrows[j] << " * C]; gr" << j << " = " << (again ? "" : "!accR ? (T) 0 : ") << "gRv[" << B.rrows[j] << " * C];\n";
+    } else {
+      for (size_t j = 0; j < B.rrows.size(); j++) s << "    r" << j << " = Rv[" << B.rrows[j] << " * C];\n";
+      s << "    if (accR || (seen >> " << bit << " & 1)) {\n";
+      for (size_t j = 0; j < B.rrows.size(); j++) s << "      gr" << j << " = gRv[" << B.rrows[j] << " * C];\n";
+      s << "    } else {\n     ";
+      for (size_t j = 0; j < B.rrows.size(); j++) s << " gr" << j << " = (T) 0;";
+      s << "\n    }\n    seen |= 1ull << " << bit << ";\n";
     }
     s << "  }\n";
     std::map<int, std::vector<const ProdTerm *>> by_o;
@@ -392,7 +443,14 @@ inline std::string generate_blocked(const std::vector<ProdTerm> &terms, const st
     if (last_of_a)
       for (size_t i = 0; i < B.lrows.size(); i++) s << "    gL[" << B.lrows[i] << " * C] = gl" << i << ";\n";
     s << "  }\n";
+    if (dealt && last_of_a) s << "  }\n";
   }
+  if (dealt)
+    for (const auto &kv : rows_r) {
+      s << "  if (nparts > 1 && !(seen >> " << index_r[kv.first] << " & 1)) {\n";
+      for (int f : kv.second) s << "    gR[" << f << " * C] = (T) 0;\n";
+      s << "  }\n";
+    }
   s << "}\n";
   return s.str();
 }

@@ -157,6 +157,40 @@ def test_blocked_generator_on_ragged_blocks(tmp_path, seed, precision):
     run_case(tmp_path, "blocked", terms, gl, gr, nout, precision, channels=3, natoms=2, seed=seed)
 
 
+PARTS_SUFFIX = """
+extern "C" void run_fwd_parts(const T *L, const T *R, T *O, int natoms, int nparts, const unsigned long long *masks)
+{
+  blockDim.x = 1; threadIdx.x = 0;
+  for (unsigned c = 0; c < (unsigned) natoms * C * nparts; c++) { blockIdx.x = c; prod_fwd(L, R, O, natoms, 1, nparts, masks); }
+}
+extern "C" void run_bwd_parts(const T *L, const T *R, const T *G, T *gL, T *gR, int natoms, int nparts, const unsigned long long *masks, long long stride)
+{
+  blockDim.x = 1; threadIdx.x = 0;
+  for (unsigned c = 0; c < (unsigned) natoms * C * nparts; c++) { blockIdx.x = c; prod_bwd(L, R, G, gL, gR, 0, 0, natoms, 1, nparts, masks, stride); }
+}
+"""
+
+
+@pytest.mark.parametrize("masks", [[1, 6], [2, 4, 1], [7, 0]])
+@pytest.mark.parametrize("seed", [1, 2])
+def test_parts_of_a_blocked_couple_add_up(tmp_path, monkeypatch, seed, masks):
+    """left groups dealt to parts, one of them without any: outputs written once, every part's right adjoint complete"""
+    monkeypatch.setitem(globals(), "HOST_SUFFIX", HOST_SUFFIX + PARTS_SUFFIX)
+    terms, gl, gr, nout = synthetic_blocks(seed)
+    lib = host_library(tmp_path, "blocked", terms, gl, gr, nout, 3, 64)
+    rng = np.random.default_rng(seed)
+    n, np_ = 2, len(masks)
+    L, R, G = rng.standard_normal((n, len(gl), 3)), rng.standard_normal((n, len(gr), 3)), rng.standard_normal((n, nout, 3))
+    ref = direct(terms, L, R, G, nout)
+    ptr = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    m = np.array(masks, np.uint64)
+    out, gL, gR = np.full(G.shape, np.nan), np.full(L.shape, np.nan), np.full((np_,) + R.shape, np.nan)
+    lib.run_fwd_parts(ptr(L), ptr(R), ptr(out), n, np_, ptr(m))
+    lib.run_bwd_parts(ptr(L), ptr(R), ptr(G), ptr(gL), ptr(gR), n, np_, ptr(m), ctypes.c_longlong(R.size))
+    for got, exp in ((out, ref[0]), (gL, ref[1]), (gR.sum(0), ref[2])):
+        assert np.abs(got - exp).max() < 1e-12 * max(1.0, np.abs(exp).max())
+
+
 def test_blocked_generator_refuses_an_output_fed_by_two_blocks(tmp_path):
     terms = (np.array([0, 1]), np.array([0, 1]), np.array([0, 0]), np.array([1.0, 2.0]))
     assert host_library(tmp_path, "blocked", terms, [0, 1], [0, 1], 1, 4, 64) is None
