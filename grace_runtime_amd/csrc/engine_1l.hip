@@ -490,14 +490,19 @@ template<class T> void Engine1L<T>::run_chunk(const RunFlags &fl, int chunk, int
     launch_reduce_fwd<T>(redrho_, ka, kf, mu, A, AA, AAA, AAAA, rho_.as<double>(), nullptr, tiles, ntiles);
   });
   stage("energy_mlp", [&] {
+    double *ea = fl.eatom || ordered_ ? eatom_.as<double>() + a0 : nullptr, *rec = ordered_ ? nullptr : scal_.as<double>();
+    if (readout_fits(en_.nlay, en_.nin[0], en_.nout[0], en_.nout[1])) {
+      hipLaunchKernelGGL(k_energy_hidden, dim3(readout_blocks(n)), dim3(256), readout_lds(en_.nout[0]), stream_, en_, mu_.as<int>(), a0, n,
+                         rho_.as<double>(), grho_.as<double>(), ea, rec, fl.energy_only ? 0 : 1, sid_ptr());
+      return;
+    }
     const size_t lds = (size_t) (4 * (2 * en_.nlay + 4) * en_.width + en_.wlds) * sizeof(double);
     const dim3 grid((unsigned) ((n + kEnergyAtomsPerBlock - 1) / kEnergyAtomsPerBlock));
     auto kern = en_.wlds > 0 ? k_energy<true> : k_energy<false>;
     if (lds > 48 * 1024)
       HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream_, en_, mu_.as<int>(), a0, n, rho_.as<double>(), grho_.as<double>(),
-                       fl.eatom || ordered_ ? eatom_.as<double>() + a0 : nullptr, ordered_ ? nullptr : scal_.as<double>(), fl.energy_only ? 0 : 1,
-                       sid_ptr());
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream_, en_, mu_.as<int>(), a0, n, rho_.as<double>(), grho_.as<double>(), ea, rec,
+                       fl.energy_only ? 0 : 1, sid_ptr());
   });
   if (fl.uq) {
     stage("uq", [&] {

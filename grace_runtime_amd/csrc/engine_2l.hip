@@ -799,8 +799,10 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
       ran_uq_ = true;
     }
     stage("energy_mlp", [&] {
-      hipLaunchKernelGGL(k_energy_2l, dim3(nc), dim3(64), (size_t) (2 * en_.nlay + 4) * en_.width * sizeof(double), stream_, en_, mu, nc,
-                         (const double *) rho_.as<double>() + (size_t) a0_ * nrho_, (const double *) I2_.as<double>(),
+      const bool hidden = readout_fits(en_.nlay, en_.nin[0], en_.nout[0], en_.nout[1]);
+      const size_t lds = hidden ? readout_lds(en_.nout[0]) : (size_t) (2 * en_.nlay + 4) * en_.width * sizeof(double);
+      hipLaunchKernelGGL(hidden ? k_energy_2l_hidden : k_energy_2l, dim3(hidden ? readout_blocks(nc) : (unsigned) nc), dim3(hidden ? 256 : 64), lds,
+                         stream_, en_, mu, nc, (const double *) rho_.as<double>() + (size_t) a0_ * nrho_, (const double *) I2_.as<double>(),
                          grho_.as<double>() + (size_t) a0_ * nrho_, gI2_.as<double>(), fl.eatom || ordered_ ? eatom_.as<double>() + a0_ : nullptr,
                          ordered_ ? nullptr : scal_.as<double>(), forces ? 1 : 0, sid_ptr() ? sid_ptr() + a0_ : nullptr);
     });

@@ -1923,6 +1923,126 @@ struct EnergyDev {
   const double *shift;        // [nel]
 };
 
+// Readout networks of one hidden layer and up to 16 inputs (every GRACE-1L and 2L readout this repository configures): 16 lanes per
+// atom, lane p takes the hidden units p, p + 16, ... with all inputs of its atom in registers, so that no lane of the group reads
+// what another one wrote.  k_energy and the first k_energy_2l give a wave to an atom, exchange every layer through LDS and are
+// bound by that chain of round trips: 22.6 us for 128 atoms, 28 for 8192, 128 for 65 536 (GRACE-1L), 81 for 32 000 (GRACE-2L).
+// Here 7.4, 10, 43 and 38 us.
+constexpr int kReadoutInputs = 16;
+constexpr int kReadoutLds = 4096;            // doubles of weights that a block stages: hidden widths up to 240
+constexpr unsigned kReadoutBlocks = 1024;    // blocks of 16 atoms; a block of a larger pass walks on and keeps its weights
+inline bool readout_fits(int nlay, int nin, int nhid, int nout)
+{
+  return nlay == 2 && nin >= 1 && nin <= kReadoutInputs && nout == 1 && nhid <= kReadoutLds / (kReadoutInputs + 1);
+}
+inline size_t readout_lds(int nhid) { return (size_t) (kReadoutInputs + 1) * nhid * sizeof(double); }
+inline unsigned readout_blocks(int natoms) { return std::min((unsigned) (natoms + 15) / 16, kReadoutBlocks); }
+
+// weights of the two layers -> LDS: [16][nhid] (rows beyond the inputs are zero), then the nhid weights of the output
+__device__ inline void readout_stage(double *lds, const double *W0, const double *W1, int nin, int nhid)
+{
+  for (int e = threadIdx.x; e < (kReadoutInputs + 1) * nhid; e += blockDim.x)
+    lds[e] = e < nin * nhid ? W0[e] : e < kReadoutInputs * nhid ? 0.0 : W1[e - kReadoutInputs * nhid];
+  __syncthreads();
+}
+// sum over the 16 lanes of an atom
+__device__ inline double readout_sum(double v)
+{
+  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 16);
+  return v;
+}
+// Output of the network for the input x of lane p (the inputs of lanes beyond the network's are zero), and, with want_grad, gscale
+// times its derivative by that input.  All 64 lanes of the wave arrive here.
+__device__ inline double readout_net(const double *lds, int nhid, double norm0, double norm1, int act, double x, int p, int want_grad, double gscale,
+                                     double &grad)
+{
+  double xs[kReadoutInputs], g[kReadoutInputs];
+#pragma unroll
+  for (int a = 0; a < kReadoutInputs; a++) { xs[a] = __shfl(x, a, 16); g[a] = 0.0; }
+  const double *w1 = lds + kReadoutInputs * nhid;
+  double e = 0.0;
+  for (int j = p; j < nhid; j += 16) {
+    double w[kReadoutInputs], s = 0.0;
+#pragma unroll
+    for (int a = 0; a < kReadoutInputs; a++) { w[a] = lds[a * nhid + j]; s += xs[a] * w[a]; }
+    s *= norm0;
+    double v, dv;
+    if (act == 1) {
+      v = tanh(s);
+      dv = 1.0 - v * v;
+    } else {
+      const double d = 1.0 + exp(-s), sg = 1.0 / d;
+      v = s / d;
+      dv = sg * (1.0 + s * (1.0 - sg));
+    }
+    e += v * w1[j];
+    const double t = gscale * w1[j] * norm1 * dv * norm0;
+#pragma unroll
+    for (int a = 0; a < kReadoutInputs; a++) g[a] += t * w[a];
+  }
+  e = readout_sum(e) * norm1;
+  if (want_grad) {
+    // every step halves the inputs that a lane still adds up: lane p is left with input p
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+      for (int a = 0; a < o; a++) {
+        const double mine = p & o ? g[a + o] : g[a], other = p & o ? g[a] : g[a + o];
+        g[a] = mine + __shfl_xor(other, o, 16);
+      }
+    grad = g[0];
+  }
+  return e;
+}
+// the legacy layer norm in front of the network (fused_cpu.h:666-682): x q, q = 1 / sqrt(mean x^2 + 1e-16), and the reverse
+__device__ inline double readout_ln(double x, int nin) { return 1.0 / sqrt(readout_sum(x * x) / nin + 1e-16); }
+__device__ inline double readout_ln_bwd(double g, double x, double q, int nin) { return q * (g - x * readout_sum(g * x) * q * q / nin); }
+// energies of the atoms of a block without structure records: one addition per block
+__device__ inline void readout_add(double esum, double *energy)
+{
+  __shared__ double eblk[4];
+  esum += __shfl_xor(esum, 16, 64);
+  esum += __shfl_xor(esum, 32, 64);
+  if ((threadIdx.x & 63) == 0) eblk[threadIdx.x >> 6] = esum;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(energy + record_of(nullptr, blockIdx.x), eblk[0] + eblk[1] + eblk[2] + eblk[3]);
+}
+
+// as k_energy below
+static __global__ __launch_bounds__(256) void k_energy_hidden(EnergyDev M, const int *__restrict__ mu, int a0, int natoms, const double *__restrict__ rho,
+                                                              double *__restrict__ grho, double *eatom_chunk, double *energy, int want_grad,
+                                                              const int *sid)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  double *lds = reinterpret_cast<double *>(smem_raw);
+  const int p = threadIdx.x & 15, nin = M.nrho - 1;
+  readout_stage(lds, M.W[0], M.W[1], nin, M.nout[0]);
+  double esum = 0.0;
+  for (int b0 = blockIdx.x * 16; b0 < natoms; b0 += gridDim.x * 16) {    // uniform over the block
+    const int at = b0 + (threadIdx.x >> 4);
+    const bool ok = at < natoms;
+    const double *r = rho + (long long) (ok ? at : 0) * M.nrho;
+    const double x0 = p < nin ? r[p + 1] : 0.0;
+    const double q = M.ln ? readout_ln(x0, nin) : 1.0;
+    double g;
+    const double e = readout_net(lds, M.nout[0], M.norm[0], M.norm[1], M.act, x0 * q, p, want_grad, M.out_scale, g);
+    if (want_grad && M.ln) g = readout_ln_bwd(g, x0, q, nin);
+    if (!ok) continue;    // no exchange between lanes below
+    if (p == 0) {
+      const double Ei = (e + r[0]) * M.out_scale + M.shift[mu[a0 + at]];
+      if (eatom_chunk) eatom_chunk[at] = Ei;
+      if (!energy) {}    // ordered mode: the records are summed from the per-atom energies afterwards
+      else if (sid) atomicAdd(energy + record_of(sid, a0 + at), Ei);
+      else esum += Ei;
+    }
+    if (!want_grad) continue;
+    double *gr = grho + (long long) at * M.nrho;
+    if (p == 0) gr[0] = M.out_scale;
+    if (p < nin) gr[p + 1] = g;
+  }
+  if (!sid && energy) readout_add(esum, energy);
+}
+
 constexpr int kEnergyAtomsPerBlock = 16;    // atoms of one block of k_energy (4 waves, 4 atoms each)
 
 // E_i = (MLP(rho[1:]) + rho[0]) out_scale + shift[mu_i] and dE/drho, fp64, one wave per atom (fused_1l.cpp:378-427;

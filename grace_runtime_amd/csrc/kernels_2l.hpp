@@ -880,6 +880,56 @@ struct Energy2Dev {
   const double *ln0;          // [nrho]     scale of the full RMSNorm of I2
 };
 
+// as k_energy_2l below, by 16 lanes per atom: networks of one hidden layer (k_energy_hidden of GRACE-1L)
+static __global__ __launch_bounds__(256) void k_energy_2l_hidden(Energy2Dev M, const int *__restrict__ mu, int natoms, const double *__restrict__ rho,
+                                                                 const double *__restrict__ I2, double *__restrict__ grho, double *__restrict__ gI2,
+                                                                 double *eatom, double *energy, int want_grad, const int *sid)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  double *lds = reinterpret_cast<double *>(smem_raw);
+  const int p = threadIdx.x & 15, nr = M.nrho, nin = nr - 1;
+  readout_stage(lds, M.W[0], M.W[1], nin, M.nout[0]);
+  const double lnI = p < nin ? M.lnI[p] : 0.0, ln0 = p < nin ? M.ln0[p + 1] : 0.0, lnF = M.ln0[0];
+  double esum = 0.0;
+  for (int b0 = blockIdx.x * 16; b0 < natoms; b0 += gridDim.x * 16) {    // uniform over the block
+    const int at = b0 + (threadIdx.x >> 4);
+    const bool ok = at < natoms;
+    const double *r = rho + (long long) (ok ? at : 0) * nr, *i2 = I2 + (long long) (ok ? at : 0) * nr;
+    const double rf = r[0], jf = i2[0], rp = p < nin ? r[p + 1] : 0.0, jp = p < nin ? i2[p + 1] : 0.0;    // channel 0, and channel p + 1
+    const double s1 = M.rms ? sqrt(readout_sum(rp * rp) / nin + M.eps) : 1.0, s0 = M.rms ? sqrt((readout_sum(jp * jp) + jf * jf) / nr + M.eps) : 1.0;
+    const double x0 = rp / s1 * lnI + jp / s0 * ln0;
+    const double q = M.ln ? readout_ln(x0, nin) : 1.0;
+    double g;
+    const double e = readout_net(lds, M.nout[0], M.norm[0], M.norm[1], M.act, x0 * q, p, want_grad, M.out_scale, g);
+    if (ok && p == 0) {
+      const double Ei = (e + rf + jf / s0 * lnF) * M.out_scale + M.shift[mu[at]];
+      if (eatom) eatom[at] = Ei;
+      if (!energy) {}    // ordered sums: the records are added from eatom afterwards
+      else if (sid) atomicAdd(energy + record_of(sid, at), Ei);
+      else esum += Ei;
+    }
+    if (!want_grad) continue;
+    if (M.ln) g = readout_ln_bwd(g, x0, q, nin);
+    // RMSNorm reverses (y_k = x_k s_k / sigma)
+    double t1 = 0.0, t0 = 0.0;
+    if (M.rms) {
+      t1 = readout_sum(g * lnI * rp);
+      t0 = readout_sum(g * ln0 * jp) + M.out_scale * lnF * jf;
+    }
+    if (!ok) continue;    // no exchange between lanes below
+    double *gr = grho + (long long) at * nr, *gi = gI2 + (long long) at * nr;
+    if (p == 0) {
+      gr[0] = M.out_scale;
+      gi[0] = M.out_scale * lnF / s0 - jf * t0 / (nr * s0 * s0 * s0);
+    }
+    if (p < nin) {
+      gr[p + 1] = g * lnI / s1 - rp * t1 / (nin * s1 * s1 * s1);
+      gi[p + 1] = g * ln0 / s0 - jp * t0 / (nr * s0 * s0 * s0);
+    }
+  }
+  if (!sid && energy) readout_add(esum, energy);
+}
+
 // E_i = (MLP(x) + rho[0] + I2[0] ln0[0] / s0) out_scale + shift,  x_k = rho[k] lnI[k-1] / s1 + I2[k] ln0[k] / s0,
 // s1 = sqrt(mean rho[1:]^2 + eps), s0 = sqrt(mean I2^2 + eps); dE/drho, dE/dI2.  One wave per atom, fp64; a layer with
 // fewer than 33 outputs splits each dot product over 64 / outputs lanes.
