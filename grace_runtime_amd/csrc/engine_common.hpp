@@ -769,7 +769,6 @@ class EngineBase : public Engine, protected BufRegistry {
     for (DevBuf *b : bufs_)
       if (!b->model_data) b->release();
     have_sid_ = false;
-    scal_.ensure((size_t) 8 * kRecordCopies * sizeof(double));    // an empty pass still clears and reads the records of one structure
     chunk_laid_out_ = 0;
     n_peak_ = 0;
     n_ = 0;
@@ -926,7 +925,6 @@ class EngineBase : public Engine, protected BufRegistry {
     nstruct_ = in.sid ? in.nstruct : 1;
     have_sid_ = in.sid != nullptr;
     sid_sorted_ = !in.sid || std::is_sorted(in.sid, in.sid + n);
-    scal_.ensure((size_t) 8 * records() * sizeof(double));
     have_rij_ = in.rij != nullptr;
     auto put = [&](DevBuf &b, const void *src, size_t bytes) {
       b.ensure(std::max<size_t>(bytes, 8));
@@ -977,7 +975,6 @@ class EngineBase : public Engine, protected BufRegistry {
     have_sid_ = in.sid != nullptr;
     sid_sorted_ = !in.sid || std::is_sorted(in.sid, in.sid + n);
     have_rij_ = in.rij != nullptr;
-    scal_.ensure((size_t) 8 * records() * sizeof(double));
     auto put = [&](DevBuf &b, const void *src, size_t bytes, hipMemcpyKind kind) {
       b.ensure(std::max<size_t>(bytes, 8));
       if (bytes) HIP_CHECK(hipMemcpyAsync(b.p, src, bytes, kind, stream_));
@@ -1058,13 +1055,12 @@ class EngineBase : public Engine, protected BufRegistry {
     if (!ran_) throw Error("fetch() before run()");
     if (nstruct != nstruct_) throw InvalidArgument("fetch_batch: the uploaded list holds " + std::to_string(nstruct_) + " structures");
     // everything the call returns goes to pinned memory as asynchronous copies behind the pass, with one wait:
-    // [records 8 records()][forces 3 n_nodes][per-atom energies n]; the zero-bond flag of the pass is in pin_flag_ already
+    // [records 8 records()][forces 3 n_nodes][per-atom energies n]; the pass leaves its zero-bond flag in pin_flag_
     const bool wf = forces && ran_forces_ && n_nodes_ > 0, we = eatom && ran_eatom_ && n_ > 0;
     const size_t nrec = (size_t) 8 * records(), nf = wf ? (size_t) 3 * n_nodes_ : 0, ne = we ? (size_t) n_ : 0;
     pin_out_.ensure((nrec + nf + ne) * sizeof(double));
     double *rec = pin_out_.as<double>(), *pf = rec + nrec, *pe = pf + nf;
-    HIP_CHECK(hipMemcpyAsync(rec, scal_.p, nrec * sizeof(double), hipMemcpyDeviceToHost, stream_));
-    if (wf) HIP_CHECK(hipMemcpyAsync(pf, f_.p, nf * sizeof(double), hipMemcpyDeviceToHost, stream_));
+    HIP_CHECK(hipMemcpyAsync(rec, out_.p, (nrec + nf) * sizeof(double), hipMemcpyDeviceToHost, stream_));    // the forces stand behind the records
     if (we) HIP_CHECK(hipMemcpyAsync(pe, eatom_.p, ne * sizeof(double), hipMemcpyDeviceToHost, stream_));
     HIP_CHECK(hipStreamSynchronize(stream_));
     check_zero_bond();
@@ -1091,11 +1087,11 @@ class EngineBase : public Engine, protected BufRegistry {
     if (eatom && ran_eatom_ && n_ > 0) HIP_CHECK(hipMemcpyAsync(eatom, eatom_.p, sizeof(double) * n_, hipMemcpyDeviceToDevice, stream_));
     HIP_CHECK(hipStreamSynchronize(stream_));
   }
-  // two atoms at one position make a bond of length 0 (bonds.h:49-62 of the reference): reported by the pass in zero_
+  // two atoms at one position make a bond of length 0 (bonds.h:49-62 of the reference): reported by the pass in pin_flag_
   void check_zero_bond()
   {
     if (n_ == 0) return;
-    // the pass sent the flag to pinned memory right after its bond filter; every caller has waited for the stream
+    // k_edge_fill writes it to the pinned memory itself; every caller has waited for the stream
     const int *zb = pin_flag_.as<int>();
     if (!zb) return;
     if (zb[0] >= 0)
@@ -1208,24 +1204,34 @@ class EngineBase : public Engine, protected BufRegistry {
     if (fl.uq && !has_uq_head_) throw InvalidArgument(who_ + ": the model has no usable UQ head (" + uq_why_ + ")");
     ev_used_ = 0;
     const int n = n_;
-    f_.ensure(std::max<size_t>((size_t) 3 * n_nodes_, 1) * sizeof(double));
+    PassClear clear{};
+    clear.nout = (long long) (8 * records()) + 3ll * n_nodes_;
+    out_.ensure((size_t) clear.nout * sizeof(double));
+    clear.out = scal_.p = out_.as<double>();
+    f_.p = scal_.p + 8 * records();
     eatom_.ensure(std::max<size_t>(n, 1) * sizeof(double));
-    HIP_CHECK(hipMemsetAsync(f_.p, 0, (size_t) 3 * n_nodes_ * sizeof(double), stream_));
-    HIP_CHECK(hipMemsetAsync(scal_.p, 0, (size_t) 8 * records() * sizeof(double), stream_));
     ran_ = true;
     n_peak_ = std::max(n_peak_, n_);
     ran_forces_ = !fl.energy_only;
     ran_vatom_ = fl.vatom && !fl.energy_only;
     if (ran_vatom_) {
-      vatom_.ensure(std::max<size_t>((size_t) 9 * n_nodes_, 1) * sizeof(double));
-      HIP_CHECK(hipMemsetAsync(vatom_.p, 0, (size_t) 9 * n_nodes_ * sizeof(double), stream_));
+      clear.nvatom = 9ll * n_nodes_;
+      vatom_.ensure((size_t) std::max<long long>(clear.nvatom, 1) * sizeof(double));
+      clear.vatom = vatom_.as<double>();
     }
     ran_eatom_ = fl.eatom;
     ran_uq_ = false;    // set by the engine that evaluates a UQ head
-    if (n == 0) return false;
+    if (n == 0) {
+      HIP_CHECK(hipMemsetAsync(clear.out, 0, (size_t) clear.nout * sizeof(double), stream_));
+      if (clear.nvatom) HIP_CHECK(hipMemsetAsync(clear.vatom, 0, (size_t) clear.nvatom * sizeof(double), stream_));
+      return false;
+    }
+    clear.zero_bond = zero_.as<int>();
+    // no pass with other bonds is in flight: whatever changes the list or the positions has waited for the stream
+    pin_flag_.ensure(2 * sizeof(int));
+    pin_flag_.as<int>()[0] = pin_flag_.as<int>()[1] = -1;
     count_.ensure(sizeof(int) * n);
     eoff_.ensure(sizeof(long long) * (n + 1));
-    HIP_CHECK(hipMemsetAsync(zero_.p, 0xFF, 2 * sizeof(int), stream_));    // (-1, -1): no bond of length zero seen
     BondSrc src{};
     src.mu = mu_.as<int>(); src.offset = offset_.as<long long>(); src.j = j_.as<int>();
     src.rij = have_rij_ ? rij_.as<double>() : nullptr;
@@ -1243,12 +1249,14 @@ class EngineBase : public Engine, protected BufRegistry {
       erow_.ensure(ecap * sizeof(int));
       ed.erow = erow_.as<int>();
     }
-    const int wpb = 4;
-    stage("edge_count", [&] { hipLaunchKernelGGL(k_edge_count, dim3((n + wpb - 1) / wpb), dim3(64 * wpb), 0, stream_, src, n, count_.as<int>(), zero_.as<int>()); });
-    stage("edge_scan", [&] { launch_scan(stream_, count_.as<int>(), n, eoff_.as<long long>()); });
-    stage("edge_fill", [&] { hipLaunchKernelGGL(k_edge_fill, dim3((n + wpb - 1) / wpb), dim3(64 * wpb), 0, stream_, src, n, eoff_.as<long long>(), ed); });
-    pin_flag_.ensure(2 * sizeof(int));
-    HIP_CHECK(hipMemcpyAsync(pin_flag_.p, zero_.p, 2 * sizeof(int), hipMemcpyDeviceToHost, stream_));    // read by check_zero_bond()
+    const dim3 grid((unsigned) ((n + 3) / 4)), block(256);
+    stage("edge_count", [&] { hipLaunchKernelGGL(k_edge_count, grid, block, 0, stream_, src, n, count_.as<int>(), clear); });
+    const bool scan = n > kFillScanAtoms;
+    if (scan) stage("edge_scan", [&] { launch_scan(stream_, count_.as<int>(), n, eoff_.as<long long>()); });
+    stage("edge_fill", [&] {
+      hipLaunchKernelGGL(scan ? k_edge_fill<false> : k_edge_fill<true>, grid, block, 0, stream_, src, n, (const int *) count_.as<int>(),
+                         eoff_.as<long long>(), ed, zero_.as<int>(), pin_flag_.as<int>());
+    });
     return true;
   }
   EngineBase(int device, const char *who, int ntypes, const std::vector<int> &type2mu, int n_elements) :
@@ -1263,7 +1271,6 @@ class EngineBase : public Engine, protected BufRegistry {
     ncu_ = prop.multiProcessorCount;
     arch_ = prop.gcnArchName;
     check(hipStreamCreate(&stream_), "hipStreamCreate");
-    scal_.ensure((size_t) 8 * kRecordCopies * sizeof(double));
     zero_.ensure(2 * sizeof(int));
   }
   ~EngineBase() override
@@ -1875,7 +1882,14 @@ class EngineBase : public Engine, protected BufRegistry {
       for (int k = 0; k < 7; k++) sum[k] += rec[8 * ((size_t) structure * record_copies() + q) + k];
   }
   // edges of the pass and its outputs (scal: energy, virial[6])
-  DevBuf count_, eoff_, zero_, ei_, ej_, emu_, rh_, r_, xr_, rc_, f_, eatom_, scal_;
+  DevBuf count_, eoff_, zero_, ei_, ej_, emu_, rh_, r_, xr_, rc_, eatom_;
+  // records of the structures, then the forces, in one buffer that is cleared and fetched at once; laid out by begin_pass()
+  struct View {
+    double *p = nullptr;
+    template<class U> U *as() const { static_assert(std::is_same<U, double>::value, "records and forces are fp64"); return p; }
+  };
+  DevBuf out_;
+  View scal_, f_;
   bool ran_ = false, ran_forces_ = false, ran_eatom_ = false, ran_uq_ = false;
   bool has_uq_head_ = false;      // set by an engine whose model carries a valid UQ head
   std::string uq_why_ = "this engine evaluates none";

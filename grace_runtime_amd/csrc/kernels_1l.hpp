@@ -180,9 +180,22 @@ __device__ inline void bond_vec(const BondSrc &s, int i, long long q, double &dx
   }
 }
 
-// one wave per atom: number of bonds with r^2 < rc^2; a bond of length 0 is recorded in zero_bond (i, j) and skipped
-static __global__ void k_edge_count(BondSrc s, int n, int *count, int *zero_bond)
+// What a pass clears before it adds to it: the records and forces (one buffer) and the per-atom virials, and the flag of a bond of
+// length zero.  k_edge_count does it, the first kernel of a pass: as fills of their own they were three launches, which with a few
+// hundred atoms the GPU waits for (the host issues a launch in about 5 us).
+struct PassClear {
+  double *out, *vatom;
+  long long nout, nvatom;
+  int *zero_bond;             // (i, j) of a bond of length zero, or (-1, -1)
+};
+
+// one wave per atom: number of bonds with 0 < r^2 < rc^2
+static __global__ void k_edge_count(BondSrc s, int n, int *count, PassClear z)
 {
+  const long long t0 = blockIdx.x * (long long) blockDim.x + threadIdx.x, step = (long long) gridDim.x * blockDim.x;
+  for (long long q = t0; q < z.nout; q += step) z.out[q] = 0.0;
+  for (long long q = t0; q < z.nvatom; q += step) z.vatom[q] = 0.0;
+  if (t0 < 2) z.zero_bond[t0] = -1;
   const int lane = threadIdx.x & 63;
   const int i = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (i >= n) return;
@@ -192,14 +205,8 @@ static __global__ void k_edge_count(BondSrc s, int n, int *count, int *zero_bond
     double dx, dy, dz;
     bond_vec(s, i, q, dx, dy, dz);
     const double rsq = dx * dx + dy * dy + dz * dz;
-    const int jj = s.j[q];
-    const double rc = s.cut[mi * s.nel + s.mu[jj]];
-    if (!(rsq < rc * rc)) continue;
-    if (rsq == 0.0) {
-      if (atomicCAS(zero_bond, -1, i) == -1) zero_bond[1] = jj;
-      continue;
-    }
-    c++;
+    const double rc = s.cut[mi * s.nel + s.mu[s.j[q]]];
+    if (rsq < rc * rc && rsq != 0.0) c++;
   }
   for (int o = 32; o > 0; o >>= 1) c += __shfl_down(c, o, 64);
   if (lane == 0) count[i] = c;
@@ -306,14 +313,37 @@ struct Edges {
   int *erow;                  // its own number (k_edge_pairs), or null
 };
 
-// one wave per atom: in-cutoff bonds in list order -> compact edge arrays at eoff[i]
-static __global__ void k_edge_fill(BondSrc s, int n, const long long *eoff, Edges e)
+// One wave per atom, four per block: in-cutoff bonds in list order -> compact edge arrays at eoff[i].  The first bond of length 0
+// that is seen is recorded in zero_bond (cleared by k_edge_count) and reported in `flag`, (i, j) in the host's pinned memory.
+// SCAN: the block also adds up the counts of the atoms in front of its own and writes its part of eoff, which saves the launch of
+// k_scan (4.6 us and the gap behind it) where a pass has few atoms.  A block reads 2 n bytes of counts on average, n^2 / 2 bytes in
+// all: 8 MB from the L2 with 4096 atoms, about what the launch costs.
+constexpr int kFillScanAtoms = 4096;
+template<bool SCAN>
+static __global__ __launch_bounds__(256) void k_edge_fill(BondSrc s, int n, const int *__restrict__ count, long long *eoff, Edges e, int *zero_bond, int *flag)
 {
-  const int lane = threadIdx.x & 63;
-  const int i = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (i >= n) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int i = blockIdx.x * 4 + wave;
+  long long w = 0;
+  if (SCAN) {
+    __shared__ int part[4];
+    int c = 0;
+    for (int q = threadIdx.x; q < (int) blockIdx.x * 4; q += 256) c += count[q];
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    if (lane == 0) part[wave] = c;
+    __syncthreads();
+    if (i >= n) return;
+    w = (long long) part[0] + part[1] + part[2] + part[3];
+    for (int k = 0; k < wave; k++) w += count[blockIdx.x * 4 + k];
+    if (lane == 0) {
+      eoff[i] = w;
+      if (i == n - 1) eoff[n] = w + count[i];
+    }
+  } else {
+    if (i >= n) return;
+    w = eoff[i];
+  }
   const int mi = s.mu[i];
-  long long w = eoff[i];
   const long long q0 = s.offset[i], q1 = s.offset[i + 1];
   for (long long base = q0; base < q1; base += 64) {
     const long long q = base + lane;
@@ -326,6 +356,10 @@ static __global__ void k_edge_fill(BondSrc s, int n, const long long *eoff, Edge
       jj = s.j[q];
       rc = s.cut[mi * s.nel + s.mu[jj]];
       keep = (rsq < rc * rc) && rsq != 0.0;
+      if (rsq == 0.0 && 0.0 < rc * rc && atomicCAS(zero_bond, -1, i) == -1) {
+        __hip_atomic_store(flag + 1, jj, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(flag, i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
     }
     const unsigned long long m = __ballot(keep);
     if (keep) {

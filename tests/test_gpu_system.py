@@ -121,3 +121,32 @@ def test_rebuild_policy_and_results(model):
         s.compute(np.full(3, 5, np.int32), pos[:3], cell, pbc)
     with pytest.raises(ValueError):
         kk.System(model, ["Mo", "W"], skin=-1.0)
+
+
+@pytest.mark.parametrize("n", [4095, 4096, 4097])
+def test_bonds_of_few_atoms_without_a_scan(model, n):
+    """up to 4096 atoms k_edge_fill adds up the counts itself; the same structure among 3 atoms more has its bonds placed by k_scan"""
+    rng = np.random.default_rng(n)
+    grid = np.stack(np.meshgrid(*[np.arange(17)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    pos, cell, types = grid * 3.2 + rng.uniform(-0.3, 0.3, (n, 3)), 17 * 3.2 * np.eye(3), rng.integers(1, 3, n).astype(np.int32)
+    one = kk.System(model, ["Mo", "W"], skin=0.5).compute(types, pos, cell, np.array([True] * 3), energies=True)
+    more = kk.Batch(model, ["Mo", "W"]).compute([n, 3], np.concatenate([types, types[:3]]), np.concatenate([pos, pos[:3]]), np.stack([cell, cell]),
+                                                np.ones((2, 3), bool), energies=True)
+    fs = max(1.0, np.abs(one["forces"]).max())
+    assert np.abs(more["energies"][:n] - one["energies"]).max() < 1e-10 * fs and np.abs(more["forces"][:n] - one["forces"]).max() < 1e-9 * fs
+    assert np.abs(more["virial"][0] - one["virial"]).max() < 1e-8 * max(1.0, np.abs(one["virial"]).max())
+
+
+def test_a_call_after_two_atoms_met(model):
+    """the flag of a bond of length zero and the outputs of the refused call leave nothing behind"""
+    pos, cell, pbc, types = cases.structure_alloy54()
+    s = kk.System(model, ["Mo", "W"], skin=40.0)              # the list is kept over the whole test
+    ref = s.compute(types, pos, cell, pbc)
+    met = pos.copy()
+    met[5] = pos[20]
+    for _ in range(2):
+        with pytest.raises(RuntimeError, match="two atoms at the same position"):
+            s.compute(types, met, cell, pbc)
+    out = s.compute(types, pos, cell, pbc)
+    assert s.rebuilds == 1
+    assert abs(out["energy"] - ref["energy"]) < 1e-10 and np.abs(out["forces"] - ref["forces"]).max() < 1e-10
