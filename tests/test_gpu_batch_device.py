@@ -280,3 +280,38 @@ def test_release_buffers_gives_the_work_memory_back(model_dir):
     eng.release_buffers()
     eng.run()
     assert eng.fetch()["energy"] == 0.0
+
+
+@pytest.mark.parametrize("far", [0, 3, 5000])
+def test_host_batches_equal_one_system_call_per_structure(model_dir, far):
+    """Batch.compute takes its lists from the device search or, for atoms more than 1024 cells away (far = 5000) and for
+    structures of more than 2^16 candidates per atom (2450 atoms with 27 images), from the cell lists of the host: the bonds are
+    those of one System call per structure, whose list is neither."""
+    rng = np.random.default_rng(11)
+    structs = [cases.structure_alloy54(), cases.structure_triclinic(), cases.structure_slab()]
+    for edges, pbc, n in [((9.0, 8.0, 7.0), (1, 1, 1), 5), ((2.4, 2.45, 2.5), (1, 1, 1), 1), ((2.4, 2.8, 9.0), (1, 1, 0), 3), ((9.0, 9.0, 9.0), (0, 0, 0), 4)]:
+        pos = np.array([[0.1, 0.2, 2.2 * q] for q in range(n)]) + rng.uniform(-0.1, 0.1, (n, 3))
+        structs.append((pos, np.diag(edges), np.array(pbc, bool), rng.integers(1, 3, n).astype(np.int32)))
+    if far == 0:
+        grid = np.stack(np.meshgrid(*[np.arange(m) for m in (13, 13, 15)], indexing="ij"), -1).reshape(-1, 3)[:2450]
+        structs.append((2.4 * grid + rng.uniform(-0.1, 0.1, grid.shape), np.diag([31.2, 31.2, 36.0]), np.ones(3, bool),
+                        rng.integers(1, 3, 2450).astype(np.int32)))
+    model = kk.Model(cases.model_file(model_dir, "mix2"))
+    natoms, types, pos, cells, pbc = _pack(structs)
+    if far:
+        moved = np.concatenate([rng.integers(-far, far + 1, (len(s[0]), 3)) * np.asarray(s[2]) @ np.asarray(s[1], float) for s in structs])
+        pos = pos + moved
+    out = kk.Batch(model, ["Mo", "W"]).compute(natoms, types, pos, cells, pbc, energies=True)
+    start = np.concatenate([[0], np.cumsum(natoms)])
+    near = np.concatenate([s[0] for s in structs])
+    one = [kk.System(model, ["Mo", "W"], skin=0.0).compute(types[a:b], near[a:b], cells[q], pbc[q], energies=True)
+           for q, (a, b) in enumerate(zip(start[:-1], start[1:]))]
+    ref = {"energy": np.array([o["energy"] for o in one]), "virial": np.stack([o["virial"] for o in one]),
+           "forces": np.concatenate([o["forces"] for o in one]), "energies": np.concatenate([o["energies"] for o in one])}
+    _compare(out, ref)
+    eo = kk.Batch(model, ["Mo", "W"]).compute(natoms, types, pos, cells, pbc, energy_only=True)
+    assert np.abs(eo["energy"] - ref["energy"]).max() < 1e-9 * max(1.0, np.abs(ref["energy"]).max())
+    bad = pos.copy()
+    bad[2, 1] = np.nan
+    with pytest.raises(ValueError, match="not finite"):
+        kk.Batch(model, ["Mo", "W"]).compute(natoms, types, bad, cells, pbc)
