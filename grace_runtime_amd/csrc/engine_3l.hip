@@ -7,7 +7,7 @@
 //   radial functions  R[e][l][n] = MLP([T_k(2x-1), emb_i, emb_j]) env(x) fac[mu_j][n]          k_radial, species form
 //   SPBF              layer 1: X[lm][n] = sum_b Y_lm R_l                                       k_scatter_a*
 //                     layers 2-3: P[li][ly][n] = sum_b Y_ly R_l(ly) M_j[li][n],               k_pair_fwd
-//                     A = cg_W^T P (sparse), X = reduce(A)                                     k_lincomb, job GEMM
+//                     A = cg_W^T P (sparse), X = reduce(A)                                     k_groups_fwd, job GEMM
 //   cp_l product q    Lp = U[g] XL, Rp = V[g] XR (job GEMMs), P = sum cg Lp Rp (product kernel), R_q = reduce(P) (job GEMM)
 //   FCRight2Left      out[f] = nof[f] (left[f] + W[t] right[from])                             k_scale_rows + job GEMM
 //   eq / rho          reduces of (X, R2, R3, R4); EquivariantRMSNorm -> message; rho -> readout kernel
@@ -15,6 +15,7 @@
 // GEMM jobs on the matrix cores (k_gemm_jobs), forward by destination and reverse by source.
 #include "engine_common.hpp"
 #include "kernels_3l.hpp"
+#include "lincomb_groups.hpp"
 #include "model_3l.hpp"
 
 namespace grhip {
@@ -97,32 +98,24 @@ template<class T> struct DevContract {
   }
 };
 
-// sparse matrix in CSR form on the device (k_lincomb)
-struct DevCsr {
-  DevBuf off, idx, rowof, val;
-  int nrow = 0, ncol = 0, rows = 8;    // rows: output rows per wave
-  void build(int nrow_, int ncol_, const std::vector<int> &row, const std::vector<int> &col, const std::vector<double> &v)
+// the sparse Clebsch-Gordan matrix as groups of rows and outputs on the device (k_groups_fwd, k_groups_bwd; lincomb_groups.hpp)
+template<class T> struct DevGroups {
+  DevBuf job, grp, idx, w;
+  int njobs = 0, nrow = 0, nout = 0;
+  int ngrp() const { return (njobs + 3) / 4; }
+  void build(const LincombGroups &h)
   {
-    nrow = nrow_;
-    ncol = ncol_;
-    rows = lincomb_rows((int) row.size(), nrow_);
-    std::vector<int> o(nrow + 1, 0), ix(row.size()), rw(row.size());
-    std::vector<double> vv(row.size());
-    for (int r : row) o[r + 1]++;
-    for (int r = 0; r < nrow; r++) o[r + 1] += o[r];
-    std::vector<int> pos(o.begin(), o.end() - 1);
-    for (size_t t = 0; t < row.size(); t++) {
-      const int q = pos[row[t]]++;
-      ix[q] = col[t];
-      rw[q] = row[t];
-      vv[q] = v[t];
-    }
-    if (ix.empty()) { ix.push_back(0); rw.push_back(0); vv.push_back(0.0); }
-    upload_vec(off, o);
-    upload_vec(idx, ix);
-    upload_vec(rowof, rw);
-    upload_vec(val, vv);
+    static_assert(sizeof(LinGroup) == sizeof(LincombGroups::Group), "one layout on both sides");
+    njobs = (int) h.job.size() - 1;
+    nrow = h.nrow;
+    nout = h.nout;
+    const std::vector<T> wt(h.w.begin(), h.w.end());
+    upload_vec(job, h.job);
+    upload_vec(grp, h.group);
+    upload_vec(idx, h.idx);
+    upload_vec(w, wt);
   }
+  dim3 grid(int natoms, int C) const { return dim3((unsigned) ((natoms + 64 / C - 1) / (64 / C) + 7) / 8 * 8 * ngrp()); }
 };
 
 // a per-atom tensor [atom][nf][w]
@@ -251,7 +244,7 @@ template<class T> struct Layer3 {
   // equivariant SPBF
   int nlmi = 0, nfA = 0;
   DevBuf zproj, mask;
-  DevCsr cg, cgt;                     // A = cg P (rows: A functions), gP = cgt gA (rows: pair functions slot * nlm + lm)
+  DevGroups<T> cg;                    // A = cg^T P, gP = cg gA (rows: pair functions slot * nlm + lm, outputs: A functions)
   DevContract<T> redA;
   ProdStage<T> p2, p3, p4;
   FcStage<T> fa, fb;
@@ -626,8 +619,7 @@ template<class T> void Engine3L<T>::build_layer(int k)
         cf.push_back(li * nlm_ + ly);
         vv.push_back(v);
       }
-    L.cg.build(L.nfA, np, rf, cf, vv);
-    L.cgt.build(np, L.nfA, cf, rf, vv);
+    L.cg.build(lincomb_groups(np, L.nfA, cf, rf, vv));
     const Model3L::Reduce &r = Model3L::by_name(m.reduce, K + "_red");
     if (r.instr.size() != 1 || r.only_invar) throw Error("GRACE-3L: " + K + "_red must be one instruction on " + K);
     instr_contract(L.redA, r, r.instr[0], L.nfA, K + "_red");
@@ -955,11 +947,9 @@ template<class T> void Engine3L<T>::layer_forward(int k, bool forces, int yw, bo
               (const T *) M_.as<T>(), pairP_.as<T>(), L.nlmi, L.CP, nl_, L.rad.noutp, yw, sink_.as<T>(), ngrp, n, spb, (const int *) nullptr);
     });
     stage(tg(k, "couple_YI").c_str(), [&] {
-      const int AT = 64 / L.CP;
-      const int ngrp = (L.nfA + 4 * L.cg.rows - 1) / (4 * L.cg.rows);
-      hipLaunchKernelGGL(k_lincomb<T>, dim3((unsigned) (((n + AT - 1) / AT + 7) / 8 * 8 * ngrp)), dim3(256), 0, stream_,
-                         L.cg.off.template as<int>(), L.cg.idx.template as<int>(), L.cg.rowof.template as<int>(), L.cg.val.template as<double>(),
-                         (const T *) pairP_.as<T>(), A_.as<T>(), npf, L.nfA, L.CP, n, L.cg.rows, ngrp);
+      hipLaunchKernelGGL(k_groups_fwd<T>, L.cg.grid(n, L.CP), dim3(256), 0, stream_, L.cg.job.template as<int>(), L.cg.grp.template as<LinGroup>(),
+                         L.cg.idx.template as<int>(), L.cg.w.template as<T>(), (const T *) pairP_.as<T>(), A_.as<T>(), npf, L.nfA, L.CP, n, L.cg.njobs,
+                         L.cg.ngrp());
     });
     stage(tg(k, "reduce_A").c_str(), [&] { cfwd_set(L.redA, A_.as<T>(), X); });
   }
@@ -1181,11 +1171,9 @@ template<class T> void Engine3L<T>::layer_backward(int k, int yw)
   gpairP_.ensure(na * npf * L.CP * s);
   stage(tg(k, "reduce_A_bwd").c_str(), [&] { cbwd_set(L.redA, gX, gA_.as<T>()); });
   stage(tg(k, "couple_YI_bwd").c_str(), [&] {
-    const int AT = 64 / L.CP;
-    const int ngrp = (npf + 4 * L.cgt.rows - 1) / (4 * L.cgt.rows);
-    hipLaunchKernelGGL(k_lincomb<T>, dim3((unsigned) (((n + AT - 1) / AT + 7) / 8 * 8 * ngrp)), dim3(256), 0, stream_,
-                       L.cgt.off.template as<int>(), L.cgt.idx.template as<int>(), L.cgt.rowof.template as<int>(), L.cgt.val.template as<double>(),
-                       (const T *) gA_.as<T>(), gpairP_.as<T>(), L.nfA, npf, L.CP, n, L.cgt.rows, ngrp);
+    hipLaunchKernelGGL(k_groups_bwd<T>, L.cg.grid(n, L.CP), dim3(256), 0, stream_, L.cg.job.template as<int>(), L.cg.grp.template as<LinGroup>(),
+                       L.cg.idx.template as<int>(), L.cg.w.template as<T>(), (const T *) gA_.as<T>(), gpairP_.as<T>(), npf, L.nfA, L.CP, n, L.cg.njobs,
+                       L.cg.ngrp());
   });
   const int spb = slots_per_block(L.nlmi, L.CP, 1024), ngrp = (L.nlmi + spb - 1) / spb, pthreads = round_up(spb * L.CP, 64);
   stage(tg(k, "pair_bwd").c_str(), [&] {

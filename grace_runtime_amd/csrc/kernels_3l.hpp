@@ -3,7 +3,7 @@
 //   k_edge_center      element of the central atom of every edge (input of the species form of the radial kernel)
 //   k_message          M[atom][li][n] = I[atom][li][n] + chem_l0_mask[li] zproj[mu_atom][n]: what a neighbour contributes to
 //                      the equivariant SPBF (bond_vectors, libgrace/src/fused_3l.cpp:1049-1083)
-//   k_lincomb          out[atom][f][n] = sum_t v_t in[atom][p_t][n]: the sparse Clebsch-Gordan matrix cg_W of the equivariant
+//   k_groups_fwd, _bwd out[atom][f][n] = sum_p W[p][f] in[atom][p][n]: the sparse Clebsch-Gordan matrix cg_W of the equivariant
 //                      SPBF and its transpose (fused_3l.cpp:1266-1272, :1443-1449)
 //   k_scale_rows       out[atom][f][n] (+)= s[f] in[atom][f][n]: the left input of an FCRight2Left layer (fused_3l.cpp:955-969)
 //   k_couple_*_lds     cp_l couple and its reverse with the atom's projections in LDS (fused_3l_cpu.h:223-276)
@@ -40,67 +40,112 @@ __global__ void k_message(const T *I, const int *mu, const T *zproj, const T *ma
   M[q] = I[q] + mask[f] * zproj[(long long) mu[at] * C + n];
 }
 
-// Sparse matrix times the per-atom tensor: out[atom][f][n] = sum_{t in row f} val[t] in[atom][idx[t]][n].  CSR by output
-// row: terms [off[f], off[f + 1]), row[t] = f.  A wave spans the channels of AT = 64 / C atoms and takes `rows`
-// consecutive output rows (lincomb_rows: about 64 terms per wave); it reads its terms 64 at a time, one per lane, and
-// walks them with lane reads, the source rows of 8 terms requested before the first is used.
-// grid: 8 ceil(ceil(atoms / AT) / 8) ngrp blocks, ngrp = ceil(nout / (4 rows)), in the order of pair_block: the row groups
-// of one atom run on one XCD shortly after each other, so a source row that several groups read comes from HBM once.
-// block 256.
-inline int lincomb_rows(int nterms, int nout)
-{
-  const int per = nout > 0 ? (nterms + nout - 1) / nout : 1;
-  int rows = 8;
-  while (rows < 64 && rows * 2 * per <= 64) rows *= 2;
-  return rows;
-}
+// The sparse Clebsch-Gordan matrix and its transpose, group by group.  The matrix of l1 x l2 -> L couples few functions at a
+// time: as a graph of pair functions (rows) and A functions (outputs) it falls into parts of at most 31 rows and 6 outputs, so
+// a wave that takes whole parts reads every source row once and writes every result once, with dense coefficients [row][6] and
+// no test per term.  Parts are joined up to kGroupOut outputs; one with more is cut into groups of kGroupOut outputs that the
+// same wave runs one after another, the reverse adding from the second group of a row on (sign bit of its index).  A job, the
+// groups of about 32 rows, belongs to one wave, which spans the channels of AT = 64 / C atoms.
+// grid: 8 ceil(ceil(atoms / AT) / 8) ngrp blocks, ngrp = ceil(jobs / 4), in the order of pair_block; block 256.
+// Bound by the pair tensor, which goes through once per direction: 3001 atoms in fp64, both layers, 7.9 GB in 1.40 ms forward and
+// 1.51 ms reverse (5.6 and 5.2 TB/s; a large copy reaches 5.4 - 5.7).  Walking the terms of one output after another, two per source
+// row in the mean, took 1.9 + 2.5 ms.  Rows go eight (forward) and four (reverse) at a time without a branch between them: their
+// indices and coefficients are scalar loads, and one by one their latencies add up (96 atoms: 38 and 32 us a launch, now 33 and 27).
+constexpr int kGroupOut = 6;
+struct LinGroup {
+  int t0, t1, t2;                // rows t0 .. t1 with coefficients, t1 .. t2 without any (the reverse writes zeros there)
+  int nout, out[kGroupOut];      // outputs, padded with the first
+};
 template<class T>
-__global__ __launch_bounds__(256) void k_lincomb(const int *__restrict__ off, const int *__restrict__ idx, const int *__restrict__ row,
-                                                 const double *__restrict__ val, const T *__restrict__ in, T *__restrict__ out, int nin, int nout,
-                                                 int C, int natoms, int rows, int ngrp)
+__global__ __launch_bounds__(256) void k_groups_fwd(const int *__restrict__ job, const LinGroup *__restrict__ grps, const int *__restrict__ idx,
+                                                    const T *__restrict__ w, const T *__restrict__ in, T *__restrict__ out, int nrow, int nout, int C,
+                                                    int natoms, int njobs, int ngrp)
 {
-  const int AT = 64 / C, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int AT = 64 / C, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int ab, grp;
   if (!pair_block(ngrp, (natoms + AT - 1) / AT, ab, grp)) return;
-  const int a0 = ab * AT, sub = lane / C, n = lane % C;
-  const bool live = a0 + sub < natoms;
-  const int r0 = (grp * 4 + wave) * rows, r1 = r0 + rows < nout ? r0 + rows : nout;
-  if (r0 >= nout) return;
-  const T *src = in + (long long) (a0 + (live ? sub : 0)) * nin * C + n;
-  T *dst = out + (long long) (a0 + (live ? sub : 0)) * nout * C + n;
-  const int t0 = off[r0], t1 = off[r1];
-  for (int f = r0; f < r1; f++)                        // rows without terms
-    if (live && off[f] == off[f + 1]) dst[(long long) f * C] = (T) 0;
-  int cur = -1;
-  T acc = (T) 0;
-  for (int base = t0; base < t1; base += 64) {
-    const int q = base + lane < t1 ? base + lane : t1 - 1;
-    const int iv = idx[q], rv = row[q];
-    const double cv = val[q];
-    const int cnt = t1 - base < 64 ? t1 - base : 64;
-    for (int k0 = 0; k0 < cnt; k0 += 8) {
+  const int jb = grp * 4 + wave;
+  if (jb >= njobs) return;
+  const int a = ab * AT + lane / C;
+  const bool live = a < natoms;
+  const T *src = in + (long long) (live ? a : ab * AT) * nrow * C + lane % C;
+  T *dst = out + (long long) (live ? a : ab * AT) * nout * C + lane % C;
+  const int g1 = job[jb + 1];
+  for (int g = job[jb]; g < g1; g++) {
+    const LinGroup G = grps[g];
+    T acc[kGroupOut] = {};
+    // no branch within eight rows: those past the end read the last one and count with coefficient 0
+    for (int t = G.t0; t < G.t1; t += 8) {
       T x[8];
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int k = k0 + u < cnt ? k0 + u : cnt - 1;
-        x[u] = src[(long long) __builtin_amdgcn_readlane(iv, k) * C];
-      }
+      for (int u = 0; u < 8; u++) x[u] = src[(long long) (idx[t + u < G.t1 ? t + u : G.t1 - 1] & 0x7fffffff) * C];
 #pragma unroll
       for (int u = 0; u < 8; u++) {
-        const int k = k0 + u;
-        if (k < cnt) {
-          const int f = __builtin_amdgcn_readlane(rv, k);
-          if (f != cur) {
-            if (cur >= 0 && live) dst[(long long) cur * C] = acc;
-            acc = (T) 0;
-            cur = f;
-          }
-          acc += (T) readlane_f64(cv, k) * x[u];
-        }
+        const T *wu = w + (long long) (t + u < G.t1 ? t + u : G.t1 - 1) * kGroupOut;
+        const T xu = t + u < G.t1 ? x[u] : (T) 0;
+#pragma unroll
+        for (int o = 0; o < kGroupOut; o++) acc[o] += wu[o] * xu;
       }
     }
+#pragma unroll
+    for (int o = 0; o < kGroupOut; o++)
+      if (o < G.nout && live) dst[(long long) G.out[o] * C] = acc[o];
   }
-  if (cur >= 0 && live) dst[(long long) cur * C] = acc;
+}
+template<class T>
+__global__ __launch_bounds__(256) void k_groups_bwd(const int *__restrict__ job, const LinGroup *__restrict__ grps, const int *__restrict__ idx,
+                                                    const T *__restrict__ w, const T *__restrict__ gout, T *__restrict__ gin, int nrow, int nout, int C,
+                                                    int natoms, int njobs, int ngrp)
+{
+  const int AT = 64 / C, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int ab, grp;
+  if (!pair_block(ngrp, (natoms + AT - 1) / AT, ab, grp)) return;
+  const int jb = grp * 4 + wave;
+  if (jb >= njobs) return;
+  const int a = ab * AT + lane / C;
+  const bool live = a < natoms;
+  const T *src = gout + (long long) (live ? a : ab * AT) * nout * C + lane % C;
+  T *dst = gin + (long long) (live ? a : ab * AT) * nrow * C + lane % C;
+  const int g1 = job[jb + 1];
+  for (int g = job[jb]; g < g1; g++) {
+    const LinGroup G = grps[g];
+    T x[kGroupOut];
+#pragma unroll
+    for (int o = 0; o < kGroupOut; o++) x[o] = src[(long long) G.out[o] * C];
+    auto row = [&](int t) {
+      const int at = idx[t];
+      T *d = dst + (long long) (at & 0x7fffffff) * C;
+      T y = at < 0 ? *d : (T) 0;
+#pragma unroll
+      for (int o = 0; o < kGroupOut; o++) y += w[(long long) t * kGroupOut + o] * x[o];
+      if (live) *d = y;
+    };
+    int t = G.t0;
+    for (; t + 4 <= G.t1; t += 4) {    // the rows of a group are different ones: their indices and coefficients are requested together
+      T y[4], *d[4];
+      int at[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        at[u] = idx[t + u];
+        d[u] = dst + (long long) (at[u] & 0x7fffffff) * C;
+        y[u] = (T) 0;
+      }
+      if ((at[0] | at[1] | at[2] | at[3]) < 0)
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (at[u] < 0) y[u] = *d[u];
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int o = 0; o < kGroupOut; o++) y[u] += w[(long long) (t + u) * kGroupOut + o] * x[o];
+      if (live)
+#pragma unroll
+        for (int u = 0; u < 4; u++) *d[u] = y[u];
+    }
+    for (; t < G.t1; t++) row(t);
+    for (; t < G.t2; t++)
+      if (live) dst[(long long) idx[t] * C] = (T) 0;
+  }
 }
 
 // grid: ceil(natoms * nf * C / 256)
