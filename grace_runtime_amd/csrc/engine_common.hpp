@@ -1358,7 +1358,7 @@ class EngineBase : public Engine, protected BufRegistry {
     sa.natoms = n;
     for (int q = 0; q < 16; q++) sa.drow[q] = drow_[q];
     const int kb = sa.C / 16;
-    const size_t lds = (size_t) 4 * 16 * sa.nlm * sizeof(T);
+    const size_t lds = (size_t) 4 * scatter_harmonics(sa.nl) * sa.nlm * sizeof(T);
     const dim3 grid((n + 3) / 4), block(256);
 #define GR_SCAT(NL_, KB_)                                                                       \
   do {                                                                                          \

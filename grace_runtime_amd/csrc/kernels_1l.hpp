@@ -1039,7 +1039,11 @@ template<class T, int MAXM, RowsOf ROWS> __global__ void k_scatter_a(ScatterArgs
 // accumulators of the wave are the atom's A.
 // The grid walks the atoms from the LAST to the first: the radial kernel, which runs right before, writes the edge rows
 // in ascending order, so the rows it wrote last are the ones still held by the memory-side cache.
-// NL = lmax + 1, KB = channels / 16.   dynamic LDS: 4 * 16 * nlm values.
+// NL = lmax + 1, KB = channels / 16.   dynamic LDS: 4 * scatter_harmonics(NL) * nlm values.
+// A wave evaluates the harmonics of the bonds of four tiles at once, one bond per lane: tile by tile 48 of 64 lanes had nothing to
+// do (GRACE-1L in fp64, 128 atoms 19.2 -> 16.9 us, 8192 126 -> 118; GRACE-2L 32 000 659 -> 626; fp32 rows, 20 000 atoms 156 -> 142).
+// From lmax 5 on, where those of 64 bonds would leave a CU one block in fp64, of a tile.
+constexpr int scatter_harmonics(int nl) { return nl <= 5 ? 64 : 16; }
 template<class T, int NL, int KB, RowsOf ROWS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_scatter_a_mfma(ScatterArgs<T> a)
 {
@@ -1048,7 +1052,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, g = lane >> 4;
-  T *Yw = reinterpret_cast<T *>(smem_raw) + wave * 16 * a.nlm;     // [16 bonds][nlm]
+  constexpr int YB = scatter_harmonics(NL);
+  T *Yw = reinterpret_cast<T *>(smem_raw) + wave * YB * a.nlm;     // [YB bonds][nlm]
   const int ia = a.natoms - 1 - (blockIdx.x * 4 + wave);
   if (ia < 0) return;
   const int i = a.a0 + ia;
@@ -1097,19 +1102,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   }
   for (long long eb = w0; eb < w1; eb += 16) {
     const int nb = (int) (w1 - eb < 16 ? w1 - eb : 16);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    if (lane < 16) {
-      if (lane < nb) {
-        const double *u = a.rh + 3 * (eb + lane);
-        sh_eval<false, T, NL - 1>(a.sh, u[0], u[1], u[2], Yw + lane * a.nlm, nullptr);
-      } else {
-        for (int q = 0; q < a.nlm; q++) Yw[lane * a.nlm + q] = (T) 0;
+    const int at = (int) (eb - w0) & (YB - 1);      // place of the tile in its round of harmonics
+    if (at == 0) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (lane < YB) {
+        if (eb + lane < w1) {
+          const double *u = a.rh + 3 * (eb + lane);
+          sh_eval<false, T, NL - 1>(a.sh, u[0], u[1], u[2], Yw + lane * a.nlm, nullptr);
+        } else {
+          for (int q = 0; q < a.nlm; q++) Yw[lane * a.nlm + q] = (T) 0;
+        }
       }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const bool more = eb + 16 < w1;
     if constexpr (PAIRS) {
       if (more) rows_of(eb + 16);
@@ -1119,7 +1127,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
       for (int s = 2 * h; s < 2 * h + 2; s++) {
         if (4 * s >= nb) continue;
-        const T *yb = Yw + (4 * s + g) * a.nlm;
+        const T *yb = Yw + (at + 4 * s + g) * a.nlm;
 #pragma unroll
         for (int l = 0; l < NL; l++) {
           const T y = c < 2 * l + 1 ? yb[l * l + c] : (T) 0;       // A operand: row m = c
@@ -1153,14 +1161,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // consecutive bytes of a table row; the 2.6 MB table of a 32-channel lmax-4 model stays in the L2), the cubic in t, times
 // the species weight.  The entries of step s + 1 are requested when those of step s have been turned into operands, and
 // arrive while the matrix instructions of step s run; x and the element of the lane's four bonds of the NEXT tile are
-// requested a tile ahead.  No radial row is read: the rows need not exist.
-template<class T, int NL, int KB> __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_scatter_a_tab(ScatterArgs<T> a)
+// requested a tile ahead.  No radial row is read: the rows need not exist.  Three waves per SIMD in fp32 (182 registers left
+// alone, 9 spilled at 168): 65 536 atoms 778 -> 674 us together with the harmonics of four tiles at once.
+template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_scatter_a_tab(ScatterArgs<T> a)
 {
   typedef typename Mfma<T>::v4 v4;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, g = lane >> 4;
-  T *Yw = reinterpret_cast<T *>(smem_raw) + wave * 16 * a.nlm;     // [16 bonds][nlm]
+  constexpr int YB = scatter_harmonics(NL);
+  T *Yw = reinterpret_cast<T *>(smem_raw) + wave * YB * a.nlm;     // [YB bonds][nlm]
   const int ia = a.natoms - 1 - (blockIdx.x * 4 + wave);
   if (ia < 0) return;
   const int i = a.a0 + ia;
@@ -1202,19 +1212,22 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256) __attribute_
     request(0);
     const bool more = eb + 16 < w1;
     if (more) geometry(eb + 16, xn, mn);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    if (lane < 16) {
-      if (lane < nb) {
-        const double *u = a.rh + 3 * (eb + lane);
-        sh_eval<false, T, NL - 1>(a.sh, u[0], u[1], u[2], Yw + lane * a.nlm, nullptr);
-      } else {
-        for (int q = 0; q < a.nlm; q++) Yw[lane * a.nlm + q] = (T) 0;
+    const int at = (int) (eb - w0) & (YB - 1);      // place of the tile in its round of harmonics
+    if (at == 0) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (lane < YB) {
+        if (eb + lane < w1) {
+          const double *u = a.rh + 3 * (eb + lane);
+          sh_eval<false, T, NL - 1>(a.sh, u[0], u[1], u[2], Yw + lane * a.nlm, nullptr);
+        } else {
+          for (int q = 0; q < a.nlm; q++) Yw[lane * a.nlm + q] = (T) 0;
+        }
       }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
     for (int q = 0; q < 4 * KB; q++) {
       const int s = q / KB, cb = q % KB;
@@ -1227,7 +1240,7 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256) __attribute_
         bv[l] = R * zc;
       }
       if (q + 1 < 4 * KB && 4 * ((q + 1) / KB) < nb) request(q + 1);
-      const T *yb = Yw + (4 * s + g) * a.nlm;
+      const T *yb = Yw + (at + 4 * s + g) * a.nlm;
 #pragma unroll
       for (int l = 0; l < NL; l++) {
         const T y = c < 2 * l + 1 ? yb[l * l + c] : (T) 0;       // A operand: row m = c
@@ -2431,6 +2444,13 @@ template<class T> struct BondBwdArgs {
   ShCoef sh;
 };
 
+// Waves per SIMD that k_bond_bwd is compiled for.  In fp32 it waits for its chain of loads, not for HBM or the atomics (without
+// them it is no faster), and left alone it takes 173 registers where 168 let a third wave in: tables, 65 536 atoms 1.85 -> 1.39 ms,
+// 3999 of GRACE-2L 183 -> 147 us; paired rows, 20 000 atoms 571 -> 536 us.  A fourth wave spills 42 registers (2.03 ms).  Rows of
+// their own serve small structures, which have one block per CU anyway (500 atoms 20.4 -> 21.9 us); from lmax 5 on, with 64
+// channels and in fp64 three waves spill.
+template<class T> constexpr int bond_bwd_waves(int kb, int nl, RowsOf rows) { return sizeof(T) == 4 && kb <= 2 && nl <= 5 && rows != RowsOf::bonds ? 3 : 1; }
+
 // One block (4 waves) per atom; a wave takes tiles of 16 bonds.  Per tile and l two tile GEMMs on the matrix cores,
 //   P[m][b] = sum_n gA[l*l + m][n] Rz[b][l][n],   Q[m][b] = sum_n gA[l*l + m][n] dRz[b][l][n]      (K = channels)
 // with the bonds as columns: lane (g, c) of the wave ends up with the rows m = drow[4 g + v] of bond c, so the sums over
@@ -2446,7 +2466,7 @@ template<class T> struct BondBwdArgs {
 // KB = channels / 16, NL = lmax + 1.  dynamic LDS: nlm (C + 2) + 4 waves x 16 bonds x 3 nlm values.
 // RowsOf::tables: the B operands are formed from the radial tables (lane (g, c): the eight columns l C + 8 g + s of bond c, four table
 // entries each, value and derivative from the same four; requested for l + 1 before the products of l).
-template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(256) void k_bond_bwd(BondBwdArgs<T> a)
+template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(256, bond_bwd_waves<T>(KB, NL, ROWS)) void k_bond_bwd(BondBwdArgs<T> a)
 {
   constexpr bool TAB = ROWS == RowsOf::tables, PAIRS = ROWS == RowsOf::pairs;
   typedef typename Mfma<T>::v4 v4;
