@@ -1,6 +1,6 @@
 """`Batch.compute_device` (gr_compute_batch_device through the C ABI): atoms and results in device memory, neighbour
-lists built on the device.  Checked against `Batch.compute` (host lists, the reference's list order) on the same
-structures: periodic, triclinic with atoms outside the cell, slab, molecule, and the small cells of the batched
+lists built on the device.  Checked against `Batch.compute` on the same structures, and `Batch.compute`, which takes small
+structures through the same search, against one `System` call per structure: periodic, triclinic with atoms outside the cell, slab, molecule, and the small cells of the batched
 workload.  The two paths sum the same bonds in different orders: 1e-9 relative.  Needs an MI355X: run with -m gpu."""
 import os
 
