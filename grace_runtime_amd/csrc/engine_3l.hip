@@ -663,8 +663,9 @@ template<class T> void Engine3L<T>::build_layer(int k)
     P.jit = P.cp.jit.ok();
     if (P.jit && P.jit_sets) {
       std::vector<unsigned long long> masks((size_t) (jit_detail::kCoupleMaxParts + 1) * jit_detail::kCoupleMaxParts, 0);
+      const auto work = jit_detail::blocked_work(h.terms, c.group_left, c.group_right);
       for (int np = 2; np <= jit_detail::kCoupleMaxParts; np++) {
-        const auto mk = jit_detail::blocked_parts(h.terms, c.group_left, c.group_right, np);
+        const auto mk = jit_detail::blocked_parts(work, np);
         if (mk.empty()) break;
         std::copy(mk.begin(), mk.end(), masks.begin() + (size_t) np * jit_detail::kCoupleMaxParts);
         P.max_parts = np;

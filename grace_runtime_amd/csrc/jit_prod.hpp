@@ -20,6 +20,7 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <array>
 #include <cstdio>
 #include <cstdlib>
 #include <map>
@@ -218,28 +219,37 @@ inline std::string generate(const std::vector<ProdTerm> &terms, int nfl, int nfr
 constexpr int kBlockRows = 16;
 constexpr int kCoupleMaxParts = 8;
 
-// Deals the left groups to n parts by falling work (outputs, and four more per block for its operands).  Empty: the list
-// cannot be dealt (more than 64 groups on a side, or fewer left groups than parts).
-inline std::vector<unsigned long long> blocked_parts(const std::vector<ProdTerm> &terms, const std::vector<int> &group_l, const std::vector<int> &group_r, int n)
+// The left groups with their work (outputs, and four more per block for its operands), the largest first: (-work, group).  Empty:
+// the list cannot be dealt (more than 64 groups on a side).  Formed once per couple; the list has up to 12 000 terms.
+inline std::vector<std::pair<double, int>> blocked_work(const std::vector<ProdTerm> &terms, const std::vector<int> &group_l, const std::vector<int> &group_r)
 {
-  std::map<int, std::map<int, std::set<int>>> outs;    // left group -> right group -> outputs
+  std::set<std::array<int, 3>> outs;    // (left group, right group, output)
   std::set<int> right;
   for (const auto &t : terms) {
-    outs[group_l[t.l]][group_r[t.r]].insert(t.o);
+    outs.insert({group_l[t.l], group_r[t.r], t.o});
     right.insert(group_r[t.r]);
   }
-  if (outs.size() > 64 || right.size() > 64 || (int) outs.size() < n) return {};
   std::vector<std::pair<double, int>> work;
-  int gi = 0;
-  for (const auto &a : outs) {
-    double w = 0.0;
-    for (const auto &b : a.second) w += 4.0 + (double) b.second.size();
-    work.push_back({-w, gi++});
+  int a = -1, b = -1;
+  for (const auto &x : outs) {
+    if (work.empty() || x[0] != a) work.push_back({0.0, (int) work.size()});
+    if (work.back().first == 0.0 || x[1] != b) work.back().first -= 4.0;
+    work.back().first -= 1.0;
+    a = x[0];
+    b = x[1];
   }
+  if (work.size() > 64 || right.size() > 64) return {};
   std::sort(work.begin(), work.end());
+  return work;
+}
+
+// Deals the left groups to n parts by falling work.  Empty: fewer left groups than parts.
+inline std::vector<unsigned long long> blocked_parts(const std::vector<std::pair<double, int>> &groups, int n)
+{
+  if ((int) groups.size() < n) return {};
   std::vector<double> load(n, 0.0);
   std::vector<unsigned long long> mask(n, 0);
-  for (const auto &w : work) {
+  for (const auto &w : groups) {
     const int q = (int) (std::min_element(load.begin(), load.end()) - load.begin());
     load[q] -= w.first;
     mask[q] |= 1ull << w.second;
