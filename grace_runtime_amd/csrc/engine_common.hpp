@@ -1646,12 +1646,13 @@ class EngineBase : public Engine, protected BufRegistry {
       if (mode == 1 || mode == 3) HIP_CHECK(hipMemcpyAsync(db, buf, count * sizeof(double), hipMemcpyHostToDevice, stream_));
     }
     if (!by_list && (first < 0 || first + n > n_nodes_)) throw InvalidArgument("the atom range of the exchange lies outside the owned and ghost atoms");
-    const dim3 grid((unsigned) ((count + 255) / 256)), block(256);
+    const size_t moved = mode == 1 ? (size_t) n * nf * CP : count;    // rows that are set are set with their padding
+    const dim3 grid((unsigned) ((moved + 255) / 256)), block(256);
     if (mode == 0 || mode == 2)
       hipLaunchKernelGGL(k_comm_pack<T>, grid, block, 0, stream_, (const T *) rows, stride, nf, C, CP, by_list ? dl : nullptr, first, n, db);
     else
-      hipLaunchKernelGGL(k_comm_unpack<T>, grid, block, 0, stream_, rows, stride, nf, C, CP, by_list ? dl : nullptr, first, n, (const double *) db,
-                         mode == 3 ? 1 : 0);
+      hipLaunchKernelGGL((mode == 3 ? k_comm_unpack<T, true> : k_comm_unpack<T, false>), grid, block, 0, stream_, rows, stride, nf, C, CP,
+                         by_list ? dl : nullptr, first, n, (const double *) db);
     HIP_CHECK(hipGetLastError());
     if (host && (mode == 0 || mode == 2)) HIP_CHECK(hipMemcpyAsync(buf, db, count * sizeof(double), hipMemcpyDeviceToHost, stream_));
     HIP_CHECK(hipStreamSynchronize(stream_));

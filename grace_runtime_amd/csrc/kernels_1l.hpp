@@ -109,7 +109,9 @@ __device__ inline void sh_eval(const ShCoef &co, double rx, double ry, double rz
 
 // Message rows to and from an exchange buffer (the pack / unpack kernels of the reference's GPU engines,
 // libgrace/include/grace/kk/grace_2l_kk.h:141-157): rows[atom][function][CP], of which nf functions x C channels travel
-// as doubles; the atoms are list[0 .. n) or first .. first + n.  add: the buffer is added to the rows (reverse exchange).
+// as doubles; the atoms are list[0 .. n) or first .. first + n.  ADD: the buffer is added to the rows (reverse exchange).
+// Else the rows are set whole: the channels C .. CP - 1 of a ghost's row, which no other kernel writes, become zero.  Readers
+// multiply them by zero weights, which is not enough where the memory held NaN.
 template<class T>
 __global__ void k_comm_pack(const T *rows, long long stride, int nf, int C, int CP, const int *list, int first, int n, double *buf)
 {
@@ -119,17 +121,19 @@ __global__ void k_comm_pack(const T *rows, long long stride, int nf, int C, int 
   const int atom = list ? list[k] : first + k;
   buf[e] = (double) rows[atom * stride + (long long) fn * CP + c];
 }
-template<class T>
-__global__ void k_comm_unpack(T *rows, long long stride, int nf, int C, int CP, const int *list, int first, int n, const double *buf, int add)
+template<class T, bool ADD>
+__global__ void k_comm_unpack(T *rows, long long stride, int nf, int C, int CP, const int *list, int first, int n, const double *buf)
 {
   const long long e = blockIdx.x * (long long) blockDim.x + threadIdx.x;
-  if (e >= (long long) n * nf * C) return;
-  const int c = (int) (e % C), fn = (int) ((e / C) % nf), k = (int) (e / ((long long) C * nf));
+  const int W = ADD ? C : CP;
+  if (e >= (long long) n * nf * W) return;
+  const int c = (int) (e % W), fn = (int) ((e / W) % nf), k = (int) (e / ((long long) W * nf));
   const int atom = list ? list[k] : first + k;
   T *dst = rows + atom * stride + (long long) fn * CP + c;
+  const double v = c < C ? buf[((long long) k * nf + fn) * C + c] : 0.0;
   // several entries of a send list may name one atom (an atom with several images): atomic add
-  if (add) atomicAdd(dst, (T) buf[e]);
-  else *dst = (T) buf[e];
+  if (ADD) atomicAdd(dst, (T) v);
+  else *dst = (T) v;
 }
 
 // plain copy of n doubles: the calibration kernel for the HBM counters (FETCH_SIZE / WRITE_SIZE per byte moved)

@@ -4,13 +4,14 @@ atoms and the ghosts its bonds reach (images of its own atoms and atoms of the o
 side by side in two host threads; their exchange callbacks move the message rows and the adjoint rows through host buffers, as
 MPI would.  The energies of the ranks add up to, and the forces folded back onto their atoms equal, the single-engine result,
 the fp64 CPU oracle on the uncut structure and the committed outputs of the compiled reference."""
+import os
 import threading
 
 import numpy as np
 import pytest
 
 import cases
-from grace_runtime_amd import kk
+from grace_runtime_amd import _lib, kk, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -201,3 +202,72 @@ def test_device_row_movers_equal_the_host_forms(model_dir):
     one = kk.Engine(kk.Model(cases.model_file(model_dir, "mix2")), ["Mo", "W"], 64)
     with pytest.raises(RuntimeError, match="no message rows"):
         one.pack_forward_host(1, np.zeros(1, np.int32))
+
+
+def self_exchange(pos, cell, pbc, types, rc):
+    """one rank that owns every atom: LAMMPS arrays with a ghost per (atom, image) that a bond reaches, and the owner of every ghost"""
+    perm, offset, j, image, shifts = kk.neighbor_search(pos, cell, pbc, rc)
+    n = len(pos)
+    slot = np.empty(n, np.int64)
+    slot[perm] = np.arange(n)
+    ghosts, rows = {}, []
+    for a in range(n):
+        row = []
+        for b in range(offset[slot[a]], offset[slot[a] + 1]):
+            nb, im = int(perm[j[b]]), int(image[b])
+            row.append(ghosts.setdefault((nb, im), n + len(ghosts)) if shifts[im].any() else nb)
+        rows.append(np.array(row, np.int32))
+    owner = np.array([a for a, _ in ghosts])
+    x = np.concatenate([pos, np.array([pos[a] + shifts[im] for a, im in ghosts])])
+    return dict(x=x, type=np.concatenate([types, types[owner]]).astype(np.int32), rows=rows, owner=owner)
+
+
+def own_all_call(eng, me, n, ghost_rows):
+    """the LAMMPS call of a self_exchange rank of n atoms; ghost_rows(rows of the owned atoms): the rows the ghosts receive"""
+    nall = len(me["x"])
+
+    def forward(layer):
+        eng.unpack_forward_host(layer, n, ghost_rows(eng.pack_forward_host(layer, np.arange(n, dtype=np.int32))))
+
+    def reverse(layer):
+        eng.unpack_reverse_host(layer, me["owner"].astype(np.int32), eng.pack_reverse_host(layer, n, nall - n))
+
+    eng.set_exchange(forward, reverse)
+    return eng.compute_lammps(n, me["type"], me["x"], np.arange(n, dtype=np.int32), np.array([len(r) for r in me["rows"]], np.int32), me["rows"],
+                              owner=None, energies=True)
+
+
+# message widths that are padded on the GPU (12 -> 16), and the padded width itself
+PADDED = {"l2mix": ("random_model_2l", {"cr": 16})}
+
+
+def leave_nan_memory(monkeypatch, folder, model, me, n, precision, engines=3):
+    """Passes of engines whose widths are the padded ones of `model` and whose ghosts receive NaN; their memory, NaN in the padding
+    channels of `model` too, goes to the pool, for the next engine that asks for buffers of these sizes."""
+    make, width = PADDED[model]
+    build = getattr(synth, make)
+    monkeypatch.setattr(synth, make, lambda **kw: build(**{**kw, **width}))
+    path = os.path.join(str(folder), "wide.npz")
+    synth.save_model(path, cases.MODELS[model]())
+    monkeypatch.undo()
+    made = [kk.Engine(kk.Model(path), ["Mo", "W"], precision) for _ in range(engines)]
+    for eng in made:
+        assert np.isnan(own_all_call(eng, me, n, lambda rows: np.full((len(me["x"]) - n, rows.shape[1]), np.nan))["forces"]).any()
+    for eng in made:
+        _lib.check(_lib.lib().gr_engine_recycle_buffers(eng._h))
+    return made
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("model", list(PADDED))
+def test_padding_channels_whatever_the_memory_held(model_dir, tmp_path, monkeypatch, model, precision):
+    pos, cell, pbc, types = cases.structure_alloy54()
+    n, me = len(pos), self_exchange(pos, cell, pbc, types, 5.0)
+    keep = leave_nan_memory(monkeypatch, tmp_path, model, me, n, precision)      # the pool lives as long as an engine does
+    eng = kk.Engine(kk.Model(cases.model_file(model_dir, model)), ["Mo", "W"], precision)
+    got = own_all_call(eng, me, n, lambda rows: rows[me["owner"]])
+    del keep
+    forces = np.array(got["forces"][:n])
+    np.add.at(forces, me["owner"], got["forces"][n:])
+    orc = cases.oracle_reference(model_dir, model, pos, cell, pbc, types)
+    cases.check_against({**got, "forces": forces}, orc, n, *((1e-10, 1e-9, 1e-10, 1e-8) if precision == 64 else (1e-6, 2e-5, 2e-6, 2e-5)))
