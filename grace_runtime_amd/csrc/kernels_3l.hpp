@@ -353,8 +353,12 @@ __global__ void k_eqnorm(EqNormDev E, const T *X, T *Y, const T *gY, T *gX, int 
     }
     for (int o = 32; o > 0; o >>= 1) vsum += __shfl_xor(vsum, o, 64);
     const double mg = cen ? vsum / Cr * E.mask[f] : 0.0;
-    for (int n = lane; n < Cr; n += 64) {
+    for (int n = lane; n < C; n += 64) {
       const long long q = (long long) f * C + n;
+      if (n >= Cr) {    // the padding is read by the products behind, with zero weights
+        if (!accumulate) go[q] = (T) 0;
+        continue;
+      }
       const double v = r * (double) gy[q] * E.aff[(long long) E.grp[f] * C + n] - kf * ((double) x[q] - mean[f]) - mg;
       go[q] = accumulate ? go[q] + (T) v : (T) v;
     }

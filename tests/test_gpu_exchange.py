@@ -237,8 +237,8 @@ def own_all_call(eng, me, n, ghost_rows):
                               owner=None, energies=True)
 
 
-# message widths that are padded on the GPU (12 -> 16), and the padded width itself
-PADDED = {"l2mix": ("random_model_2l", {"cr": 16})}
+# message widths that are padded on the GPU (12 -> 16, 20 -> 32), and the padded width itself
+PADDED = {"l2mix": ("random_model_2l", {"cr": 16}), "l3pad": ("random_model_3l", {"channels": 32})}
 
 
 def leave_nan_memory(monkeypatch, folder, model, me, n, precision, engines=3):
