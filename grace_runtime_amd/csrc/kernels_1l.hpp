@@ -1165,8 +1165,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // consecutive bytes of a table row; the 2.6 MB table of a 32-channel lmax-4 model stays in the L2), the cubic in t, times
 // the species weight.  The entries of step s + 1 are requested when those of step s have been turned into operands, and
 // arrive while the matrix instructions of step s run; x and the element of the lane's four bonds of the NEXT tile are
-// requested a tile ahead.  No radial row is read: the rows need not exist.  Three waves per SIMD in fp32 (182 registers left
-// alone, 9 spilled at 168): 65 536 atoms 778 -> 674 us together with the harmonics of four tiles at once.
+// requested a tile ahead.  No radial row is read: the rows need not exist.  Three waves per SIMD in fp32: 32 channels
+// and lmax 4 take 182 registers left alone and spill 9 at 168, 65 536 atoms 778 -> 674 us together with the harmonics of four tiles
+// at once; 16 channels and lmax 6 take 187 and spill 18, 8192 atoms 96 -> 95 us; the other forms fit without spills.
 template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_scatter_a_tab(ScatterArgs<T> a)
 {
   typedef typename Mfma<T>::v4 v4;
@@ -2452,7 +2453,8 @@ template<class T> struct BondBwdArgs {
 // them it is no faster), and left alone it takes 173 registers where 168 let a third wave in: tables, 65 536 atoms 1.85 -> 1.39 ms,
 // 3999 of GRACE-2L 183 -> 147 us; paired rows, 20 000 atoms 571 -> 536 us.  A fourth wave spills 42 registers (2.03 ms).  Rows of
 // their own serve small structures, which have one block per CU anyway (500 atoms 20.4 -> 21.9 us); from lmax 5 on, with 64
-// channels and in fp64 three waves spill.
+// channels and in fp64 three waves spill.  Of the forms compiled for three waves one spills, paired rows of 32 channels and lmax 4
+// (200 registers left alone, 10 spilled): the form that the 20 000 atoms above take.
 template<class T> constexpr int bond_bwd_waves(int kb, int nl, RowsOf rows) { return sizeof(T) == 4 && kb <= 2 && nl <= 5 && rows != RowsOf::bonds ? 3 : 1; }
 
 // One block (4 waves) per atom; a wave takes tiles of 16 bonds.  Per tile and l two tile GEMMs on the matrix cores,
