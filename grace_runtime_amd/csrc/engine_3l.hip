@@ -663,7 +663,7 @@ template<class T> void Engine3L<T>::build_layer(int k)
     P.jit = P.cp.jit.ok();
     if (P.jit && P.jit_sets) {
       std::vector<unsigned long long> masks((size_t) (jit_detail::kCoupleMaxParts + 1) * jit_detail::kCoupleMaxParts, 0);
-      const auto work = jit_detail::blocked_work(h.terms, c.group_left, c.group_right);
+      const auto work = jit_detail::blocked_work(h.terms, c.group_left, c.group_right, c.nfunc);
       for (int np = 2; np <= jit_detail::kCoupleMaxParts; np++) {
         const auto mk = jit_detail::blocked_parts(work, np);
         if (mk.empty()) break;
