@@ -404,7 +404,6 @@ template<class T> class Engine3L final : public EngineBase {
     cbwd(c, gout, gX, c.all_src ? 0 : 1);
   }
   int couple_parts(const ProdStage<T> &p, int n) const;
-  DevBuf couple_part_;    // the right operand's adjoints of the parts of a reverse couple
   void couple_fwd(ProdStage<T> &p, const T *Lp, int nfl, const T *Rp, int nfr, T *out);
   void couple_bwd(ProdStage<T> &p, const T *Lp, int nfl, const T *Rp, int nfr, const T *g, T *gL, T *gR);
   void scale_rows(const T *in, const DevBuf &s, T *out, int nf, int w, int accumulate)
@@ -708,6 +707,11 @@ template<class T> void Engine3L<T>::build_layer(int k)
   build_prod(L.p3, "3", L.nR2, L.wR, nX, L.X.w, L.L3, L.R3p, L.nR3, false);
   build_fc(L.fb, K + "_2b");
   build_prod(L.p4, "4", L.nR2, L.wR, L.nR2, L.wR, L.L4, L.R4p, L.nR4, true);
+  // the parts of a reverse couple leave the right operand's adjoint in P_, which holds the layer's longest product
+  int longest = 0;
+  for (const ProdStage<T> *p : {&L.p2, &L.p3, &L.p4}) longest = std::max(longest, p->nfunc * p->rankP);
+  for (auto &pr : {std::make_pair(&L.p2, &L.R2p), std::make_pair(&L.p3, &L.R3p), std::make_pair(&L.p4, &L.R4p)})
+    pr.first->max_parts = std::max(1, std::min(pr.first->max_parts, longest / std::max(1, pr.second->nf * pr.first->rankP)));
   // ---- eq (layers 1-2) and rho reduces of (X, R2, R3, R4)
   const std::string xname = L.equiv ? K + "_red" : K;
   const std::string srcs[4] = {xname, K + "_2_red", K + "_3_red", K + "_4_red"};
@@ -804,10 +808,7 @@ template<class T> void Engine3L<T>::couple_bwd(ProdStage<T> &p, const T *Lp, int
     const unsigned long long *masks = parts > 1 ? p.masks.template as<unsigned long long>() + parts * jit_detail::kCoupleMaxParts : nullptr;
     long long stride = (long long) n * nfr * KP;
     T *gRp = gR;
-    if (parts > 1) {
-      couple_part_.ensure((size_t) parts * stride * sizeof(T));
-      gRp = couple_part_.as<T>();
-    }
+    if (parts > 1) gRp = P_.as<T>();    // the product of the forward pass, which nothing reads any more
     void *args[] = {(void *) &Lp,  (void *) &Rp,  (void *) &g,     (void *) &gL,    (void *) &gRp,   (void *) &acc,
                     (void *) &acc, (void *) &nat, (void *) &one,   (void *) &parts, (void *) &masks, (void *) &stride};    // the last three: block-structured
     const long long cols = (long long) n * KP;

@@ -150,6 +150,22 @@ def test_automatic_chunk_counts_what_the_paired_rows_keep(model_dir, model):
     assert kept[0] - kept[256] >= 16 * len(j) / n * 1000 / 1048576 - 1 > 0
 
 
+def test_few_atoms_take_no_more_memory_per_atom(model_dir):
+    """GRACE-3L deals the couples of few atoms (below 1408 with 64 channels and 256 CUs) to blocks that leave an adjoint each: in memory
+    that the pass holds anyway, which the automatic chunk counts"""
+    m, L, held, energy = kk.Model(cases.model_file(model_dir, "config4")), _lib.lib(), {}, {}
+    for n in (96, 2880):                                  # dimers: the same bonds per atom
+        eng = kk.Engine(m, ["Mo", "W"], 64)
+        eng.set_chunksize(0)
+        base = L.gr_memory_in_use()
+        i = np.arange(n)
+        out = eng.compute(1 + i % 2, np.arange(n + 1), i ^ 1, rij=np.where(i % 2, -1.0, 1.0)[:, None] * np.array([1.5, 1.2, 1.0]))
+        held[n], energy[n] = L.gr_memory_in_use() - base, out["energy"] / n
+        del eng
+    assert abs(energy[96] - energy[2880]) < 1e-10
+    assert held[96] / 96 < held[2880] / 2880 + 4 * 2 ** 20 / 96        # the parts of the reduces: up to 2 MB; those of the couples took 30
+
+
 def test_outputs_accumulate_on_request(model_dir):
     """GR_FLAG_ACCUMULATE: the outputs of a call are added to the caller's values (libgrace/include/grace/system.h:66-75)"""
     pos, cell, pbc, types = cases.structure_alloy54()
