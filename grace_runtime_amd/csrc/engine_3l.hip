@@ -766,8 +766,13 @@ template<class T> void Engine3L<T>::build_layer(int k)
 }
 
 // Blocks that share the atoms of a couple: as many as keep 11 waves per CU (a wave runs one atom of 64 channels, and few atoms
-// wait for the loads of one wave each).  The nine couples of a pass, forward + reverse + sums of the parts, 1 / 2 / 4 / 8 parts:
-// 96 atoms fp64 1337, 801, 562, 523 us; 701 fp32 1134, 862, 771, 807; 3001 fp64 5253, 5378, 5799, 6406.
+// wait for the loads of one wave each).  The nine couples of a pass of the benchmark model, forward + reverse + sums of the parts, us
+// with 1 / 2 / 4 / 8 parts:
+//   atoms      96                350                   701                    1000                   2000                   3001
+//   fp64  1431 856 618 579   1688 1128 958 935   2082 1629 1537 1684   2416 1993 2119 2271   3607 3761 3958 4368   5379 5485 5819 6449
+//   fp32   976 595 426 397   1037  694 575 561   1298  969  840  864   1441 1116 1070 1179   2045 1833 2113 2234   2616 2770 3036 3327
+// The line gives 8, 8, 4, 2, 1 and 1: within 4 % of the best there, and at 200, 500 and 1400 atoms, in both precisions except for
+// 2000 atoms in fp32, where two parts would be a tenth quicker.
 template<class T> int Engine3L<T>::couple_parts(const ProdStage<T> &p, int n) const
 {
   const int waves = std::max(1, n * p.rankP / 64);
