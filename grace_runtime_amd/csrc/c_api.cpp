@@ -1351,14 +1351,12 @@ int gr_compute_batch_uq(gr_engine *e, int nstruct, const int *natoms, const int 
       if (!e->bnl) e->bnl = std::make_unique<grhip::BatchDeviceNeighbors>();
       grhip::BatchDeviceNeighbors &nl = *e->bnl;
       nl.build_from_host(nstruct, natoms, N, positions, cells, pbc, rc, e->bnl_stream);
-      if (hipStreamSynchronize(e->bnl_stream) != hipSuccess) throw grhip::Error("the device neighbour search failed");
       grhip::DeviceCsr in;
       in.n = (int) N;
       in.types = types;
       in.nb = nl.nb;
       in.offset = nl.offset.as<int64_t>();
-      in.j = nl.j.as<int>();
-      in.rij = nl.rij.as<double>();
+      in.fill = [&nl](int *j, double *rij, hipStream_t st) { nl.fill(j, rij, st); };
       in.nstruct = nstruct;
       in.sid = nl.sid.data();
       live(e).upload_device(in);
@@ -1521,8 +1519,7 @@ int gr_compute_batch_device_uq(gr_engine *e, int nstruct, const int *natoms, con
         in.types = ty.data();
         in.nb = nl.nb;
         in.offset = nl.offset.as<int64_t>();
-        in.j = nl.j.as<int>();
-        in.rij = nl.rij.as<double>();
+        in.fill = [&nl](int *j, double *rij, hipStream_t st) { nl.fill(j, rij, st); };
         in.nstruct = ns;
         in.sid = nl.sid.data();
         live(e).upload_device(in);

@@ -7,7 +7,10 @@
 #include "model_2l.hpp"
 #include "model_3l.hpp"
 
+#include <hip/hip_runtime_api.h>
+
 #include <cstdint>
+#include <functional>
 #include <memory>
 #include <string>
 #include <vector>
@@ -55,6 +58,7 @@ struct DeviceCsr {
   const double *shifts = nullptr;     // host [nimages][3]
   int64_t nimages = 0;
   const double *rij = nullptr;        // device [nb][3] bond vectors, in place of (image, x, shifts)
+  std::function<void(int *j, double *rij, hipStream_t stream)> fill;    // in place of j and rij: writes both, on the stream it is given
   int nstruct = 1;                    // several independent structures in one list:
   const int *sid = nullptr;           // host [n] structure of every atom, or null for one structure
   int n_nodes = 0;                    // as CsrInput::n_nodes: types has n_nodes entries, j indexes 0 .. n_nodes - 1

@@ -955,7 +955,8 @@ class EngineBase : public Engine, protected BufRegistry {
     HIP_CHECK(hipSetDevice(device_));
     if (in.n < 0) throw InvalidArgument("negative atom count");
     const int n = in.n, nn = std::max(in.n, in.n_nodes);
-    if (nn > n && (in.sid || !in.rij)) throw InvalidArgument("a list with ghost atoms holds one structure and gives its bond vectors");
+    const bool vectors = in.rij || in.fill;
+    if (nn > n && (in.sid || !vectors)) throw InvalidArgument("a list with ghost atoms holds one structure and gives its bond vectors");
     std::vector<int> mu(nn);
     for (int a = 0; a < nn; a++) {
       if (in.types[a] < 1 || in.types[a] > ntypes_) throw InvalidArgument("types must be 1 .. len(species)");
@@ -974,7 +975,7 @@ class EngineBase : public Engine, protected BufRegistry {
     nstruct_ = in.sid ? in.nstruct : 1;
     have_sid_ = in.sid != nullptr;
     sid_sorted_ = !in.sid || std::is_sorted(in.sid, in.sid + n);
-    have_rij_ = in.rij != nullptr;
+    have_rij_ = vectors;
     auto put = [&](DevBuf &b, const void *src, size_t bytes, hipMemcpyKind kind) {
       b.ensure(std::max<size_t>(bytes, 8));
       if (bytes) HIP_CHECK(hipMemcpyAsync(b.p, src, bytes, kind, stream_));
@@ -986,13 +987,19 @@ class EngineBase : public Engine, protected BufRegistry {
     ntiles_ = (int) tiles.size() / 16;
     put(tiles_, tiles.data(), sizeof(int) * tiles.size(), hipMemcpyHostToDevice);
     put(offset_, in.offset, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToDevice);
-    put(j_, in.j, sizeof(int) * in.nb, hipMemcpyDeviceToDevice);
     if (have_sid_) put(sid_, in.sid, sizeof(int) * n, hipMemcpyHostToDevice);
-    if (have_rij_) put(rij_, in.rij, sizeof(double) * 3 * in.nb, hipMemcpyDeviceToDevice);
-    else {
-      put(image_, in.image, sizeof(int) * in.nb, hipMemcpyDeviceToDevice);
-      put(x_, in.x, sizeof(double) * 3 * n, hipMemcpyDeviceToDevice);
-      put(shifts_, in.shifts, sizeof(double) * 3 * in.nimages, hipMemcpyHostToDevice);
+    if (in.fill) {
+      j_.ensure(std::max<size_t>(sizeof(int) * (size_t) in.nb, 8));
+      rij_.ensure(std::max<size_t>(sizeof(double) * 3 * (size_t) in.nb, 8));
+      in.fill(j_.as<int>(), rij_.as<double>(), stream_);
+    } else {
+      put(j_, in.j, sizeof(int) * in.nb, hipMemcpyDeviceToDevice);
+      if (have_rij_) put(rij_, in.rij, sizeof(double) * 3 * in.nb, hipMemcpyDeviceToDevice);
+      else {
+        put(image_, in.image, sizeof(int) * in.nb, hipMemcpyDeviceToDevice);
+        put(x_, in.x, sizeof(double) * 3 * n, hipMemcpyDeviceToDevice);
+        put(shifts_, in.shifts, sizeof(double) * 3 * in.nimages, hipMemcpyHostToDevice);
+      }
     }
     HIP_CHECK(hipStreamSynchronize(stream_));
     ran_ = false;

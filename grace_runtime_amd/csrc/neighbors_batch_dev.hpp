@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void k_bnl_pairs(const BnlStruct *__restrict__
 class BatchDeviceNeighbors {
  public:
   int64_t nb = 0;
-  DevBuf offset, j, rij;          // [N + 1] i64, [nb] i32, [nb][3] f64
+  DevBuf offset;                  // [N + 1] i64
   std::vector<int> sid;           // structure of every atom (host)
 
   // Whether a batch whose positions are on the host may have its lists from here, with the bonds that the cell lists of
@@ -166,8 +166,9 @@ class BatchDeviceNeighbors {
     build(nstruct, natoms, x_.as<double>(), cells, pbc, cutoff, stream);
   }
 
-  // natoms [nstruct] (host), pos [N][3] (device), cells [nstruct][3][3] and pbc [nstruct][3] (host).  A direction is
-  // periodic when its flag is set and its cell vector is not zero; the other cell vectors are not read.
+  // Bonds of every atom (offset, nb); fill() writes them.  natoms [nstruct] (host), pos [N][3] (device), cells [nstruct][3][3] and
+  // pbc [nstruct][3] (host).  A direction is periodic when its flag is set and its cell vector is not zero; the other cell vectors
+  // are not read.  The stream has been waited for on return.
   void build(int nstruct, const int *natoms, const double *pos, const double *cells, const unsigned char *pbc, double cutoff,
              hipStream_t stream)
   {
@@ -186,6 +187,8 @@ class BatchDeviceNeighbors {
     sid.resize((size_t) N);
     for (int s = 0; s < nstruct; s++) std::fill(sid.begin() + tab[s].first, sid.begin() + tab[s].first + tab[s].n, s);
     nb = 0;
+    n_ = (int) N;
+    rc2_ = cutoff * cutoff;
     offset.ensure(sizeof(long long) * (size_t) (N + 1));
     if (N == 0) {
       const long long z = 0;
@@ -202,22 +205,29 @@ class BatchDeviceNeighbors {
     hipLaunchKernelGGL(k_bnl_wrap, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, stream, tab_.as<BnlStruct>(), sid_.as<int>(), pos,
                        xw_.as<double>(), n);
     const dim3 grid((unsigned) ((n + 3) / 4)), block(256);
-    hipLaunchKernelGGL(k_bnl_pairs<false>, grid, block, 0, stream, tab_.as<BnlStruct>(), sid_.as<int>(), xw_.as<double>(), cutoff * cutoff, n,
+    hipLaunchKernelGGL(k_bnl_pairs<false>, grid, block, 0, stream, tab_.as<BnlStruct>(), sid_.as<int>(), xw_.as<double>(), rc2_, n,
                        count_.as<int>(), (const long long *) nullptr, (int *) nullptr, (double *) nullptr);
     launch_scan(stream, count_.as<int>(), n, offset.as<long long>());
     long long total = 0;
     HIP_CHECK(hipMemcpyAsync(&total, offset.as<long long>() + n, sizeof(total), hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(stream));    // also: the host tables above are free to go
     nb = total;
-    j.ensure(sizeof(int) * (size_t) std::max<int64_t>(nb, 1));
-    rij.ensure(sizeof(double) * 3 * (size_t) std::max<int64_t>(nb, 1));
-    hipLaunchKernelGGL(k_bnl_pairs<true>, grid, block, 0, stream, tab_.as<BnlStruct>(), sid_.as<int>(), xw_.as<double>(), cutoff * cutoff, n,
-                       (int *) nullptr, (const long long *) offset.as<long long>(), j.as<int>(), rij.as<double>());
+  }
+  // j [nb] and rij [nb][3] of the bonds that build() counted, into the memory of whoever uses them: a list of 28 bytes per bond is
+  // held once
+  void fill(int *j, double *rij, hipStream_t stream) const
+  {
+    if (nb == 0) return;
+    hipLaunchKernelGGL(k_bnl_pairs<true>, dim3((unsigned) ((n_ + 3) / 4)), dim3(256), 0, stream, tab_.as<BnlStruct>(), sid_.as<int>(), xw_.as<double>(), rc2_,
+                       n_, (int *) nullptr, (const long long *) offset.as<long long>(), j, rij);
     HIP_CHECK(hipGetLastError());
   }
 
  private:
   DevBuf tab_, sid_, xw_, count_, x_;
+  int n_ = 0;
+  double rc2_ = 0.0;
 
   static void fill_cell(const double *cell, const unsigned char *pbc, double cutoff, BnlStruct &b)
   {

@@ -282,6 +282,31 @@ def test_release_buffers_gives_the_work_memory_back(model_dir):
     assert eng.fetch()["energy"] == 0.0
 
 
+@pytest.mark.parametrize("arrays", ["host", "device"])
+def test_the_list_of_a_batch_is_held_once(model_dir, arrays):
+    """28 bytes per bond, which are what an engine holds that is given the same list"""
+    pos, cell, pbc, types = cases.structure_alloy54()
+    copies, n = 100, len(pos)
+    perm, offset, j, image, shifts = kk.neighbor_search(pos, cell, pbc, 5.0)
+    x, nb = pos[perm], len(j)
+    rij = x[j] - np.repeat(x, np.diff(offset), axis=0) + shifts[image]
+    base = kk.memory_in_use()
+    eng = _engine(model_dir, "mix2", ["Mo", "W"])
+    eng.compute(np.tile(types[perm], copies), np.concatenate([[0], np.cumsum(np.tile(np.diff(offset), copies))]),
+                np.concatenate([j + q * n for q in range(copies)]), rij=np.tile(rij, (copies, 1)))
+    given = kk.memory_in_use() - base
+    del eng
+    base = kk.memory_in_use()
+    b = kk.Batch(kk.Model(cases.model_file(model_dir, "mix2")), ["Mo", "W"])
+    b.keep_buffers = True
+    batch = _pack([(pos, cell, pbc, types)] * copies)
+    out = b.compute(*batch, energies=True) if arrays == "host" else _device_run(b, *batch)
+    searched = kk.memory_in_use() - base
+    assert np.abs(out["energy"] - out["energy"][0]).max() < 1e-9 * abs(out["energy"][0])
+    # beside the list the search keeps 72 bytes per atom and a table of 200 per cell; every buffer is allocated an eighth larger
+    assert searched < given + 1.125 * (200 * copies * n + 300 * copies) + 65536 < given + 1.125 * 28 * nb * copies / 2
+
+
 @pytest.mark.parametrize("far", [0, 3, 5000])
 def test_host_batches_equal_one_system_call_per_structure(model_dir, far):
     """Batch.compute takes its lists from the device search or, for atoms more than 1024 cells away (far = 5000) and for
