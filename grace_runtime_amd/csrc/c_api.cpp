@@ -1506,13 +1506,12 @@ int gr_compute_batch_device_uq(gr_engine *e, int nstruct, const int *natoms, con
         while (g1 < nstruct && start[g1 + 1] - start[g0] <= fit) g1++;
         const int ns = g1 - g0;
         const int64_t a0 = start[g0], na = start[g1] - a0;
-        nl.build(ns, natoms + g0, positions + 3 * a0, cells + 9 * (size_t) g0, pbc + 3 * (size_t) g0, rc, e->bnl_stream);
         // atom types: 4 bytes per atom to the host, where the element tiles of the tile GEMMs are laid out
         e->pin_types.ensure(sizeof(int) * (size_t) std::max<int64_t>(na, 1));    // pinned: the copy is a DMA, not a staged one
         int *ty_pinned = e->pin_types.as<int>();
         if (na > 0 && hipMemcpyAsync(ty_pinned, types + a0, sizeof(int) * (size_t) na, hipMemcpyDeviceToHost, e->bnl_stream) != hipSuccess)
           throw grhip::Error("copy of the atom types failed");
-        if (hipStreamSynchronize(e->bnl_stream) != hipSuccess) throw grhip::Error("the device neighbour search failed");
+        nl.build(ns, natoms + g0, positions + 3 * a0, cells + 9 * (size_t) g0, pbc + 3 * (size_t) g0, rc, e->bnl_stream);    // waits for the types too
         const std::vector<int> ty(ty_pinned, ty_pinned + na);
         grhip::DeviceCsr in;
         in.n = (int) na;

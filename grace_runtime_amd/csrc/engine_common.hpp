@@ -964,11 +964,16 @@ class EngineBase : public Engine, protected BufRegistry {
       if (mu[a] < 0)
         throw Error(who_ + ": atom " + std::to_string(a) + " of unmapped type " + std::to_string(in.types[a]) + " in the atom list");
     }
-    HIP_CHECK(hipStreamSynchronize(stream_));
     if (in.nstruct < 1) throw InvalidArgument("the number of structures must be positive");
     if (in.sid)
       for (int a = 0; a < n; a++)
         if (in.sid[a] < 0 || in.sid[a] >= in.nstruct) throw InvalidArgument("structure index of an atom out of range");
+    HIP_CHECK(hipStreamSynchronize(stream_));
+    if (in.fill) {    // first, so that the list is written while the host lays out the tiles
+      j_.ensure(std::max<size_t>(sizeof(int) * (size_t) in.nb, 8));
+      rij_.ensure(std::max<size_t>(sizeof(double) * 3 * (size_t) in.nb, 8));
+      in.fill(j_.as<int>(), rij_.as<double>(), stream_);
+    }
     n_ = n;
     n_nodes_ = nn;
     nb_ = in.nb;
@@ -976,23 +981,19 @@ class EngineBase : public Engine, protected BufRegistry {
     have_sid_ = in.sid != nullptr;
     sid_sorted_ = !in.sid || std::is_sorted(in.sid, in.sid + n);
     have_rij_ = vectors;
+    mu_host_.assign(mu.begin(), mu.begin() + n);    // the central atoms: they make the element tiles
+    chunk_laid_out_ = 0;
+    const std::vector<int> tiles = element_tiles(mu_host_, nelem_, tile_el_);
+    ntiles_ = (int) tiles.size() / 16;
     auto put = [&](DevBuf &b, const void *src, size_t bytes, hipMemcpyKind kind) {
       b.ensure(std::max<size_t>(bytes, 8));
       if (bytes) HIP_CHECK(hipMemcpyAsync(b.p, src, bytes, kind, stream_));
     };
     put(mu_, mu.data(), sizeof(int) * nn, hipMemcpyHostToDevice);
-    mu_host_.assign(mu.begin(), mu.begin() + n);    // the central atoms: they make the element tiles
-    chunk_laid_out_ = 0;
-    const std::vector<int> tiles = element_tiles(mu_host_, nelem_, tile_el_);
-    ntiles_ = (int) tiles.size() / 16;
     put(tiles_, tiles.data(), sizeof(int) * tiles.size(), hipMemcpyHostToDevice);
     put(offset_, in.offset, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToDevice);
     if (have_sid_) put(sid_, in.sid, sizeof(int) * n, hipMemcpyHostToDevice);
-    if (in.fill) {
-      j_.ensure(std::max<size_t>(sizeof(int) * (size_t) in.nb, 8));
-      rij_.ensure(std::max<size_t>(sizeof(double) * 3 * (size_t) in.nb, 8));
-      in.fill(j_.as<int>(), rij_.as<double>(), stream_);
-    } else {
+    if (!in.fill) {
       put(j_, in.j, sizeof(int) * in.nb, hipMemcpyDeviceToDevice);
       if (have_rij_) put(rij_, in.rij, sizeof(double) * 3 * in.nb, hipMemcpyDeviceToDevice);
       else {
