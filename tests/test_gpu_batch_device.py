@@ -1,7 +1,8 @@
 """`Batch.compute_device` (gr_compute_batch_device through the C ABI): atoms and results in device memory, neighbour
-lists built on the device.  Checked against `Batch.compute` on the same structures, and `Batch.compute`, which takes small
-structures through the same search, against one `System` call per structure: periodic, triclinic with atoms outside the cell, slab, molecule, and the small cells of the batched
-workload.  The two paths sum the same bonds in different orders: 1e-9 relative.  Needs an MI355X: run with -m gpu."""
+lists built on the device, and `Batch.compute`, which takes small structures through the same search and others through lists
+of the host.  Checked against one `System` call per structure, whose list is neither: periodic, triclinic with atoms outside the cell,
+slab, molecule, and the small cells of the batched workload.  The paths sum the same bonds in different orders: 1e-9 relative.
+Needs an MI355X: run with -m gpu."""
 import os
 
 import numpy as np
@@ -53,6 +54,13 @@ def _compare(out, ref):
     assert np.abs(out["energies"] - ref["energies"]).max() < 1e-9 * fs
 
 
+def _one_by_one(model, species, structs):
+    """one System call per structure, as _compare takes it"""
+    one = [kk.System(model, species, skin=0.0).compute(np.asarray(t, np.int32), x, c, np.asarray(p, bool), energies=True) for x, c, p, t in structs]
+    return {"energy": np.array([o["energy"] for o in one]), "virial": np.stack([o["virial"] for o in one]),
+            "forces": np.concatenate([o["forces"] for o in one]), "energies": np.concatenate([o["energies"] for o in one])}
+
+
 def test_device_lists_over_few_and_many_images(model_dir):
     """cells whose images number 1, 9, 27, 63, 64 or more per step of the search, 125 and 343 (more than the table of shifts holds)"""
     rng = np.random.default_rng(5)
@@ -63,30 +71,34 @@ def test_device_lists_over_few_and_many_images(model_dir):
         pos = np.array([[0.1, 0.2, 2.2 * q] for q in range(n)]) + rng.uniform(-0.1, 0.1, (n, 3)) + np.array(edges) * np.array(pbc) * rng.integers(-2, 3, (n, 3))
         structs.append((pos, np.diag(edges), np.array(pbc, bool), rng.integers(1, 3, n)))
     natoms, types, pos, cells, pbc = _pack(structs)
-    b = kk.Batch(_engine(model_dir, "mix2", ["Mo", "W"]).model, ["Mo", "W"])
-    ref = b.compute(natoms, types, pos, cells, pbc, energies=True)
-    _compare(_device_run(b, natoms, types, pos, cells, pbc), ref)
+    model = kk.Model(cases.model_file(model_dir, "mix2"))
+    _compare(_device_run(kk.Batch(model, ["Mo", "W"]), natoms, types, pos, cells, pbc), _one_by_one(model, ["Mo", "W"], structs))
 
 
 @pytest.mark.parametrize("name", ["mix2", "l2mix", "l3mix"])
-def test_device_batch_equals_host_batch(model_dir, name):
+def test_batches_equal_one_system_call_per_structure(model_dir, name):
+    """compute_device, and compute over both searches: with one atom 1100 cells away the lists of all structures are the host's"""
     eng = _engine(model_dir, name, ["Mo", "W"])
     mol = cases.structure_molecule()
     structs = [cases.structure_alloy54(), cases.structure_triclinic(), cases.structure_slab(),
                (mol[0], np.zeros((3, 3)), mol[2], mol[3])]
     natoms, types, pos, cells, pbc = _pack(structs)
     b = kk.Batch(eng.model, ["Mo", "W"])
-    ref = b.compute(natoms, types, pos, cells, pbc, energies=True)
+    ref = _one_by_one(eng.model, ["Mo", "W"], structs)
     out = _device_run(b, natoms, types, pos, cells, pbc)
     assert b.passes == 1
     _compare(out, ref)
+    _compare(b.compute(natoms, types, pos, cells, pbc, energies=True), ref)
+    far = pos.copy()
+    far[60] += 1100 * cells[1, 1]
+    _compare(b.compute(natoms, types, far, cells, pbc, energies=True), ref)
+    for x in (pos, far):
+        eo = b.compute(natoms, types, x, cells, pbc, energy_only=True)
+        assert np.abs(eo["energy"] - ref["energy"]).max() < 1e-9 * max(1.0, np.abs(ref["energy"]).max())
     eo = _device_run(b, natoms, types, pos, cells, pbc, energy_only=True, energies=False)
     assert np.abs(eo["energy"] - ref["energy"]).max() < 1e-9 * max(1.0, np.abs(ref["energy"]).max())
     # a second call with fewer structures reuses the buffers
-    sub = _pack(structs[1:3])
-    out2 = _device_run(b, *sub)
-    ref2 = b.compute(*sub, energies=True)
-    _compare(out2, ref2)
+    _compare(_device_run(b, *_pack(structs[1:3])), _one_by_one(eng.model, ["Mo", "W"], structs[1:3]))
 
 
 def test_small_cells_with_several_images_per_direction(model_dir):
@@ -100,7 +112,7 @@ def test_small_cells_with_several_images_per_direction(model_dir):
     structs.append((np.array([[0.1, 0.2, 0.3]]), np.diag([3.0, 3.2, 2.8]), [True, True, True], np.array([2], np.int32)))
     natoms, types, pos, cells, pbc = _pack(structs)
     b = kk.Batch(eng.model, ["Al", "Ni", "Ti"])
-    ref = b.compute(natoms, types, pos, cells, pbc, energies=True)
+    ref = _one_by_one(eng.model, ["Al", "Ni", "Ti"], structs)
     out = _device_run(b, natoms, types, pos, cells, pbc)
     assert b.passes == 1
     _compare(out, ref)
@@ -327,12 +339,7 @@ def test_host_batches_equal_one_system_call_per_structure(model_dir, far):
         moved = np.concatenate([rng.integers(-far, far + 1, (len(s[0]), 3)) * np.asarray(s[2]) @ np.asarray(s[1], float) for s in structs])
         pos = pos + moved
     out = kk.Batch(model, ["Mo", "W"]).compute(natoms, types, pos, cells, pbc, energies=True)
-    start = np.concatenate([[0], np.cumsum(natoms)])
-    near = np.concatenate([s[0] for s in structs])
-    one = [kk.System(model, ["Mo", "W"], skin=0.0).compute(types[a:b], near[a:b], cells[q], pbc[q], energies=True)
-           for q, (a, b) in enumerate(zip(start[:-1], start[1:]))]
-    ref = {"energy": np.array([o["energy"] for o in one]), "virial": np.stack([o["virial"] for o in one]),
-           "forces": np.concatenate([o["forces"] for o in one]), "energies": np.concatenate([o["energies"] for o in one])}
+    ref = _one_by_one(model, ["Mo", "W"], structs)
     _compare(out, ref)
     eo = kk.Batch(model, ["Mo", "W"]).compute(natoms, types, pos, cells, pbc, energy_only=True)
     assert np.abs(eo["energy"] - ref["energy"]).max() < 1e-9 * max(1.0, np.abs(ref["energy"]).max())

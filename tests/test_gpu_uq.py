@@ -101,7 +101,8 @@ def test_uq_errors(model_dir):
 @pytest.mark.parametrize("name", ["uq2", "uq2l", "uq3l"])
 def test_batches_return_uq_per_atom_in_the_callers_order(model_dir, name):
     """Batch.compute(uq=True) and the gamma / atomic_sigma / gmm_cluster outputs of Batch.compute_device
-    (python/kk/kk_api.h:116-156) against one System call per structure, in one pass and in passes of one structure"""
+    (python/kk/kk_api.h:116-156) against one System call per structure, in one pass and in passes of one structure, and with one atom
+    1100 cells away, where Batch.compute takes the lists of its pass from the host, whose atom order is not the caller's"""
     import torch
     model = kk.Model(cases.model_file(model_dir, name))
     structs = [cases.structure_alloy54(), cases.structure_triclinic(), cases.structure_slab()]
@@ -114,8 +115,10 @@ def test_batches_return_uq_per_atom_in_the_callers_order(model_dir, name):
     want = {k: np.concatenate([o[k] for o in one]) for k in ("gamma", "atomic_sigma", "gmm_cluster")}
     b = kk.Batch(model, ["Mo", "W"])
     dev = torch.device("cuda", kk.device())
-    for max_nall in (1 << 21, 1):
-        out = b.compute(natoms, types, pos, cells, pbc, uq=True, max_nall=max_nall)
+    far = pos.copy()
+    far[60] += 1100 * cells[1, 1]
+    for x, max_nall in ((pos, 1 << 21), (pos, 1), (far, 1 << 21)):
+        out = b.compute(natoms, types, x, cells, pbc, uq=True, max_nall=max_nall)
         assert b.passes == (1 if max_nall > 1 else 3)
         assert np.array_equal(out["gmm_cluster"], want["gmm_cluster"])
         assert np.abs(out["gamma"] / want["gamma"] - 1).max() < 1e-9 and np.abs(out["atomic_sigma"] / want["atomic_sigma"] - 1).max() < 1e-9
