@@ -1,7 +1,7 @@
 """The element-dependent reduces (k_reduce_fwd, k_reduce_sum, k_reduce_bwd) where their launches can go wrong: a function of the
 chain that several functions of I1 and rho collect at once (more than two feeds of one adjoint row take a second launch that
-adds), tiles that are whole, part or one atom over, and structures and batches on both sides of the number of tiles from which
-a reduce is no longer split over several blocks.  Against the fp64 oracle at the bounds of the other parity tests."""
+adds), a layer of more reduces than one launch takes, tiles that are whole, part or one atom over, and structures and batches on
+both sides of the number of tiles from which a reduce is no longer split over several blocks.  Against the fp64 oracle at the bounds of the other parity tests."""
 import os
 
 import numpy as np
@@ -61,13 +61,32 @@ def test_one_function_collected_several_times(model_dir, tmp_path, model, extra,
     assert np.abs(out["forces"] - forces).max() < tf * fs
 
 
-# copies of a cell of two or more tiles (two species: every cell's tiles hold both): the reduces of the batch are split over
-# blocks below 4 x 256 / 5 tiles
+def _many_functions_model(base, tmp_path):
+    """the model with four more functions of I1, from A and AA alone, which feed I beside the first four: nine reduces of layer 1
+    where a launch takes eight"""
+    d = dict(np.load(base, allow_pickle=False))
+    nf = int(d["I1_n_funcs"][0])
+    assert nf == 4
+    d["I1_n_funcs"] = d["I1_n_funcs"] * 2
+    for src in ("I1_{}_A", "I1_{}_AA", "I_{}_I1"):
+        for key, plus in (("collect_ind", nf if src.startswith("I_") else 0), ("w_l_tile", 0), ("total_sum_ind", 0 if src.startswith("I_") else nf)):
+            old = d[src.format(key)]
+            d[src.format(key)] = np.concatenate([old, old + plus])
+    path = os.path.join(str(tmp_path), "functions.npz")
+    np.savez(path, **d)
+    return path
+
+
+# copies of a cell of two or more tiles (two species: every cell's tiles hold both).  With 256 CUs the five reduces of layer 1 go to
+# 512 / (5 x tiles) blocks each, no more than an eighth of their functions: one tile, three blocks up to 34 tiles, two up to 51, one
+# beyond; the single reduce of layer 2 is whole from 257 tiles on.  With nine reduces the eight of the first launch are whole from
+# 33 tiles on, the ninth is in parts.  Tiles of these batches: 17 atoms x copies / 16 and up to one more
 @pytest.mark.parametrize("model,natoms,copies,precision", [
-    ("grace_2l_small", 2, 1, 64), ("config5", 2, 1, 64), ("config5", 15, 1, 64), ("config5", 17, 1, 32), ("grace_2l_small", 17, 2, 64), ("config5", 17, 50, 64),
-    ("grace_2l_small", 17, 150, 64), ("config5", 17, 150, 64), ("config5", 17, 150, 32)])
-def test_few_and_many_tiles(model_dir, model, natoms, copies, precision):
-    path = _base(model_dir, model)
+    ("grace_2l_small", 2, 1, 64), ("config5", 2, 1, 64), ("config5", 15, 1, 64), ("config5", 17, 1, 32), ("grace_2l_small", 17, 2, 64), ("config5", 17, 31, 64),
+    ("config5", 17, 40, 64), ("config5", 17, 40, 32), ("grace_2l_small", 17, 40, 64), ("config5", 17, 50, 64), ("grace_2l_small", 17, 150, 64),
+    ("config5", 17, 150, 64), ("config5", 17, 150, 32), ("config5", 17, 245, 64), ("functions", 17, 1, 64), ("functions", 17, 20, 32), ("functions", 17, 40, 64)])
+def test_few_and_many_tiles(model_dir, tmp_path, model, natoms, copies, precision):
+    path = _many_functions_model(_base(model_dir, "config5"), tmp_path) if model == "functions" else _base(model_dir, model)
     species = [str(n) for n in kk.Model(path).element_names][:2]
     rng = np.random.default_rng(natoms)
     grid = np.array([[x, y, z] for x in range(3) for y in range(3) for z in range(2)])[:natoms]
