@@ -9,7 +9,7 @@
 //   k_gemm_jobs                  FC forward / reverse as tile GEMMs on MFMA               (fused_cpu.h:349-364)
 //   k_prod_fwd / k_prod_bwd      channel-wise CG products                                 (fused_cpu.h:409-475)
 //   k_reduce_fwd / k_reduce_bwd  rho reduce with per-element weights                      (fused_cpu.h:637-649)
-//   k_energy                     fp64 readout MLP and its reverse                         (fused_1l.cpp:378-427)
+//   k_energy_hidden, k_energy    fp64 readout MLP and its reverse                         (fused_1l.cpp:378-427)
 //   k_bond_bwd                   per-bond force, pair scatter, virial                     (fused_cpu.h:836-860,1027-1050)
 #pragma once
 

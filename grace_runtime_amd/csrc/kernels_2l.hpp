@@ -8,7 +8,7 @@
 //   k_pair_bwd_mfma, k_pair_bwd[_async]  its reverse: per-bond force of layer 2, dE/dI_j added to the neighbour's row
 //                  (bond_yi_bwd_g, bond_yi_commit, bond_scatter_bwd_t, bond_force: fused_cpu.h:836-942,1027-1050); the first
 //                  forms the sums over m on the matrix cores, the others on the vector unit
-//   k_energy_2l    readout with the two RMSNorms, fp64 (libgrace/src/fused_2l.cpp:548-615)
+//   k_energy_2l_hidden, k_energy_2l    readout with the two RMSNorms, fp64 (libgrace/src/fused_2l.cpp:548-615)
 //
 // The vector gather kernels run one block per atom with one thread per (slot, channel): a thread keeps its 2l+1 .. nlm
 // accumulators (or adjoints) in registers and walks the atom's bonds; everything that is the same for the whole block

@@ -1,8 +1,8 @@
-// Neighbour lists of many structures at once, built on the GPU from positions that already live there: the list of
+// Neighbour lists of many structures at once, built on the GPU: from positions that already live there the list of
 // Batch::compute_device of the reference's GPU module (python/kk/kk_api.h:141-146; its own device list is
-// libgrace/include/grace/kk/neighbors_kk.h BatchNeighborListKK).  Positions never visit the host; cells, periodic flags
-// and atom counts come from the host as in the reference.  Batch::compute sends its positions up and takes its lists from here
-// too where serves() allows it.
+// libgrace/include/grace/kk/neighbors_kk.h BatchNeighborListKK), whose positions never visit the host; cells,
+// periodic flags and atom counts come from the host as in the reference.  Batch::compute sends its positions up and takes its lists
+// from here too where serves() allows it.
 //
 // The batches this serves hold hundreds of small cells, so the search is the direct one: per structure the atoms are
 // wrapped into the cell along its periodic directions, and one wave per atom walks the (neighbour, image) candidates

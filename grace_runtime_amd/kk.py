@@ -775,8 +775,9 @@ class Batch:
         pb = np.ascontiguousarray(pbc, dtype=np.uint8)
         flags = (FLAG_ENERGY_ONLY if energy_only else 0) | (FLAG_EATOM if energies else 0)
         nth = len(os.sched_getaffinity(0)) if hasattr(os, "sched_getaffinity") else 1
-        # every structure's list is built on the host (in parallel); the structures go through the GPU in passes of whole
-        # structures with at most max_nall atoms (python/kk/kk_core.cpp:1311-1347: ONE pass unless the batch is larger)
+        # lists: from the search on the GPU when all structures of a pass are small, else built on the host (in parallel), as
+        # gr_compute_batch decides; the structures go through the GPU in passes of whole structures with at most max_nall atoms
+        # (python/kk/kk_core.cpp:1311-1347: ONE pass unless the batch is larger)
         start = np.concatenate([[0], np.cumsum(natoms, dtype=np.int64)])
         # after an allocation failure: a fresh engine and passes of half as many atoms, down to 16384, from the first
         # structure again (every pass overwrites its outputs); python/kk/kk_core.cpp:1452-1484 compute_with_retry

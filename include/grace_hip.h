@@ -354,7 +354,9 @@ int gr_system_list_get(gr_system *s, int64_t *perm, int64_t *offset, int32_t *j,
  * list, one engine pass, per-structure energies and virials).
  * gr_compute_batch: natoms [nstruct], types / positions of all atoms structure after structure, cells [nstruct][3][3],
  * pbc [nstruct][3]; per structure the bonds of gr_compute, from the device search of gr_compute_batch_device for small
- * structures, else from lists built on `nthreads` host threads (open directions padded); energy [nstruct], virial [nstruct][6], forces [N][3] and eatom [N] in the caller's atom order.
+ * structures (that of ALL structures of the call, if each has at most 2^16 candidates per atom and no atom is 1024 cells out),
+ * else from lists built on `nthreads` host threads (open directions padded); energy [nstruct], virial [nstruct][6],
+ * forces [N][3] and eatom [N] in the caller's atom order.
  * gr_engine_upload_batch / gr_engine_fetch_batch: the resident form for a caller with its own lists: one CSR list over
  * all atoms (no bond may join two structures) and the structure of every atom. */
 int gr_compute_batch(gr_engine *e, int nstruct, const int *natoms, const int *types, const double *positions, const double *cells,
