@@ -777,9 +777,10 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
       else radR1_.launch(stream_, ncu_, radR1_.has_tables() ? nullptr : ones_.as<T>(), eb, ecnt, xr_.as<double>(), emu_.as<int>(), R1, dR1, n_edges, nullptr, true);
     });
     stage("pair_fwd", [&] {
-      const size_t lds = (size_t) 2 * kAsyncChunkFwd * (pthreads + radR1_.noutp) * sizeof(T);
-      GR_PAIR(k_pair_fwd, dim3(nc), dim3(pthreads), lds, stream_, eoff, ej_.as<int>(), YG_.as<T>(), (const T *) R1, (const T *) M, P, nslot_, CRP_,
-              nl_, radR1_.noutp, yw, sink_.as<T>(), 0, nc, nslot_, rows.erow);
+      PairFwdArgs<T> pf{};
+      pf.eoff = eoff; pf.ej = ej_.as<int>(); pf.erow = rows.erow; pf.Y = YG_.as<T>(); pf.R1 = R1; pf.M = M; pf.P = P;
+      pf.nslot = nslot_; pf.C = CRP_; pf.noutp = radR1_.noutp; pf.ystride = yw; pf.natoms = nc;
+      launch_pair_fwd<T>(pf, nl_, 4 * ncu_, stream_);
     });
     stage("reduce_B", [&] { gemm(jB_, CRP_ / 16, C2P_ / 16, P, npf, B, nB_, 0); });
     chain_forward(c2_, "_L2", B);

@@ -944,14 +944,11 @@ template<class T> void Engine3L<T>::layer_forward(int k, bool forces, int yw, bo
     const int npf = L.nlmi * nlm_;
     pairP_.ensure(na * npf * L.CP * s);
     A_.ensure(na * L.nfA * L.CP * s);
-    const int spb = slots_per_block(L.nlmi, L.CP, 512), ngrp = (L.nlmi + spb - 1) / spb;
     stage(tg(k, "pair_fwd").c_str(), [&] {
-      const int pt = round_up(spb * L.CP, 64);
-      // rows of CP values and of noutp values go to LDS 16 bytes at a time
-      if ((L.CP * s) % 16 || (L.rad.noutp * s) % 16) throw Error("GRACE-3L: pair kernels need rows that are multiples of 16 bytes");
-      const size_t lds = (size_t) 2 * kAsyncChunkFwd * (pt + L.rad.noutp) * s;
-      GR_PAIR(k_pair_fwd, dim3((unsigned) ((n + 7) / 8 * 8 * ngrp)), dim3(pt), lds, stream_, eoff, ej_.as<int>(), YG_.as<T>(), (const T *) Rl,
-              (const T *) M_.as<T>(), pairP_.as<T>(), L.nlmi, L.CP, nl_, L.rad.noutp, yw, sink_.as<T>(), ngrp, n, spb, (const int *) nullptr);
+      PairFwdArgs<T> pf{};
+      pf.eoff = eoff; pf.ej = ej_.as<int>(); pf.Y = YG_.as<T>(); pf.R1 = Rl; pf.M = M_.as<T>(); pf.P = pairP_.as<T>();
+      pf.nslot = L.nlmi; pf.C = L.CP; pf.noutp = L.rad.noutp; pf.ystride = yw; pf.natoms = n;
+      launch_pair_fwd<T>(pf, nl_, 4 * ncu_, stream_);
     });
     stage(tg(k, "couple_YI").c_str(), [&] {
       hipLaunchKernelGGL(k_groups_fwd<T>, L.cg.grid(n, L.CP), dim3(256), 0, stream_, L.cg.job.template as<int>(), L.cg.grp.template as<LinGroup>(),
