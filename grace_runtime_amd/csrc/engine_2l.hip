@@ -836,7 +836,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
         pa.gM = gM_.as<T>(); pa.bsum = bsum_ptr();
         pa.nslot = nslot_; pa.nI = nI_; pa.C = CRP_; pa.noutp = radR1_.noutp; pa.natoms = nc;
         for (int q = 0; q < 16; q++) pa.drow[q] = drow_[q];
-        launch_pair_bwd_mfma(mp, pa, nl_, stream_);
+        launch_pair_bwd_mfma<T, true>(mp, pa, nl_, stream_);
       } else if (ordered_) {
         GR_PAIR_ORD(GR_ARGS)
       } else if (ch == 8) {

@@ -1206,7 +1206,7 @@ template<class T> void Engine3L<T>::layer_backward(int k, int yw)
       pa.gM = gM_.as<T>(); pa.bsum = bsum_ptr();
       pa.nslot = pa.nI = L.nlmi; pa.C = L.CP; pa.noutp = L.rad.noutp; pa.natoms = n;
       for (int q = 0; q < 16; q++) pa.drow[q] = drow_[q];
-      launch_pair_bwd_mfma(mp, pa, nl_, stream_);
+      launch_pair_bwd_mfma<T, false>(mp, pa, nl_, stream_);
     } else if (ordered_) {
       GR_PAIR_ORD(GR_ARGS, po)
       const long long nwork = 3 * (long long) (ecnt_ >= 0 ? ecnt_ : std::max<int64_t>(nb_, 1)) + 9ll * n;

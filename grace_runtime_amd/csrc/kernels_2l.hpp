@@ -704,16 +704,19 @@ __global__ void k_pair_bwd_async(const long long *__restrict__ eoff, const int *
 // A wave owns 16 channels of up to kPairMfmaSlots slots of one atom and works alone: nothing is staged for the block and no barrier
 // stands inside its loop.  Only the adjoint tiles, which every bond reads, sit in LDS ([slot][lm][16], its own area); the
 // harmonics, the radial rows and the message rows of the neighbours come from memory into registers in the layout in which
-// they are used.  The harmonics and radial rows of l + 1 are requested before the products of l, those of the next chunk's
-// l = 0 before the products of the last l, the neighbours' rows of the next chunk as soon as the last products have used
-// this chunk's and before the atomic additions of this chunk are sent (the counter of outstanding memory operations is in
-// order: a load behind an atomic waits for it).
-// Measured against its predecessor, whose block copied chunks of 16 bonds to LDS one chunk ahead and met at a barrier per
-// chunk (the compiler waits for ALL copies in flight before the next LDS read, so each chunk began by waiting for the copies
-// of the one after it): GRACE-2L, 32 000 atoms fp64 5.28 -> 3.94 ms, 3999 atoms fp32 0.443 -> 0.343, 107 atoms 44 -> 35 us;
-// GRACE-3L, both layers, 3001 atoms fp64 17.3 -> 14.5 ms, 701 fp32 3.09 -> 2.41, 96 atoms 0.80 -> 0.59.  The vector kernels
-// are behind both everywhere.  What bounds it: in fp64 the matrix work (6.4 ms of the 14.5) next to the traffic of the message
-// rows and of the atomic additions to their adjoints, which are written through (35 GB, 7 ms at the copy rate).
+// they are used.  The harmonics of the next l are requested before the products of one, the neighbours' rows of the next chunk as
+// soon as the last products have used this chunk's and before the atomic additions of this chunk are sent (the counter of
+// outstanding memory operations is in order: a load behind an atomic waits for it); the longest l comes first, so that the
+// first loads behind the atomics have its products to arrive under.
+// fp32 and fp64 matrix instructions do not run beside vector instructions of another wave of the SIMD (2000 x 4 fp64 MFMA of one wave
+// 243 us, 128 000 fp64 multiply-adds of another 292, both together 525), so what counts is their sum: l = 0, whose harmonic is
+// a constant without gradient, takes no matrix step, the last function of an even l (5 = 4 + 1, 9 = 8 + 1) is added by the vector unit
+// through its lane-broadcast operand instead of a step of its own (27 steps for three sums at lmax 5 instead of 36), and
+// addresses are a uniform base and a constant offset.  Kernel alone, before / now: GRACE-2L, 8000 atoms fp64 1.11 / 1.00 ms, 3999 atoms
+// fp32 396 / 341 us; GRACE-3L, 72 slots, 3001 atoms fp64 9.2 / 9.05 ms, 36 slots 4.62 / 4.39, 72 slots, 701 atoms fp32 1.63 / 1.54, 96 atoms
+// 0.318 / 0.300.  The vector kernels are behind everywhere.  What bounds it: in fp64 the matrix and vector work (5.2 of the 9.05
+// ms) next to the atomic additions, which are written through (1.6 ms of it); which neighbour's rows are read makes no difference.
+// Radial rows one l ahead: 2 % in fp32 rows per bond, spills elsewhere; contiguous ranges of atoms per XCD 8 % slower.
 // grid: as k_pair_bwd (pair_block, groups of wpb spw slots); block: 64 (C / 16) wpb threads, dynamic LDS per wave:
 // (spw NLM + 3) 16 values.
 template<class T> struct PairMfmaArgs {
@@ -727,58 +730,104 @@ template<class T> struct PairMfmaArgs {
   int drow[16];    // accumulator row of (lane / 16, register)
 };
 
-constexpr int pair_mfma_steps(int l) { return (2 * l + 1 + 3) / 4; }
+// Matrix steps of l (four k each): l odd, the last holds three; l even, the function left over goes to the vector unit
+constexpr int pair_mfma_steps(int l) { return (l + 1) / 2; }
+constexpr bool pair_mfma_rest(int l) { return l > 0 && l % 2 == 0; }
+// value of lane Q of every row of 16 lanes
+template<int Q> __device__ inline double row_bcast(double x)
+{
+  long long v = __builtin_bit_cast(long long, x);
+  v = __builtin_amdgcn_update_dpp(v, v, 0x150 + Q, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, v);
+}
+template<int Q> __device__ inline float row_bcast(float x)
+{
+  const int v = __builtin_bit_cast(int, x);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(v, v, 0x150 + Q, 0xf, 0xf, true));
+}
 // slots of a wave: the message values, their adjoints and the adjoint tiles of 4 x 36 functions are what fits two waves per
 // SIMD in fp64 (registers and LDS)
 constexpr int kPairMfmaSlots = 4;
 inline size_t pair_mfma_wave_lds(int nl, int spw, size_t value_bytes) { return ((size_t) spw * nl * nl + 3) * 16 * value_bytes; }
 
-// What a wave holds while it walks the bonds of its atom
-template<class T, int NL, int NQ> __device__ inline void pair_bwd_wave(const PairMfmaArgs<T> &a, int i, int s0, int n0, const T *Bw)
+// A wave walks the bonds of its atom, 16 at a time.  Per chunk the l are taken in the order NL - 1, 1, 2 .. NL - 2: the
+// longest first, since the loads behind the atomic additions of the chunk before wait for those.
+template<class T, int NL, int NQ, bool PAIRS> __device__ inline void pair_bwd_wave(const PairMfmaArgs<T> &a, int i, int s0, int n0, const T *Bw)
 {
   typedef typename Mfma<T>::v4 v4;
-  constexpr int NLM = NL * NL;
+  typedef const char __attribute__((address_space(1))) *bytes_t;
+  typedef const T __attribute__((address_space(1))) *value_t;
+  constexpr int NLM = NL * NL, NS = NL - 1, TS = (int) sizeof(T);
+  constexpr bool EARLY = NS >= 3;    // the message rows are read for the last time by the products of the last step
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int C = a.C;
-  const long long e0 = a.eoff[i], e1 = a.eoff[i + 1];
+  auto scalar = [](long long x) {
+    return (long long) (unsigned) __builtin_amdgcn_readfirstlane((int) x) | (long long) __builtin_amdgcn_readfirstlane((int) (x >> 32)) << 32;
+  };
+  const long long e0 = scalar(a.eoff[i]), e1 = scalar(a.eoff[i + 1]);
   const int nchunk = (int) ((e1 - e0 + 15) / 16);
   if (nchunk == 0) return;
   int rows[4];
 #pragma unroll
   for (int v = 0; v < 4; v++) rows[v] = a.drow[4 * g + v];
   const int myrow = a.drow[4 * g + (c & 3)];             // the bond whose sums lane (g, c < 4) ends up with
-  // bond of a row of chunk ch; rows beyond the last bond read it again, what they give is not used
-  auto bond = [&](int ch, int row) {
-    const long long e = e0 + 16ll * ch + row;
-    return e < e1 ? e : e1 - 1;
+  // a uniform base in scalar registers and an offset of the lane, in bytes: the empty statements keep the compiler from adding
+  // the two ahead of their use (it would keep, and spill, an address per l)
+  auto uniform = [](const T *p) {
+    bytes_t b = (bytes_t) p;
+    asm("" : "+s"(b));
+    return b;
   };
-  // the chunk requested next: its first bond, the neighbours of the lane's four bonds, their radial rows and the lane's row of
-  // the harmonics, both in values from the chunk's first (pair_rows() sees to it that they fit)
-  const int *rowlist = a.erow ? a.erow : a.ej;            // no branch in the loop: see `pin`
+  auto load = [](bytes_t b, unsigned offset, int values) {
+    asm("" : "+v"(offset) : "s"(b));
+    return *(value_t) (b + offset + values * TS);
+  };
+  // The chunk requested next: its first bond, the neighbours of the lane's four bonds, their radial rows (PAIRS: addresses, else
+  // bytes from the chunk's first) and, in bytes from the chunk's first, the lane's row of the harmonics and the row whose left-over
+  // functions it holds for its row of 16 lanes.  Bonds beyond the last read the last, what they give is not used.
+  const int *rowlist = PAIRS ? a.erow : a.ej;
   long long base = e0;
-  int jn[4], ro[4], yo = 0;
+  int jn[4];
+  const T *pr[4];
+  unsigned ro[4], yo = 0, yro = 0;
   auto next_bonds = [&](int ch) {
     base = e0 + 16ll * ch;
+    const int last = e1 - 1 - base > 15 ? 15 : (int) (e1 - 1 - base);      // negative behind the last chunk
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      const long long e = bond(ch, rows[v]);
-      jn[v] = a.ej[e];
-      const int er = rowlist[e];
-      ro[v] = (a.erow ? er - (int) base : (int) (e - base)) * a.noutp + n0 + c;
+      const int r = rows[v] < last ? rows[v] : last;
+      jn[v] = a.ej[base + r];
+      if (PAIRS) pr[v] = a.R1 + (long long) rowlist[base + r] * a.noutp + n0 + c;
+      else ro[v] = (unsigned) ((r < 0 ? 0 : r) * a.noutp + n0 + c) * TS;
     }
-    yo = (int) (bond(ch, c) - base) * a.ystr + g;
+    const int ry = c < last ? c : last, rr = myrow < last ? myrow : last;
+    if (last < 0) base = e1 - 1;
+    yo = (unsigned) ((ry < 0 ? 0 : ry) * a.ystr + g) * TS;
+    yro = (unsigned) ((rr < 0 ? 0 : rr) * a.ystr) * TS;
+  };
+  auto request_r = [&](T (&R)[4], T (&dR)[4], int l) {
+    if (PAIRS) {
+      const long long d = reinterpret_cast<const char *>(a.dR1) - reinterpret_cast<const char *>(a.R1) + (long long) l * C * TS;
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        R[v] = pr[v][l * C];
+        dR[v] = *reinterpret_cast<const T *>(reinterpret_cast<const char *>(pr[v]) + d);
+      }
+    } else {
+      const bytes_t Rb = uniform(a.R1 + base * a.noutp + l * C), dRb = uniform(a.dR1 + base * a.noutp + l * C);
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        R[v] = load(Rb, ro[v], 0);
+        dR[v] = load(dRb, ro[v], 0);
+      }
+    }
   };
   T m[NQ][4];
-  auto request_m = [&]() {
+  auto request_m = [&](int q) {
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const T *mp = a.M + ((long long) jn[v] * a.nslot + s0) * C + n0 + c;
-#pragma unroll
-      for (int q = 0; q < NQ; q++) m[q][v] = mp[q * C];
-    }
+    for (int v = 0; v < 4; v++) m[q][v] = a.M[((long long) jn[v] * a.nslot + s0 + q) * C + n0 + c];
   };
-  // an offset of zero that the compiler cannot see through: addresses formed with it stay where they are used instead of
-  // being computed for all l ahead of the loop (and spilled)
+  // an offset of zero that the compiler cannot see through: LDS reads stay where they are used
   auto opaque = []() {
     int z = 0;
     asm volatile("" : "+v"(z));
@@ -787,19 +836,24 @@ template<class T, int NL, int NQ> __device__ inline void pair_bwd_wave(const Pai
   // keeps the accumulation of x where it stands: the compiler otherwise moves the multiply-adds of all l behind the loop, to
   // the branch that uses their sum, and spills every matrix product
   auto pin = [](T &x) { asm volatile("" : "+v"(x)); };
-  auto request_y = [&](T (&y)[3][3], int l) {
-    const T *Y = a.YG + base * a.ystr;
-    const int yz = yo + opaque();
+  // y[k][s]: the lane's operand of matrix step s; for l even y[k][steps]: the left-over function of its bond `myrow`
+  auto request_y = [&](T (&y)[3][4], int l) {
+    const bytes_t Yb = uniform(a.YG + base * a.ystr);
 #pragma unroll
-    for (int s = 0; s < pair_mfma_steps(l); s++)
+    for (int k = 0; k < 3; k++) {
 #pragma unroll
-      for (int k = 0; k < 3; k++) y[k][s] = Y[yz + k * NLM + l * l + 4 * s];
+      for (int s = 0; s < pair_mfma_steps(l); s++) y[k][s] = load(Yb, yo, k * NLM + l * l + 4 * s);
+      if (pair_mfma_rest(l)) y[k][pair_mfma_steps(l)] = load(Yb, yro, k * NLM + l * l + 2 * l);
+    }
   };
+  auto order = [](int t) { return t == 0 ? NL - 1 : t; };
   const T *Bl = Bw + g * 16 + c;
+  const T y00 = a.YG[e0 * a.ystr];                        // the harmonic of l = 0: the same for every bond
   next_bonds(0);
-  T y[3][3], yn[3][3];
-  request_y(y, 0);
-  request_m();
+  T y[3][4], yn[3][4], R[4], dR[4], R0[4], dR0[4];
+  if (NS > 0) request_y(y, order(0));
+#pragma unroll
+  for (int q = 0; q < NQ; q++) request_m(q);
   for (int ch = 0; ch < nchunk; ch++) {
     const int nb = (int) (e1 - e0 - 16ll * ch < 16 ? e1 - e0 - 16ll * ch : 16);
     int jc[4];
@@ -813,37 +867,57 @@ template<class T, int NL, int NQ> __device__ inline void pair_bwd_wave(const Pai
       for (int v = 0; v < 4; v++) sI[q][v] = (T) 0;
 #pragma unroll
     for (int v = 0; v < 4; v++) pE[v] = p1[v] = p2[v] = (T) 0;
+    // l = 0: no gradient, and a sum that is the same for every bond
+    auto add_l0 = [&]() {
+      const int bz = opaque();
 #pragma unroll
-    for (int l = 0; l < NL; l++) {
-      // the radial rows of this l arrive under its first products, the harmonics of the next under all of them
-      T R[4], dR[4];
-      {
-        const T *Rb = a.R1 + base * a.noutp, *dRb = a.dR1 + base * a.noutp;
-        const int z = opaque();
+      for (int q = 0; q < NQ; q++) {
+        const T s = y00 * Bw[bz + q * NLM * 16 + c];
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-          const int o = ro[v] + l * C + z;
-          R[v] = Rb[o];
-          dR[v] = dRb[o];
+          sI[q][v] += R0[v] * s;
+          pE[v] += dR0[v] * (s * m[q][v]);
+          pin(sI[q][v]); pin(pE[v]);
         }
       }
-      if (l + 1 < NL) {
-        request_y(yn, l + 1);
-      } else {                      // behind the last chunk: the last bond again
-        next_bonds(ch + 1);
-        request_y(yn, 0);
-      }
+    };
+    if (NS == 0) {
+      request_r(R0, dR0, 0);
+      next_bonds(ch + 1);
+      add_l0();
+    }
+#pragma unroll
+    for (int t = 0; t < NS; t++) {
+      const int l = order(t);
+      // the radial rows of this l arrive under its first products, the harmonics of the next step under all of them
+      request_r(R, dR, l);
+      if (l == 1) request_r(R0, dR0, 0);
+      if (t + 1 == NS) next_bonds(ch + 1);
+      request_y(yn, order(t + 1 < NS ? t + 1 : 0));
       const int bz = opaque();
       __builtin_amdgcn_sched_barrier(0);
-      // k beyond 2 l + 1: zero in the harmonics (the adjoint rows read there belong to l + 1, or are the zero rows at the end)
-      const int last = pair_mfma_steps(l) - 1;
-      const bool in = 4 * last + g < 2 * l + 1;
+      if (!pair_mfma_rest(l)) {    // the fourth k of the last step: zero in the harmonics (the adjoint row read there is another one)
+        const int last = pair_mfma_steps(l) - 1;
 #pragma unroll
-      for (int k = 0; k < 3; k++) y[k][last] = in ? y[k][last] : (T) 0;
+        for (int k = 0; k < 3; k++) y[k][last] = g < 3 ? y[k][last] : (T) 0;
+      }
       T U[4] = {0, 0, 0, 0}, V1[4] = {0, 0, 0, 0}, V2[4] = {0, 0, 0, 0};
+      const int rest = pair_mfma_steps(l);
 #pragma unroll
       for (int q = 0; q < NQ; q++) {
         v4 aS = {0, 0, 0, 0}, a1 = {0, 0, 0, 0}, a2 = {0, 0, 0, 0};
+        if (pair_mfma_rest(l)) {
+          const T b = Bw[bz + (q * NLM + l * l + 2 * l) * 16 + c];
+          T yq[3];
+#pragma unroll
+          for (int k = 0; k < 3; k++) {
+            yq[k] = y[k][rest];
+            if (TS == 8) pin(yq[k]);        // in fp64 the twelve broadcast values of an l would be spilled: formed for every slot
+          }
+          aS = v4{row_bcast<0>(yq[0]) * b, row_bcast<1>(yq[0]) * b, row_bcast<2>(yq[0]) * b, row_bcast<3>(yq[0]) * b};
+          a1 = v4{row_bcast<0>(yq[1]) * b, row_bcast<1>(yq[1]) * b, row_bcast<2>(yq[1]) * b, row_bcast<3>(yq[1]) * b};
+          a2 = v4{row_bcast<0>(yq[2]) * b, row_bcast<1>(yq[2]) * b, row_bcast<2>(yq[2]) * b, row_bcast<3>(yq[2]) * b};
+        }
 #pragma unroll
         for (int s = 0; s < pair_mfma_steps(l); s++) {
           const T bq = Bl[bz + (q * NLM + l * l + 4 * s) * 16];
@@ -860,6 +934,7 @@ template<class T, int NL, int NQ> __device__ inline void pair_bwd_wave(const Pai
           pin(sI[q][v]); pin(U[v]); pin(V1[v]); pin(V2[v]);
         }
         __builtin_amdgcn_sched_barrier(0);
+        if (EARLY && t + 1 == NS) request_m(q);
       }
 #pragma unroll
       for (int v = 0; v < 4; v++) {
@@ -868,12 +943,16 @@ template<class T, int NL, int NQ> __device__ inline void pair_bwd_wave(const Pai
         p2[v] += R[v] * V2[v];
         pin(pE[v]); pin(p1[v]); pin(p2[v]);
       }
+      if (l == 1) add_l0();
 #pragma unroll
       for (int k = 0; k < 3; k++)
 #pragma unroll
-        for (int q = 0; q < 3; q++) y[k][q] = yn[k][q];
+        for (int q = 0; q < 4; q++) y[k][q] = yn[k][q];
     }
-    request_m();
+    if (!EARLY) {
+#pragma unroll
+      for (int q = 0; q < NQ; q++) request_m(q);
+    }
     __builtin_amdgcn_sched_barrier(0);
     // dE/dI of the neighbours
 #pragma unroll
@@ -912,7 +991,7 @@ template<class T, int NL, int NQ> __device__ inline void pair_bwd_wave(const Pai
   }
 }
 
-template<class T, int NL>
+template<class T, int NL, bool PAIRS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 2))) void k_pair_bwd_mfma(PairMfmaArgs<T> a)
 {
   constexpr int NLM = NL * NL;
@@ -932,10 +1011,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  if (nq == 4) pair_bwd_wave<T, NL, 4>(a, i, s0, n0, Bw);
-  else if (nq == 3) pair_bwd_wave<T, NL, 3>(a, i, s0, n0, Bw);
-  else if (nq == 2) pair_bwd_wave<T, NL, 2>(a, i, s0, n0, Bw);
-  else if (nq == 1) pair_bwd_wave<T, NL, 1>(a, i, s0, n0, Bw);
+  if (nq == 4) pair_bwd_wave<T, NL, 4, PAIRS>(a, i, s0, n0, Bw);
+  else if (nq == 3) pair_bwd_wave<T, NL, 3, PAIRS>(a, i, s0, n0, Bw);
+  else if (nq == 2) pair_bwd_wave<T, NL, 2, PAIRS>(a, i, s0, n0, Bw);
+  else if (nq == 1) pair_bwd_wave<T, NL, 1, PAIRS>(a, i, s0, n0, Bw);
 }
 
 // Values per row of the harmonics and their two gradient components in memory: at least 3 nlm + 3 (the last MFMA step of
@@ -974,11 +1053,23 @@ inline PairMfmaPlan pair_mfma_plan(int nslot, int C, int nl, size_t value_bytes,
 // 4 %: a block keeps its place until its last wave is done)
 inline int pair_mfma_waves(int asked) { return asked > 0 ? asked : 1; }
 
-template<class T> inline void launch_pair_bwd_mfma(const PairMfmaPlan &p, PairMfmaArgs<T> a, int nl, hipStream_t stream)
+template<class T, bool PAIRS> inline auto pair_bwd_kernel(int nl) -> void (*)(PairMfmaArgs<T>)
 {
-  void (*kern)(PairMfmaArgs<T>) = nl == 1 ? k_pair_bwd_mfma<T, 1> : nl == 2 ? k_pair_bwd_mfma<T, 2> : nl == 3 ? k_pair_bwd_mfma<T, 3>
-                                : nl == 4 ? k_pair_bwd_mfma<T, 4> : nl == 5 ? k_pair_bwd_mfma<T, 5> : nl == 6 ? k_pair_bwd_mfma<T, 6>
-                                                                                                            : k_pair_bwd_mfma<T, 7>;
+  switch (nl) {
+    case 1: return k_pair_bwd_mfma<T, 1, PAIRS>;
+    case 2: return k_pair_bwd_mfma<T, 2, PAIRS>;
+    case 3: return k_pair_bwd_mfma<T, 3, PAIRS>;
+    case 4: return k_pair_bwd_mfma<T, 4, PAIRS>;
+    case 5: return k_pair_bwd_mfma<T, 5, PAIRS>;
+    case 6: return k_pair_bwd_mfma<T, 6, PAIRS>;
+    default: return k_pair_bwd_mfma<T, 7, PAIRS>;
+  }
+}
+// PAIRS: engines whose bonds may share radial rows (erow); without, erow is never set
+template<class T, bool PAIRS> inline void launch_pair_bwd_mfma(const PairMfmaPlan &p, PairMfmaArgs<T> a, int nl, hipStream_t stream)
+{
+  void (*kern)(PairMfmaArgs<T>) = pair_bwd_kernel<T, false>(nl);
+  if constexpr (PAIRS) if (a.erow) kern = pair_bwd_kernel<T, true>(nl);
   if (p.lds > 48 * 1024)
     HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int) p.lds));
   a.spw = p.spw;

@@ -159,7 +159,7 @@ template<class T> static void run_bwd(const Problem<T> &p, const int *drow)
   a.eoff = eoff; a.ej = ej; a.erow = erow; a.YG = Y; a.R1 = R; a.dR1 = dR; a.M = M; a.gP = gP; a.gM = gM; a.bsum = bsum;
   a.nslot = p.nslot; a.nI = p.nslot; a.C = p.C; a.noutp = p.noutp; a.natoms = p.natoms;
   for (int q = 0; q < 16; q++) a.drow[q] = drow[q];
-  launch_pair_bwd_mfma<T>(plan, a, p.nl, 0);
+  launch_pair_bwd_mfma<T, true>(plan, a, p.nl, 0);
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipDeviceSynchronize());
   const std::vector<T> gotM = download(gM, nM);
