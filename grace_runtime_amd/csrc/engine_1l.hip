@@ -346,7 +346,7 @@ void Engine1L<T>::launch_radial(long long e_begin, long long e_count, const doub
                                 const long long *n_edges, bool tables, const PairedRows &rows)
 {
   if (rows.on) rad_.launch_paired(stream_, ncu_, rows, Rz, dRz);
-  else rad_.launch(stream_, ncu_, z_.as<T>(), e_begin, e_count, x, emu, Rz, dRz, n_edges, nullptr, tables);
+  else rad_.launch(stream_, ncu_, z_.as<T>(), e_begin, e_count, x, emu, Rz, dRz, n_edges, nullptr, tables, nb_);
 }
 
 template<class T> void Engine1L<T>::run(const RunFlags &fl)

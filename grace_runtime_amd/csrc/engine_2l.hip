@@ -672,7 +672,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     if (!tab_inside)
       stage("radial_R", [&] {
         if (rows.on) radR_.launch_paired(stream_, ncu_, rows, Rz, dRz);
-        else radR_.launch(stream_, ncu_, zA_.as<T>(), eb, ecnt, xr_.as<double>(), emu_.as<int>(), Rz, dRz, n_edges, nullptr, true);
+        else radR_.launch(stream_, ncu_, zA_.as<T>(), eb, ecnt, xr_.as<double>(), emu_.as<int>(), Rz, dRz, n_edges, nullptr, true, nb_);
       });
     ScatterArgs<T> sa{};
     sa.tb = tbR;
@@ -774,7 +774,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     T *R1 = moved_back(R1_.as<T>(), eb * radR1_.noutp), *dR1 = moved_back(dR1_.as<T>(), eb * radR1_.noutp);
     stage("radial_R1", [&] {
       if (rows.on) radR1_.launch_paired(stream_, ncu_, rows, R1, dR1);
-      else radR1_.launch(stream_, ncu_, radR1_.has_tables() ? nullptr : ones_.as<T>(), eb, ecnt, xr_.as<double>(), emu_.as<int>(), R1, dR1, n_edges, nullptr, true);
+      else radR1_.launch(stream_, ncu_, radR1_.has_tables() ? nullptr : ones_.as<T>(), eb, ecnt, xr_.as<double>(), emu_.as<int>(), R1, dR1, n_edges, nullptr, true, nb_);
     });
     stage("pair_fwd", [&] {
       PairFwdArgs<T> pf{};

@@ -931,7 +931,7 @@ template<class T> void Engine3L<T>::layer_forward(int k, bool forces, int yw, bo
   L.dR.ensure(ecap_ * L.rad.noutp * s);
   T *Rl = moved_back(L.R.template as<T>(), eb_ * L.rad.noutp), *dRl = moved_back(L.dR.template as<T>(), eb_ * L.rad.noutp);
   stage(tg(k, "radial").c_str(), [&] {
-    L.rad.launch(stream_, ncu_, L.fac.template as<T>(), eb_, ecnt_, xr_.as<double>(), emu_.as<int>(), Rl, dRl, n_edges, emi_.as<int>(), true);
+    L.rad.launch(stream_, ncu_, L.fac.template as<T>(), eb_, ecnt_, xr_.as<double>(), emu_.as<int>(), Rl, dRl, n_edges, emi_.as<int>(), true, nb_);
   });
   L.X.buf.ensure(L.X.bytes(na, s));
   T *X = L.X.buf.template as<T>();

@@ -464,9 +464,9 @@ template<class T> struct DevRadial {
   // z: [nel][CP] species weights of the neighbour (null, only where tables are used: rows without weights); e_count < 0: the
   // edge count is read from *n_edges on the device; emi: element of the central atom of every edge (species form only)
   // tables: use the radial tables when the engine was asked for them (the plain form only); otherwise, and for the debug
-  // entry points, the MLP is evaluated for every bond
+  // entry points, the MLP is evaluated for every bond.  listed: no more edges than this where e_count < 0 (< 0: not known)
   void launch(hipStream_t stream, int ncu, const T *z, long long e_begin, long long e_count, const double *x, const int *emu, T *Rz, T *dRz,
-              const long long *n_edges, const int *emi = nullptr, bool tables = false)
+              const long long *n_edges, const int *emi = nullptr, bool tables = false, long long listed = -1)
   {
     if (tables && has_tables()) {
       ensure_tables(stream, ncu);
@@ -478,14 +478,14 @@ template<class T> struct DevRadial {
                          mode == 1 ? emi : (const int *) nullptr, (const int *) sp_of_mu.as<int>(), (int) species_mu.size());
       return;
     }
-    launch_mlp(stream, ncu, z, e_begin, e_count, x, emu, Rz, dRz, n_edges, emi);
+    launch_mlp(stream, ncu, z, e_begin, e_count, x, emu, Rz, dRz, n_edges, emi, listed);
   }
   // only the listed rows, without the species weights (the plain form; no tables)
   void launch_paired(hipStream_t stream, int ncu, const PairedRows &rows, T *Rz, T *dRz)
   {
     RadialArgs<T> ra = mlp_args(nullptr, 0, -1, rows.x, nullptr, Rz, dRz, rows.n, nullptr);
     ra.uid = rows.uid;
-    run_mlp<true>(stream, ncu, ra);
+    run_mlp<true>(stream, ncu, ra, -1);
   }
   // tables requested (spline_n > 0) and, in the species form, within the memory they may take
   bool has_tables()
@@ -557,10 +557,10 @@ template<class T> struct DevRadial {
   }
   // the radial MLP itself for every edge of the range
   void launch_mlp(hipStream_t stream, int ncu, const T *z, long long e_begin, long long e_count, const double *x, const int *emu, T *Rz, T *dRz,
-                  const long long *n_edges, const int *emi)
+                  const long long *n_edges, const int *emi, long long listed = -1)
   {
     if (mode == 1 && !emi) throw Error("radial kernel: the species form needs the central element of every edge");
-    run_mlp<false>(stream, ncu, mlp_args(z, e_begin, e_count, x, emu, Rz, dRz, n_edges, emi));
+    run_mlp<false>(stream, ncu, mlp_args(z, e_begin, e_count, x, emu, Rz, dRz, n_edges, emi), e_count >= 0 ? e_count : listed);
   }
   RadialArgs<T> mlp_args(const T *z, long long e_begin, long long e_count, const double *x, const int *emu, T *Rz, T *dRz, const long long *n_edges,
                          const int *emi) const
@@ -590,8 +590,20 @@ template<class T> struct DevRadial {
     if constexpr (!LISTED) if (mode == 1) kern = hb == 4 ? k_radial<T, 4, 0, 1, W2L, false> : k_radial<T, 8, 0, 1, W2L, false>;
     return kern;
   }
-  template<bool LISTED> void run_mlp(hipStream_t stream, int ncu, const RadialArgs<T> &ra)
+  // most: no more edges than this (< 0: not known).  Up to three tiles of 16 edges per CU at width 64 and two at width 128 the
+  // waves of a block share a tile (times at k_radial_few).
+  template<bool LISTED> void run_mlp(hipStream_t stream, int ncu, const RadialArgs<T> &ra, long long most)
   {
+    const long long tiles = (most + 15) / 16;
+    if (!LISTED && most > 0 && tiles <= (hb == 4 ? 3 : 2) * (long long) ncu) {
+      auto few = mode == 1 ? (hb == 4 ? k_radial_few<T, 4, 0, 1> : k_radial_few<T, 8, 0, 1>)
+               : hb == 4   ? (act == 1 ? k_radial_few<T, 4, 1, 0> : k_radial_few<T, 4, 0, 0>)
+                           : (act == 1 ? k_radial_few<T, 8, 1, 0> : k_radial_few<T, 8, 0, 0>);
+      const size_t bytes = (size_t) radial_few_lds(hb) * sizeof(T);
+      if (bytes > 48 * 1024) HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(few), hipFuncAttributeMaxDynamicSharedMemorySize, (int) bytes));
+      hipLaunchKernelGGL(few, dim3((unsigned) tiles), dim3(64 * hb), bytes, stream, ra);
+      return;
+    }
     const int threads = radial_threads(hb, mode, w2_in_lds != 0);
     auto kern = w2_in_lds ? mlp_kernel<true, LISTED>() : mlp_kernel<false, LISTED>();
     HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));

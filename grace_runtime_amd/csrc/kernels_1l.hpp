@@ -894,6 +894,176 @@ template<class T, int HB, int ACT, int MODE, bool W2L, bool LISTED> __global__ _
   }
 }
 
+// barrier of a block that exchanges through LDS only: __syncthreads would also wait for the loads and stores in flight
+__device__ inline void lds_barrier()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// k_radial for few edges: the HB waves of a block share a tile of 16 edges.  Wave w forms row block w of both hidden layers, whose
+// values go to LDS in the order in which the next layer takes them (an accumulator register is one k of the next operand), and
+// the column blocks w, w + HB .. of the output; the sums are those of k_radial in the same order.  The weights come from L2, those of
+// layer 1 and of a wave's first column block ahead of everything else.  In k_radial a wave walks the whole network for its tile
+// (29 700 cycles of matrix instructions in fp64 at width 64, 132 000 at width 128) behind the copy of all weights to LDS, however
+// many SIMDs have nothing to do.
+// Measured, k_radial / k_radial_few, us: width 64, 160 outputs, fp64 8 tiles 27 / 12, 371 tiles 30 / 19, 768 32 / 27, 1024 33 / 34; fp32 371
+// tiles 20 / 13, 768 22 / 18, 1024 23 / 21; width 128, 384 outputs, fp64 128 tiles 89 / 35, 371 93 / 67, 512 95 / 73, 768 100 / 106; fp32 371
+// tiles 65 / 38, 512 66 / 40, 1024 71 / 74.  What bounds it: one tile per CU takes the latency of its three layers (the activations
+// of 16 values per wave run at one wave per SIMD), more tiles take turns.
+// dynamic LDS: radial_few_lds(HB) values.
+constexpr int radial_few_lds(int hb) { return 2 * 2 * hb * 4 * 64; }
+template<class T, int HB, int ACT, int MODE> __global__ __launch_bounds__(64 * HB, HB == 4 ? 3 : 2) void k_radial_few(RadialArgs<T> a)
+{
+  typedef typename Mfma<T>::v4 v4;
+  constexpr int NS = HB * 4;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  T *const hs = reinterpret_cast<T *>(smem_raw);          // [stage][value, tangent][row block, register][lane]
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const long long cnt = a.e_count >= 0 ? a.e_count : *a.n_edges - a.e_begin;
+  const long long ntiles = (cnt + 15) / 16;
+  const int p = a.p;
+  const double cf0 = 0.5 * (p + 1) * (p + 2), cf1 = (double) p * (p + 2), cf2 = 0.5 * p * (p + 1), cfd = 0.5 * p * (p + 1) * (p + 2);
+  const int KZ = a.C >> 4;
+  // weights of the next 16 steps of a layer; behind those of layer 1 come those of the wave's first column block, and so on
+  constexpr int PF = 16;
+  T wq[PF];
+  const T *const wl1 = a.w1 + (w * NS) * 64 + lane, *const wl2 = a.w2 + lane;
+  auto column = [&](int cb) { return wl2 + (long long) cb * NS * 64; };
+  // value and tangent of stage `stage` times NS steps of weights, of which the first PF wait in wq; next: the weights after them
+  auto multiply = [&](int stage, const T *weights, const T *next, bool rows, v4 &h, v4 &dh) {
+    const T *hp = hs + stage * 2 * NS * 64 + lane;
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+      const T wv = wq[q % PF];
+      wq[q % PF] = q + PF < NS ? weights[(q + PF) * 64] : next[(q + PF - NS) * 64];
+      const T x = hp[q * 64], dx = hp[(NS + q) * 64];
+      h = rows ? Mfma<T>::mma(x, wv, h) : Mfma<T>::mma(wv, x, h);
+      dh = rows ? Mfma<T>::mma(dx, wv, dh) : Mfma<T>::mma(wv, dx, dh);
+      if (q % 8 == 7) __builtin_amdgcn_sched_barrier(0);    // or the operands of all steps are read ahead, and spilled
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < PF; q++) wq[q] = wl1[q * 64];
+  auto put = [&](int stage, const v4 &h, const v4 &dh) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      hs[((stage * 2 + 0) * NS + w * 4 + v) * 64 + lane] = h[v];
+      hs[((stage * 2 + 1) * NS + w * 4 + v) * 64 + lane] = dh[v];
+    }
+  };
+  auto activate = [&](v4 &h, v4 &dh) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      T s_ = h[v], d_ = dh[v];
+      act_pair<T, ACT>(s_, d_);
+      h[v] = s_; dh[v] = d_;
+    }
+  };
+  for (long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const long long eloc = tile * 16 + c;
+    const double x = eloc < cnt ? a.x[a.e_begin + eloc] : 0.5;
+    int row_v[4], zrow[4];
+    double xv[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int rl = a.drow[g * 4 + v];
+      const bool ok = tile * 16 + rl < cnt;
+      row_v[v] = ok ? rl * a.noutp : -1;
+      zrow[v] = (ok ? a.emu[a.e_begin + tile * 16 + rl] : 0) * a.C + c;
+      xv[v] = MODE == 1 && ok ? a.x[a.e_begin + tile * 16 + rl] : 0.5;
+    }
+    // basis, as in k_radial
+    T h0[kMaxRadBasis / 4], dh0[kMaxRadBasis / 4];
+    {
+      const double xpm = ipow(x, p - 1), xp = xpm * x, xp1 = xp * x, xp2 = xp1 * x;
+      const double fc = 1.0 - cf0 * xp + cf1 * xp1 - cf2 * xp2;
+      const double dfc = cfd * (-xpm + 2.0 * xp - xp1);
+      const double t = 2.0 * x - 1.0;
+      double Tp = 1.0, Tc = t, dTp = 0.0, dTc = 2.0;
+#pragma unroll
+      for (int s = 0; s < kMaxRadBasis / 4; s++) { h0[s] = (T) 0; dh0[s] = (T) 0; }
+      for (int k = 0; k < a.nrb; k++) {
+        const double gk = MODE == 1 ? Tc : Tc * fc, dgk = MODE == 1 ? dTc : dTc * fc + Tc * dfc;
+        if ((k & 3) == g) {
+#pragma unroll
+          for (int s = 0; s < kMaxRadBasis / 4; s++)
+            if (s == (k >> 2)) { h0[s] = (T) gk; dh0[s] = (T) dgk; }
+        }
+        const double Tn = 2.0 * t * Tc - Tp, dTn = 2.0 * (2.0 * Tc + t * dTc) - dTp;
+        Tp = Tc; dTp = dTc; Tc = Tn; dTc = dTn;
+      }
+    }
+    // ---- layer 0, row block w
+    {
+      v4 h = {0, 0, 0, 0}, dh = {0, 0, 0, 0};
+#pragma unroll
+      for (int s = 0; s < kMaxRadBasis / 4; s++)
+        if (s < a.ks0) {
+          const T wv = a.w0[(w * a.ks0 + s) * 64 + lane];
+          h = Mfma<T>::mma(wv, h0[s], h);
+          dh = Mfma<T>::mma(wv, dh0[s], dh);
+        }
+      if (MODE == 1) {
+        const long long ee = a.e_begin + (eloc < cnt ? eloc : 0);
+        const T *bi = a.bias_i + (long long) a.emi[ee] * (HB * 16), *bj = a.bias_j + (long long) a.emu[ee] * (HB * 16);
+#pragma unroll
+        for (int v = 0; v < 4; v++) h[v] += bi[w * 16 + a.drow[g * 4 + v]] + bj[w * 16 + a.drow[g * 4 + v]];
+      }
+      activate(h, dh);
+      put(0, h, dh);
+    }
+    lds_barrier();
+    // ---- layer 1, row block w
+    {
+      v4 h = {0, 0, 0, 0}, dh = {0, 0, 0, 0};
+      multiply(0, wl1, w < a.nob ? column(w) : wl1, false, h, dh);
+      if (MODE == 1) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) h[v] += a.bias1[w * 16 + a.drow[g * 4 + v]];
+      }
+      activate(h, dh);
+      put(1, h, dh);
+    }
+    lds_barrier();
+    // ---- layer 2, column blocks w, w + HB, ..
+    T env_v[4], denv_v[4];
+    if (MODE == 1) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const double xpm = ipow(xv[v], p - 1), xp = xpm * xv[v], xp1 = xp * xv[v], xp2 = xp1 * xv[v];
+        env_v[v] = (T) (1.0 - cf0 * xp + cf1 * xp1 - cf2 * xp2);
+        denv_v[v] = (T) (cfd * (-xpm + 2.0 * xp - xp1));
+      }
+    }
+    const long long first = (a.e_begin + tile * 16) * a.noutp;
+    T *const Rt = a.Rz + first, *const dRt = a.dRz + first;
+    for (int cb = w; cb < a.nob; cb += HB) {
+      T z[4];
+      const int kn = (cb & (KZ - 1)) * 16;
+#pragma unroll
+      for (int v = 0; v < 4; v++) z[v] = a.z[zrow[v] + kn];
+      v4 acc = {0, 0, 0, 0}, dacc = {0, 0, 0, 0};
+      multiply(1, column(cb), cb + HB < a.nob ? column(cb + HB) : wl1, true, acc, dacc);
+      const int col = cb * 16 + c;
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        if (row_v[v] >= 0) {
+          const int o = row_v[v] + col;
+          if (MODE == 1) {
+            Rt[o] = (T) (acc[v] * env_v[v] * z[v]);
+            dRt[o] = (T) ((dacc[v] * env_v[v] + acc[v] * denv_v[v]) * z[v]);
+          } else {
+            Rt[o] = (T) (acc[v] * z[v]);
+            dRt[o] = (T) (dacc[v] * z[v]);
+          }
+        }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // A basis
 // ---------------------------------------------------------------------------------------------------------------
@@ -1436,14 +1606,6 @@ __global__ __launch_bounds__(512) void k_gemm_jobs(GemmJobs<T> J, const T *X0, i
 }
 
 // ---- the jobs of a launch with one width of inputs and one of outputs, in the two shapes that few and many atom tiles need ----
-// barrier of a block that exchanges through LDS only: __syncthreads would also wait for the loads and stores in flight
-__device__ inline void lds_barrier()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // k_gemm_few: a wave owns ONE 16 x 16 tile of the output (an atom tile and a column block), so that a structure of a few
 // atom tiles still puts a wave on every SIMD, and the segments of a job are dealt to S waves whose sums meet in LDS (in the
 // order of the waves).  No operand passes through LDS and no wave waits for another before the end: both operands come from
