@@ -1407,13 +1407,14 @@ class EngineBase : public Engine, protected BufRegistry {
   {
     for (int q = 0; q < 16; q++) ba.drow[q] = drow_[q];
     const int kb = ba.C / 16;
-    const size_t lds = ((size_t) ba.nlm * (ba.C + 2) + (size_t) 4 * 16 * ba.nlm * 3) * sizeof(T);
+    const size_t lds = ((size_t) ba.nlm * (ba.C + 2) + (size_t) 4 * 16 * ba.nlm * 3) * sizeof(T);      // four tiles of bonds
     if (kb != 1 && kb != 2 && kb != 4) throw Error("bond backward: channel width must be 16, 32 or 64");
+    if (ba.tb.F && ba.noutp != ba.nl * ba.C) throw Error("bond backward: rows of the radial tables of another width");
 #define GR_BB(KB, NL)                                                                                  \
   do {                                                                                                 \
     auto kern = ba.tb.F ? k_bond_bwd<T, KB, NL, RowsOf::tables> : k_bond_bwd<T, KB, NL, RowsOf::bonds>; \
     if constexpr (PAIRS) if (ba.erow) kern = k_bond_bwd<T, KB, NL, RowsOf::pairs>;                     \
-    hipLaunchKernelGGL(kern, dim3(n), dim3(256), lds, stream_, ba);                                    \
+    hipLaunchKernelGGL(kern, dim3(n), dim3(64 * bond_bwd_block<T>()), lds, stream_, ba);               \
   } while (0)
 #define GR_BB_NL(NL) case NL: if (kb == 1) GR_BB(1, NL); else if (kb == 2) GR_BB(2, NL); else GR_BB(4, NL); break
     switch (ba.nl) {

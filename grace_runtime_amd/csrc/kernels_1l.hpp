@@ -1087,29 +1087,54 @@ __device__ inline int table_interval(double x, int N, double &t)
   t = sx - k;
   return k;
 }
-// the four table entries of column col in interval k (requested here, used by table_value)
-template<class T> __device__ inline void table_request(const RadialTable<T> &tb, int k, int col, int noutp, T (&raw)[4])
+// What the cubic of an interval takes from the bond, formed once for all its columns: t, and in fp64 the length of an interval, in
+// fp32 2 t and 3 t^2.
+template<class T> struct TableBond {
+  T t, u, w;
+};
+template<class T> __device__ inline TableBond<T> table_bond(double t, int N)
 {
-  if constexpr (sizeof(T) == 4) {
-    const T *c = tb.F + (long long) k * 4 * noutp + col;
-    raw[0] = c[0]; raw[1] = c[noutp]; raw[2] = c[2 * noutp]; raw[3] = c[3 * noutp];
+  if constexpr (sizeof(T) == 8) return {t, 1.0 / N, 0.0};
+  else return {(T) t, (T) 2 * (T) t, (T) 3 * (T) t * (T) t};
+}
+// Entry q of the four of interval k, column col: NOUT, the width of the rows, is a constant where these are used, so that the
+// entries stand at constant distances from one (fp64: two) addresses of a bond.
+template<class T> struct TableRow {
+  const T *f, *d;
+};
+template<class T, int NOUT> __device__ inline TableRow<T> table_row(const RadialTable<T> &tb, int k, int col)
+{
+  if constexpr (sizeof(T) == 8) return {tb.F + (long long) k * NOUT + col, tb.D + (long long) k * NOUT + col};
+  else return {tb.F + (long long) k * 4 * NOUT + col, nullptr};
+}
+template<int NOUT, class T> __device__ inline const T *table_entry(const TableRow<T> &r, int q)
+{
+  if constexpr (sizeof(T) == 8) return (q & 1 ? r.d : r.f) + (q >> 1) * NOUT;    // f0, d0, f1, d1
+  else return r.f + q * NOUT;
+}
+// The cubic of the four entries: fp64 from value and derivative at both ends, fp32 as stored.  (The fp64 slope in the Hermite basis,
+// (f1 - f0) 6 t (1 - t) + .., is half the operations and as accurate, but its rounding, eps N f, is another: 8e-14 of a virial.)
+template<class T> struct TableCubic {
+  T a0, a1, a2, a3;
+};
+template<class T> __device__ inline TableCubic<T> table_cubic(T e0, T e1, T e2, T e3, const TableBond<T> &b)
+{
+  if constexpr (sizeof(T) == 8) {
+    const T a1 = e1 * b.u, d1 = e3 * b.u;
+    return {e0, a1, (T) -3 * e0 - (T) 2 * a1 + (T) 3 * e2 - d1, (T) 2 * e0 + a1 - (T) 2 * e2 + d1};
   } else {
-    const T *f = tb.F + (long long) k * noutp + col, *d = tb.D + (long long) k * noutp + col;
-    raw[0] = f[0]; raw[1] = d[0]; raw[2] = f[noutp]; raw[3] = d[noutp];    // f0, f0', f1, f1'
+    return {e0, e1, e2, e3};
   }
 }
-// R(t) and, with DERIV, dR/dx of the cubic of the interval
-template<class T, bool DERIV> __device__ inline void table_value(const T (&raw)[4], T t, T h, T fN, T &R, T &dR)
+template<class T> __device__ inline T table_value(const TableCubic<T> &a, const TableBond<T> &b)
 {
-  T a0 = raw[0], a1 = raw[1], a2 = raw[2], a3 = raw[3];
-  if constexpr (sizeof(T) == 8) {
-    const T f1 = a2, d1 = a3 * h;
-    a1 *= h;
-    a2 = (T) -3 * a0 - (T) 2 * a1 + (T) 3 * f1 - d1;
-    a3 = (T) 2 * a0 + a1 - (T) 2 * f1 + d1;
-  }
-  R = a0 + t * (a1 + t * (a2 + t * a3));
-  if (DERIV) dR = (a1 + t * ((T) 2 * a2 + t * (T) 3 * a3)) * fN;
+  return a.a0 + b.t * (a.a1 + b.t * (a.a2 + b.t * a.a3));
+}
+// dR/dt, of which dR/dx is N times
+template<class T> __device__ inline T table_slope(const TableCubic<T> &a, const TableBond<T> &b)
+{
+  if constexpr (sizeof(T) == 8) return a.a1 + b.t * ((T) 2 * a.a2 + b.t * (T) 3 * a.a3);
+  else return a.a1 + b.u * a.a2 + b.w * a.a3;
 }
 
 // Where a kernel takes the radial functions of a bond from: its own row, the radial tables, or the row of its pair of atoms
@@ -1335,9 +1360,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // consecutive bytes of a table row; the 2.6 MB table of a 32-channel lmax-4 model stays in the L2), the cubic in t, times
 // the species weight.  The entries of step s + 1 are requested when those of step s have been turned into operands, and
 // arrive while the matrix instructions of step s run; x and the element of the lane's four bonds of the NEXT tile are
-// requested a tile ahead.  No radial row is read: the rows need not exist.  Three waves per SIMD in fp32: 32 channels
-// and lmax 4 take 182 registers left alone and spill 9 at 168, 65 536 atoms 778 -> 674 us together with the harmonics of four tiles
-// at once; 16 channels and lmax 6 take 187 and spill 18, 8192 atoms 96 -> 95 us; the other forms fit without spills.
+// requested a tile ahead.  No radial row is read: the rows need not exist.  Three waves per SIMD in fp32, with the harmonics of
+// four tiles at once: 65 536 atoms 778 -> 674 us.  No branch in a tile, constant distances between the entries of a bond: 32 768
+// atoms fp32 355 -> 331 us, 3999 atoms of 78 bonds 73.5 -> 63.4, 4001 atoms fp64 95.6 -> 95.4 (without the scheduling barrier 97).
 template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_scatter_a_tab(ScatterArgs<T> a)
 {
   typedef typename Mfma<T>::v4 v4;
@@ -1352,7 +1377,6 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) ==
   const long long w0 = a.eoff[i], w1 = a.eoff[i + 1];
   const int C = a.C;
   const RadialTable<T> tb = a.tb;
-  const T h = (T) (1.0 / tb.N), fN = (T) tb.N;
   v4 acc[NL][KB];
 #pragma unroll
   for (int l = 0; l < NL; l++)
@@ -1371,22 +1395,22 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) ==
     }
   };
   // one (step, 16-column block) at a time: NL x 4 entries in flight per lane
-  T raw[NL][4], zc = (T) 0, tt = (T) 0;
+  T raw[NL][4], zc = (T) 0;
+  double tt = 0.0;
   auto request = [&](int q) {    // q = s KB + cb
     const int s = q / KB, cb = q % KB;
-    double t;
-    const int k = table_interval(xs[s], tb.N, t);
-    tt = (T) t;
+    const int k = table_interval(xs[s], tb.N, tt);
     zc = tb.z[ms[s] * C + cb * 16 + c];
+    const TableRow<T> row = table_row<T, NL * KB * 16>(tb, k, c);
 #pragma unroll
-    for (int l = 0; l < NL; l++) table_request(tb, k, l * C + cb * 16 + c, a.noutp, raw[l]);
+    for (int l = 0; l < NL; l++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) raw[l][e] = table_entry<NL * KB * 16>(row, e)[(l * KB + cb) * 16];
   };
   if (w0 < w1) geometry(w0, xs, ms);
   for (long long eb = w0; eb < w1; eb += 16) {
-    const int nb = (int) (w1 - eb < 16 ? w1 - eb : 16);
     request(0);
-    const bool more = eb + 16 < w1;
-    if (more) geometry(eb + 16, xn, mn);
+    if (eb + 16 < w1) geometry(eb + 16, xn, mn);
     const int at = (int) (eb - w0) & (YB - 1);      // place of the tile in its round of harmonics
     if (at == 0) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1403,24 +1427,22 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) ==
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
+    // a step without a bond reads the tile's first again and multiplies with harmonics of zero: no branch in the tile
 #pragma unroll
     for (int q = 0; q < 4 * KB; q++) {
       const int s = q / KB, cb = q % KB;
-      if (4 * s >= nb) continue;                      // a step with no bond: neither evaluated nor multiplied
       T bv[NL];
+      const TableBond<T> bond = table_bond<T>(tt, tb.N);
 #pragma unroll
-      for (int l = 0; l < NL; l++) {
-        T R, dR;
-        table_value<T, false>(raw[l], tt, h, fN, R, dR);
-        bv[l] = R * zc;
-      }
-      if (q + 1 < 4 * KB && 4 * ((q + 1) / KB) < nb) request(q + 1);
+      for (int l = 0; l < NL; l++) bv[l] = table_value(table_cubic(raw[l][0], raw[l][1], raw[l][2], raw[l][3], bond), bond) * zc;
+      if (q + 1 < 4 * KB) request(q + 1);
       const T *yb = Yw + (at + 4 * s + g) * a.nlm;
 #pragma unroll
       for (int l = 0; l < NL; l++) {
         const T y = c < 2 * l + 1 ? yb[l * l + c] : (T) 0;       // A operand: row m = c
         acc[l][cb] = Mfma<T>::mma(y, bv[l], acc[l][cb]);
       }
+      if (sizeof(T) == 8) __builtin_amdgcn_sched_barrier(0);    // entries of a later step requested early spill in fp64
     }
 #pragma unroll
     for (int s = 0; s < 4; s++) { xs[s] = xn[s]; ms[s] = mn[s]; }
@@ -2615,11 +2637,18 @@ template<class T> struct BondBwdArgs {
 // them it is no faster), and left alone it takes 173 registers where 168 let a third wave in: tables, 65 536 atoms 1.85 -> 1.39 ms,
 // 3999 of GRACE-2L 183 -> 147 us; paired rows, 20 000 atoms 571 -> 536 us.  A fourth wave spills 42 registers (2.03 ms).  Rows of
 // their own serve small structures, which have one block per CU anyway (500 atoms 20.4 -> 21.9 us); from lmax 5 on, with 64
-// channels and in fp64 three waves spill.  Of the forms compiled for three waves one spills, paired rows of 32 channels and lmax 4
-// (200 registers left alone, 10 spilled): the form that the 20 000 atoms above take.
+// channels and in fp64 three waves spill.  Of the forms compiled for three waves two spill at 32 channels and lmax 4: tables 22
+// registers, paired rows 17.
 template<class T> constexpr int bond_bwd_waves(int kb, int nl, RowsOf rows) { return sizeof(T) == 4 && kb <= 2 && nl <= 5 && rows != RowsOf::bonds ? 3 : 1; }
 
-// One block (4 waves) per atom; a wave takes tiles of 16 bonds.  Per tile and l two tile GEMMs on the matrix cores,
+// Tiles of 16 bonds whose harmonics a wave evaluates at once, a bond per lane, and waves of a block.  One tile at a time leaves 48
+// lanes idle in the harmonics, half of the vector instructions of a tile in fp32.  Two tiles: paired rows, 8192 atoms fp32 198 -> 178 us,
+// tables, 3999 atoms of 78 bonds 156 -> 150; in fp64, where the harmonics of two tiles leave LDS for six waves of a CU, 203 -> 225 us
+// (tables, 4001 atoms), 21 -> 25 (128 atoms).
+template<class T> constexpr int bond_bwd_tiles() { return sizeof(T) == 4 ? 2 : 1; }
+template<class T> constexpr int bond_bwd_block() { return 4 / bond_bwd_tiles<T>(); }
+
+// One block per atom; a wave takes rounds of HT tiles of 16 bonds.  Per tile and l two tile GEMMs on the matrix cores,
 //   P[m][b] = sum_n gA[l*l + m][n] Rz[b][l][n],   Q[m][b] = sum_n gA[l*l + m][n] dRz[b][l][n]      (K = channels)
 // with the bonds as columns: lane (g, c) of the wave ends up with the rows m = drow[4 g + v] of bond c, so the sums over
 // m are four terms in the lane and two exchanges between the lane groups, and lane c < 16 -- the lane that evaluated
@@ -2631,166 +2660,195 @@ template<class T> constexpr int bond_bwd_waves(int kb, int nl, RowsOf rows) { re
 // the harmonics' gradients are kept as their two components along e1 and e2: two sums per bond instead of three, and a
 // third less LDS per block (three blocks per CU instead of two).  gA of the atom sits in LDS as [lm][C + 2]
 // (the pad spreads the rows over the banks); the radial rows of l + 1 are requested before the products of l.
-// KB = channels / 16, NL = lmax + 1.  dynamic LDS: nlm (C + 2) + 4 waves x 16 bonds x 3 nlm values.
+// KB = channels / 16, NL = lmax + 1.  dynamic LDS: nlm (C + 2) + 4 tiles x 16 bonds x 3 nlm values.
+// l = 0 has no gradient: its radial function is neither read nor evaluated, its derivative is (a tenth of the rows at lmax 4).  With
+// that, the harmonics of a bond in one row and fewer address instructions: paired rows, 8192 atoms fp64 280 -> 254 us, fp32 226 ->
+// 198; tables, 3999 atoms fp32 166 -> 156, 4001 atoms fp64 211 -> 204, and the tiles two at a time above.
 // RowsOf::tables: the B operands are formed from the radial tables (lane (g, c): the eight columns l C + 8 g + s of bond c, four table
 // entries each, value and derivative from the same four; requested for l + 1 before the products of l).
-template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(256, bond_bwd_waves<T>(KB, NL, ROWS)) void k_bond_bwd(BondBwdArgs<T> a)
+template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 * bond_bwd_block<T>(), bond_bwd_waves<T>(KB, NL, ROWS)) void k_bond_bwd(BondBwdArgs<T> a)
 {
+  constexpr int HT = bond_bwd_tiles<T>(), NW = bond_bwd_block<T>();
   constexpr bool TAB = ROWS == RowsOf::tables, PAIRS = ROWS == RowsOf::pairs;
   typedef typename Mfma<T>::v4 v4;
   constexpr int KS = KB * 4, C = KB * 16, CS = C + 2, NLM = NL * NL;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *gAl = reinterpret_cast<T *>(smem_raw);                          // [NLM][CS]
-  T *Ysh = gAl + NLM * CS;                                           // [4 waves][16][NLM]
-  T *Gsh = Ysh + 4 * 16 * NLM;                                       // [4 waves][16][2][NLM]: gradient . e1, gradient . e2
-  __shared__ double red[4][9];
+  T *Hsh = gAl + NLM * CS;                                           // [NW waves][16 HT][3][NLM]: harmonics, gradient . e1, gradient . e2
+  __shared__ double red[NW][9];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int c = lane & 15, g = lane >> 4;
   const int i = a.a0 + blockIdx.x;
-  const long long e0 = a.eoff[i], e1 = a.eoff[i + 1];
+  const long long e0 = a.eoff[i], e1_ = a.eoff[i + 1];
   {
     const T *gAi = a.gA + (long long) blockIdx.x * NLM * C;
-    for (int q = t; q < NLM * C; q += 256) gAl[(q / C) * CS + q % C] = gAi[q];
+    for (int q = t; q < NLM * C; q += 64 * NW) gAl[(q / C) * CS + q % C] = gAi[q];
   }
   __syncthreads();
-  T *Yw = Ysh + wave * 16 * NLM, *Gw = Gsh + wave * 16 * 2 * NLM;
+  T *Hw = Hsh + wave * HT * 16 * 3 * NLM;
   int mrow[4];
+  const T *hrow0 = Hw + c * 3 * NLM, *hrow[4];
 #pragma unroll
-  for (int v = 0; v < 4; v++) mrow[v] = a.drow[4 * g + v];
+  for (int v = 0; v < 4; v++) {
+    mrow[v] = a.drow[4 * g + v];
+    hrow[v] = hrow0 + mrow[v];
+  }
   double fi[3] = {0, 0, 0}, vir[6] = {0, 0, 0, 0, 0, 0};
-  const int ntile = (int) ((e1 - e0 + 15) / 16);
-  for (int tile = wave; tile < ntile; tile += 4) {
-    const long long eb = e0 + (long long) tile * 16;
-    const int nb = (int) (e1 - eb < 16 ? e1 - eb : 16);
-    const bool colok = c < nb;                      // B operand column = bond c of the tile
+  const int ntile = (int) ((e1_ - e0 + 15) / 16);
+  for (int round = wave; round * HT < ntile; round += NW) {
+    const long long er = e0 + (long long) round * HT * 16;
+    const int nr = (int) (e1_ - er < 16 * HT ? e1_ - er : 16 * HT);      // bonds of the round
     // rows read by this lane: without tables step s of lane group g is channel 8 (s / 2) + 2 g + s % 2 (CH), so that the
     // four lane groups read 64 consecutive bytes of a bond's row in one instruction; with tables channel g KS + s
-    const long long ec = eb + (colok ? c : 0), row = PAIRS ? (long long) a.erow[ec] : ec;
-    const T *rp = a.Rz + row * a.noutp + (TAB ? g * KS : 2 * g);
-    const T *dp = a.dRz + row * a.noutp + (TAB ? g * KS : 2 * g);
 #define CH(s_) (TAB ? (s_) : 8 * ((s_) >> 1) + ((s_) & 1))
+    const T *rp = nullptr, *dp = nullptr;
     T x[2][KS], dx[2][KS];
     // tables: interval, offset and species weights of bond c, and the entries of l = 0
     // (four columns at a time: the entries of the next four are requested before the products of these four)
     constexpr int KH = 4;
-    T raw[TAB ? KH : 1][4], zc[TAB || PAIRS ? KS : 1], tt = (T) 0;
-    int tk = 0;
-    const T th = TAB ? (T) (1.0 / a.tb.N) : (T) 0, tN = TAB ? (T) a.tb.N : (T) 0;
-    if constexpr (TAB) {
-      const long long e = eb + (colok ? c : 0);
-      double t;
-      tk = table_interval(a.tb.x[e], a.tb.N, t);
-      tt = (T) t;
-      const int mu = a.tb.emu[e];
+    T raw[4][TAB ? KH : 1], zc[TAB || PAIRS ? KS : 1];
+    TableBond<T> tt{};
+    TableRow<T> trow{};
+    // four columns from column `col` of the lane's eight on
+    auto request = [&](int col) {
+      constexpr int V = 16 / (int) sizeof(T);
+      typedef T piece __attribute__((ext_vector_type(16 / sizeof(T))));
 #pragma unroll
-      for (int s = 0; s < KS; s++) zc[s] = a.tb.z[mu * C + g * KS + s];
-    } else {
+      for (int e = 0; e < 4; e++)
 #pragma unroll
-      for (int s = 0; s < KS; s++) { x[0][s] = rp[CH(s)]; dx[0][s] = dp[CH(s)]; }
-      if constexpr (PAIRS) {
-        const int mu = a.emu[ec];
+        for (int q = 0; q < KH / V; q++) {
+          const piece w = *reinterpret_cast<const piece *>(table_entry<NL * C>(trow, e) + col + q * V);
 #pragma unroll
-        for (int s = 0; s < KS; s++) zc[s] = a.z[mu * C + 2 * g + CH(s)];
+          for (int s = 0; s < V; s++) raw[e][q * V + s] = w[s];
+        }
+    };
+    // the first rows (table entries) of the tile from bond eb on: of l = 0, whose gradient is zero, the derivative alone
+    auto begin = [&](long long eb) {
+      const long long e = eb + (eb + c < e1_ ? c : 0);
+      if constexpr (TAB) {
+        double t;
+        const int tk = table_interval(a.tb.x[e], a.tb.N, t);
+        tt = table_bond<T>(t, a.tb.N);
+        trow = table_row<T, NL * C>(a.tb, tk, g * KS);
+        const int mu = a.tb.emu[e];
+#pragma unroll
+        for (int s = 0; s < KS; s++) zc[s] = a.tb.z[mu * C + g * KS + s];
+        request(0);
+      } else {
+        const long long row = PAIRS ? (long long) a.erow[e] : e;
+        rp = a.Rz + row * a.noutp + 2 * g;
+        dp = a.dRz + row * a.noutp + 2 * g;
+#pragma unroll
+        for (int s = 0; s < KS; s++) dx[0][s] = dp[CH(s)];
+        if constexpr (PAIRS) {
+          const int mu = a.emu[e];
+#pragma unroll
+          for (int s = 0; s < KS; s++) zc[s] = a.z[mu * C + 2 * g + CH(s)];
+        }
       }
-    }
-    // geometry of bond `lane` (lanes below nb), kept for the end of the tile
+    };
+    begin(er);
+    // geometry of bond `lane` (lanes below nr), kept for the end of the round
     double u0 = 0, u1 = 0, u2 = 1, br = 1, brc = 1;
     double e1[3] = {1, 0, 0}, e2[3] = {0, 1, 0};
     int jj = 0;
-    if (lane < nb) {
-      const long long e = eb + lane;
+    if (lane < nr) {
+      const long long e = er + lane;
       u0 = a.rh[3 * e]; u1 = a.rh[3 * e + 1]; u2 = a.rh[3 * e + 2];
       br = a.r[e]; brc = a.rc[e]; jj = a.ej[e];
       const double u[3] = {u0, u1, u2};
       tangent_basis(u, e1, e2);
-      sh_eval<true, T, NL - 1>(a.sh, u0, u1, u2, Yw + lane * NLM, Gw + lane * 2 * NLM, e1, e2, Gw + lane * 2 * NLM + NLM);
+      T *h = Hw + lane * 3 * NLM;
+      sh_eval<true, T, NL - 1>(a.sh, u0, u1, u2, h, h + NLM, e1, e2, h + 2 * NLM);
     }
-    if constexpr (TAB) {
-#pragma unroll
-      for (int s = 0; s < KH; s++) table_request(a.tb, tk, g * KS + s, a.noutp, raw[s]);
-    }
-    // LDS writes of this wave visible to its other lanes (the Y / G region is private to the wave)
+    // LDS writes of this wave visible to its other lanes (its harmonics are private to the wave)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    double px = 0, p1 = 0, p2 = 0;
+    double px_r = 0, p1_r = 0, p2_r = 0;      // of bond er + lane
+    for (int ht = 0; ht < HT; ht++) {
+      const long long eb = er + 16 * ht;
+      if (HT > 1 && eb >= e1_) break;
+      const bool colok = eb + c < e1_;                // B operand column = bond c of the tile
+      double px = 0, p1 = 0, p2 = 0;
 #pragma unroll
-    for (int l = 0; l < NL; l++) {
-      const int cur = TAB ? 0 : (l & 1), nxt = cur ^ 1;
-      if constexpr (!TAB) {
-        if (l + 1 < NL) {
+      for (int l = 0; l < NL; l++) {
+        const int cur = TAB ? 0 : (l & 1), nxt = cur ^ 1;
+        if constexpr (!TAB) {
+          if (l + 1 < NL) {
 #pragma unroll
-          for (int s = 0; s < KS; s++) { x[nxt][s] = rp[(l + 1) * C + CH(s)]; dx[nxt][s] = dp[(l + 1) * C + CH(s)]; }
-        }
-      }
-      v4 aP = {0, 0, 0, 0}, aQ = {0, 0, 0, 0};
-      // A operand: row m = c of gA_l^T, k = g KS + s
-      const T *ga = gAl + (l * l + (c < 2 * l + 1 ? c : 0)) * CS + (TAB ? g * KS : 2 * g);
-      if constexpr (TAB) {
-#pragma unroll
-        for (int hb = 0; hb < KS; hb += KH) {
-          T xv[KH], dxv[KH];
-#pragma unroll
-          for (int s = 0; s < KH; s++) {
-            T R, dR;
-            table_value<T, true>(raw[s], tt, th, tN, R, dR);
-            xv[s] = R * zc[hb + s];
-            dxv[s] = dR * zc[hb + s];
-          }
-          // the next four columns: of this l, or the first four of l + 1
-          if (hb + KH < KS) {
-#pragma unroll
-            for (int s = 0; s < KH; s++) table_request(a.tb, tk, l * C + g * KS + hb + KH + s, a.noutp, raw[s]);
-          } else if (l + 1 < NL) {
-#pragma unroll
-            for (int s = 0; s < KH; s++) table_request(a.tb, tk, (l + 1) * C + g * KS + s, a.noutp, raw[s]);
-          }
-#pragma unroll
-          for (int s = 0; s < KH; s++) {
-            const T w = c < 2 * l + 1 ? ga[hb + s] : (T) 0;
-            aP = Mfma<T>::mma(w, xv[s], aP);
-            aQ = Mfma<T>::mma(w, dxv[s], aQ);
+            for (int s = 0; s < KS; s++) { x[nxt][s] = rp[(l + 1) * C + CH(s)]; dx[nxt][s] = dp[(l + 1) * C + CH(s)]; }
           }
         }
-      } else {
+        v4 aP = {0, 0, 0, 0}, aQ = {0, 0, 0, 0};
+        // A operand: row m = c of gA_l^T, k = g KS + s
+        const T *ga = gAl + (l * l + (c < 2 * l + 1 ? c : 0)) * CS + (TAB ? g * KS : 2 * g);
+        if constexpr (TAB) {
 #pragma unroll
-        for (int s = 0; s < KS; s++) {
-          const T w = c < 2 * l + 1 ? ga[CH(s)] : (T) 0;
-          T xs = x[cur][s], dxs = dx[cur][s];
-          if constexpr (PAIRS) {
-            xs *= zc[s];
-            dxs *= zc[s];
+          for (int hb = 0; hb < KS; hb += KH) {
+            T xv[KH], dxv[KH];
+#pragma unroll
+            for (int s = 0; s < KH; s++) {
+              const TableCubic<T> cubic = table_cubic(raw[0][s], raw[1][s], raw[2][s], raw[3][s], tt);
+              xv[s] = l > 0 ? table_value(cubic, tt) * zc[hb + s] : (T) 0;
+              dxv[s] = table_slope(cubic, tt) * zc[hb + s];
+            }
+            // the next four columns: of this l, or the first four of l + 1
+            if (hb + KH < KS) request(l * C + hb + KH);
+            else if (l + 1 < NL) request((l + 1) * C);
+#pragma unroll
+            for (int s = 0; s < KH; s++) {
+              const T w = c < 2 * l + 1 ? ga[hb + s] : (T) 0;
+              if (l > 0) aP = Mfma<T>::mma(w, xv[s], aP);
+              aQ = Mfma<T>::mma(w, dxv[s], aQ);
+            }
           }
-          aP = Mfma<T>::mma(w, xs, aP);
-          aQ = Mfma<T>::mma(w, dxs, aQ);
+        } else {
+#pragma unroll
+          for (int s = 0; s < KS; s++) {
+            const T w = c < 2 * l + 1 ? ga[CH(s)] : (T) 0;
+            T dxs = dx[cur][s];
+            if constexpr (PAIRS) dxs *= zc[s];
+            if (l > 0) {
+              T xs = x[cur][s];
+              if constexpr (PAIRS) xs *= zc[s];
+              aP = Mfma<T>::mma(w, xs, aP);
+            }
+            aQ = Mfma<T>::mma(w, dxs, aQ);
+          }
         }
-      }
-      if (colok) {
+        // rows m > 2 l hold zeros (their operand is zero) and take the harmonics of m = 0; what a column without a bond gives is not used
+        if (colok)      // ends a scheduling region: without it the l of a tile run into each other and spill (740 -> 1180 us)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-          if (mrow[v] < 2 * l + 1) {
-            const int lm = l * l + mrow[v];
-            const T *G = Gw + c * 2 * NLM + lm;
-            px += (double) (Yw[c * NLM + lm] * aQ[v]);
-            p1 += (double) (G[0] * aP[v]);
-            p2 += (double) (G[NLM] * aP[v]);
+          int m = mrow[v];
+          asm volatile("" : "+v"(m));      // or the compiler keeps (and spills) an address per l and v ahead of the tiles
+          const T *h = (m < 2 * l + 1 ? hrow[v] : hrow0) + ht * 16 * 3 * NLM + l * l;
+          px += (double) (h[0] * aQ[v]);
+          if (l > 0) {
+            p1 += (double) (h[NLM] * aP[v]);
+            p2 += (double) (h[2 * NLM] * aP[v]);
           }
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
+      if (HT > 1 && ht + 1 < HT && eb + 16 < e1_) begin(eb + 16);
+      // sum over the four lane groups (the rows m of a bond are spread over them); lane group ht keeps the sums of tile ht
+      px += __shfl_xor(px, 16, 64); p1 += __shfl_xor(p1, 16, 64); p2 += __shfl_xor(p2, 16, 64);
+      px += __shfl_xor(px, 32, 64); p1 += __shfl_xor(p1, 32, 64); p2 += __shfl_xor(p2, 32, 64);
+      if (HT == 1 || g == ht) { px_r = px; p1_r = p1; p2_r = p2; }
     }
-    // sum over the four lane groups (the rows m of a bond are spread over them)
-    px += __shfl_xor(px, 16, 64); p1 += __shfl_xor(p1, 16, 64); p2 += __shfl_xor(p2, 16, 64);
-    px += __shfl_xor(px, 32, 64); p1 += __shfl_xor(p1, 32, 64); p2 += __shfl_xor(p2, 32, 64);
-    if (lane < nb) {
+    if (TAB) px_r *= (double) a.tb.N;      // the slopes are per interval
+    if (lane < nr) {
       if (a.bsum) {
-        const double *b = a.bsum + 3 * (eb + lane);
-        px += b[0]; p1 += b[1]; p2 += b[2];
+        const double *b = a.bsum + 3 * (er + lane);
+        px_r += b[0]; p1_r += b[1]; p2_r += b[2];
       }
-      const double dEdr = px / brc, t1 = p1 / br, t2 = p2 / br;
+      const double dEdr = px_r / brc, t1 = p1_r / br, t2 = p2_r / br;
       const double fv[3] = {dEdr * u0 + t1 * e1[0] + t2 * e2[0], dEdr * u1 + t1 * e1[1] + t2 * e2[1], dEdr * u2 + t1 * e1[2] + t2 * e2[2]};
       for (int d = 0; d < 3; d++) {
         fi[d] += fv[d];
-        if (a.fedge) a.fedge[3 * (eb + lane) + d] = (a.ordered_add ? a.fedge[3 * (eb + lane) + d] : 0.0) + fv[d];
+        if (a.fedge) a.fedge[3 * (er + lane) + d] = (a.ordered_add ? a.fedge[3 * (er + lane) + d] : 0.0) + fv[d];
         else atomicAdd(&a.f[3 * (long long) jj + d], -fv[d]);
       }
       const double ddx = -u0 * br, ddy = -u1 * br, ddz = -u2 * br;
@@ -2818,9 +2876,11 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(256,
     for (int k = 0; k < 9; k++) red[wave][k] = vsum[k];
   __syncthreads();
   if (t < 9) {
-    const double s = red[0][t] + red[1][t] + red[2][t] + red[3][t];
+    double s = red[0][t];
+#pragma unroll
+    for (int w = 1; w < NW; w++) s += red[w][t];
     if (a.fcen) a.fcen[9 * (long long) i + t] = (a.ordered_add ? a.fcen[9 * (long long) i + t] : 0.0) + s;
-    else if (e1 > e0) {
+    else if (e1_ > e0) {
       if (t < 3) atomicAdd(&a.f[3 * (long long) i + t], s);
       else {
         atomicAdd(&a.virial[record_of(a.sid, i) + t - 3], s);
