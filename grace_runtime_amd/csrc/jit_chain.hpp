@@ -81,6 +81,7 @@ struct ChainSpec {
 };
 
 constexpr int kChainMaxParts = 8;
+constexpr size_t kLdsPerCu = 160 * 1024;
 struct ChainParts {
   bool used = false;
   unsigned long long mask[kChainMaxParts] = {};    // groups of every part
@@ -104,7 +105,7 @@ struct ChainKernels {
   ChainParts parts[kChainMaxParts + 1];
   unsigned long long keep0 = 0;    // functions of X0 whose stored adjoint the reverse adds to
   bool ok() const { return mod != nullptr; }
-  // parts of a launch over n atoms: as many as leave every block its own CU (the LDS of a block fills one)
+  // parts of a launch over n atoms: as many as leave every block its own CU
   int parts_for(int n, int ncu) const
   {
     const int blocks = (n + atoms_per_block - 1) / atoms_per_block;
@@ -396,7 +397,45 @@ inline bool generate_chain(const ChainSpec &sp, ChainCode &out)
   for (const Path &p : paths) XM = std::max(XM, p.M);
   for (const Fc1Path &p : f1) XM = std::max(XM, p.M);
   const int XR = XM * NA;    // rows of a hand-over buffer
-
+  // Blocks on a CU.  The LDS of a block holds a row for every function of X0 (of its adjoint in the reverse) and the hand-over
+  // buffers of the longest path.  In fp64 that used to fill a CU, whose one wave per SIMD then waits at every LDS read, barrier and
+  // weight request.  Without FC22 two blocks fit when a path is handed over in pieces and, where that is not enough, the rows of
+  // X0 that FC1 works on and those that the paths of P2 work on take turns in the same LDS (layer 2 of a model with parity:
+  // 25 and 25 of 49 functions).  Measured, 8192 atoms, fp64, layer 1 / layer 2 of GRACE-2L: forward 204 -> 161 / 215 -> 165 us,
+  // reverse 269 -> 212 / 284 -> 232; up to 2048 atoms, where a CU has one block either way: forward 51 -> 48 / 52 -> 49, reverse 64
+  // -> 68 / 63 -> 68.  In fp32 two blocks fit as it is and a third pays in the forward of layer 2 (32 768 atoms: 387 -> 355 us;
+  // layer 1, which had three: 344 -> 351 and 8192 atoms 91 -> 87); the reverse with three: 440 -> 459 us.  With FC22 (GRACE-1L) the
+  // values of a group stay in registers until P4, and two blocks' worth of registers spills: 304 -> 324 us.
+  std::vector<char> in_fc1(nf0, 0), in_p2(nf0, 0);    // functions of X0 that the matrix steps of FC1 / of the paths of P2 read
+  for (const Fc1Path &p : f1)
+    for (int i = 0; i < p.M; i++) in_fc1[p.f0 + i] = in_fc1[p.r0 + i] = 1;
+  for (const Path &p : paths)
+    for (int i = 0; i < p.M; i++) {
+      if (p.any && p.l21) in_p2[p.r21 + i] = 1;
+      if (p.any && p.l22) in_p2[p.r22 + i] = 1;
+    }
+  if (sp.fuse3 && sp.prod3_right_x0)
+    for (const auto &kv : p3_by_l)
+      for (const ProdTerm *t : kv.second) in_p2[t->r] = 1;
+  auto row_map = [&](const std::vector<char> &in) {    // compact row of every function, the number of rows in [nf0]
+    std::vector<int> row(nf0 + 1, 0);
+    for (int f = 0; f < nf0; f++) row[f + 1] = row[f] + (in[f] ? 1 : 0);
+    return row;
+  };
+  std::vector<int> all_rows(nf0 + 1);
+  std::iota(all_rows.begin(), all_rows.end(), 0);
+  const std::vector<int> fc1_rows = row_map(in_fc1), p2_rows = row_map(in_p2);
+  const int turns_rows = std::max(fc1_rows[nf0], p2_rows[nf0]);
+  const size_t row_bytes = (size_t) NA * S * (f32 ? sizeof(float) : sizeof(double));
+  struct Layout { int piece; bool turns; int blocks; };    // functions of a piece, rows of X0 in turns, blocks on a CU (1: not bounded)
+  auto layout = [&](int piece, int blocks, int extra_rows) {    // of pieces of at most so many functions
+    const Layout whole{XM, false, 1};
+    if (sp.have22) return whole;
+    const int m = std::min(XM, piece);
+    auto fits = [&](int rows) { return blocks * (size_t) (rows + 2 * m + extra_rows) * row_bytes <= kLdsPerCu; };
+    if (!fits(nf0) && !fits(turns_rows)) return whole;
+    return Layout{m, !fits(nf0), blocks};
+  };
   // ---- source
   std::ostringstream s;
   s << "typedef " << (f32 ? "float" : "double") << " T;\n";
@@ -493,6 +532,32 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   }
 }
 )";
+  s << R"(
+// One column block of one function with one output, the two segments by two waves: D = W_seg B (segment `seg` of wf), written to Y.
+template<int NNEXT>
+__device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * KS], T (&wn)[2 * KS], const T *wq, const T *B, T *Y, int rb, int seg, int lane)
+{
+  const int g = lane >> 4, c = lane & 15;
+  const int it = c < NA ? c : NA - 1;
+  T b[KS];
+#pragma unroll
+  for (int q = 0; q < KS; q++) b[q] = B[it * S + g + 4 * q];
+  __builtin_amdgcn_sched_barrier(0);
+  v4 d = {0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < KS; q++) {
+    d = MMA(seg ? wf[KS + q] : wf[q], b[q], d);
+    if (2 * q < NNEXT) wn[2 * q] = LDW(wq, 2 * q);
+    if (2 * q + 1 < NNEXT) wn[2 * q + 1] = LDW(wq, 2 * q + 1);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (c < NA) {
+    T *y = Y + c * S + rb * 16;
+#pragma unroll
+    for (int v = 0; v < 4; v++) y[DROW[4 * g + v]] = d[v];
+  }
+}
+)";
   auto woff = [&](const WaveUnits &u) {
     std::ostringstream o;
     o << "(wave == 0 ? " << u.off[0] << "LL : wave == 1 ? " << u.off[1] << "LL : wave == 2 ? " << u.off[2] << "LL : " << u.off[3] << "LL)";
@@ -574,42 +639,77 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   auto guard = [&](bool split, size_t gi) { return split ? "if (mask >> " + std::to_string(gi) + " & 1) " : std::string(); };
   // owner_of_p3[o]: a group whose part owns output o of P3 (all groups that give to o are in one part)
   auto emit_forward = [&](bool split) {
-  s << "extern \"C\" __global__ __launch_bounds__(256) void chain_fwd" << (split ? "_part" : "") << "(const T *__restrict__ X0, T *__restrict__ X1, T *__restrict__ P2, "
+  const Layout lay = split ? Layout{XM, false, 1} : layout(5, f32 ? 3 : 2, 1);
+  const int PM = lay.piece, PR = PM * NA;    // functions of a piece, rows of a hand-over buffer
+  s << "extern \"C\" __global__ __launch_bounds__(256" << (lay.blocks > 1 ? ", " + std::to_string(lay.blocks) : std::string()) << ") void chain_fwd" << (split ? "_part" : "") << "(const T *__restrict__ X0, T *__restrict__ X1, T *__restrict__ P2, "
        "T *__restrict__ P21, T *__restrict__ P22, T *__restrict__ P3, T *__restrict__ P4, const T *__restrict__ W, int natoms, int one"
     << mask_args(split) << ")\n{\n";
   if (split) mask_pick();
   {
     std::ostringstream d;
-    d << "__shared__ T L0[" << nf0 * NA * S << "], LX[" << XR * S << "], LY1[" << XR * S << "], LY2[" << XR * S << "];";
+    d << "__shared__ T L0[" << (lay.turns ? turns_rows : nf0) * NA * S << "], LX[" << PR * S << "], LY1[" << PR * S << "]";
+    d << (sp.have22 ? ", LY2[" : ", LZ[") << (sp.have22 ? PR : NA) * S << "];";    // LZ: unused, and left out, where `halves` is false
     common_head(d.str().c_str());
   }
   s << "  X0 += at * " << nf0 << " * C + n; X1 += at * " << nf0 << " * C + n; P2 += at * " << nP2 << " * C + n; P21 += at * " << nP2
     << " * C + n; P22 += at * " << nP2 << " * C + n; P3 += at * " << std::max(nP3, 1) << " * C + n; P4 += at * " << std::max(nP4, 1) << " * C + n;\n";
-  for (int f = 0; f < nf0; f++) s << "  L0[" << f * NA * S << " + col] = X0[" << f << " * C];\n";
+  const std::vector<int> &r1 = lay.turns ? fc1_rows : all_rows, &r2 = lay.turns ? p2_rows : all_rows;
+  for (int f = 0; f < nf0; f++)
+    if (!lay.turns || in_fc1[f]) s << "  L0[" << r1[f] * NA * S << " + col] = X0[" << f << " * C];\n";
   for (int f = 0; f < nf0; f++) s << "  T " << x1(f) << ";\n";
   if (sp.fuse3)
     for (int o = 0; o < nP3; o++) s << "  T p3_" << o << " = (T) 0;\n";
   // the steps of the forward kernel: FC1 paths, then the paths of P2 with an FC phase, group by group
   steps.clear();
   step = 0;
-  for (size_t q = 0; q < f1.size(); q++) steps.push_back(&wu_f1[q]);
+  auto pieces = [&](int M) { return M <= PM ? 1 : 1 + (M - PM + 3) / 4; };    // of four functions, the last one of up to PM
+  for (size_t q = 0; q < f1.size(); q++)
+    for (int k = 0; k < pieces(f1[q].M); k++) steps.push_back(&wu_f1[q]);
   for (const auto &g : order)
     for (int q : g)
-      if (paths[q].any && (paths[q].l21 || paths[q].l22)) steps.push_back(&wu_p[q]);
+      if (paths[q].any && (paths[q].l21 || paths[q].l22))
+        for (int k = 0; k < pieces(paths[q].M); k++) steps.push_back(&wu_p[q]);
   request_wf(0);
+  // One FC step of m functions with one output into Y: a pair of waves per row block takes the column blocks (two functions) in
+  // turn.  When their number is odd and the last one holds one function, its two segments go to the two pairs instead, the right
+  // one to row 0 of Z, and the column threads add them.
+  const bool halves = sp.have22 || (size_t) ((lay.turns ? turns_rows : nf0) + 2 * PM + 1) * row_bytes <= kLdsPerCu;
+  auto other = [&](const std::string &Y) { return Y == "LY2" ? "LY1" : sp.have22 ? "LY2" : "LZ"; };
+  auto in_halves = [&](int m) { return halves && m % 4 == 1; };
+  auto one_output = [&](const StepArgs &wf, int m, const std::string &b0, const std::string &b1, const std::string &Y) {
+    const int whole = in_halves(m) ? m - 1 : m;
+    const std::string last = " + " + std::to_string((m - 1) * NA * S);
+    if (whole > 0)
+      s << "      fc_rows<2, " << whole * NA << ", 2, " << wf.nnext << ", 0>(" << wf.bufs << ", " << b0 << ", " << b1 << ", " << Y << ", wave >> 1, wave & 1, 0, lane);\n";
+    if (in_halves(m))
+      s << "      fc_half<" << (whole > 0 ? "0" : wf.nnext) << ">(" << wf.bufs << ", (wave < 2 ? " << b0 << " : " << b1 << ")" << last << ", wave < 2 ? " << Y << last << " : " << other(Y)
+        << ", wave & 1, wave >> 1, lane);\n";
+  };
+  auto result = [&](int m, int i, const std::string &Y) {
+    const std::string v = Y + "[" + std::to_string(i * NA * S) + " + col]";
+    return in_halves(m) && i == m - 1 ? "(" + v + " + " + other(Y) + "[col])" : v;
+  };
   // FC1
   for (size_t q = 0; q < f1.size(); q++) {
     const Fc1Path &p = f1[q];
-    s << "  {    // FC1, functions " << p.f0 << " .. " << p.f0 + p.M - 1 << "\n";
-    const StepArgs wf = begin_step(split && q + 1 == f1.size());
-    s << "    SYNC();\n";
-    s << "    fc_rows<2, " << p.M * NA << ", 2, " << wf.nnext << ", 0>(" << wf.bufs << ", L0 + " << p.f0 * NA * S << ", L0 + " << p.r0 * NA * S << ", LY1, wave >> 1, wave & 1, 0, lane);\n";
-    s << "    SYNC();\n";
-    for (int i = 0; i < p.M; i++) {
-      const int f = p.f0 + i;
-      s << "    " << x1(f) << " = (T) " << lit(sp.fc1.nof[f], f32) << " * LY1[" << i * NA * S << " + col]; X1[" << f << " * C] = " << x1(f) << ";\n";
+    for (int k = 0; k < pieces(p.M); k++) {
+      const int i0 = 4 * k, m = k + 1 < pieces(p.M) ? 4 : p.M - i0;
+      s << "  {    // FC1, functions " << p.f0 + i0 << " .. " << p.f0 + i0 + m - 1 << "\n";
+      const StepArgs wf = begin_step(split && q + 1 == f1.size() && k + 1 == pieces(p.M));
+      s << "    SYNC();\n";
+      one_output(wf, m, "L0 + " + std::to_string(r1[p.f0 + i0] * NA * S), "L0 + " + std::to_string(r1[p.r0 + i0] * NA * S), "LY1");
+      s << "    SYNC();\n";
+      for (int i = 0; i < m; i++) {
+        const int f = p.f0 + i0 + i;
+        s << "    " << x1(f) << " = (T) " << lit(sp.fc1.nof[f], f32) << " * " << result(m, i, "LY1") << "; X1[" << f << " * C] = " << x1(f) << ";\n";
+      }
+      s << "  }\n";
     }
-    s << "  }\n";
+  }
+  if (lay.turns) {
+    s << "  int later = 0;\n  __asm__ volatile(\"\" : \"+s\"(later));\n";
+    for (int f = 0; f < nf0; f++)
+      if (in_p2[f]) s << "  L0[" << r2[f] * NA * S << " + col] = X0[later + " << f << " * C];\n";
   }
   // P2 paths, group by group
   for (size_t gi = 0; gi < order.size(); gi++) {
@@ -633,10 +733,13 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
       const Path &p = paths[q];
       if (!p.any) continue;
       const bool gemm = p.l21 || p.l22;
-      s << "    {    // path " << q << ": functions " << p.f0 << " .. " << p.f0 + p.M - 1 << "\n";
-      const StepArgs wf = gemm ? begin_step(split && q == last_step) : StepArgs();
-      for (int i = 0; i < p.M; i++) {
-        const int f = p.f0 + i;
+      for (int k = 0; k < pieces(p.M); k++) {
+      const int i0 = 4 * k, m = k + 1 < pieces(p.M) ? 4 : p.M - i0, f0 = p.f0 + i0;
+      const bool both = p.l21 && p.l22;
+      s << "    {    // path " << q << ": functions " << f0 << " .. " << f0 + m - 1 << "\n";
+      const StepArgs wf = gemm ? begin_step(split && q == last_step && k + 1 == pieces(p.M)) : StepArgs();
+      for (int i = 0; i < m; i++) {
+        const int f = f0 + i;
         const auto it = p2_by_o.find(f);
         const std::string e = sum_terms(it == p2_by_o.end() ? std::vector<const ProdTerm *>() : it->second,
                                         [&](const ProdTerm *t) { return x1(t->l) + " * " + x1(t->r); });
@@ -647,36 +750,42 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
       }
       if (gemm) {
         s << "      SYNC();\n";
-        if (p.l21 && p.l22)
-          s << "      fc_rows<2, " << p.M * NA << ", 1, " << wf.nnext << ", 0>(" << wf.bufs << ", LX, L0 + (wave < 2 ? " << p.r21 * NA * S << " : " << p.r22 * NA * S
+        if (both)
+          s << "      fc_rows<2, " << m * NA << ", 1, " << wf.nnext << ", 0>(" << wf.bufs << ", LX, L0 + (wave < 2 ? " << r2[p.r21 + i0] * NA * S << " : " << r2[p.r22 + i0] * NA * S
             << "), wave < 2 ? LY1 : LY2, 0, wave & 1, 0, lane);\n";
         else
-          s << "      fc_rows<2, " << p.M * NA << ", 2, " << wf.nnext << ", 0>(" << wf.bufs << ", LX, L0 + " << (p.l22 ? p.r22 : p.r21) * NA * S << ", " << (p.l22 ? "LY2" : "LY1")
-            << ", wave >> 1, wave & 1, 0, lane);\n";
+          one_output(wf, m, "LX", "L0 + " + std::to_string(r2[(p.l22 ? p.r22 : p.r21) + i0] * NA * S), p.l22 ? "LY2" : "LY1");
         s << "      SYNC();\n";
-        for (int i = 0; i < p.M; i++) {
-          const int f = p.f0 + i;
+        std::set<int> sums;
+        auto value = [&](int i, const std::string &Y) { return both ? Y + "[" + std::to_string(i * NA * S) + " + col]" : result(m, i, Y); };
+        for (int i = 0; i < m; i++) {
+          const int f = f0 + i;
           if (live21[f]) {
-            s << "      { const T v = (T) " << lit(sp.fc21.nof[f], f32) << " * LY1[" << i * NA * S << " + col]; ST(P21[" << f << " * C], v);";
+            s << "      { const T v = (T) " << lit(sp.fc21.nof[f], f32) << " * " << value(i, "LY1") << "; ST(P21[" << f << " * C], v);";
             const auto it = p3_by_l.find(f);
             if (sp.fuse3 && it != p3_by_l.end())
-              for (const ProdTerm *t : it->second)
+              for (const ProdTerm *t : it->second) {
+                sums.insert(t->o);
                 s << " p3_" << t->o << " += (T) " << lit(t->c, f32) << " * v * "
-                  << (sp.prod3_right_x0 ? "L0[" + std::to_string(t->r * NA * S) + " + col]" : x1(t->r)) << ";";    // X0 is resident in LDS
+                  << (sp.prod3_right_x0 ? "L0[" + std::to_string(r2[t->r] * NA * S) + " + col]" : x1(t->r)) << ";";    // X0 is resident in LDS
+              }
             s << " }\n";
           }
           if (live22[f]) {
-            s << "      " << v2(f) << " = (T) " << lit(sp.fc22.nof[f], f32) << " * LY2[" << i * NA * S << " + col]; ST(P22[" << f << " * C], " << v2(f)
+            s << "      " << v2(f) << " = (T) " << lit(sp.fc22.nof[f], f32) << " * " << value(i, "LY2") << "; ST(P22[" << f << " * C], " << v2(f)
               << ");\n";
-            for (const auto *m : {&p4_by_l, &p4_by_r}) {
-              const auto it = m->find(f);
-              if (it != m->end())
+            for (const auto *mp : {&p4_by_l, &p4_by_r}) {
+              const auto it = mp->find(f);
+              if (it != mp->end())
                 for (const ProdTerm *t : it->second) outs4.insert(t->o);
             }
           }
         }
+        // the sums of P3 are taken here: the compiler otherwise leaves them to the end and keeps every value until then
+        for (int o : sums) s << "      __asm__ volatile(\"\" : \"+v\"(p3_" << o << "));\n";
       }
       s << "    }\n";
+      }
     }
     if (!outs4.empty()) {
       s << "    {\n";
@@ -696,7 +805,12 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
 
   // =========================================================== reverse
   auto emit_reverse = [&](bool split) -> bool {
-  s << "extern \"C\" __global__ __launch_bounds__(256) void chain_bwd" << (split ? "_part" : "") << "(const T *__restrict__ X0, const T *__restrict__ X1, const T *__restrict__ P21, "
+  const Layout lay = split || f32 ? Layout{XM, false, 1} : layout(6, 2, 0);
+  const int PM = lay.piece, PR = PM * NA;
+  const std::vector<int> &r1 = lay.turns ? fc1_rows : all_rows, &r2 = lay.turns ? p2_rows : all_rows;
+  const char *pipe = lay.blocks > 1 ? "0" : "1";
+  auto pieces = [&](int M) { return (M + PM - 1) / PM; };
+  s << "extern \"C\" __global__ __launch_bounds__(256" << (lay.blocks > 1 ? ", " + std::to_string(lay.blocks) : std::string()) << ") void chain_bwd" << (split ? "_part" : "") << "(const T *__restrict__ X0, const T *__restrict__ X1, const T *__restrict__ P21, "
        "const T *__restrict__ P22, const T *__restrict__ gP2, const T *__restrict__ gP3, const T *__restrict__ gP4, const T *__restrict__ gP21, "
        "T *__restrict__ gX0, "
        "const T *__restrict__ W, int natoms, int one"
@@ -707,7 +821,7 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   }
   {
     std::ostringstream d;
-    d << "__shared__ T LG[" << nf0 * NA * S << "], LX1[" << XR * S << "], LX2[" << XR * S << "], LY[" << XR * S << "];";
+    d << "__shared__ T LG[" << (lay.turns ? turns_rows : nf0) * NA * S << "], LX1[" << PR * S << "], LX2[" << PR * S << "], LY[" << PR * S << "];";
     common_head(d.str().c_str());
   }
   s << "  X0 += at * " << nf0 << " * C + n; X1 += at * " << nf0 << " * C + n; P21 += at * " << nP2 << " * C + n; P22 += at * " << nP2
@@ -716,7 +830,7 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
 
   for (int f = 0; f < nf0; f++)
     if (sp.fc1.live[f]) s << "  const T " << x1(f) << " = X1[" << f << " * C];\n";
-  if (sp.prod3_right_x0 && sp.fuse3)
+  if (sp.prod3_right_x0 && sp.fuse3 && !lay.turns)
     for (int f = 0; f < nf0; f++) s << "  const T x0_" << f << " = X0[" << f << " * C];\n";
   for (int f = 0; f < nf0; f++) s << "  T g1_" << f << " = (T) 0;\n";
   if (sp.fuse3)
@@ -746,7 +860,8 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
     }
   }
   for (int f = 0; f < nf0; f++)
-    s << "    LG[" << f * NA * S << " + col] = " << (sp.prod3_right_x0 && sp.fuse3 ? "gx0_" + std::to_string(f) : std::string("(T) 0")) << ";\n";
+    if (!lay.turns || in_p2[f])
+    s << "    LG[" << r2[f] * NA * S << " + col] = " << (sp.prod3_right_x0 && sp.fuse3 ? "gx0_" + std::to_string(f) : std::string("(T) 0")) << ";\n";
   s << "  }\n";
   // the P22 rows and the P4 adjoints of a group are requested one path ahead of the group (behind the column phase of the
   // last path of the group before it, whose own rows are dead by then), so that they arrive during that path's matrix phase
@@ -785,8 +900,10 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   step = 0;
   for (const auto &g : order)
     for (int q : g)
-      if (paths[q].any && (paths[q].l21 || paths[q].l22)) steps.push_back(&wu_pb[q]);
-  for (size_t q = 0; q < f1.size(); q++) steps.push_back(&wu_f1b[q]);
+      if (paths[q].any && (paths[q].l21 || paths[q].l22))
+        for (int k = 0; k < pieces(paths[q].M); k++) steps.push_back(&wu_pb[q]);
+  for (size_t q = 0; q < f1.size(); q++)
+    for (int k = 0; k < pieces(f1[q].M); k++) steps.push_back(&wu_f1b[q]);
   if (!split) request_wf(0);
   for (size_t gi = 0; gi < order.size(); gi++) {
     const auto &g = order[gi];
@@ -817,15 +934,27 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
       const Path &p = paths[q];
       if (!p.any) continue;
       const bool gemm = p.l21 || p.l22;
-      s << "    for (int ip = 0; ip < one; ip++) {    // path " << q << ": functions " << p.f0 << " .. " << p.f0 + p.M - 1 << "\n";
+      for (int k = 0; k < pieces(p.M); k++) {
+      const int i0 = k * PM, m = std::min(PM, p.M - i0), f0 = p.f0 + i0;
+      const bool last_piece = k + 1 == pieces(p.M);
+      s << "    for (int ip = 0; ip < one; ip++) {    // path " << q << ": functions " << f0 << " .. " << f0 + m - 1 << "\n";
       s << "      const T *P22w = P22v + ip, *gP4w = gP4v + ip, *gP2w = gP2 + it + ip, *gP21w = gP21 + it + ip;\n";
       // the adjoints that the reduces left on this path's functions: requested here, used behind the matrix phase
-      for (int i = 0; i < p.M; i++)
-        if (keep2[p.f0 + i] && p2_by_o.count(p.f0 + i)) s << "      const T gk_" << p.f0 + i << " = gP2w[" << p.f0 + i << " * C];\n";
-      const StepArgs wf = gemm ? begin_step(split && q == last_gemm) : StepArgs();
+      for (int i = 0; i < m; i++)
+        if (keep2[f0 + i] && p2_by_o.count(f0 + i)) s << "      const T gk_" << f0 + i << " = gP2w[" << f0 + i << " * C];\n";
+      const StepArgs wf = gemm ? begin_step(split && q == last_gemm && last_piece) : StepArgs();
+      if (gemm && lay.turns && sp.prod3_right_x0 && sp.fuse3 && p.l21) {
+        std::set<int> right;
+        for (int i = 0; i < m; i++) {
+          const auto it = p3_by_l.find(f0 + i);
+          if (live21[f0 + i] && it != p3_by_l.end())
+            for (const ProdTerm *t : it->second) right.insert(t->r);
+        }
+        for (int f : right) s << "      const T x0_" << f << " = X0[it + ip + " << f << " * C];\n";
+      }
       if (gemm) {
-        for (int i = 0; i < p.M; i++) {
-          const int f = p.f0 + i;
+        for (int i = 0; i < m; i++) {
+          const int f = f0 + i;
           if (p.l21) {
             if (live21[f]) {
               const auto it = p3_by_l.find(f);
@@ -862,7 +991,7 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
             }
           }
         }
-        if (q == last_gemm && next_group < order.size()) {
+        if (q == last_gemm && last_piece && next_group < order.size()) {
           group_loads(next_group, "P22w", "gP4w", "      ");
           next_requested = true;
         }
@@ -871,12 +1000,12 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
         const char *b0 = p.l21 ? "LX1" : "LX2";
         const int rr = p.l21 ? p.r21 : p.r22;
         if (p.l21 && p.l22 && p.r21 != p.r22) { out.why = "the two layers of a path read different right inputs"; return false; }
-        s << "      fc_rows<" << wu_pb[q].nseg << ", " << p.M * NA << ", 1, " << wf.nnext << ", 1>(" << wf.bufs << ", " << b0 << ", LX2, wave < 2 ? LY : LG + " << rr * NA * S
+        s << "      fc_rows<" << wu_pb[q].nseg << ", " << m * NA << ", 1, " << wf.nnext << ", " << pipe << ">(" << wf.bufs << ", " << b0 << ", LX2, wave < 2 ? LY : LG + " << r2[rr + i0] * NA * S
           << ", 0, wave & 1, wave >> 1, lane);\n";
         s << "      SYNC();\n";
       }
-      for (int i = 0; i < p.M; i++) {
-        const int f = p.f0 + i;
+      for (int i = 0; i < m; i++) {
+        const int f = f0 + i;
         const auto it = p2_by_o.find(f);
         if (it == p2_by_o.end()) continue;
         if (!gemm && !keep2[f]) continue;
@@ -892,8 +1021,23 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
         s << " }\n";
       }
       s << "    }\n";
+      }
     }
     if (!next_requested && next_group < order.size()) group_loads(next_group, "P22v", "gP4v", "    ");
+    s << "  }\n";
+  }
+  std::vector<char> keep0 = sp.keepX0;
+  keep0.resize(nf0, 0);
+  auto kept = [&](int f) { return !split && (keep0[f] || !sp.fuse3) ? " + gX0[" + std::to_string(f) + " * C]" : std::string(); };
+  if (lay.turns) {
+    s << "  {\n";
+    for (int f = 0; f < nf0; f++)
+      if (in_p2[f]) s << "    const T t_" << f << " = LG[" << r2[f] * NA * S << " + col];\n";
+    for (int f = 0; f < nf0; f++) {
+      const std::string t = in_p2[f] ? "t_" + std::to_string(f) : std::string("(T) 0");
+      if (in_fc1[f]) s << "    LG[" << r1[f] * NA * S << " + col] = " << t << ";\n";
+      else s << "    gX0[" << f << " * C] = " << t << kept(f) << ";\n";
+    }
     s << "  }\n";
   }
   // reverse of FC1
@@ -901,32 +1045,30 @@ __device__ inline __attribute__((always_inline)) void fc_rows(const T (&wf)[2 * 
   for (size_t q = 0; q < f1.size(); q++) {
     const Fc1Path &p = f1[q];
     const bool same = p.r0 == p.f0;
-    s << "  {    // FC1 reverse, functions " << p.f0 << " .. " << p.f0 + p.M - 1 << "\n";
+    for (int k = 0; k < pieces(p.M); k++) {
+    const int i0 = k * PM, m = std::min(PM, p.M - i0), f0 = p.f0 + i0;
+    s << "  {    // FC1 reverse, functions " << f0 << " .. " << f0 + m - 1 << "\n";
     const StepArgs wf = begin_step();
-    for (int i = 0; i < p.M; i++) {
-      const int f = p.f0 + i;
+    for (int i = 0; i < m; i++) {
+      const int f = f0 + i;
       s << "    LX1[" << i * NA * S << " + col] = (T) " << lit(sp.fc1.nof[f], f32) << " * g1_" << f << ";\n";
     }
     s << "    SYNC();\n";
     if (same)
-      s << "    fc_rows<2, " << p.M * NA << ", 2, " << wf.nnext << ", 1>(" << wf.bufs << ", LX1, LX1, LG + " << p.f0 * NA * S << ", wave >> 1, wave & 1, 1, lane);\n";
+      s << "    fc_rows<2, " << m * NA << ", 2, " << wf.nnext << ", " << pipe << ">(" << wf.bufs << ", LX1, LX1, LG + " << r1[f0] * NA * S << ", wave >> 1, wave & 1, 1, lane);\n";
     else
-      s << "    fc_rows<1, " << p.M * NA << ", 1, " << wf.nnext << ", 1>(" << wf.bufs << ", LX1, LX1, LG + (wave < 2 ? " << p.f0 * NA * S << " : " << p.r0 * NA * S << "), 0, wave & 1, 1, lane);\n";
+      s << "    fc_rows<1, " << m * NA << ", 1, " << wf.nnext << ", " << pipe << ">(" << wf.bufs << ", LX1, LX1, LG + (wave < 2 ? " << r1[f0] * NA * S << " : " << r1[p.r0 + i0] * NA * S << "), 0, wave & 1, 1, lane);\n";
     s << "    SYNC();\n";
     s << "  }\n";
+    }
   }
   // when left and right rows of FC1 differ, two waves may add to one row in the same phase only if the rows of a path's two
   // sides are disjoint
   for (const Fc1Path &p : f1)
     if (p.r0 != p.f0 && p.r0 < p.f0 + p.M && p.f0 < p.r0 + p.M) { out.why = "fc1: left and right rows of a path overlap"; return false; }
   s << "  {\n";
-  std::vector<char> keep0 = sp.keepX0;
-  keep0.resize(nf0, 0);
-  for (int f = 0; f < nf0; f++) {
-    s << "    gX0[" << f << " * C] = LG[" << f * NA * S << " + col]";
-    if (!split && (keep0[f] || !sp.fuse3)) s << " + gX0[" << f << " * C]";
-    s << ";\n";
-  }
+  for (int f = 0; f < nf0; f++)
+    if (!lay.turns || in_fc1[f]) s << "    gX0[" << f << " * C] = LG[" << r1[f] * NA * S << " + col]" << kept(f) << ";\n";
   s << "  }\n}\n";
   return true;
   };

@@ -168,3 +168,31 @@ def test_chain_in_parts(model_dir, model, natoms, precision):
     assert sums == (set() if natoms > 1024 else {"chain_sum"} if model == "ch20" else {"chain_sum_L1", "chain_sum_L2"})
     ref = (g1.compute_1l if model == "ch20" else g2.compute_2l)(om, types[perm] - 1, offset, j, rij)
     cases.check_against(out, ref, natoms, *((1e-10, 1e-9, 1e-10, 1e-9) if precision == 64 else (1e-6, 2e-5, 1e-5, 1e-5)))
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("natoms", [1025, 2041, 4105])
+def test_blocks_that_share_a_cu(model_dir, natoms, precision):
+    """the whole form of both chains of GRACE-2L, whose paths are handed over in pieces of four to six functions and whose rows of
+    X0 take turns in layer 2, against the stages: one block per CU, the last one of a single atom; one CU without a block; twice
+    as many blocks as CUs and one.  The two differ in the order in which 64 terms are added, which moves a sum by at most 64 eps
+    of its terms (1.4e-14, 7.6e-6); forces come through both layers, both ways, and get ten times the bound of the energies."""
+    from grace_runtime_amd import synth
+    from oracle import grace_oracle_2l as g2
+    path = cases.model_file(model_dir, "config3")
+    pos, cell = synth.bcc_supercell(3.165, 13)
+    rng = np.random.default_rng(natoms)
+    pos = synth.jitter(pos, 0.05, 3)[np.sort(rng.permutation(len(pos))[:natoms])]
+    om = g2.Model2L(path)
+    types = rng.integers(1, om.n_elements + 1, natoms).astype(np.int32)
+    perm, offset, j, image, shifts = kk.neighbor_search(pos, cell, [True] * 3, float(np.max(om.cut)))
+    rij = cases.bond_vectors(pos, perm, offset, j, image, shifts)
+    species = [s.decode() for s in om.d["element_names"]]
+    out = []
+    for fused in (True, False):
+        eng = _engine(path, species, precision, fused)
+        eng.set_profile(True)
+        out.append(eng.compute(types[perm], offset, j, rij=rij, energies=True))
+        assert ("chain_bwd_L2" in eng.stage_times()) == fused
+    same = 1e-11 if precision == 64 else 2e-5
+    cases.check_against(out[0], out[1], natoms, same, 10 * same, same, 10 * same)
