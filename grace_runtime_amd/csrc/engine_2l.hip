@@ -23,7 +23,7 @@ template<class T> struct Chain {
   // the whole chain as one generated kernel per direction (jit_chain.hpp); not ok(): the stage-by-stage kernels run
   ChainKernels fused;
   DevBuf fusedW;            // fragment-ordered weights
-  bool fuse3 = true;        // P3 = XX1 x X inside the chain kernels (few outputs) or as the product kernels below (many)
+  bool fuse3 = true;        // P3 = XX1 x X inside the chain kernels or as the product kernels below
   std::string fused_note;
   ~Chain() { fused.release(); }
   DevBuf X1, XX, XX1, XXX, XX2, XXXX, gX, gX1, gXX, gXX1, gXXX, gXX2, gXXXX;
@@ -170,6 +170,7 @@ void Engine2L<T>::build_chain(Chain<T> &c, const char *tag, int nf, int KP, cons
     if (jit_compile_chain(("chain" + t).c_str(), sp, arch_, c.fused, w, c.fused_note)) {
       std::vector<T> wt(w.begin(), w.end());
       upload_vec(c.fusedW, wt);
+      c.fuse3 = c.fused.fuse3;    // also with many outputs, where the kernels form them path by path
     } else {
       log_message(1, std::string("GRACE-2L: the dense chain") + tag + " runs stage by stage (" + c.fused_note + ")");
     }

@@ -69,9 +69,10 @@ struct ChainSpec {
   int nP3 = 0;
   std::vector<ProdTerm> prod3;
   bool prod3_right_x0 = false;
-  // P3 inside the kernels (its outputs are accumulated in registers: for the few scalar outputs of a readout chain) or left to
-  // the product kernels of the caller (many outputs): the forward kernel then only writes P21, the reverse kernel reads the
-  // adjoint of P21 from gP21, and the adjoint of X0 that the reverse of P3 leaves in gX0 is added to, for every function
+  // P3 inside the kernels with its outputs accumulated in registers (the few scalar outputs of a readout chain).  More outputs
+  // are inside as well if each of them is fed by one path of P2 (`stream3` in generate_chain).  Else P3 is left to the product
+  // kernels of the caller: the forward kernel then only writes P21, the reverse kernel reads the adjoint of P21 from gP21, and
+  // the adjoint of X0 that the reverse of P3 leaves in gX0 is added to, for every function
   bool fuse3 = true;
   int nP4 = 0;
   std::vector<ProdTerm> prod4;
@@ -93,6 +94,7 @@ struct ChainCode {
   std::string why;
   int atoms_per_block = 0;
   double flops_per_atom = 0.0;    // of the FC layers of one direction (live functions, padded widths; 2 per multiply-add)
+  bool fuse3 = true;              // P3 is inside the kernels
   ChainParts parts[kChainMaxParts + 1];    // [p]: the groups dealt to p parts (p >= 2); used == false: not available
 };
 
@@ -102,6 +104,7 @@ struct ChainKernels {
   hipFunction_t fwd = nullptr, bwd = nullptr, fwd_part = nullptr, bwd_part = nullptr;
   int atoms_per_block = 0, nf0 = 0, C = 0;
   double flops_per_atom = 0.0;
+  bool fuse3 = true;               // P3 is inside the kernels
   ChainParts parts[kChainMaxParts + 1];
   unsigned long long keep0 = 0;    // functions of X0 whose stored adjoint the reverse adds to
   bool ok() const { return mod != nullptr; }
@@ -273,6 +276,17 @@ inline bool generate_chain(const ChainSpec &sp, ChainCode &out)
           (p.l22 && (p.tl22 < 0 || p.tl22 >= sp.fc22.ntiles || p.tr22 < 0 || p.tr22 >= sp.fc22.ntiles))) { out.why = "weight tile out of range"; return false; }
     }
   }
+  // ---- P3 path by path: with many outputs, each fed by one path, a path forms its own from the values it has at hand and the rows
+  // of X0 in LDS, and the reverse reads their adjoints where it reads the path's rows of P21.  P21 is then read once and its adjoint
+  // never stored.  Layer 1 of GRACE-2L (113 outputs, which all at once spilled 1100 registers), 8192 atoms, fp64: forward 161 -> 183
+  // us in place of a product kernel of 131, reverse 211 -> 344 in place of one of 216 (in pieces of four functions: 35 registers
+  // spill; 374 in pieces of six, 395 with the adjoint of X0 taken behind the matrix phase).  107 atoms: 34 + 38 us of the
+  // product kernels saved; the passes of 107, 3999 (fp32) and 32 000 atoms 444 -> 392, 1329 -> 1279 us and 16.3 -> 15.8 ms.
+  bool one_path = true;
+  for (const auto &kv : p3_by_o)
+    for (const ProdTerm *t : kv.second) one_path = one_path && path_of[t->l] == path_of[kv.second[0]->l];
+  const bool stream3 = one_path && p3_by_o.size() > 24, fuse3 = sp.fuse3 || stream3;
+  out.fuse3 = fuse3;
   // ---- groups: paths joined by P4 terms
   std::vector<int> grp(paths.size());
   std::iota(grp.begin(), grp.end(), 0);
@@ -402,7 +416,7 @@ inline bool generate_chain(const ChainSpec &sp, ChainCode &out)
   // weight request.  Without FC22 two blocks fit when a path is handed over in pieces and, where that is not enough, the rows of
   // X0 that FC1 works on and those that the paths of P2 work on take turns in the same LDS (layer 2 of a model with parity:
   // 25 and 25 of 49 functions).  Measured, 8192 atoms, fp64, layer 1 / layer 2 of GRACE-2L: forward 204 -> 161 / 215 -> 165 us,
-  // reverse 269 -> 212 / 284 -> 232; up to 2048 atoms, where a CU has one block either way: forward 51 -> 48 / 52 -> 49, reverse 64
+  // reverse 269 -> 212 / 284 -> 232 (without P3); up to 2048 atoms, where a CU has one block either way: forward 51 -> 48 / 52 -> 49, reverse 64
   // -> 68 / 63 -> 68.  In fp32 two blocks fit as it is and a third pays in the forward of layer 2 (32 768 atoms: 387 -> 355 us;
   // layer 1, which had three: 344 -> 351 and 8192 atoms 91 -> 87); the reverse with three: 440 -> 459 us.  With FC22 (GRACE-1L) the
   // values of a group stay in registers until P4, and two blocks' worth of registers spills: 304 -> 324 us.
@@ -414,7 +428,7 @@ inline bool generate_chain(const ChainSpec &sp, ChainCode &out)
       if (p.any && p.l21) in_p2[p.r21 + i] = 1;
       if (p.any && p.l22) in_p2[p.r22 + i] = 1;
     }
-  if (sp.fuse3 && sp.prod3_right_x0)
+  if (fuse3 && sp.prod3_right_x0)
     for (const auto &kv : p3_by_l)
       for (const ProdTerm *t : kv.second) in_p2[t->r] = 1;
   auto row_map = [&](const std::vector<char> &in) {    // compact row of every function, the number of rows in [nf0]
@@ -657,7 +671,7 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
   for (int f = 0; f < nf0; f++)
     if (!lay.turns || in_fc1[f]) s << "  L0[" << r1[f] * NA * S << " + col] = X0[" << f << " * C];\n";
   for (int f = 0; f < nf0; f++) s << "  T " << x1(f) << ";\n";
-  if (sp.fuse3)
+  if (fuse3 && !stream3)
     for (int o = 0; o < nP3; o++) s << "  T p3_" << o << " = (T) 0;\n";
   // the steps of the forward kernel: FC1 paths, then the paths of P2 with an FC phase, group by group
   steps.clear();
@@ -733,6 +747,16 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
       const Path &p = paths[q];
       if (!p.any) continue;
       const bool gemm = p.l21 || p.l22;
+      std::set<int> outs3;    // outputs of P3 that this path feeds
+      if (stream3) {
+        for (int i = 0; i < p.M; i++) {
+          const auto it = p3_by_l.find(p.f0 + i);
+          if (it != p3_by_l.end())
+            for (const ProdTerm *t : it->second) outs3.insert(t->o);
+        }
+        if (!outs3.empty()) s << "    {\n";
+        for (int o : outs3) s << "    T p3_" << o << " = (T) 0;\n";
+      }
       for (int k = 0; k < pieces(p.M); k++) {
       const int i0 = 4 * k, m = k + 1 < pieces(p.M) ? 4 : p.M - i0, f0 = p.f0 + i0;
       const bool both = p.l21 && p.l22;
@@ -763,7 +787,7 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
           if (live21[f]) {
             s << "      { const T v = (T) " << lit(sp.fc21.nof[f], f32) << " * " << value(i, "LY1") << "; ST(P21[" << f << " * C], v);";
             const auto it = p3_by_l.find(f);
-            if (sp.fuse3 && it != p3_by_l.end())
+            if (fuse3 && it != p3_by_l.end())
               for (const ProdTerm *t : it->second) {
                 sums.insert(t->o);
                 s << " p3_" << t->o << " += (T) " << lit(t->c, f32) << " * v * "
@@ -786,6 +810,8 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
       }
       s << "    }\n";
       }
+      for (int o : outs3) s << "    P3[" << o << " * C] = p3_" << o << ";\n";
+      if (!outs3.empty()) s << "    }\n";
     }
     if (!outs4.empty()) {
       s << "    {\n";
@@ -796,8 +822,9 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
     s << "  }\n";
   }
   s << "  {\n";
-  if (sp.fuse3)
-    for (int o = 0; o < nP3; o++) s << "    " << guard(split, (size_t) owner_of_p3[o]) << "P3[" << o << " * C] = p3_" << o << ";\n";
+  for (int o = 0; o < nP3 && fuse3; o++)
+    if (!stream3) s << "    " << guard(split, (size_t) owner_of_p3[o]) << "P3[" << o << " * C] = p3_" << o << ";\n";
+    else if (!p3_by_o.count(o)) s << "    " << (split ? "if (blockIdx.y == 0) " : "") << "P3[" << o << " * C] = (T) 0;\n";
   for (int o = 0; o < nP4; o++)
     if (!p4_by_o.count(o)) s << "    " << (split ? "if (blockIdx.y == 0) " : "") << "P4[" << o << " * C] = (T) 0;\n";
   s << "  }\n}\n\n";
@@ -805,7 +832,7 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
 
   // =========================================================== reverse
   auto emit_reverse = [&](bool split) -> bool {
-  const Layout lay = split || f32 ? Layout{XM, false, 1} : layout(6, 2, 0);
+  const Layout lay = split || f32 ? Layout{XM, false, 1} : layout(stream3 ? 4 : 6, 2, 0);
   const int PM = lay.piece, PR = PM * NA;
   const std::vector<int> &r1 = lay.turns ? fc1_rows : all_rows, &r2 = lay.turns ? p2_rows : all_rows;
   const char *pipe = lay.blocks > 1 ? "0" : "1";
@@ -830,17 +857,18 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
 
   for (int f = 0; f < nf0; f++)
     if (sp.fc1.live[f]) s << "  const T " << x1(f) << " = X1[" << f << " * C];\n";
-  if (sp.prod3_right_x0 && sp.fuse3 && !lay.turns)
+  const bool x0_rows = sp.prod3_right_x0 && fuse3 && (lay.turns || stream3);    // rows of X0 are read by the paths that need them
+  if (sp.prod3_right_x0 && fuse3 && !x0_rows)
     for (int f = 0; f < nf0; f++) s << "  const T x0_" << f << " = X0[" << f << " * C];\n";
   for (int f = 0; f < nf0; f++) s << "  T g1_" << f << " = (T) 0;\n";
-  if (sp.fuse3)
+  if (fuse3 && !stream3)
     for (int o = 0; o < nP3; o++) s << "  const T g3_" << o << " = gP3[" << o << " * C];\n";
   auto gr = [&](int f) { return (sp.prod3_right_x0 ? "gx0_" : "g1_") + std::to_string(f); };
   // the reverse of P3 with respect to its right operand needs P21 only here: all of it up front, with every load in flight
   // at once, instead of a load per path whose latency nothing hides (one wave per SIMD)
   // (when the right operand is X0 the sums are the initial values of the LDS rows in which the adjoint of X0 is gathered)
   s << "  {\n";
-  if (sp.fuse3) {
+  if (fuse3 && !stream3) {
     if (sp.prod3_right_x0)
       for (int f = 0; f < nf0; f++) s << "    T gx0_" << f << " = (T) 0;\n";
     if (split) {
@@ -861,7 +889,7 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
   }
   for (int f = 0; f < nf0; f++)
     if (!lay.turns || in_p2[f])
-    s << "    LG[" << r2[f] * NA * S << " + col] = " << (sp.prod3_right_x0 && sp.fuse3 ? "gx0_" + std::to_string(f) : std::string("(T) 0")) << ";\n";
+    s << "    LG[" << r2[f] * NA * S << " + col] = " << (sp.prod3_right_x0 && fuse3 && !stream3 ? "gx0_" + std::to_string(f) : std::string("(T) 0")) << ";\n";
   s << "  }\n";
   // the P22 rows and the P4 adjoints of a group are requested one path ahead of the group (behind the column phase of the
   // last path of the group before it, whose own rows are dead by then), so that they arrive during that path's matrix phase
@@ -943,14 +971,30 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
       for (int i = 0; i < m; i++)
         if (keep2[f0 + i] && p2_by_o.count(f0 + i)) s << "      const T gk_" << f0 + i << " = gP2w[" << f0 + i << " * C];\n";
       const StepArgs wf = gemm ? begin_step(split && q == last_gemm && last_piece) : StepArgs();
-      if (gemm && lay.turns && sp.prod3_right_x0 && sp.fuse3 && p.l21) {
-        std::set<int> right;
+      if (fuse3 && p.l21) {
+        std::set<int> right, outs3;
+        std::map<int, std::vector<const ProdTerm *>> by_r;
         for (int i = 0; i < m; i++) {
           const auto it = p3_by_l.find(f0 + i);
-          if (live21[f0 + i] && it != p3_by_l.end())
-            for (const ProdTerm *t : it->second) right.insert(t->r);
+          if (it == p3_by_l.end()) continue;
+          for (const ProdTerm *t : it->second) {
+            right.insert(t->r);
+            outs3.insert(t->o);
+            by_r[t->r].push_back(t);
+          }
         }
-        for (int f : right) s << "      const T x0_" << f << " = X0[it + ip + " << f << " * C];\n";
+        if (stream3) {
+          for (int o : outs3) s << "      const T g3_" << o << " = gP3[it + ip + " << o << " * C];\n";
+          for (int i = 0; i < m; i++)
+            if (p3_by_l.count(f0 + i)) s << "      const T p_" << f0 + i << " = P21[it + ip + " << f0 + i << " * C];\n";
+        }
+        if (x0_rows)
+          for (int f : right) s << "      const T x0_" << f << " = X0[it + ip + " << f << " * C];\n";
+        // the adjoint of P3's right operand: this thread's own elements of the rows, which no wave adds to between two steps
+        if (stream3)
+          for (const auto &kv : by_r)
+            s << "      " << (sp.prod3_right_x0 ? "LG[" + std::to_string(r2[kv.first] * NA * S) + " + col]" : "g1_" + std::to_string(kv.first)) << " += "
+              << sum_terms(kv.second, [&](const ProdTerm *t) { return "g3_" + std::to_string(t->o) + " * p_" + std::to_string(t->l); }) << ";\n";
       }
       if (gemm) {
         for (int i = 0; i < m; i++) {
@@ -960,7 +1004,7 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
               const auto it = p3_by_l.find(f);
               const std::vector<const ProdTerm *> none;
               const auto &ts = it == p3_by_l.end() ? none : it->second;
-              if (sp.fuse3)
+              if (fuse3)
                 s << "      LX1[" << i * NA * S << " + col] = (T) " << lit(sp.fc21.nof[f], f32) << " * ("
                   << sum_terms(ts, [&](const ProdTerm *t) { return "g3_" + std::to_string(t->o) + " * " + xr(t->r); }) << ");\n";
               else
@@ -1028,7 +1072,7 @@ __device__ inline __attribute__((always_inline)) void fc_half(const T (&wf)[2 * 
   }
   std::vector<char> keep0 = sp.keepX0;
   keep0.resize(nf0, 0);
-  auto kept = [&](int f) { return !split && (keep0[f] || !sp.fuse3) ? " + gX0[" + std::to_string(f) + " * C]" : std::string(); };
+  auto kept = [&](int f) { return !split && (keep0[f] || !fuse3) ? " + gX0[" + std::to_string(f) + " * C]" : std::string(); };
   if (lay.turns) {
     s << "  {\n";
     for (int f = 0; f < nf0; f++)
@@ -1147,9 +1191,10 @@ inline bool jit_compile_chain(const char *name, const ChainSpec &sp, const std::
   k.bwd = jk.bwd;
   k.atoms_per_block = code.atoms_per_block;
   k.nf0 = sp.nf0;
+  k.fuse3 = code.fuse3;
   k.C = sp.C;
   for (int f = 0; f < sp.nf0 && f < 64; f++)
-    if (!sp.fuse3 || (f < (int) sp.keepX0.size() && sp.keepX0[f])) k.keep0 |= 1ull << f;
+    if (!code.fuse3 || (f < (int) sp.keepX0.size() && sp.keepX0[f])) k.keep0 |= 1ull << f;
   if (parts)
     for (int p = 0; p <= kChainMaxParts; p++) k.parts[p] = code.parts[p];
   k.flops_per_atom = code.flops_per_atom;
