@@ -581,7 +581,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
   const long long *n_edges = eoff_.as<long long>() + n;
   const bool forces = !fl.energy_only;
   if (ordered_ && forces) ordered_begin();
-  bsum_begin(forces && !ordered_ && pair_mfma_ != 0 && pair_mfma_plan(nslot_, CRP_, nl_, sizeof(T), pair_mfma_waves(pair_waves_)).ok);
+  bsum_begin(forces && !ordered_ && pair_mfma_ != 0 && pair_mfma_plan(nslot_, CRP_, nl_, sizeof(T), pair_mfma_waves(pair_waves_)).ok, false);
   // row of an edge: Y[nlm] and, for forces, the two tangential gradients D1[nlm], D2[nlm] and padding (pair_row_stride)
   const int yw = forces ? pair_row_stride(nlm_, sizeof(T)) : nlm_;
   YG_.ensure(ecap_all * yw * sizeof(T));
@@ -691,9 +691,14 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     stage("reduce_rho_I1", [&] { reduce_fwd(red1_, c1_, A, rho_.as<double>() + (size_t) a0_ * nrho_, I1_.as<T>()); });
     stage("reduce_I", [&] { gemm(jI_, PI1_ / 16, CRP_ / 16, (const T *) I1_.as<T>(), nI1_, M + (size_t) a0_ * nslot_ * CRP_, nslot_, 0); });
   }
+  if (forces) gM_.ensure(nnodes * nI_ * CRP_ * sizeof(T));
   stage("fill_slot", [&] {
-    hipLaunchKernelGGL(k_fill_slot<T>, dim3((unsigned) ((nnodes * CRP_ + 255) / 256)), dim3(256), 0, stream_, mu_.as<int>(), zB0_.as<T>(), M, n_nodes_,
-                       nslot_, nI_, CRP_);
+    typedef unsigned long long word;    // rows of gM hold a multiple of 16 values
+    const unsigned fill = (unsigned) ((nnodes * CRP_ + 255) / 256);
+    const long long n0 = forces ? (long long) (nnodes * nI_ * CRP_ * sizeof(T) / sizeof(word)) : 0, n1 = bsum_on_ ? (long long) (bsum_bytes() / sizeof(word)) : 0;
+    const unsigned clear = (unsigned) ((n0 + n1 + 256 * kClearWords - 1) / (256 * kClearWords));
+    hipLaunchKernelGGL(k_fill_slot<T>, dim3(fill + clear), dim3(256), 0, stream_, mu_.as<int>(), zB0_.as<T>(), M, n_nodes_, nslot_, nI_, CRP_, fill, gM_.as<word>(), n0,
+                       bsum_.as<word>(), n1);
   });
   exchange_forward(1);
 
@@ -710,9 +715,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
   if ((CRP_ * sizeof(T)) % 16 || (radR1_.noutp * sizeof(T)) % 16) throw Error("GRACE-2L: pair kernels need rows that are multiples of 16 bytes");
   if (forces) {
     gP_.ensure(na * npf * CRP_ * sizeof(T));
-    gM_.ensure(nnodes * nI_ * CRP_ * sizeof(T));
     if (ordered_) gMe_.ensure(ecap * nI_ * CRP_ * sizeof(T));
-    stage("zero_gM", [&] { HIP_CHECK(hipMemsetAsync(gM_.p, 0, nnodes * nI_ * CRP_ * sizeof(T), stream_)); });
   }
 #define GR_PAIR1(K_, N_, grid_, block_, lds_, ...)                                                                       \
   {                                                                                                                      \

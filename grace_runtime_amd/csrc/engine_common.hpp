@@ -1935,13 +1935,14 @@ class EngineBase : public Engine, protected BufRegistry {
   DevBuf bsum_;
   bool bsum_on_ = false;
   double *bsum_ptr() const { return bsum_on_ ? bsum_.as<double>() : nullptr; }
-  void bsum_begin(bool on)
+  size_t bsum_bytes() const { return (size_t) 3 * std::max<int64_t>(nb_, 1) * sizeof(double); }
+  void bsum_begin(bool on, bool clear = true)    // clear == false: the caller clears bsum_bytes() of them
   {
     bsum_on_ = on;
     if (!on) return;
-    const size_t bytes = (size_t) 3 * std::max<int64_t>(nb_, 1) * sizeof(double);
+    const size_t bytes = bsum_bytes();
     bsum_.ensure(bytes);
-    stage("zero_bond_sums", [&] { HIP_CHECK(hipMemsetAsync(bsum_.p, 0, bytes, stream_)); });
+    if (clear) stage("zero_bond_sums", [&] { HIP_CHECK(hipMemsetAsync(bsum_.p, 0, bytes, stream_)); });
   }
   int pair_waves_ = pair_waves_switch();    // waves of a block of that kernel; 0: those of one group of slots
   static int pair_waves_switch()

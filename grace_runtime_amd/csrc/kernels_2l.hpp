@@ -52,9 +52,22 @@ template<class T> __global__ void k_sh_edges(ShCoef sh, const double *rh, const 
   }
 }
 
-// M[atom][slot][n] = z[mu_atom][n]
-template<class T> __global__ void k_fill_slot(const int *mu, const T *z, T *M, int natoms, int nslot, int slot, int C)
+// M[atom][slot][n] = z[mu_atom][n] by the first `fill_blocks` blocks; the others clear what the reverse pair kernel adds to (two
+// arrays of 8-byte words, 4 a thread).  As two fills of their own the arrays cost 3 us each below some thousand atoms.
+constexpr int kClearWords = 4;
+template<class T> __global__ __launch_bounds__(256) void k_fill_slot(const int *mu, const T *z, T *M, int natoms, int nslot, int slot, int C, unsigned fill_blocks,
+                                                                     unsigned long long *clear0, long long n0, unsigned long long *clear1, long long n1)
 {
+  if (blockIdx.x >= fill_blocks) {
+    const long long first = (long long) (blockIdx.x - fill_blocks) * (256 * kClearWords) + threadIdx.x;
+#pragma unroll
+    for (int w = 0; w < kClearWords; w++) {
+      const long long q = first + w * 256;
+      if (q < n0) clear0[q] = 0;
+      else if (q < n0 + n1) clear1[q - n0] = 0;
+    }
+    return;
+  }
   const long long q = blockIdx.x * (long long) blockDim.x + threadIdx.x;
   if (q >= (long long) natoms * C) return;
   const int at = (int) (q / C), n = (int) (q % C);
