@@ -1362,7 +1362,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // arrive while the matrix instructions of step s run; x and the element of the lane's four bonds of the NEXT tile are
 // requested a tile ahead.  No radial row is read: the rows need not exist.  Three waves per SIMD in fp32, with the harmonics of
 // four tiles at once: 65 536 atoms 778 -> 674 us.  No branch in a tile, constant distances between the entries of a bond: 32 768
-// atoms fp32 355 -> 331 us, 3999 atoms of 78 bonds 73.5 -> 63.4, 4001 atoms fp64 95.6 -> 95.4 (without the scheduling barrier 97).
+// atoms fp32 355 -> 331 us, 3999 atoms of 78 bonds 73.5 -> 63.4, 4001 atoms fp64 95.6 -> 95.4 (without the scheduling barrier 97);
+// both column blocks of a 32-channel step requested a step ahead in fp32: 32 768 atoms 335 -> 327 us.
 template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_scatter_a_tab(ScatterArgs<T> a)
 {
   typedef typename Mfma<T>::v4 v4;
@@ -1394,22 +1395,24 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) ==
       m[s] = tb.emu[e];
     }
   };
-  // one (step, 16-column block) at a time: NL x 4 entries in flight per lane
-  T raw[NL][4], zc = (T) 0;
-  double tt = 0.0;
+  // one (step, 16-column block) at a time, QB of them requested ahead: QB x NL x 4 entries in flight per lane
+  constexpr int QB = sizeof(T) == 4 && KB == 2 ? 2 : 1;
+  T raw[QB][NL][4], zc[QB];
+  double tt[QB];
   auto request = [&](int q) {    // q = s KB + cb
     const int s = q / KB, cb = q % KB;
-    const int k = table_interval(xs[s], tb.N, tt);
-    zc = tb.z[ms[s] * C + cb * 16 + c];
+    const int k = table_interval(xs[s], tb.N, tt[q % QB]);
+    zc[q % QB] = tb.z[ms[s] * C + cb * 16 + c];
     const TableRow<T> row = table_row<T, NL * KB * 16>(tb, k, c);
 #pragma unroll
     for (int l = 0; l < NL; l++)
 #pragma unroll
-      for (int e = 0; e < 4; e++) raw[l][e] = table_entry<NL * KB * 16>(row, e)[(l * KB + cb) * 16];
+      for (int e = 0; e < 4; e++) raw[q % QB][l][e] = table_entry<NL * KB * 16>(row, e)[(l * KB + cb) * 16];
   };
   if (w0 < w1) geometry(w0, xs, ms);
   for (long long eb = w0; eb < w1; eb += 16) {
-    request(0);
+#pragma unroll
+    for (int q = 0; q < QB; q++) request(q);
     if (eb + 16 < w1) geometry(eb + 16, xn, mn);
     const int at = (int) (eb - w0) & (YB - 1);      // place of the tile in its round of harmonics
     if (at == 0) {
@@ -1432,10 +1435,11 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) ==
     for (int q = 0; q < 4 * KB; q++) {
       const int s = q / KB, cb = q % KB;
       T bv[NL];
-      const TableBond<T> bond = table_bond<T>(tt, tb.N);
+      const TableBond<T> bond = table_bond<T>(tt[q % QB], tb.N);
+      const auto &w = raw[q % QB];
 #pragma unroll
-      for (int l = 0; l < NL; l++) bv[l] = table_value(table_cubic(raw[l][0], raw[l][1], raw[l][2], raw[l][3], bond), bond) * zc;
-      if (q + 1 < 4 * KB) request(q + 1);
+      for (int l = 0; l < NL; l++) bv[l] = table_value(table_cubic(w[l][0], w[l][1], w[l][2], w[l][3], bond), bond) * zc[q % QB];
+      if (q + QB < 4 * KB) request(q + QB);
       const T *yb = Yw + (at + 4 * s + g) * a.nlm;
 #pragma unroll
       for (int l = 0; l < NL; l++) {
@@ -2637,13 +2641,14 @@ template<class T> struct BondBwdArgs {
 // them it is no faster), and left alone it takes 173 registers where 168 let a third wave in: tables, 65 536 atoms 1.85 -> 1.39 ms,
 // 3999 of GRACE-2L 183 -> 147 us; paired rows, 20 000 atoms 571 -> 536 us.  A fourth wave spills 42 registers (2.03 ms).  Rows of
 // their own serve small structures, which have one block per CU anyway (500 atoms 20.4 -> 21.9 us); from lmax 5 on, with 64
-// channels and in fp64 three waves spill.  Of the forms compiled for three waves two spill at 32 channels and lmax 4: tables 22
-// registers, paired rows 17.
+// channels and in fp64 three waves spill.  Of the forms compiled for three waves one spills, tables at 32 channels and lmax 4 (two
+// registers): the unit vector of a bond is read again behind its tiles and the addresses of a row's harmonics are formed where
+// they are used, 32 768 atoms 725 -> 665 us, 3999 atoms of 78 bonds 153 -> 142, paired rows, 8192 atoms 178 -> 163 (21 and 16 spilled).
 template<class T> constexpr int bond_bwd_waves(int kb, int nl, RowsOf rows) { return sizeof(T) == 4 && kb <= 2 && nl <= 5 && rows != RowsOf::bonds ? 3 : 1; }
 
 // Tiles of 16 bonds whose harmonics a wave evaluates at once, a bond per lane, and waves of a block.  One tile at a time leaves 48
 // lanes idle in the harmonics, half of the vector instructions of a tile in fp32.  Two tiles: paired rows, 8192 atoms fp32 198 -> 178 us,
-// tables, 3999 atoms of 78 bonds 156 -> 150; in fp64, where the harmonics of two tiles leave LDS for six waves of a CU, 203 -> 225 us
+// tables, 3999 atoms of 78 bonds 156 -> 153; in fp64, where the harmonics of two tiles leave LDS for six waves of a CU, 203 -> 225 us
 // (tables, 4001 atoms), 21 -> 25 (128 atoms).
 template<class T> constexpr int bond_bwd_tiles() { return sizeof(T) == 4 ? 2 : 1; }
 template<class T> constexpr int bond_bwd_block() { return 4 / bond_bwd_tiles<T>(); }
@@ -2687,11 +2692,10 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 *
   __syncthreads();
   T *Hw = Hsh + wave * HT * 16 * 3 * NLM;
   int mrow[4];
-  const T *hrow0 = Hw + c * 3 * NLM, *hrow[4];
+  const T *hrow0 = Hw + c * 3 * NLM;
 #pragma unroll
   for (int v = 0; v < 4; v++) {
     mrow[v] = a.drow[4 * g + v];
-    hrow[v] = hrow0 + mrow[v];
   }
   double fi[3] = {0, 0, 0}, vir[6] = {0, 0, 0, 0, 0, 0};
   const int ntile = (int) ((e1_ - e0 + 15) / 16);
@@ -2823,7 +2827,7 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 *
         for (int v = 0; v < 4; v++) {
           int m = mrow[v];
           asm volatile("" : "+v"(m));      // or the compiler keeps (and spills) an address per l and v ahead of the tiles
-          const T *h = (m < 2 * l + 1 ? hrow[v] : hrow0) + ht * 16 * 3 * NLM + l * l;
+          const T *h = hrow0 + (m < 2 * l + 1 ? m : 0) + ht * 16 * 3 * NLM + l * l;
           px += (double) (h[0] * aQ[v]);
           if (l > 0) {
             p1 += (double) (h[NLM] * aP[v]);
@@ -2840,6 +2844,12 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 *
     }
     if (TAB) px_r *= (double) a.tb.N;      // the slopes are per interval
     if (lane < nr) {
+      if (sizeof(T) == 4) {      // read again: held over the tiles they are 6 of the 168 registers
+        int again = 0;
+        asm volatile("" : "+s"(again));
+        const long long e = er + lane + again;
+        u0 = a.rh[3 * e]; u1 = a.rh[3 * e + 1]; u2 = a.rh[3 * e + 2];
+      }
       if (a.bsum) {
         const double *b = a.bsum + 3 * (er + lane);
         px_r += b[0]; p1_r += b[1]; p2_r += b[2];
