@@ -1537,7 +1537,8 @@ class EngineBase : public Engine, protected BufRegistry {
 
   // ---- the generated chain kernels (ChainKernels, jit_chain.hpp) over n atoms, in parts where n is small (parts_for) ----
   // Measured, GRACE-1L with 128 atoms (5 parts): forward 69 -> 32 us, reverse 87 -> 43 us with the sum of the parts;
-  // GRACE-2L with 107 atoms: the four launches 51 + 52 + 58 + 62 -> 19 + 21 + 30 + 29 us.
+  // GRACE-2L with 107 atoms: the four launches 51 + 52 + 58 + 62 -> 19 + 21 + 30 + 29 us (37 + 47 since P3 of layer 1, two launches of
+  // 34 + 38 us, is inside them).
   template<class T, class K>
   void launch_chain_fwd(K &ck, int n, const T *X0, T *X1, T *P2, T *P21, T *P22, T *P3, T *P4, const T *W)
   {
@@ -1682,7 +1683,7 @@ class EngineBase : public Engine, protected BufRegistry {
   // ---- one radial row for both directions of a bond (k_edge_pairs) ----
   // want_pairs_: set by an engine before begin_pass(), from pair_rows_min() bonds of the list on.  Measured: GRACE-1L with
   // 475 136 bonds, network 0.548 -> 0.281 ms, search 0.035 ms; GRACE-2L with 2.5 M bonds, both networks 6.0 -> 2.76 ms, search
-  // 0.16 ms, of the kernels that gather the rows k_pair_fwd 1.40 -> 1.64 ms and the others as before.  Not with tables, where
+  // 0.16 ms, of the kernels that gather the rows k_pair_fwd (then through LDS) 1.40 -> 1.64 ms and the others as before.  Not with tables, where
   // a row costs its stores only (312 018 bonds: 0.080 -> 0.047 ms, less than the search and the gathers).  The rows of a chunk
   // are addressed with 32-bit offsets (k_pair_bwd_mfma), which bounds it from above.
   // The search of a short list takes some 20 us whatever the list, and a network that has few tiles of 16 rows for each SIMD

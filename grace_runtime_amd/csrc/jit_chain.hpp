@@ -410,14 +410,13 @@ inline bool generate_chain(const ChainSpec &sp, ChainCode &out)
   int XM = 1;
   for (const Path &p : paths) XM = std::max(XM, p.M);
   for (const Fc1Path &p : f1) XM = std::max(XM, p.M);
-  const int XR = XM * NA;    // rows of a hand-over buffer
   // Blocks on a CU.  The LDS of a block holds a row for every function of X0 (of its adjoint in the reverse) and the hand-over
   // buffers of the longest path.  In fp64 that used to fill a CU, whose one wave per SIMD then waits at every LDS read, barrier and
   // weight request.  Without FC22 two blocks fit when a path is handed over in pieces and, where that is not enough, the rows of
   // X0 that FC1 works on and those that the paths of P2 work on take turns in the same LDS (layer 2 of a model with parity:
   // 25 and 25 of 49 functions).  Measured, 8192 atoms, fp64, layer 1 / layer 2 of GRACE-2L: forward 204 -> 161 / 215 -> 165 us,
-  // reverse 269 -> 212 / 284 -> 232 (without P3); up to 2048 atoms, where a CU has one block either way: forward 51 -> 48 / 52 -> 49, reverse 64
-  // -> 68 / 63 -> 68.  In fp32 two blocks fit as it is and a third pays in the forward of layer 2 (32 768 atoms: 387 -> 355 us;
+  // reverse 269 -> 212 / 284 -> 232 (layer 1 without its P3, above); up to 2048 atoms, where a CU has one block either way: forward
+  // 51 -> 48 / 52 -> 49, reverse 64 -> 68 / 63 -> 68.  In fp32 two blocks fit as it is and a third pays in the forward of layer 2 (32 768 atoms: 387 -> 355 us;
   // layer 1, which had three: 344 -> 351 and 8192 atoms 91 -> 87); the reverse with three: 440 -> 459 us.  With FC22 (GRACE-1L) the
   // values of a group stay in registers until P4, and two blocks' worth of registers spills: 304 -> 324 us.
   std::vector<char> in_fc1(nf0, 0), in_p2(nf0, 0);    // functions of X0 that the matrix steps of FC1 / of the paths of P2 read
