@@ -74,6 +74,66 @@ def model_l2mix():
     return d
 
 
+def with_fourth_order(d, seed):
+    """`d` (a GRACE-2L model of body order 3 from synth) with the fourth-order stage of both layers: XXXX = XX2 x XX2 with the
+    invariants of structure_1l in layer 1; in layer 2 those of every pair of groups of BB that share L and parity (XX2 and its
+    product as in the reference's container, libgrace/include/grace/model_2l.h:22-175).  A group of functions is a run of
+    fc_*1_w_tile_left with one tile."""
+    rng = np.random.default_rng(seed)
+    s = synth.structure_1l(int(d["lmax"][0]))
+    for k in s:
+        if "AA2" in k or "AAAA" in k:
+            d[k] = s[k]
+    tile = d["fc_BB1_w_tile_left"]
+    first = np.flatnonzero(np.concatenate([[True], np.diff(tile) != 0]))
+    size = np.diff(np.append(first, len(tile)))
+    terms, nout = [], 0
+    for q in range(len(first)):
+        for p in range(q + 1):
+            if d["fc_BB1_collect_from"][first[p]] == d["fc_BB1_collect_from"][first[q]]:      # the same piece of B: L and parity
+                terms += [(nout, first[q] + m, first[p] + m, 1.0 / size[q]) for m in range(size[q])]
+                nout += 1
+    o, l, r, c = zip(*terms)
+    i64 = lambda v: np.array([v], dtype=np.int64)    # noqa: E731
+    d.update(prod_BBBB_left_ind=np.array(l, np.int32), prod_BBBB_right_ind=np.array(r, np.int32), prod_BBBB_m_sum_ind=np.array(o, np.int32),
+             prod_BBBB_cg_coeff=np.array(c), prod_BBBB_n_output_funcs=i64(nout), prod_BBBB_n_cg_terms=i64(len(c)), prod_BBBB_lmax=i64(0),
+             prod_BBBB_Lmax=i64(0))
+    for k in ("w_tile_left", "w_tile_right", "collect_to", "collect_from", "norm_out_factor"):
+        d["fc_BB2_" + k] = d["fc_BB1_" + k].copy()
+    for X in ("AA", "BB"):
+        for k in ("norm_left", "norm_right", "n_out", "left_coefs"):
+            d[f"fc_{X}2_{k}"] = d[f"fc_{X}1_{k}"]
+        for k in ("w_left", "w_right"):
+            d[f"fc_{X}2_{k}"] = rng.standard_normal(d[f"fc_{X}1_{k}"].shape)
+    for pfx, X in (("I1", "A"), ("rho", "A"), ("I2", "B")):
+        n, src = int(d[f"prod_{4 * X}_n_output_funcs"][0]), 4 * X
+        n_el, n_out, n_in, _ = d[f"{pfx}_reduce_{X}_W"].shape
+        d[f"{pfx}_collect_ind_{src}"] = np.arange(n, dtype=np.int32)
+        d[f"{pfx}_w_l_tile_{src}"] = np.arange(n, dtype=np.int32)
+        d[f"{pfx}_total_sum_ind_{src}"] = np.zeros((n, 1), np.int32)
+        d[f"{pfx}_w_shape_{src}"] = i64(n)
+        d[f"{pfx}_reduce_{src}_W"] = rng.standard_normal((n_el, n_out, n_in, n))
+        d[f"{pfx}_reduce_{src}_norm"] = d[f"{pfx}_reduce_{X}_norm"]
+        d[f"{pfx}_n_in_{src}"] = d[f"{pfx}_n_in_{X}"]
+        d[f"{pfx}_instruction_names"] = np.append(d[f"{pfx}_instruction_names"], np.array([src.encode()], dtype="|S8"))
+    return d
+
+
+def model_l2ord4():
+    """GRACE-2L, two elements, lmax 3, body order 4 in both layers, 20 channels (padded to 32, the width of the fused dense chain):
+    the third product of layer 1 has more than 24 outputs"""
+    return with_fourth_order(synth.random_model_2l(lmax=3, n_elements=2, element_names=("Mo", "W"), embedding_size=8, nradbase=8, c1=20, cr=12, c2=20,
+                                                   i1_width=10, hidden=32, rho_n_out=9, energy_hidden=16, rcut=5.0, inv_avg_n_neigh=1.0 / 26.0,
+                                                   seed=14), seed=15)
+
+
+def model_l2deep():
+    """GRACE-2L, two elements, lmax 5, 20 channels: the eleven functions of l = 5 are two paths of the fused dense chain, and outputs
+    of the third product are fed by both"""
+    return synth.random_model_2l(lmax=5, n_elements=2, element_names=("Mo", "W"), embedding_size=8, nradbase=8, c1=20, cr=12, c2=20, i1_width=10,
+                                 hidden=32, rho_n_out=9, energy_hidden=16, rcut=5.0, inv_avg_n_neigh=1.0 / 26.0, seed=16)
+
+
 def model_l3mix():
     """GRACE-3L, two elements with pair-specific cutoffs, lmax 2, messages with both parities"""
     d = synth.random_model_3l(lmax=2, n_elements=2, element_names=("Mo", "W"), embedding_size=8, nradbase=10, channels=16,
@@ -183,8 +243,8 @@ def model_uq3l():
     return d
 
 
-MODELS = {"ch20": model_ch20, "ch3": model_ch3, "ch48": model_ch48, "chleg": model_chleg, "uq3l": model_uq3l, "uq2l": model_uq2l, "uq2": model_uq2, "l3mix": model_l3mix, "l3wide": model_l3wide, "l3pad": model_l3pad, "l3el": model_l3el, "l3nat": model_l3nat, "config4": model_config4, "config5": model_config5, "config1": model_config1, "mix2": model_mix2, "cut2": model_cut2, "config3": model_config3, "l2mix": model_l2mix}
-LAYERS = {"ch20": 1, "ch3": 1, "ch48": 1, "chleg": 1, "uq3l": 3, "uq2l": 2, "uq2": 1, "l3mix": 3, "l3wide": 3, "l3pad": 3, "l3el": 3, "l3nat": 3, "config4": 3, "config5": 2, "config1": 1, "mix2": 1, "cut2": 1, "config3": 2, "l2mix": 2}
+MODELS = {"ch20": model_ch20, "ch3": model_ch3, "ch48": model_ch48, "chleg": model_chleg, "uq3l": model_uq3l, "uq2l": model_uq2l, "uq2": model_uq2, "l3mix": model_l3mix, "l3wide": model_l3wide, "l3pad": model_l3pad, "l3el": model_l3el, "l3nat": model_l3nat, "config4": model_config4, "config5": model_config5, "config1": model_config1, "mix2": model_mix2, "cut2": model_cut2, "config3": model_config3, "l2mix": model_l2mix, "l2ord4": model_l2ord4, "l2deep": model_l2deep}
+LAYERS = {"ch20": 1, "ch3": 1, "ch48": 1, "chleg": 1, "uq3l": 3, "uq2l": 2, "uq2": 1, "l3mix": 3, "l3wide": 3, "l3pad": 3, "l3el": 3, "l3nat": 3, "config4": 3, "config5": 2, "config1": 1, "mix2": 1, "cut2": 1, "config3": 2, "l2mix": 2, "l2ord4": 2, "l2deep": 2}
 
 
 def write_model(name, directory):

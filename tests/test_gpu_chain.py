@@ -144,6 +144,24 @@ def test_compiled_kernels_are_kept_on_disk_for_the_next_process(model_dir, tmp_p
     assert not os.path.exists(tmp_path / "home" / ".cache" / "grace_hip")
 
 
+@pytest.mark.parametrize("model,species,precision,fused,files", [("config3", ["Al", "Co", "Ni", "Ti"], 64, "1", 2), ("l2ord4", ["Mo", "W"], 64, "1", 2),
+                                                                 ("l2deep", ["Mo", "W"], 32, "1", 4), ("config3", ["Al", "Co", "Ni", "Ti"], 64, "0", 4),
+                                                                 ("l2ord4", ["Mo", "W"], 64, "0", 6)])
+def test_a_two_layer_engine_compiles_what_a_pass_launches(model_dir, tmp_path, model, species, precision, fused, files):
+    """the code objects that creating an engine leaves on disk: the chain of each layer, with the third product of a chain that leaves
+    it outside, or without chains all products of both layers"""
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = (f"import sys; sys.path.insert(0, {root!r})\n"
+            "from grace_runtime_amd import kk\n"
+            f"kk.Engine(kk.Model({cases.model_file(model_dir, model)!r}), {species!r}, {precision})\n")
+    env = dict(os.environ, GRACE_HIP_CACHE=str(tmp_path), GRACE_HIP_CHAIN=fused)
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env, timeout=110)
+    assert res.returncode == 0, res.stderr
+    assert len(os.listdir(tmp_path)) == files
+
+
 @pytest.mark.parametrize("precision", [64, 32])
 @pytest.mark.parametrize("natoms", [9, 350, 1020, 1030])
 @pytest.mark.parametrize("model", ["ch20", "config3"])
