@@ -379,7 +379,7 @@ template<class T> void Engine1L<T>::run(const RunFlags &fl)
   const size_t na = (size_t) round_up(cs, 16);
   paired_ = false;
   if (!tables_in_kernels()) {    // with tables evaluated inside the kernels the rows do not exist
-    pair_rows(cs, ecap, noutp_, ebound);
+    pair_rows(cs, ebound);
     Rz_.ensure(ecap * noutp_ * sizeof(T));
     dRz_.ensure(ecap * noutp_ * sizeof(T));
   }

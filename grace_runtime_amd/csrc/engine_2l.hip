@@ -640,7 +640,7 @@ template<class T> void Engine2L<T>::run(const RunFlags &fl)
     cur_ntiles_ = chunk_tile_off_[(size_t) q + 1] - chunk_tile_off_[(size_t) q];
   };
   const size_t na = cap_, nnodes = (size_t) n_nodes_;
-  pair_rows(cs, ecap, std::max(radR_.noutp, radR1_.noutp), ebound);
+  pair_rows(cs, ebound);
 
   // buffers of the whole structure
   rho_.ensure((size_t) n * nrho_ * sizeof(double));

@@ -1684,8 +1684,8 @@ class EngineBase : public Engine, protected BufRegistry {
   // want_pairs_: set by an engine before begin_pass(), from pair_rows_min() bonds of the list on.  Measured: GRACE-1L with
   // 475 136 bonds, network 0.548 -> 0.281 ms, search 0.035 ms; GRACE-2L with 2.5 M bonds, both networks 6.0 -> 2.76 ms, search
   // 0.16 ms, of the kernels that gather the rows k_pair_fwd (then through LDS) 1.40 -> 1.64 ms and the others as before.  Not with tables, where
-  // a row costs its stores only (312 018 bonds: 0.080 -> 0.047 ms, less than the search and the gathers).  The rows of a chunk
-  // are addressed with 32-bit offsets (k_pair_bwd_mfma), which bounds it from above.
+  // a row costs its stores only (312 018 bonds: 0.080 -> 0.047 ms, less than the search and the gathers).  Not from 2^31 listed
+  // bonds on: the numbers of rows are 32-bit integers (begin_pass).
   // The search of a short list takes some 20 us whatever the list, and a network that has few tiles of 16 rows for each SIMD
   // does not get quicker by half when half of them go.  The line is at three tiles per SIMD of listed bonds and one network in
   // fp64, where a tile takes twice as long as in fp32; two networks share one search.  A call with own rows over one with
@@ -1708,10 +1708,10 @@ class EngineBase : public Engine, protected BufRegistry {
   static constexpr double kPairRowBytes = 2 * sizeof(int) + sizeof(double);    // erow_, uid_, ux_, per bond
   bool want_pairs_ = false, paired_ = false;
   int pair_chunks_ = 0;
-  // chunks of cs atoms; chunk_edges: bonds of the largest; bounds: first bond of every chunk (empty: one chunk of all atoms)
-  void pair_rows(int cs, size_t chunk_edges, int noutp, const std::vector<long long> &bounds)
+  // chunks of cs atoms; bounds: first bond of every chunk (empty: one chunk of all atoms)
+  void pair_rows(int cs, const std::vector<long long> &bounds)
   {
-    paired_ = want_pairs_ && (double) chunk_edges * noutp < 2147483647.0;
+    paired_ = want_pairs_;
     if (!paired_) return;
     const int n = n_, nch = pair_chunks_ = (n + cs - 1) / cs;
     uid_.ensure((size_t) nb_ * sizeof(int));

@@ -83,6 +83,22 @@ def test_shared_rows_of_the_vector_pair_kernels(model_dir, shared_from_one_bond,
     _check(model_dir, "l2mix", variant, precision, chunk)
 
 
+@pytest.mark.parametrize("model,species", [("config1", ["W"]), ("config3", ["Al", "Co", "Ni", "Ti"])])
+def test_shared_rows_beyond_32_bit_offsets(model_dir, model, species):
+    """one pass over 14 M bonds, whose rows of 160 values hold more than 2^31, against the same structure in chunks whose rows hold
+    fewer; both at the fp32 gate of the reference (a bond that a chunk cuts has two rows, whose arguments differ in rounding)"""
+    pos, cell = synth.bcc_supercell(2.4, 38)
+    pos = synth.jitter(pos, 0.05, 6)
+    types = np.random.default_rng(6).integers(1, len(species) + 1, len(pos)).astype(np.int32)
+    out = {}
+    for chunk in (0, 32768):
+        s = kk.System(kk.Model(cases.model_file(model_dir, model)), species, skin=0.0, chunksize=chunk, precision=32)
+        out[chunk] = s.compute(types, pos, cell, [True] * 3, energies=True)
+        bonds, rows = s.engine.edge_count(), s.engine.radial_rows()
+        assert bonds * 160 > 2**31 and (rows == bonds / 2 if chunk == 0 else bonds / 2 < rows < bonds)
+    cases.check_against(out[0], out[32768], len(pos), 1e-6, 2e-5, 1e-5, 1e-5)
+
+
 def _check(model_dir, model, variant, precision, chunk):
     path = cases.model_file(model_dir, model)
     types, offset, j, rij = _list(variant)
