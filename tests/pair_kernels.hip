@@ -2,76 +2,16 @@
 // same sums in fp64 on the host:
 //
 //   pair_kernels fwd|bwd 64|32 <lmax + 1>
+//   pair_kernels compare <value> <wanted value> <bound>     the comparison itself, on the host
 //
 // Sizes: channels that fill a wave, half a wave, or part of one; slots that leave the last wave partly empty; atoms with no bond,
-// fewer and more bonds than a chunk; a radial row per bond and per pair of atoms; launches that count as few and as many waves.
-// Bound of a value: (longest chain of additions) eps (sum of the absolute terms).  Prints the worst ratio of difference to bound.
-#include <algorithm>
-#include <cmath>
-#include <cstdio>
-#include <cstdlib>
+// fewer and more bonds than a chunk; a radial row per bond and per pair of atoms; launches that count as few and as many waves;
+// adjoints for every slot (GRACE-3L) and for all but the last (GRACE-2L), with values behind them that have to stay.
+// Bound of a value: (longest chain of additions) eps (sum of the absolute terms).  Prints the worst ratio of difference to bound,
+// 1e300 where a difference is no number or a value without a bound differs.
+#include "kernel_program.hpp"
+
 #include <cstring>
-#include <map>
-#include <stdexcept>
-#include <vector>
-
-#include <hip/hip_runtime.h>
-
-struct Error : std::runtime_error {
-  using std::runtime_error::runtime_error;
-};
-#define HIP_CHECK(expr)                                                                         \
-  do {                                                                                          \
-    const hipError_t err_ = (expr);                                                             \
-    if (err_ != hipSuccess) throw Error(std::string(#expr) + ": " + hipGetErrorString(err_));   \
-  } while (0)
-#include "../grace_runtime_amd/csrc/kernels_2l.hpp"
-
-using namespace grhip;
-
-template<class U> static U *upload(const std::vector<U> &v)
-{
-  U *p = nullptr;
-  HIP_CHECK(hipMalloc(&p, std::max<size_t>(v.size(), 1) * sizeof(U)));
-  if (!v.empty()) HIP_CHECK(hipMemcpy(p, v.data(), v.size() * sizeof(U), hipMemcpyHostToDevice));
-  return p;
-}
-template<class U> static std::vector<U> download(const U *p, size_t n)
-{
-  std::vector<U> v(n);
-  if (n) HIP_CHECK(hipMemcpy(v.data(), p, n * sizeof(U), hipMemcpyDeviceToHost));
-  return v;
-}
-
-static unsigned long long state = 1;
-static double uniform()    // in [-1, 1)
-{
-  state = state * 6364136223846793005ull + 1442695040888963407ull;
-  return (double) (state >> 11) / 4503599627370496.0 - 1.0;
-}
-template<class T> static std::vector<T> randoms(size_t n)
-{
-  std::vector<T> v(n);
-  for (T &x : v) x = (T) uniform();
-  return v;
-}
-
-// accumulator row of (lane / 16, register) of a 16x16x4 MFMA, from the product of rows 0 .. 15 with ones
-template<class T> static void probe(int *drow)
-{
-  std::vector<T> A(64, (T) 0), B(64, (T) 0);
-  for (int q = 0; q < 16; q++) {
-    A[4 * q] = (T) q;    // k = 0 alone
-    B[q] = (T) 1;
-  }
-  T *dA = upload(A), *dB = upload(B), *dD = upload(std::vector<T>(256, (T) -1));
-  hipLaunchKernelGGL(k_mfma_probe<T>, dim3(1), dim3(64), 0, 0, dA, dB, dD);
-  HIP_CHECK(hipDeviceSynchronize());
-  const std::vector<T> D = download(dD, 256);
-  for (int g = 0; g < 4; g++)
-    for (int v = 0; v < 4; v++) drow[4 * g + v] = (int) D[(16 * g) * 4 + v];
-  for (void *p : {(void *) dA, (void *) dB, (void *) dD}) HIP_CHECK(hipFree(p));
-}
 
 template<class T> struct Problem {
   int natoms, nslot, C, nl, nlm, noutp, ystr;
@@ -107,9 +47,8 @@ template<class T> struct Problem {
 static double worst = 0.0;
 static void compare(double got, double want, double bound)
 {
-  const double d = std::fabs(got - want);
-  if (!(d <= bound) && d / std::max(bound, 1e-300) > worst) worst = bound > 0 ? d / bound : 1e300;
-  else if (bound > 0) worst = std::max(worst, d / bound);
+  const double d = std::fabs(got - want), ratio = bound > 0 ? d / bound : d == 0 ? 0.0 : 1e300;
+  if (!(ratio <= worst)) worst = ratio <= 1e300 ? ratio : 1e300;    // not a number: neither comparison holds
 }
 
 template<class T> static void run_fwd(const Problem<T> &p, int simds)
@@ -145,24 +84,30 @@ template<class T> static void run_fwd(const Problem<T> &p, int simds)
     if (q) HIP_CHECK(hipFree(q));
 }
 
-template<class T> static void run_bwd(const Problem<T> &p, const int *drow)
+// nI: slots that have an adjoint
+template<class T> static void run_bwd(const Problem<T> &p, const int *drow, int nI)
 {
   const double eps = sizeof(T) == 4 ? 1.1920929e-7 : 2.220446049250313e-16;
   const PairMfmaPlan plan = pair_mfma_plan(p.nslot, p.C, p.nl, sizeof(T), pair_mfma_waves(0));
   if (!plan.ok || plan.ystr != p.ystr) throw Error("no plan");
-  const size_t E = p.ej.size(), nM = (size_t) p.natoms * p.nslot * p.C;
+  const size_t E = p.ej.size(), nM = (size_t) p.natoms * nI * p.C;
   long long *eoff = upload(p.eoff);
   int *ej = upload(p.ej), *erow = p.erow.empty() ? nullptr : upload(p.erow);
-  T *Y = upload(p.Y), *R = upload(p.R), *dR = upload(p.dR), *M = upload(p.M), *gP = upload(p.gP), *gM = upload(std::vector<T>(nM, (T) 0));
+  T *Y = upload(p.Y), *R = upload(p.R), *dR = upload(p.dR), *M = upload(p.M), *gP = upload(p.gP), *gM = nullptr;
+  {
+    std::vector<T> zeros(nM, (T) 0);
+    zeros.resize(nM + p.C, (T) 3);    // what a slot without an adjoint would add to behind the last atom
+    gM = upload(zeros);
+  }
   double *bsum = upload(std::vector<double>(3 * E, 0.0));
   PairMfmaArgs<T> a{};
   a.eoff = eoff; a.ej = ej; a.erow = erow; a.YG = Y; a.R1 = R; a.dR1 = dR; a.M = M; a.gP = gP; a.gM = gM; a.bsum = bsum;
-  a.nslot = p.nslot; a.nI = p.nslot; a.C = p.C; a.noutp = p.noutp; a.natoms = p.natoms;
+  a.nslot = p.nslot; a.nI = nI; a.C = p.C; a.noutp = p.noutp; a.natoms = p.natoms;
   for (int q = 0; q < 16; q++) a.drow[q] = drow[q];
   launch_pair_bwd_mfma<T, true>(plan, a, p.nl, 0);
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipDeviceSynchronize());
-  const std::vector<T> gotM = download(gM, nM);
+  const std::vector<T> gotM = download(gM, nM + p.C);
   const std::vector<double> gotB = download(bsum, 3 * E);
   std::vector<double> wantM(nM, 0.0), magM(nM, 0.0), wantB(3 * E, 0.0), magB(3 * E, 0.0);
   for (int i = 0; i < p.natoms; i++)
@@ -173,11 +118,14 @@ template<class T> static void run_bwd(const Problem<T> &p, const int *drow)
             for (int n = 0; n < p.C; n++) {
               const double g = p.gP[(((size_t) i * p.nslot + s) * p.nlm + f) * p.C + n], r = p.R[p.row(e) * p.noutp + l * p.C + n],
                            d = p.dR[p.row(e) * p.noutp + l * p.C + n];
-              const size_t jm = ((size_t) p.ej[e] * p.nslot + s) * p.C + n;
-              const double mv = p.M[jm], y = p.Y[e * p.ystr + f], y1 = p.Y[e * p.ystr + p.nlm + f], y2 = p.Y[e * p.ystr + 2 * p.nlm + f];
+              const size_t jm = ((size_t) p.ej[e] * nI + s) * p.C + n;
+              const double mv = p.M[((size_t) p.ej[e] * p.nslot + s) * p.C + n];
+              const double y = p.Y[e * p.ystr + f], y1 = p.Y[e * p.ystr + p.nlm + f], y2 = p.Y[e * p.ystr + 2 * p.nlm + f];
               const double t[4] = {g * r * y, g * d * y * mv, g * r * y1 * mv, g * r * y2 * mv};
-              wantM[jm] += t[0];
-              magM[jm] += std::fabs(t[0]);
+              if (s < nI) {
+                wantM[jm] += t[0];
+                magM[jm] += std::fabs(t[0]);
+              }
               for (int k = 0; k < 3; k++) {
                 wantB[3 * e + k] += t[k + 1];
                 magB[3 * e + k] += std::fabs(t[k + 1]);
@@ -185,7 +133,10 @@ template<class T> static void run_bwd(const Problem<T> &p, const int *drow)
             }
   // additions a value goes through: the functions of an l, the l, the slots of a wave; then the bonds of a target, or lanes and waves
   const double chain = p.nlm + p.nl + 4.0;
-  for (size_t q = 0; q < nM; q++) compare((double) gotM[q], wantM[q], eps * (chain + (double) E) * magM[q]);
+  std::vector<int> into(p.natoms, 0);
+  for (int j : p.ej) into[j]++;
+  for (size_t q = 0; q < nM; q++) compare((double) gotM[q], wantM[q], eps * (chain + into[q / ((size_t) nI * p.C)]) * magM[q]);
+  for (int n = 0; n < p.C; n++) compare((double) gotM[nM + n], 3.0, 0.0);
   for (size_t q = 0; q < 3 * E; q++) compare(gotB[q], wantB[q], eps * (chain + p.nslot + p.C) * magB[q]);
   for (void *q : {(void *) eoff, (void *) ej, (void *) erow, (void *) Y, (void *) R, (void *) dR, (void *) M, (void *) gP, (void *) gM, (void *) bsum})
     if (q) HIP_CHECK(hipFree(q));
@@ -202,14 +153,19 @@ template<class T> static void run(bool fwd, int nl)
           if (C == 80 && natoms > 1 && nslot > 2) continue;    // the host's sums
           const Problem<T> p(natoms, nslot, C, nl, pairs != 0);
           if (fwd) for (int simds : {1, 1 << 20}) run_fwd<T>(p, simds);
-          else run_bwd<T>(p, drow);
+          else for (int nI = std::max(1, nslot - 1); nI <= nslot; nI++) run_bwd<T>(p, drow, nI);
         }
 }
 
 int main(int argc, char **argv)
 {
+  if (argc == 5 && std::strcmp(argv[1], "compare") == 0) {
+    compare(std::atof(argv[2]), std::atof(argv[3]), std::atof(argv[4]));
+    std::printf("%.6g\n", worst);
+    return 0;
+  }
   if (argc != 4) {
-    std::fprintf(stderr, "usage: pair_kernels fwd|bwd 64|32 <lmax + 1>\n");
+    std::fprintf(stderr, "usage: pair_kernels fwd|bwd 64|32 <lmax + 1>\n       pair_kernels compare <value> <wanted value> <bound>\n");
     return 2;
   }
   try {
