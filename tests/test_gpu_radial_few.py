@@ -1,6 +1,10 @@
 """k_radial_few, which shares a tile of 16 bonds among the waves of a block where there are few tiles, against k_radial: the same
 sums in the same order, so every value agrees in every bit whatever number of bonds a call has (radial MLP:
 libgrace/include/grace/radial_x.h:11-60)."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -8,6 +12,8 @@ import cases
 from grace_runtime_amd import kk, synth
 
 pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def wide(path):
@@ -31,3 +37,18 @@ def test_few_and_many_bonds_give_the_same_bits(model_dir, tmp_path, model, speci
     for n in (1, 15, 16, 17, 255, 16 * 256 + 1, line):
         r, dr = engine.debug_radial(x[:n], mu[:n])
         assert np.array_equal(r, R[:n]) and np.array_equal(dr, dR[:n])
+
+
+@pytest.mark.parametrize("hidden", [64, 128])
+@pytest.mark.parametrize("precision", [64, 32])
+def test_species_form_gives_the_same_bits(precision, hidden):
+    """the networks of GRACE-3L, launched by themselves (tests/radial_kernels.hip): with ordered sums a chunk of a structure is to give
+    the same rows on either side of the line between the two kernels"""
+    exe = os.path.join(ROOT, "tests", "build", "radial_kernels")
+    if not os.path.exists(exe):
+        sys.path.insert(0, ROOT)
+        import __graft_entry__
+        exe = __graft_entry__.build_kernel_program("radial_kernels")
+    r = subprocess.run([exe, str(precision), str(hidden)], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr
+    assert int(r.stdout) == 0
