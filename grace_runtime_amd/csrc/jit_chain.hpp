@@ -279,9 +279,12 @@ inline bool generate_chain(const ChainSpec &sp, ChainCode &out)
   // ---- P3 path by path: with many outputs, each fed by one path, a path forms its own from the values it has at hand and the rows
   // of X0 in LDS, and the reverse reads their adjoints where it reads the path's rows of P21.  P21 is then read once and its adjoint
   // never stored.  Layer 1 of GRACE-2L (113 outputs, which all at once spilled 1100 registers), 8192 atoms, fp64: forward 161 -> 183
-  // us in place of a product kernel of 131, reverse 211 -> 344 in place of one of 216 (in pieces of four functions: 35 registers
+  // us in place of a product kernel of 131, reverse 211 -> 344 in place of one of 216 (in pieces of four functions: 30 registers
   // spill; 374 in pieces of six, 395 with the adjoint of X0 taken behind the matrix phase).  107 atoms: 34 + 38 us of the
   // product kernels saved; the passes of 107, 3999 (fp32) and 32 000 atoms 444 -> 392, 1329 -> 1279 us and 16.3 -> 15.8 ms.
+  // Together with FC22, whose values stay in registers (body order 4, lmax 3, 56 outputs; no register spills): the pass of 54 atoms
+  // 310 -> 287 us, 2000 754 -> 712, 32 000 8.02 -> 7.50 ms, fp32 260 -> 238, 529 -> 489, 4.36 -> 3.97.
+  // Paths are cut at maxM functions: from lmax 5 on an output is fed by both parts of a path, and P3 stays outside.
   bool one_path = true;
   for (const auto &kv : p3_by_o)
     for (const ProdTerm *t : kv.second) one_path = one_path && path_of[t->l] == path_of[kv.second[0]->l];
@@ -416,7 +419,7 @@ inline bool generate_chain(const ChainSpec &sp, ChainCode &out)
   // X0 that FC1 works on and those that the paths of P2 work on take turns in the same LDS (layer 2 of a model with parity:
   // 25 and 25 of 49 functions).  Measured, 8192 atoms, fp64, layer 1 / layer 2 of GRACE-2L: forward 204 -> 161 / 215 -> 165 us,
   // reverse 269 -> 212 / 284 -> 232 (layer 1 without its P3, above); up to 2048 atoms, where a CU has one block either way: forward
-  // 51 -> 48 / 52 -> 49, reverse 64 -> 68 / 63 -> 68.  In fp32 two blocks fit as it is and a third pays in the forward of layer 2 (32 768 atoms: 387 -> 355 us;
+  // 51 -> 48 / 52 -> 49, reverse 64 -> 68 / 63 -> 68.  In layer 2 the reverse spills 28 registers.  In fp32 two blocks fit as it is and a third pays in the forward of layer 2 (32 768 atoms: 387 -> 355 us;
   // layer 1, which had three: 344 -> 351 and 8192 atoms 91 -> 87); the reverse with three: 440 -> 459 us.  With FC22 (GRACE-1L) the
   // values of a group stay in registers until P4, and two blocks' worth of registers spills: 304 -> 324 us.
   std::vector<char> in_fc1(nf0, 0), in_p2(nf0, 0);    // functions of X0 that the matrix steps of FC1 / of the paths of P2 read

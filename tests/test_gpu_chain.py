@@ -214,3 +214,39 @@ def test_blocks_that_share_a_cu(model_dir, natoms, precision):
         assert ("chain_bwd_L2" in eng.stage_times()) == fused
     same = 1e-11 if precision == 64 else 2e-5
     cases.check_against(out[0], out[1], natoms, same, 10 * same, same, 10 * same)
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("model", ["l2ord4", "l2deep"])
+def test_third_product_of_many_outputs(model_dir, model, precision):
+    """l2ord4: P3 path by path together with the fourth-order stage, whose values stay in registers (layer 1); l2deep: the paths of
+    l = 5 are cut at nine functions and an output is fed by both parts, so P3 stays outside of the chain kernels (both layers in
+    fp32; in fp64 the rows of layer 2 do not fit the LDS and it runs stage by stage).  In parts (9 and 250 atoms) and whole (1030),
+    against the oracle and against the stages, bounds as above."""
+    from grace_runtime_amd import synth
+    from oracle import grace_oracle_2l as g2
+    path = cases.model_file(model_dir, model)
+    om = g2.Model2L(path)
+    engines = [_engine(path, ["Mo", "W"], precision, fused) for fused in (True, False)]
+    same = 1e-11 if precision == 64 else 2e-5
+    for natoms in (9, 250, 1030):
+        pos, cell = synth.bcc_supercell(3.165, 9)
+        rng = np.random.default_rng(natoms)
+        pos = synth.jitter(pos, 0.05, 3)[np.sort(rng.permutation(len(pos))[:natoms])]
+        types = rng.integers(1, 3, natoms).astype(np.int32)
+        perm, offset, j, image, shifts = kk.neighbor_search(pos, cell, [True] * 3, float(np.max(om.cut)))
+        rij = cases.bond_vectors(pos, perm, offset, j, image, shifts)
+        out = []
+        for eng in engines:
+            eng.set_profile(True)
+            out.append(eng.compute(types[perm], offset, j, rij=rij, energies=True))
+        names = set(engines[0].stage_times())
+        chains = {"_L1"} if model == "l2deep" and precision == 64 else {"_L1", "_L2"}
+        assert {s[9:] for s in names if s.startswith("chain_bwd")} == chains
+        # the 71 functions of layer 2 of l2deep are more than a chain in parts keeps track of
+        assert {s[9:] for s in names if s.startswith("chain_sum")} == (set() if natoms > 1024 else chains if model == "l2ord4" else {"_L1"})
+        assert all((f"prod_3{t}" in names and f"prod_3_bwd{t}" in names) == (model == "l2deep") for t in chains)
+        cases.check_against(out[0], out[1], natoms, same, 10 * same, same, 10 * same)
+        if natoms <= 250:
+            ref = g2.compute_2l(om, types[perm] - 1, offset, j, rij)
+            cases.check_against(out[0], ref, natoms, *((1e-10, 1e-9, 1e-10, 1e-9) if precision == 64 else (1e-6, 2e-5, 1e-5, 1e-5)))
