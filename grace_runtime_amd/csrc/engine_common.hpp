@@ -1407,7 +1407,7 @@ class EngineBase : public Engine, protected BufRegistry {
   {
     for (int q = 0; q < 16; q++) ba.drow[q] = drow_[q];
     const int kb = ba.C / 16;
-    const size_t lds = ((size_t) ba.nlm * (ba.C + 2) + (size_t) 4 * 16 * ba.nlm * 3) * sizeof(T);      // four tiles of bonds
+    const size_t lds = ((size_t) ba.nlm * (ba.C + 2) + (size_t) 4 * 16 * bond_bwd_row(ba.nlm)) * sizeof(T);      // four tiles of bonds
     if (kb != 1 && kb != 2 && kb != 4) throw Error("bond backward: channel width must be 16, 32 or 64");
     if (ba.tb.F && ba.noutp != ba.nl * ba.C) throw Error("bond backward: rows of the radial tables of another width");
 #define GR_BB(KB, NL)                                                                                  \

@@ -2657,6 +2657,10 @@ template<class T> constexpr int bond_bwd_waves(int kb, int nl, RowsOf rows) { re
 // (tables, 4001 atoms), 21 -> 25 (128 atoms).
 template<class T> constexpr int bond_bwd_tiles() { return sizeof(T) == 4 ? 2 : 1; }
 template<class T> constexpr int bond_bwd_block() { return 4 / bond_bwd_tiles<T>(); }
+// Values of a bond in LDS, its harmonics and their two gradient components: odd, so that the 16 bonds of a tile, which are read at
+// once, start in different banks.  As 3 nlm values, which is even from lmax 1 on for every second lmax and 48 at lmax 3: 3456 atoms of 58
+// bonds, lmax 3 fp64, paired rows of 16 channels 97.7 -> 70.0 us, of 32 113.6 -> 92.2, of 64 223.5 -> 204.4.
+constexpr int bond_bwd_row(int nlm) { return 3 * nlm | 1; }
 
 // One block per atom; a wave takes rounds of HT tiles of 16 bonds.  Per tile and l two tile GEMMs on the matrix cores,
 //   P[m][b] = sum_n gA[l*l + m][n] Rz[b][l][n],   Q[m][b] = sum_n gA[l*l + m][n] dRz[b][l][n]      (K = channels)
@@ -2670,7 +2674,7 @@ template<class T> constexpr int bond_bwd_block() { return 4 / bond_bwd_tiles<T>(
 // the harmonics' gradients are kept as their two components along e1 and e2: two sums per bond instead of three, and a
 // third less LDS per block (three blocks per CU instead of two).  gA of the atom sits in LDS as [lm][C + 2]
 // (the pad spreads the rows over the banks); the radial rows of l + 1 are requested before the products of l.
-// KB = channels / 16, NL = lmax + 1.  dynamic LDS: nlm (C + 2) + 4 tiles x 16 bonds x 3 nlm values.
+// KB = channels / 16, NL = lmax + 1.  dynamic LDS: nlm (C + 2) + 4 tiles x 16 bonds x bond_bwd_row(nlm) values.
 // l = 0 has no gradient: its radial function is neither read nor evaluated, its derivative is (a tenth of the rows at lmax 4).  With
 // that, the harmonics of a bond in one row and fewer address instructions: paired rows, 8192 atoms fp64 280 -> 254 us, fp32 226 ->
 // 198; tables, 3999 atoms fp32 166 -> 156, 4001 atoms fp64 211 -> 204, and the tiles two at a time above.
@@ -2681,10 +2685,10 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 *
   constexpr int HT = bond_bwd_tiles<T>(), NW = bond_bwd_block<T>();
   constexpr bool TAB = ROWS == RowsOf::tables, PAIRS = ROWS == RowsOf::pairs;
   typedef typename Mfma<T>::v4 v4;
-  constexpr int KS = KB * 4, C = KB * 16, CS = C + 2, NLM = NL * NL;
+  constexpr int KS = KB * 4, C = KB * 16, CS = C + 2, NLM = NL * NL, HS = bond_bwd_row(NLM);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *gAl = reinterpret_cast<T *>(smem_raw);                          // [NLM][CS]
-  T *Hsh = gAl + NLM * CS;                                           // [NW waves][16 HT][3][NLM]: harmonics, gradient . e1, gradient . e2
+  T *Hsh = gAl + NLM * CS;                                           // [NW waves][16 HT][HS]: harmonics, gradient . e1, gradient . e2
   __shared__ double red[NW][9];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int c = lane & 15, g = lane >> 4;
@@ -2695,9 +2699,9 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 *
     for (int q = t; q < NLM * C; q += 64 * NW) gAl[(q / C) * CS + q % C] = gAi[q];
   }
   __syncthreads();
-  T *Hw = Hsh + wave * HT * 16 * 3 * NLM;
+  T *Hw = Hsh + wave * HT * 16 * HS;
   int mrow[4];
-  const T *hrow0 = Hw + c * 3 * NLM;
+  const T *hrow0 = Hw + c * HS;
 #pragma unroll
   for (int v = 0; v < 4; v++) {
     mrow[v] = a.drow[4 * g + v];
@@ -2767,7 +2771,7 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 *
       br = a.r[e]; brc = a.rc[e]; jj = a.ej[e];
       const double u[3] = {u0, u1, u2};
       tangent_basis(u, e1, e2);
-      T *h = Hw + lane * 3 * NLM;
+      T *h = Hw + lane * HS;
       sh_eval<true, T, NL - 1>(a.sh, u0, u1, u2, h, h + NLM, e1, e2, h + 2 * NLM);
     }
     // LDS writes of this wave visible to its other lanes (its harmonics are private to the wave)
@@ -2832,7 +2836,7 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 *
         for (int v = 0; v < 4; v++) {
           int m = mrow[v];
           asm volatile("" : "+v"(m));      // or the compiler keeps (and spills) an address per l and v ahead of the tiles
-          const T *h = hrow0 + (m < 2 * l + 1 ? m : 0) + ht * 16 * 3 * NLM + l * l;
+          const T *h = hrow0 + (m < 2 * l + 1 ? m : 0) + ht * 16 * HS + l * l;
           px += (double) (h[0] * aQ[v]);
           if (l > 0) {
             p1 += (double) (h[NLM] * aP[v]);
