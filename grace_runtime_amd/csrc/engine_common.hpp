@@ -1406,6 +1406,7 @@ class EngineBase : public Engine, protected BufRegistry {
   template<class T, bool PAIRS> void launch_bond_bwd(BondBwdArgs<T> ba, int n)
   {
     for (int q = 0; q < 16; q++) ba.drow[q] = drow_[q];
+    ba.tiles = bond_bwd_tiles<T>(!one_order() && n <= 2 * ncu_);
     const int kb = ba.C / 16;
     const size_t lds = ((size_t) ba.nlm * (ba.C + 2) + (size_t) 4 * 16 * bond_bwd_row(ba.nlm)) * sizeof(T);      // four tiles of bonds
     if (kb != 1 && kb != 2 && kb != 4) throw Error("bond backward: channel width must be 16, 32 or 64");
@@ -1414,7 +1415,7 @@ class EngineBase : public Engine, protected BufRegistry {
   do {                                                                                                 \
     auto kern = ba.tb.F ? k_bond_bwd<T, KB, NL, RowsOf::tables> : k_bond_bwd<T, KB, NL, RowsOf::bonds>; \
     if constexpr (PAIRS) if (ba.erow) kern = k_bond_bwd<T, KB, NL, RowsOf::pairs>;                     \
-    hipLaunchKernelGGL(kern, dim3(n), dim3(64 * bond_bwd_block<T>()), lds, stream_, ba);               \
+    hipLaunchKernelGGL(kern, dim3(n), dim3(256 / ba.tiles), lds, stream_, ba);                          \
   } while (0)
 #define GR_BB_NL(NL) case NL: if (kb == 1) GR_BB(1, NL); else if (kb == 2) GR_BB(2, NL); else GR_BB(4, NL); break
     switch (ba.nl) {
@@ -1426,7 +1427,7 @@ class EngineBase : public Engine, protected BufRegistry {
   }
   // With ordered sums a GRACE-1L result does not depend on the chunk size: kernels whose sums have another order are then not
   // chosen by the number of atoms of a pass (k_gemm_few deals the segments of a job to four waves, chain_bwd_part the groups of
-  // a chain to several blocks).
+  // a chain to several blocks, k_bond_bwd in fp32 the tiles of an atom's bonds to two waves or four).
   bool one_order() const { return ordered_ && layers() == 1; }
   // Which launches with one input width take k_gemm_few / k_gemm_wide: all of 64 x 64 channels, and those whose blocks of
   // k_gemm_jobs (16 atom tiles each) would leave CUs idle.

@@ -2638,6 +2638,7 @@ template<class T> struct BondBwdArgs {
   int ordered_add;            // ordered mode: add to what fedge / fcen hold (a later layer of the same pass) instead of storing
   int a0;
   int C, nl, nlm, noutp;
+  int tiles;                  // tiles of 16 bonds of a round (bond_bwd_tiles)
   int drow[16];               // accumulator row of (lane / 16, register)
   ShCoef sh;
 };
@@ -2654,9 +2655,10 @@ template<class T> constexpr int bond_bwd_waves(int kb, int nl, RowsOf rows) { re
 // Tiles of 16 bonds whose harmonics a wave evaluates at once, a bond per lane, and waves of a block.  One tile at a time leaves 48
 // lanes idle in the harmonics, half of the vector instructions of a tile in fp32.  Two tiles: paired rows, 8192 atoms fp32 198 -> 178 us,
 // tables, 3999 atoms of 78 bonds 156 -> 153; in fp64, where the harmonics of two tiles leave LDS for six waves of a CU, 203 -> 225 us
-// (tables, 4001 atoms), 21 -> 25 (128 atoms).
-template<class T> constexpr int bond_bwd_tiles() { return sizeof(T) == 4 ? 2 : 1; }
-template<class T> constexpr int bond_bwd_block() { return 4 / bond_bwd_tiles<T>(); }
+// (tables, 4001 atoms), 21 -> 25 (128 atoms).  Up to two atoms per CU (few) four waves of one tile each are quicker than two of two,
+// one tile / two, 58 bonds, us: lmax 4, 32 channels, 128 atoms 17.4 / 20.0, 432 21.0 / 22.5, 686 32.3 / 24.5; lmax 6 20.5 / 24.7, 26.2 /
+// 30.5, 39.8 / 33.4; with tables 19.6 / 21.9, 23.4 / 25.4, 27.4 / 28.9.
+template<class T> constexpr int bond_bwd_tiles(bool few) { return sizeof(T) == 4 && !few ? 2 : 1; }
 // Values of a bond in LDS, its harmonics and their two gradient components: odd, so that the 16 bonds of a tile, which are read at
 // once, start in different banks.  As 3 nlm values, which is even from lmax 1 on for every second lmax and 48 at lmax 3: 3456 atoms of 58
 // bonds, lmax 3 fp64, paired rows of 16 channels 97.7 -> 70.0 us, of 32 113.6 -> 92.2, of 64 223.5 -> 204.4.
@@ -2680,16 +2682,16 @@ constexpr int bond_bwd_row(int nlm) { return 3 * nlm | 1; }
 // 198; tables, 3999 atoms fp32 166 -> 156, 4001 atoms fp64 211 -> 204, and the tiles two at a time above.
 // RowsOf::tables: the B operands are formed from the radial tables (lane (g, c): the eight columns l C + 8 g + s of bond c, four table
 // entries each, value and derivative from the same four; requested for l + 1 before the products of l).
-template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 * bond_bwd_block<T>(), bond_bwd_waves<T>(KB, NL, ROWS)) void k_bond_bwd(BondBwdArgs<T> a)
+template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(256, bond_bwd_waves<T>(KB, NL, ROWS)) void k_bond_bwd(BondBwdArgs<T> a)
 {
-  constexpr int HT = bond_bwd_tiles<T>(), NW = bond_bwd_block<T>();
+  const int HT = sizeof(T) == 4 ? a.tiles : 1, NW = 4 / HT;
   constexpr bool TAB = ROWS == RowsOf::tables, PAIRS = ROWS == RowsOf::pairs;
   typedef typename Mfma<T>::v4 v4;
   constexpr int KS = KB * 4, C = KB * 16, CS = C + 2, NLM = NL * NL, HS = bond_bwd_row(NLM);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *gAl = reinterpret_cast<T *>(smem_raw);                          // [NLM][CS]
   T *Hsh = gAl + NLM * CS;                                           // [NW waves][16 HT][HS]: harmonics, gradient . e1, gradient . e2
-  __shared__ double red[NW][9];
+  __shared__ double red[4][9];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int c = lane & 15, g = lane >> 4;
   const int i = a.a0 + blockIdx.x;
@@ -2781,7 +2783,7 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 *
     double px_r = 0, p1_r = 0, p2_r = 0;      // of bond er + lane
     for (int ht = 0; ht < HT; ht++) {
       const long long eb = er + 16 * ht;
-      if (HT > 1 && eb >= e1_) break;
+      if (sizeof(T) == 4 && eb >= e1_) break;
       const bool colok = eb + c < e1_;                // B operand column = bond c of the tile
       double px = 0, p1 = 0, p2 = 0;
 #pragma unroll
@@ -2845,11 +2847,11 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 *
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (HT > 1 && ht + 1 < HT && eb + 16 < e1_) begin(eb + 16);
+      if (sizeof(T) == 4 && ht + 1 < HT && eb + 16 < e1_) begin(eb + 16);
       // sum over the four lane groups (the rows m of a bond are spread over them); lane group ht keeps the sums of tile ht
       px += __shfl_xor(px, 16, 64); p1 += __shfl_xor(p1, 16, 64); p2 += __shfl_xor(p2, 16, 64);
       px += __shfl_xor(px, 32, 64); p1 += __shfl_xor(p1, 32, 64); p2 += __shfl_xor(p2, 32, 64);
-      if (HT == 1 || g == ht) { px_r = px; p1_r = p1; p2_r = p2; }
+      if (sizeof(T) == 8 || g == ht) { px_r = px; p1_r = p1; p2_r = p2; }
     }
     if (TAB) px_r *= (double) a.tb.N;      // the slopes are per interval
     if (lane < nr) {
@@ -2896,7 +2898,6 @@ template<class T, int KB, int NL, RowsOf ROWS> __global__ __launch_bounds__(64 *
   __syncthreads();
   if (t < 9) {
     double s = red[0][t];
-#pragma unroll
     for (int w = 1; w < NW; w++) s += red[w][t];
     if (a.fcen) a.fcen[9 * (long long) i + t] = (a.ordered_add ? a.fcen[9 * (long long) i + t] : 0.0) + s;
     else if (e1_ > e0) {

@@ -45,3 +45,25 @@ def test_bonds_around_the_tile_sizes(model_dir, monkeypatch, n, model, species, 
     rows = kk.System(m, species, skin=0.0, precision=precision, spline=200).compute(types, pos, cell, pbc)
     assert abs(inside["energy"] - rows["energy"]) / n < tol * fs
     assert np.abs(inside["forces"] - rows["forces"]).max() < 10 * tol * fs
+
+
+@pytest.mark.parametrize("tables", [0, 200])
+@pytest.mark.parametrize("model,species,cutoff", [("config1", ["W"], 6.0), ("mix2", ["Mo", "W"], 5.0)])
+@pytest.mark.parametrize("n", SIZES)
+def test_many_atoms_with_bonds_around_the_tile_sizes(model_dir, n, model, species, cutoff, tables):
+    """fp32, where the bond reverse takes one tile at a time up to two atoms per CU and two beyond: a cluster among as many copies as
+    make more atoms than that, against the cluster by itself; forces, which the two forms give in the same terms, and the virial"""
+    m = kk.Model(cases.model_file(model_dir, model))
+    pos = cluster(n, 0.49 * cutoff)
+    types = (np.arange(n) % len(species) + 1).astype(np.int32)
+    copies = 520 // n + 1
+    side = int(np.ceil(copies ** (1.0 / 3.0)))
+    at = np.stack(np.unravel_index(np.arange(copies), (side,) * 3), -1) * 3.0 * cutoff
+    many = (pos[None] + at[:, None]).reshape(-1, 3)
+    pbc = [False, False, False]
+    one = kk.System(m, species, skin=0.0, precision=32, spline=tables).compute(types, pos, 30.0 * np.eye(3), pbc)
+    out = kk.System(m, species, skin=0.0, precision=32, spline=tables).compute(np.tile(types, copies), many, 200.0 * np.eye(3), pbc)
+    fs = max(1.0, np.abs(one["forces"]).max())
+    tol = 2e-6
+    assert np.abs(out["forces"].reshape(copies, n, 3) - one["forces"]).max() < 10 * tol * fs
+    assert np.abs(out["virial"] - copies * one["virial"]).max() < 100 * tol * fs * copies
