@@ -1363,9 +1363,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // requested a tile ahead.  No radial row is read: the rows need not exist.  Three waves per SIMD in fp32, with the harmonics of
 // four tiles at once: 65 536 atoms 778 -> 674 us.  No branch in a tile, constant distances between the entries of a bond: 32 768
 // atoms fp32 355 -> 331 us, 3999 atoms of 78 bonds 73.5 -> 63.4, 4001 atoms fp64 95.6 -> 95.4 (without the scheduling barrier 97);
-// both column blocks of a 32-channel step requested a step ahead in fp32: 32 768 atoms 335 -> 327 us.  fp64, which computes more
-// than it waits, ends a tile behind its last step with a bond (58 bonds an atom: 15 steps for 16): 3456 atoms, 16 channels, lmax 6
-// 83.5 -> 76.1 us, lmax 4 55.3 -> 51.9, 32 channels 92.2 -> 91.7.
+// both column blocks of a 32-channel step requested a step ahead in fp32: 32 768 atoms 335 -> 327 us.  In fp64 with 16
+// channels a tile ends behind its last step with a bond (58 bonds an atom: 15 steps for 16): lmax 6, 3456 atoms 84.3 -> 77.8 us, 128 atoms
+// 32.6 -> 29.1, lmax 4 56.8 -> 52.9 and 19.9 -> 18.9; not with 32, 93.3 -> 92.6 and 26.5 -> 29.4.
 template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_scatter_a_tab(ScatterArgs<T> a)
 {
   typedef typename Mfma<T>::v4 v4;
@@ -1399,7 +1399,7 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) ==
   };
   // one (step, 16-column block) at a time, QB of them requested ahead: QB x NL x 4 entries in flight per lane
   constexpr int QB = sizeof(T) == 4 && KB == 2 ? 2 : 1;
-  constexpr bool SHORT = sizeof(T) == 8;    // a tile ends behind its last step with a bond
+  constexpr bool SHORT = sizeof(T) == 8 && KB == 1;    // a tile ends behind its last step with a bond
   T raw[QB][NL][4], zc[QB];
   double tt[QB];
   auto request = [&](int q) {    // q = s KB + cb
@@ -1433,7 +1433,7 @@ template<class T, int NL, int KB> __global__ __launch_bounds__(256, sizeof(T) ==
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    // fp32: a step without a bond reads the tile's first again and multiplies with harmonics of zero, no branch in the tile
+    // not SHORT: a step without a bond reads the tile's first again and multiplies with harmonics of zero, no branch in the tile
     const int steps = SHORT ? ((int) (w1 - eb < 16 ? w1 - eb : 16) + 3) / 4 * KB : 4 * KB;
 #pragma unroll
     for (int q = 0; q < 4 * KB; q++) {
