@@ -380,6 +380,8 @@ template<int NL, class T> __device__ inline __attribute__((always_inline)) void 
 // 395, 3001 atoms fp64 3.53 -> 3.26 ms, 96 atoms 127 -> 99 us.  What bounds it: instruction issue (in fp64 the 42 multiply-adds of a
 // slot, channel and bond at lmax 5 are 1.1 of the 3.26 ms, the stores of P 0.8): with the rows of all neighbours, or all radial
 // rows, the same it is at most 12 % faster.  Two bonds ahead instead of one: the same; one slot per lane instead of two: 1.6 x the time.
+// Behind the form through LDS in one range only: fp64, a row per bond, 5 slots of 32 channels, lmax 4, whose waves
+// fit the GPU once up to 2048 atoms (2000 atoms 90 -> 82 us, 3456 142 -> 150, 5488 206 -> 214, 8192 297 -> 286).
 template<class T> struct PairFwdArgs {
   const long long *eoff;
   const int *ej, *erow;    // erow: radial row of every bond (k_edge_pairs), or null: row e
@@ -496,7 +498,7 @@ template<class T, int NL, int NQ> inline void launch_pair_fwd_q(PairFwdArgs<T> a
   hipLaunchKernelGGL((k_pair_fwd<T, NL, NQ>), dim3((unsigned) ((a.natoms + 7) / 8 * 8 * a.ngrp)), dim3(64 * a.wpb), 0, stream, a);
 }
 // Slots of a lane at NL and C: the groups of slots even; where every wave would have a SIMD to itself anyway (simds: of the
-// GPU) more waves with fewer slots (107 atoms of GRACE-2L: 32 us with three slots, 28 with two, 25 with one)
+// GPU) more waves with fewer slots (107 atoms of GRACE-2L: 31.4 us with three slots, 28.1 with two, 28.3 with one)
 template<class T, int NL> inline void launch_pair_fwd_l(const PairFwdArgs<T> &a, int simds, hipStream_t stream)
 {
   constexpr int MAXQ = pair_fwd_slots(NL * NL, sizeof(T));
@@ -1030,9 +1032,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   else if (nq == 1) pair_bwd_wave<T, NL, 1, PAIRS>(a, i, s0, n0, Bw);
 }
 
-// Values per row of the harmonics and their two gradient components in memory: at least 3 nlm + 3 (the last MFMA step of
-// the largest l reads up to three values past the row's third part: zeros), a whole number of 16-byte pieces, and 16
-// consecutive rows in different LDS banks (fp64: rows 2 (mod 4) values apart, fp32: 4 (mod 8))
+// Values per row of the harmonics and their two gradient components in memory: more than 3 nlm (the last matrix step of an odd
+// lmax reads one value past the row's third part, which the kernel replaces by zero), a whole number of 16-byte pieces, and an
+// odd number of pairs (fp64) or fours (fp32), which kept 16 rows in different banks while the kernel copied them to LDS
 inline int pair_row_stride(int nlm, size_t value_bytes)
 {
   int v = 3 * nlm + 3;

@@ -1,5 +1,5 @@
 """Atoms with few and uneven numbers of bonds through the GRACE-2L and GRACE-3L engines against the CPU oracle.  The
-neighbour gather and its reverse walk an atom's bonds in chunks of 4 or 8 that are copied to LDS one chunk ahead: a
+neighbour gather walks an atom's bonds two at a time, its reverse in chunks of 16, or of 4 or 8 in the vector kernels: a
 dilute, non-periodic cloud gives atoms with 0, 1, 2 ... bonds, so every length of a last chunk, the single-chunk atoms
 and the atoms without any bond occur in one structure (reference behaviour: atom_yi / bond_yi_bwd of
 libgrace/include/grace/fused_cpu.h:836-1025 loop over whatever bonds an atom has).  Needs an MI355X: run with -m gpu."""
